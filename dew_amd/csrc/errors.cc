@@ -56,6 +56,7 @@ const char* dew_moe_kernels(void) {
          "grouped_gemm<bf16 window>,256,256 | 128,64,3,v_mfma_f32_32x32x16_bf16,gemm_t: each group's window of 64-token steps of bf16 lhs_t rows x the bf16 rhs_t bank; tensor scales on the sums\n"
          "transpose_columns,128 tokens x 64 columns/block,-,-,4,-,bf16 [tokens x dim] transposed (or its NVFP4 values along the tokens): rows or bf16 bank atoms\n"
          "quantize_columns,128 tokens x 64 columns/block,-,-,4,-,bf16 [tokens x dim] -> e4m3 along the tokens and transposed: operand rows or bank atoms + e8m0 scales\n"
+         "quantize_matrices,128 depths x 128 columns/block,-,-,8,-,bf16|f32 weights (either way round) -> a prepared bank of fp8 128x128 blocks | mxfp8 | nvfp4\n"
          "absmax + quantize_rows_nvfp4,1 row/wave,-,-,4,-,bf16 rows -> bf16 (e2m1 code x e4m3 scale) + the tensor scale\n"
          "combine,8 columns/lane,-,-,4,-,bf16 slots x f32 weights\n";
 }

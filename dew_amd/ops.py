@@ -181,6 +181,14 @@ def group_offsets(sizes: torch.Tensor) -> torch.Tensor:
     return offsets
 
 
+def block_offsets(blocks: torch.Tensor, unit: int) -> torch.Tensor:
+    """`[0, cumsum(unit * blocks)]` int32 `[groups + 1]`: the groups' offsets where each holds whole blocks of `unit` rows."""
+    _device(blocks, "group_blocks", torch.int32)
+    offsets = torch.empty(blocks.numel() + 1, dtype=torch.int32, device=blocks.device)
+    _lib.check(_lib.library().dew_moe_block_offsets(_ptr(blocks), blocks.numel(), unit, _ptr(offsets), _stream()), "dew_moe_block_offsets")
+    return offsets
+
+
 # ---- dispatch -----------------------------------------------------------------------------------------
 
 
@@ -335,6 +343,34 @@ def prepare(bank) -> PreparedBank:
         at = out.tensor_scale - buffer.data_ptr()
         tensor = buffer[at:at + 4 * experts].view(torch.float32)
     return PreparedBank(out, (experts, depth, width), (buffer, scales, tensor))
+
+
+RECIPE_FORMATS = {"blockwise_fp8": _lib.W_FP8_BLOCK, "mxfp8": _lib.W_MXFP8, "nvfp4": _lib.W_NVFP4}
+"""The bank a recipe's product multiplies."""
+
+
+def quantize_matrices(w: torch.Tensor, recipe: str) -> PreparedBank:
+    """`w [E, K, N]` (bf16 or fp32; contiguous, or the transpose of contiguous memory, read where it lies) quantized for a
+    recipe's product straight into its prepared bank (`dew_moe_quantize_matrices`): the bytes that quantizing `w` to the
+    recipe's bank of `formats` and preparing that would give."""
+    kmajor = not w.is_contiguous()
+    _device(w.transpose(1, 2) if kmajor else w, "w")
+    if w.dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"w must be torch.bfloat16 or torch.float32, got {w.dtype}")
+    if recipe not in RECIPE_FORMATS:
+        raise KernelError(f"a recipe's matrices are quantized for one of {list(RECIPE_FORMATS)}, not {recipe!r}")
+    fmt = RECIPE_FORMATS[recipe]
+    experts, depth, width = w.shape
+    lib = _lib.library()
+    buffer = torch.empty(max(lib.dew_moe_quantized_matrices_bytes(fmt, experts, depth, width), 16), dtype=torch.uint8, device=w.device)
+    out = _lib.Bank()
+    _lib.check(lib.dew_moe_quantize_matrices(_ptr(w), fmt, int(w.dtype == torch.float32), int(kmajor), experts, depth, width, _ptr(buffer), out,
+                                             _stream()), "dew_moe_quantize_matrices")
+    tensor = None
+    if fmt == _lib.W_NVFP4:
+        at = out.tensor_scale - buffer.data_ptr()
+        tensor = buffer[at:at + 4 * experts].view(torch.float32)
+    return PreparedBank(out, (experts, depth, width), (buffer, None, tensor))
 
 
 # ---- products -----------------------------------------------------------------------------------------

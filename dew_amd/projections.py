@@ -71,10 +71,34 @@ def rows_quantized(x: torch.Tensor) -> QuantizedRows:
     return QuantizedRows(*ops.quantize_rows_fp8(x.contiguous()))
 
 
+def _bank(w, recipe: str, bank_types: tuple, quantized):
+    """The bank a recipe's product multiplies: `w` itself where it is one already, else its matrices quantized: on the device
+    straight into the prepared layout (`ops.quantize_matrices`, one pass over `w` as it lies), where their extents fit it,
+    else by `quantized`, which also refuses the extents that no bank has."""
+    if isinstance(w, bank_types):
+        return w
+    whole = SCALE_DEPTH * (2 if recipe == "nvfp4" else 1)    # (an NVFP4 bank's depth is whole 256s)
+    if w.is_cuda and w.dim() == 3 and w.shape[0] >= 1 and w.shape[1] and w.shape[2] and w.shape[1] % whole == 0 and w.shape[2] % SCALE_DEPTH == 0:
+        if w.dtype not in (torch.bfloat16, torch.float32):
+            w = w.to(torch.float32)
+        if not (w.is_contiguous() or w.transpose(1, 2).is_contiguous()) or w.data_ptr() % 16:
+            w = w.clone(memory_format=torch.contiguous_format)
+        return ops.quantize_matrices(w, recipe)
+    return quantized(w)
+
+
 def _offsets(group_sizes, rows: int, device) -> torch.Tensor:
     if group_sizes is None:
         return torch.tensor([0, rows], dtype=torch.int32, device=device)
     return gemm.GroupSizes.of(group_sizes).offsets
+
+
+def _groups(group_blocks, device) -> gemm.GroupSizes:
+    """The groups from their counts of whole 128-row blocks (a list, or counts on the device): their row offsets, which is all
+    that a product reads of them."""
+    if isinstance(group_blocks, gemm.GroupSizes):
+        return group_blocks
+    return gemm.GroupSizes(None, ops.block_offsets(torch.as_tensor(group_blocks, device=device).to(torch.int32).contiguous(), SCALE_DEPTH))
 
 
 def blockwise_fp8_product(lhs: QuantizedRows, kernel, group_sizes, *, out_dtype=torch.bfloat16, bias=None,
@@ -95,9 +119,8 @@ def blockwise_fp8_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torc
     """Each group's rows of `x [rows, depth]` times its matrix of `w [groups, depth, width]` in the blockwise FP8
     recipe; group `g` holds `group_blocks[g]` whole 128-row blocks, in order (src/dew/nn/kernels/projections.py:
     50-60). `w` is the weights (quantized here, `blocks_quantized`) or a bank already quantized."""
-    bank = w if isinstance(w, (formats.Fp8Blocks, ops.PreparedBank)) else blocks_quantized(w)
-    sizes = (torch.as_tensor(group_blocks, device=x.device).to(torch.int32) * SCALE_DEPTH).contiguous()
-    return blockwise_fp8_product(rows_quantized(x), bank, sizes, out_dtype=out_dtype)
+    bank = _bank(w, "blockwise_fp8", (formats.Fp8Blocks, ops.PreparedBank), blocks_quantized)
+    return blockwise_fp8_product(rows_quantized(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
 
 
 def recipe_projection(rows: torch.Tensor, matrix, group_sizes=None, *, out_dtype=torch.bfloat16, bias=None,
@@ -119,7 +142,7 @@ def recipe_projection(rows: torch.Tensor, matrix, group_sizes=None, *, out_dtype
             stacked = matrix if matrix.dim() == 3 else matrix[None]
             if stacked.shape[1] % SCALE_DEPTH or stacked.shape[2] % SCALE_DEPTH or (recipe == "nvfp4" and stacked.shape[1] % 256):
                 return None  # (an NVFP4 bank's depth is whole 256s)
-            bank = formats.MxFp8.quantized(stacked) if recipe == "mxfp8" else nvfp4_matrices(stacked)
+            bank = _bank(stacked, recipe, (), formats.MxFp8.quantized if recipe == "mxfp8" else nvfp4_matrices)
         if bias is not None:
             bias = bias.reshape(bank.shape[0], bank.shape[2]).to(torch.float32).contiguous()
         if group_sizes is None:
@@ -133,7 +156,7 @@ def recipe_projection(rows: torch.Tensor, matrix, group_sizes=None, *, out_dtype
         stacked = matrix if matrix.dim() == 3 else matrix[None]
         if stacked.shape[1] % SCALE_DEPTH or stacked.shape[2] % SCALE_DEPTH:
             return None
-        bank = blocks_quantized(stacked)
+        bank = _bank(stacked, recipe, (), blocks_quantized)
     if bias is not None:
         bias = bias.reshape(bank.shape[0], bank.shape[2]).to(torch.float32).contiguous()  # widened as it is stored (:141)
     return blockwise_fp8_product(rows_quantized(rows), bank, group_sizes, out_dtype=out_dtype, bias=bias)
@@ -177,9 +200,8 @@ def mxfp8_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torch.bfloat
     """Each group's rows of `x [rows, depth]` times its matrix of `w [groups, depth, width]` in the MXFP8 recipe, both
     quantized along the depth (src/dew/nn/kernels/projections.py:231-258); group `g` holds `group_blocks[g]` whole
     128-row blocks. `w` is the weights (quantized here) or an MXFP8 bank already quantized."""
-    bank = w if isinstance(w, (formats.MxFp8, ops.PreparedBank)) else formats.MxFp8.quantized(w)
-    sizes = (torch.as_tensor(group_blocks, device=x.device).to(torch.int32) * SCALE_DEPTH).contiguous()
-    return mxfp8_product(mxfp8_rows(x), bank, sizes, out_dtype=out_dtype)
+    bank = _bank(w, "mxfp8", (formats.MxFp8, ops.PreparedBank), formats.MxFp8.quantized)
+    return mxfp8_product(mxfp8_rows(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
 
 
 # ---- the NVFP4 recipe ------------------------------------------------------------------------------------
@@ -229,17 +251,11 @@ def nvfp4_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torch.bfloat
     """Each group's rows of `x [rows, depth]` times its matrix of `w [groups, depth, width]` in the NVFP4 recipe, both
     quantized along the depth (src/dew/nn/kernels/projections.py:261-275); group `g` holds `group_blocks[g]` whole
     128-row blocks. `w` is the weights (quantized here, `nvfp4_matrices`) or an NVFP4 bank already quantized."""
-    bank = w if isinstance(w, (formats.NvFp4, ops.PreparedBank)) else nvfp4_matrices(w)
-    sizes = (torch.as_tensor(group_blocks, device=x.device).to(torch.int32) * SCALE_DEPTH).contiguous()
-    return nvfp4_block_product(nvfp4_rows(x), bank, sizes, out_dtype=out_dtype)
+    bank = _bank(w, "nvfp4", (formats.NvFp4, ops.PreparedBank), nvfp4_matrices)
+    return nvfp4_block_product(nvfp4_rows(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
 
 
 # ---- the recipes' gradients ------------------------------------------------------------------------------
-
-
-def _group_offsets(group_blocks, device) -> torch.Tensor:
-    sizes = torch.as_tensor(group_blocks, device=device).to(torch.int64) * SCALE_DEPTH
-    return torch.cat([sizes.new_zeros(1), sizes.cumsum(0)]).to(torch.int32).contiguous()
 
 
 def kernel_gradient(x: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, mx: bool, out_dtype=torch.bfloat16) -> torch.Tensor:
@@ -250,21 +266,24 @@ def kernel_gradient(x: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, m
     `group_blocks[g]` whole 128-token blocks; an empty group's gradient is zero."""
     codes, scales = ops.quantize_columns(x.contiguous(), mx=mx, as_bank=False)
     bank = ops.quantize_columns(cotangent.contiguous(), mx=mx, as_bank=True)
-    return ops.kernel_gradient_mxfp8(codes, scales, bank, _group_offsets(group_blocks, x.device), out_dtype=out_dtype)
+    return ops.kernel_gradient_mxfp8(codes, scales, bank, _groups(group_blocks, x.device).offsets, out_dtype=out_dtype)
 
 
 def blockwise_fp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):
     """`_projection_backward` (src/dew/nn/kernels/projections.py:211-224) -> (d_x, d_w). The input's gradient is the
     recipe's own product of the requantized cotangent and the matrices' blocks transposed (a 128 x 128 block and its
-    scale transpose as they are); the matrices' is `kernel_gradient`."""
-    d_x = blockwise_fp8_projection(cotangent, w.transpose(1, 2).contiguous(), group_blocks, out_dtype=x.dtype)
+    scale transpose as they are; the quantizer reads `w` where it lies, either way round); the matrices' is
+    `kernel_gradient`."""
+    group_blocks = _groups(group_blocks, x.device)    # once for both products
+    d_x = blockwise_fp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
     return d_x, kernel_gradient(x, cotangent, group_blocks, mx=False, out_dtype=out_dtype)
 
 
 def mxfp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):
     """`_mx_backward` (src/dew/nn/kernels/projections.py:263-275) -> (d_x, d_w): the MXFP8 product of the cotangent and
     the matrices, both quantized along the width, and `kernel_gradient` with a scale every 32 tokens."""
-    d_x = mxfp8_projection(cotangent, w.transpose(1, 2).contiguous(), group_blocks, out_dtype=x.dtype)
+    group_blocks = _groups(group_blocks, x.device)    # once for both products
+    d_x = mxfp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
     return d_x, kernel_gradient(x, cotangent, group_blocks, mx=True, out_dtype=out_dtype)
 
 
@@ -273,10 +292,11 @@ def nvfp4_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, g
     and the matrices, both quantized along the width; and each group's tokens contracted over `x` and the cotangent
     quantized along the tokens, every 16 a scale. The decoded operands short of their tensor scales are exact in bf16,
     so the contraction is the bf16 kernel gradient with both tensor scales applied to its fp32 sums."""
-    d_x = nvfp4_projection(cotangent, w.transpose(1, 2).contiguous(), group_blocks, out_dtype=x.dtype)
+    group_blocks = _groups(group_blocks, x.device)    # once for both products
+    d_x = nvfp4_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
     rows, rows_scale = ops.transpose_columns(x.contiguous(), nvfp4=True, as_bank=False)
     bank, bank_scale = ops.transpose_columns(cotangent.contiguous(), nvfp4=True, as_bank=True)
-    d_w = ops.kernel_gradient_bf16(rows, bank, _group_offsets(group_blocks, x.device), lhs_scale=rows_scale, rhs_scale=bank_scale,
+    d_w = ops.kernel_gradient_bf16(rows, bank, _groups(group_blocks, x.device).offsets, lhs_scale=rows_scale, rhs_scale=bank_scale,
                                    out_dtype=out_dtype)
     return d_x, d_w
 

@@ -206,6 +206,8 @@ int dew_moe_capacity_admit(const int32_t* indices, int32_t sequences, int32_t le
 /* offsets[E+1] = exclusive prefix of group sizes[E] (implicit in jax.lax.ragged_dot's group_sizes,
  * src/dew/nn/kernels/xla_products.py:86-115; explicit at src/dew/nn/moe.py:1172).                        */
 int dew_moe_group_offsets(const int32_t* sizes, int32_t experts, int32_t* offsets, void* stream);
+/* The same of sizes counted in whole blocks of `unit` rows (a recipe's `group_blocks`, unit 128).                    */
+int dew_moe_block_offsets(const int32_t* blocks, int32_t groups, int32_t unit, int32_t* offsets, void* stream);
 
 /* ---- One-time weight re-layout -----------------------------------------------------------------------
  * The GEMM kernels read a bank re-laid into MFMA-fragment order (exact: a permutation of the codes; the
@@ -221,6 +223,16 @@ int dew_moe_group_offsets(const int32_t* sizes, int32_t experts, int32_t* offset
 size_t dew_moe_prepared_bytes(int32_t format, int32_t experts, int32_t depth, int32_t width);
 int dew_moe_prepare_bank(const dew_moe_bank* reference, void* prepared, dew_moe_bank* out /* host */,
                          void* stream);
+
+/* A recipe's weight matrices w [E, K, N] (bf16, or fp32 where w_is_f32; with kmajor held [E, N, K], the same memory as the
+ * transposed product's matrices) quantized straight into the prepared bank of the recipe's product: DEW_MOE_W_FP8_BLOCK
+ * (`blocks_quantized` src/dew/nn/kernels/projections.py:185-196), DEW_MOE_W_MXFP8 (`MxFp8.quantized` src/dew/nn/kernels/
+ * formats.py:195-229) or DEW_MOE_W_NVFP4 under one tensor scale (src/dew/nn/kernels/projections.py:243-247), bit for bit what
+ * quantizing and then preparing gives. K and N whole 128s; `prepared` holds dew_moe_quantized_matrices_bytes() bytes, 256-byte
+ * aligned. An NVFP4 bank keeps its format tag whatever its scales, so the call waits for nothing and may be captured.  */
+size_t dew_moe_quantized_matrices_bytes(int32_t format, int32_t experts, int32_t depth, int32_t width);
+int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
+                              int32_t width, void* prepared, dew_moe_bank* out /* host */, void* stream);
 
 /* The descriptor of a bank prepared earlier, from the buffer alone: for a binding that holds the prepared bytes as an
  * opaque array (an XLA buffer) and the bank's format tag and extents as static attributes. `format` is the PREPARED
