@@ -9,11 +9,12 @@ from pathlib import Path
 
 LIBRARY = Path(__file__).resolve().parent / "libdew_moe_hip.so"
 
+EINVAL = 1
 W_FP8_BLOCK, W_FP8_CHANNEL, W_NVFP4, W_MXFP4, W_MXFP8, W_BF16, W_MXFP4_BLOCKS = 1, 2, 3, 4, 5, 6, 7
 LAYOUT_REFERENCE, LAYOUT_PREPARED, LAYOUT_REFERENCE_KMAJOR = 0, 1, 2
 SCORE_SOFTMAX, SCORE_SIGMOID, SCORE_SQRTSOFTPLUS = 0, 1, 2
 SECOND_TERM_E4M3, SECOND_TERM_E2M3, TERMS_E2M3_PAIR = 0, 1, 2
-GATE_SILU, GATE_GELU_TANH = 0, 1
+GATE_SILU, GATE_GELU_TANH, GATE_INTERLEAVED = 0, 1, 2
 GROUP_TOP2, GROUP_MAX = 0, 1
 
 EXPORTS = (
@@ -23,6 +24,7 @@ EXPORTS = (
     "dew_moe_gateup_interleaved", "dew_moe_split_rows", "dew_moe_grouped_gemm_split", "dew_moe_gateup_swiglu_split", "dew_moe_gateup_swiglu_split_out", "dew_moe_split_rows_fp6", "dew_moe_gateup_swiglu_split_fp6_out", "dew_moe_grouped_gemm_split_blocks", "dew_moe_route_sown", "dew_moe_balance_bias", "dew_moe_quantize_rows_nvfp4", "dew_moe_quantize_columns_fp8", "dew_moe_quantize_columns_mxfp8", "dew_moe_kernel_gradient_mxfp8", "dew_moe_transpose_columns", "dew_moe_transpose_groups", "dew_moe_quantize_columns_nvfp4", "dew_moe_kernel_gradient_bf16", "dew_moe_quantize_rows_mxfp8", "dew_moe_grouped_gemm_mxfp8_rows", "dew_moe_quantize_rows_fp8", "dew_moe_grouped_gemm_fp8_rows", "dew_moe_gateup_swiglu", "dew_moe_swiglu", "dew_moe_swiglu_clamped", "dew_moe_gated_product", "dew_moe_scale_rows", "dew_moe_gate_rows", "dew_moe_gate_rows_add_f32", "dew_moe_gateup_gated", "dew_moe_silu", "dew_moe_relu2", "dew_moe_prefers_split_rows", "dew_moe_swiglu_mlp_split_workspace_bytes", "dew_moe_swiglu_mlp_split", "dew_moe_gated_mlp_split", "dew_moe_capacity_admit", "dew_moe_route_with", "dew_moe_route_call", "dew_moe_route_blocks_workspace_bytes", "dew_moe_route_blocks", "dew_moe_combine",
     "dew_moe_rows_f16", "dew_moe_gateup_gated_f16", "dew_moe_split_rows_e2m3_pair", "dew_moe_gateup_swiglu_split_e2m3_pair_out",
     "dew_moe_block_offsets", "dew_moe_quantized_matrices_bytes", "dew_moe_quantize_matrices",
+    "dew_moe_layer_workspace_bytes", "dew_moe_layer_forward",
 )
 """Every symbol include/dew_moe_hip.h declares."""
 
@@ -43,6 +45,12 @@ class Router(ctypes.Structure):
                 ("groups_per_token", ctypes.c_int32), ("group_score", ctypes.c_int32),
                 ("bias_in_weights", ctypes.c_int32), ("weight_sum_epsilon", ctypes.c_float), ("weight_sum_min", ctypes.c_float),
                 ("fill_excluded", ctypes.c_int32), ("excluded_group_score", ctypes.c_float), ("logit_softcap", ctypes.c_float)]
+
+
+class Layer(ctypes.Structure):
+    """`dew_moe_layer` of include/dew_moe_hip.h."""
+
+    _fields_ = [("router", Router), ("gating", ctypes.c_int32), ("limit", ctypes.c_float), ("shared", ctypes.c_int32)]
 
 
 class KernelError(RuntimeError):
@@ -136,6 +144,8 @@ def library() -> ctypes.CDLL:
         "dew_moe_route_blocks_workspace_bytes": (size, [i32, i32, i32]),
         "dew_moe_route_blocks": (i32, [c.POINTER(Router), ptr, ptr, ptr, i32, i32, i32, ptr, size, ptr, ptr, ptr, ptr, ptr]),
         "dew_moe_route_call": (i32, [c.POINTER(Router), ptr, ptr, ptr, ptr, ptr, ptr, i32, ptr, ptr, ptr, ptr, ptr]),
+        "dew_moe_layer_workspace_bytes": (size, [ptr, ptr, ptr, ptr, i32, i32, i32]),
+        "dew_moe_layer_forward": (i32, [ptr] * 10 + [i32, i32, i32, ptr, ptr, size, ptr]),
         "dew_moe_combine": (i32, [ptr, ptr, ptr, ptr, i32, i32, i32, ptr]),
     }
     for name, (restype, argtypes) in prototypes.items():

@@ -12,10 +12,11 @@ weights in fp32 and rounds once, which is at least as accurate as a bf16 sum of 
 """
 
 import dataclasses
+import functools
 
 import torch
 
-from . import gemm, ops
+from . import gemm, layer_call, ops
 from .moe import Gathered, _Module, _at, _implementation, _sorted_locally, expert_matrix, expert_projection, rounded_operand
 
 SWIGLU_LIMIT = 7.0
@@ -91,6 +92,37 @@ class GptOssMLP(_Module):
     @property
     def routes_experts(self) -> bool:
         return True
+
+    @functools.cached_property
+    def _one_call(self):
+        """The layer's fixed part for `layer_call.forward`, or None where its options are not among those the one call covers."""
+        if self.implementation != "auto" or self.dispatch not in ("auto", "global") or self.capacity_factor is not None or self.dtype not in (
+                None, torch.bfloat16):
+            return None
+        router = ops.router_description(self.num_local_experts, self.num_experts_per_tok, "softmax", True, 1.0, 1, 1, "top2", False,
+                                        ops.WEIGHT_SUM_EPSILON, 0.0, None, None)
+        return layer_call.described(router, ops._lib.GATE_INTERLEAVED, SWIGLU_LIMIT, False)
+
+    def apply(self, variables: dict, *args, **kwargs):
+        if len(args) == 1 and not kwargs and self._one_call is not None:
+            out = self._applied(variables, args[0])
+            if out is not None:
+                return out
+        return super().apply(variables, *args, **kwargs)
+
+    def _applied(self, variables: dict, x):
+        """`apply(variables, x)` as one call, or None where the separate calls answer (and raise what is wrong)."""
+        params = variables.get("params")
+        router, held = _at(params, ("router",)), _at(params, ("experts",))
+        try:
+            banks = (expert_matrix(variables, ("experts",), "gate_up_proj"), None, expert_matrix(variables, ("experts",), "down_proj"))
+            biases = (held["gate_up_proj_bias"], held["down_proj_bias"])
+            kernel, bias = router["kernel"], router["bias"]
+        except (KeyError, TypeError):
+            return None
+        if biases[0] is None or biases[1] is None or x.shape[-1] != self.hidden_size:
+            return None
+        return layer_call.forward(self._one_call, x, kernel, bias, None, banks, biases)
 
     @property
     def experts(self) -> GptOssExperts:

@@ -17,11 +17,12 @@ no other compute path here.
 """
 
 import dataclasses
+import functools
 from typing import Callable, NamedTuple
 
 import torch
 
-from . import formats, gemm, ops
+from . import formats, gemm, layer_call, ops
 from .gemm import GroupSizes
 
 GROUPED_MATMULS = ("auto", "hip", "xla", "pallas")
@@ -521,6 +522,46 @@ class SparseMLP(_Module):
     router_softcap: float | None = None
     """The router's switches (`Router`'s fields of the same names; `router_softcap` is its `logit_softcap`,
     src/dew/nn/moe.py:1440-1446)."""
+
+    @functools.cached_property
+    def _one_call(self):
+        """The layer's fixed part for `layer_call.forward`, or None where its options are not among those the one call covers."""
+        plain = (self.activation in ops.GATES and self.implementation == "auto" and self.dispatch in ("auto", "global")
+                 and self.dtype in (None, torch.bfloat16) and self.fused and self.capacity_factor is None and not self.shared_gate
+                 and self.latent_features is None and not self.scale_inputs and self.hash_vocab is None and not self.media_bias
+                 and self.routing_block is None and self.block_experts is None and self.score_function in ops.SCORES
+                 and self.group_score in ops.GROUP_SCORES and (self.swiglu_limit is None or self.swiglu_limit > 0)
+                 and (self.expert_bias or not self.bias_in_weights) and (self.router_softcap is None or self.router_softcap > 0))
+        # (a shared expert runs inside the routed launches where its gating and width are the routed experts': `__call__`)
+        joins = self.fuse_shared and self.shared == self.hidden_features and self.swiglu_limit is None and self.activation == "swiglu"
+        if not plain or (self.shared is not None and not joins):
+            return None
+        router = ops.router_description(self.num_experts, self.top_k, self.score_function, self.normalize_weights, self.routed_scaling_factor,
+                                        self.expert_groups, self.groups_per_token, self.group_score, self.bias_in_weights,
+                                        self.weight_sum_epsilon, self.weight_sum_min, self.excluded_group_score, self.router_softcap)
+        return layer_call.described(router, ops.GATES[self.activation], self.swiglu_limit or 0.0, self.shared is not None)
+
+    def apply(self, variables: dict, *args, **kwargs):
+        if len(args) == 1 and not kwargs and self._one_call is not None:
+            out = self._applied(variables, args[0])
+            if out is not None:
+                return out
+        return super().apply(variables, *args, **kwargs)
+
+    def _applied(self, variables: dict, x):
+        """`apply(variables, x)` as one call, or None where the separate calls answer (and raise what is wrong)."""
+        bias = None
+        if self.expert_bias and (bias := _at(variables.get("moe"), ("gate", "e_score_correction_bias"))) is None:
+            return None
+        try:
+            banks = tuple(expert_matrix(variables, ("experts", name)) for name in EXPERT_AXES)
+            if self.shared is not None:
+                banks = with_shared_expert(banks, tuple(expert_matrix(variables, ("shared_experts", name)) for name in EXPERT_AXES))
+        except KeyError:
+            return None
+        if banks is None or banks[2].shape[2] != self.out_features:
+            return None
+        return layer_call.forward(self._one_call, x, _at(variables.get("params"), ("gate", "kernel")), None, bias, banks)
 
     @property
     def gate(self) -> Router:

@@ -12,7 +12,7 @@ from ._lib import KernelError
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())   # (`current_stream()` builds a stream object first)
 
 
 def _device(tensor: torch.Tensor, name: str, dtype=None) -> torch.Tensor:
@@ -40,6 +40,17 @@ def device_check() -> None:
 WEIGHT_SUM_EPSILON = 1e-20
 """What a renormalization adds to the chosen weights' sum (`WEIGHT_SUM_EPSILON`, src/dew/nn/moe.py:181)."""
 
+SCORES = {"softmax": _lib.SCORE_SOFTMAX, "sigmoid": _lib.SCORE_SIGMOID, "sqrtsoftplus": _lib.SCORE_SQRTSOFTPLUS}
+GROUP_SCORES = {"top2": _lib.GROUP_TOP2, "max": _lib.GROUP_MAX}
+
+
+def router_description(experts, top_k, score_function, normalize_weights, routed_scaling_factor, expert_groups, groups_per_token, group_score,
+                       bias_in_weights, weight_sum_epsilon, weight_sum_min, excluded_group_score, logit_softcap) -> _lib.Router:
+    """A router's switches (`route`'s of the same names) as the C ABI takes them."""
+    return _lib.Router(experts, top_k, SCORES[score_function], int(bool(normalize_weights)), float(routed_scaling_factor), expert_groups,
+                       groups_per_token, GROUP_SCORES[group_score], int(bool(bias_in_weights)), float(weight_sum_epsilon), float(weight_sum_min),
+                       int(excluded_group_score is not None), float(excluded_group_score or 0.0), float(logit_softcap or 0.0))
+
 
 def route(logits: torch.Tensor, top_k: int, *, score_function: str = "softmax", normalize_weights: bool = True,
           bias: torch.Tensor | None = None, routed_scaling_factor: float = 1.0, expert_groups: int = 1,
@@ -53,12 +64,10 @@ def route(logits: torch.Tensor, top_k: int, *, score_function: str = "softmax", 
     experts to use in place of the router's own choice (a replayed record, a hash table's rows), for the tokens `covered`
     (bool `[...]`) marks, all of them where it is None; the weights are the router's for those experts. `media` (bool
     `[...]`) marks the tokens whose experts are chosen by `media_bias [E]` in place of `bias`."""
-    scores = {"softmax": _lib.SCORE_SOFTMAX, "sigmoid": _lib.SCORE_SIGMOID, "sqrtsoftplus": _lib.SCORE_SQRTSOFTPLUS}
-    group_scores = {"top2": _lib.GROUP_TOP2, "max": _lib.GROUP_MAX}
-    if score_function not in scores:
-        raise KernelError(f"score_function must be one of {list(scores)}, got {score_function!r}")
-    if group_score not in group_scores:
-        raise KernelError(f"group_score must be one of {list(group_scores)}, got {group_score!r}")
+    if score_function not in SCORES:
+        raise KernelError(f"score_function must be one of {list(SCORES)}, got {score_function!r}")
+    if group_score not in GROUP_SCORES:
+        raise KernelError(f"group_score must be one of {list(GROUP_SCORES)}, got {group_score!r}")
     _device(logits, "logits", torch.float32)
     if bias is not None:
         _device(bias, "bias", torch.float32)
@@ -87,10 +96,8 @@ def route(logits: torch.Tensor, top_k: int, *, score_function: str = "softmax", 
     indices = torch.empty((*logits.shape[:-1], top_k), dtype=torch.int32, device=logits.device)
     activated = torch.empty_like(logits) if sown else None
     log_z = torch.empty(logits.shape[:-1], dtype=torch.float32, device=logits.device) if sown else None
-    router = _lib.Router(experts, top_k, scores[score_function], int(bool(normalize_weights)), float(routed_scaling_factor),
-                         expert_groups, groups_per_token, group_scores[group_score], int(bool(bias_in_weights)),
-                         float(weight_sum_epsilon), float(weight_sum_min), int(excluded_group_score is not None),
-                         float(excluded_group_score or 0.0), float(logit_softcap or 0.0))
+    router = router_description(experts, top_k, score_function, normalize_weights, routed_scaling_factor, expert_groups, groups_per_token,
+                                group_score, bias_in_weights, weight_sum_epsilon, weight_sum_min, excluded_group_score, logit_softcap)
     _lib.check(_lib.library().dew_moe_route_call(router, _ptr(logits), _ptr(bias), _ptr(media_bias), _ptr(media), _ptr(given), _ptr(covered),
                                                  tokens, _ptr(weights), _ptr(indices), _ptr(activated), _ptr(log_z), _stream()), "dew_moe_route")
     return (weights, indices, activated, log_z) if sown else (weights, indices)
@@ -103,9 +110,8 @@ def route_blocks(logits: torch.Tensor, top_k: int, blocks: torch.Tensor, block_e
     """`route` under LLaDA2.2's block routing: `logits [rows, length, E]`, `blocks [rows, length]` int32 numbering each
     token's block within its row from 0 (negative: padding); a token chooses among the `block_experts` experts its block
     scores best, a block's score for an expert being its best token's selection (the reference's `Router.block_mask`)."""
-    scores = {"softmax": _lib.SCORE_SOFTMAX, "sigmoid": _lib.SCORE_SIGMOID, "sqrtsoftplus": _lib.SCORE_SQRTSOFTPLUS}
-    if score_function not in scores:
-        raise KernelError(f"score_function must be one of {list(scores)}, got {score_function!r}")
+    if score_function not in SCORES:
+        raise KernelError(f"score_function must be one of {list(SCORES)}, got {score_function!r}")
     _device(logits, "logits", torch.float32), _device(blocks, "blocks", torch.int32)
     if logits.dim() != 3 or blocks.shape != logits.shape[:2]:
         raise KernelError(f"block routing takes logits [rows, length, E] and blocks [rows, length], got {tuple(logits.shape)} and {tuple(blocks.shape)}")
@@ -118,9 +124,8 @@ def route_blocks(logits: torch.Tensor, top_k: int, blocks: torch.Tensor, block_e
     indices = torch.empty((rows, length, top_k), dtype=torch.int32, device=logits.device)
     activated = torch.empty_like(logits) if sown else None
     log_z = torch.empty((rows, length), dtype=torch.float32, device=logits.device) if sown else None
-    router = _lib.Router(experts, top_k, scores[score_function], int(bool(normalize_weights)), float(routed_scaling_factor), 1, 1,
-                         _lib.GROUP_TOP2, int(bool(bias_in_weights)), float(weight_sum_epsilon), float(weight_sum_min), 0, 0.0,
-                         float(logit_softcap or 0.0))
+    router = router_description(experts, top_k, score_function, normalize_weights, routed_scaling_factor, 1, 1, "top2", bias_in_weights,
+                                weight_sum_epsilon, weight_sum_min, None, logit_softcap)
     library = _lib.library()
     workspace = torch.empty(max(library.dew_moe_route_blocks_workspace_bytes(rows, length, experts), 4) // 4 + 1, dtype=torch.int32, device=logits.device)
     _lib.check(library.dew_moe_route_blocks(router, _ptr(logits), _ptr(bias), _ptr(blocks), rows, length, block_experts, _ptr(workspace),

@@ -546,6 +546,27 @@ int dew_moe_combine(const void* slots /* bf16 [T,k,D] */, const float* weights /
                     const void* addend /* nullable */, void* out /* bf16 [T,D] */, int32_t tokens,
                     int32_t top_k, int32_t width, void* stream);
 
+/* ---- A sparse layer's forward pass as one call -------------------------------------------------------
+ * SparseMLP.__call__ (src/dew/nn/moe.py:1488-1503) and GptOssMLP.__call__ (src/dew/nn/gpt_oss.py:129-171) from the tokens to
+ * the layer's output: gate logits, routing, sort, expert products, combine. `gate`, `up`, `down` are prepared banks; an
+ * interleaved layer's `gate` is its gate_up bank and `up` NULL. `up_bias` [E, 2F] and `down_bias` [E, D] are an interleaved
+ * layer's (nullable). split_terms: DEW_MOE_SECOND_TERM_* where the products may run on split rows, -1 never; f16_rows_from:
+ * the average rows a group from which a general NVFP4 pair runs on f16 rows, -1 never.                                      */
+enum { DEW_MOE_GATE_INTERLEAVED = 2 };
+typedef struct dew_moe_layer {
+  dew_moe_router router;
+  int32_t gating;  /* DEW_MOE_GATE_*                                                                       */
+  float limit;     /* the clamp before the gate; 0 for none (interleaved: above 0)                         */
+  int32_t shared;  /* 1: the banks' last expert, behind the router's, is one that every token takes        */
+} dew_moe_layer;
+size_t dew_moe_layer_workspace_bytes(const dew_moe_layer* layer, const dew_moe_bank* gate, const dew_moe_bank* up /* nullable */,
+                                     const dew_moe_bank* down, int32_t tokens, int32_t split_terms, int32_t f16_rows_from);
+int dew_moe_layer_forward(const dew_moe_layer* layer, const void* x /* bf16 [T,D] */, const float* gate_kernel /* [D,E] */,
+                          const float* gate_bias /* nullable [E], on the logits */, const float* selection_bias /* nullable [E] */,
+                          const dew_moe_bank* gate, const dew_moe_bank* up, const dew_moe_bank* down, const float* up_bias,
+                          const float* down_bias, int32_t tokens, int32_t split_terms, int32_t f16_rows_from, void* out /* bf16 [T,D] */,
+                          void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif
