@@ -1,0 +1,142 @@
+// The stable counting sort of routed slots by expert as one block runs it, shared by the sort's own launch and by the
+// router's launch of a decode step.
+#pragma once
+
+#include "common.h"
+
+namespace dew {
+
+struct PermuteParams {
+  const int32_t* ids;  // [slots]
+  int32_t* sizes;      // [experts]
+  int32_t* offsets;    // [experts + 1]
+  int32_t* order;      // [slots]
+  int32_t* rows;       // [slots]
+  int32_t* counts;     // workspace [blocks][buckets]
+  int32_t* bases;      // workspace [blocks][buckets]
+  // `slots` sorted positions: the `routed` = tokens * top_k slots of `ids`, then `slots - routed` rows that every token
+  // sends to one always-on (shared) expert, which sorts as group `experts`. `groups` = the groups written (experts, or
+  // experts + 1 with a shared one); bucket `groups` collects the dropped slots (an id outside [0, experts)), last.
+  int slots, routed, experts, groups, top_k, blocks, buckets;
+};
+
+__device__ __forceinline__ int bucket_of_id(const PermuteParams& p, int id) { return (id < 0 || id >= p.experts) ? p.groups : id; }
+
+__device__ __forceinline__ int bucket_of(const PermuteParams& p, int slot) {
+  return slot >= p.routed ? p.experts /* a shared expert's row */ : bucket_of_id(p, p.ids[slot]);
+}
+
+// The row of the activations a slot reads: its token, or for a shared expert's row the token it is.
+__device__ __forceinline__ int row_of(const PermuteParams& p, int slot) {
+  return slot < p.routed ? slot / p.top_k : slot - p.routed;
+}
+
+// The whole sort in one block for at most kSmallSlots slots (a decode step, a small prefill): the block
+// counts, scans and scatters, each wavefront a contiguous run of the slots, with the LDS histogram as the only
+// intermediate.
+// Measured under graph replay, sixteen wavefronts: 2048 slots 5.1 to 6.8 us (four wavefronts: 7.9 to 10.0), 4096 slots
+// 7.5 us against 11.4 us for the three launches, 8192 slots the same either way.
+constexpr int kSmallSlots = 4096;      // beyond this three launches over many blocks are as fast or faster
+constexpr int kSmallThreads = 1024;    // sixteen wavefronts, where their counters fit the LDS a launch may take unasked
+constexpr int kNarrowSmallSlots = 2048;  // the four-wavefront form's reach, for more buckets than that
+// `running`: LDS, [THREADS / 64][buckets] then [buckets + 1] totals. `id_of(slot)`: a routed slot's expert.
+template <int THREADS, class IdOf>
+__device__ __forceinline__ void sort_small(const PermuteParams& p, int32_t* running, IdOf id_of) {
+  constexpr int kWaves = THREADS / 64;
+  int32_t* totals = running + kWaves * p.buckets;
+  const int lane = threadIdx.x % 64;
+  const int wave = threadIdx.x / 64;
+  for (int i = threadIdx.x; i < kWaves * p.buckets; i += THREADS) running[i] = 0;
+  __syncthreads();
+  int32_t* mine = running + wave * p.buckets;
+  const int segment = ((p.slots + THREADS - 1) / THREADS) * 64;  // contiguous slots per wavefront
+  const int rounds = segment / 64;
+  const int wave_begin = wave * segment;
+  // a lane's buckets stay in registers between the count and the scatter (one round trip to the indices, not two)
+  constexpr int kMaxRounds = (THREADS == kSmallThreads ? kSmallSlots : kNarrowSmallSlots) / THREADS;
+  int kept[kMaxRounds];
+#pragma unroll
+  for (int round = 0; round < kMaxRounds; ++round) {
+    const int slot = wave_begin + round * 64 + lane;
+    kept[round] = (round < rounds && slot < p.slots) ? (slot < p.routed ? bucket_of_id(p, id_of(slot)) : p.experts) : p.buckets;
+  }
+#pragma unroll
+  for (int round = 0; round < kMaxRounds; ++round)
+    if (kept[round] < p.buckets) atomicAdd(&mine[kept[round]], 1);
+  __syncthreads();
+  for (int b = threadIdx.x; b < p.buckets; b += THREADS) {
+    int sum = 0;
+    for (int w = 0; w < kWaves; ++w) sum += running[w * p.buckets + b];
+    totals[b] = sum;
+  }
+  __syncthreads();
+  if (threadIdx.x < 64) {  // exclusive scan of the bucket totals by one wavefront, 64 buckets a round
+    int carried = 0;
+    for (int base = 0; base < p.buckets; base += 64) {
+      const int b = base + lane;
+      const int size = b < p.buckets ? totals[b] : 0;
+      int inclusive = size;
+#pragma unroll
+      for (int offset = 1; offset < 64; offset <<= 1) {
+        const int other = __shfl_up(inclusive, offset, 64);
+        if (lane >= offset) inclusive += other;
+      }
+      if (b < p.buckets) totals[b] = carried + inclusive - size;
+      carried += __shfl(inclusive, 63, 64);
+    }
+    if (lane == 0) totals[p.buckets] = carried;
+  }
+  __syncthreads();
+  for (int b = threadIdx.x; b < p.buckets; b += THREADS) {
+    const int start = totals[b];
+    if (b < p.groups) {
+      p.sizes[b] = totals[b + 1] - start;
+      p.offsets[b] = start;
+    } else {
+      p.offsets[p.groups] = start;
+    }
+    int next = start;
+    for (int w = 0; w < kWaves; ++w) {
+      const int count = running[w * p.buckets + b];
+      running[w * p.buckets + b] = next;
+      next += count;
+    }
+  }
+  __syncthreads();
+  int bits = 1;
+  while ((1 << bits) < p.buckets) ++bits;
+#pragma unroll
+  for (int round = 0; round < kMaxRounds; ++round) {
+    if (round >= rounds) continue;  // (the same for the whole block)
+    const int slot = wave_begin + round * 64 + lane;
+    const int bucket = kept[round];
+    const bool valid = bucket < p.buckets;
+    unsigned long long same = __ballot(valid);
+    for (int bit = 0; bit < bits; ++bit) {
+      const bool set = (bucket >> bit) & 1;
+      const unsigned long long vote = __ballot(set);
+      same &= set ? vote : ~vote;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull));
+    const int count = __popcll(same);
+    int position = 0;
+    if (valid) position = mine[bucket] + rank;
+    // The running positions are the wavefront's own (no other wavefront touches them), so no block barrier is needed,
+    // only an order between this wavefront's lanes: every lane's read above before the one lane's write below, and that
+    // write before the next round's reads. The wavefront-scope fences state that order to the compiler and the memory
+    // model (they cost no instruction: a wavefront's LDS operations are issued and served in order).
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (valid && rank == count - 1) mine[bucket] = position + 1;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (valid) {
+      p.order[position] = slot;
+      p.rows[position] = row_of(p, slot);
+    }
+  }
+}
+
+}  // namespace dew
