@@ -1124,3 +1124,41 @@ def test_the_gateup_launch_on_two_e2m3_terms_multiplies_the_values_the_rows_hold
     whole = ops.swiglu_mlp_split(x.cuda(), pg, pu, pd, od, gather=gd, terms="e2m3x2")
     apart = ops.grouped_gemm_split_blocks(*ops.gateup_swiglu_split_out(*pieces, pg, pu, od, gather=gd, terms="e2m3x2"), pd, od)
     assert torch.equal(whole, apart)
+
+
+@pytest.mark.parametrize("quant", ("fp8_block", "fp8_channel", "mxfp4", "nvfp4", "bf16"))
+@pytest.mark.parametrize("sizes", ([1], [0, 33, 0, 32, 1, 7], [3] * 70))
+def test_few_tiles_launch_returns_the_tiled_launchs_bits(quant, sizes):
+    """The decode launch (a wavefront a strip of 32 columns) against the 32-row tiles it stands in for: ragged and empty groups,
+    a group of more than one tile, more experts than a wavefront's lanes, rows that no expert owns."""
+    from dew_amd import codecs, formats, ops
+
+    generator = torch.Generator("cuda").manual_seed(3)
+    normal = lambda *shape: torch.randn(shape, generator=generator, device="cuda")
+    experts, depth, width, rows = len(sizes), 768, 256, sum(sizes) + 5
+
+    def bank(depth, width):
+        w = normal(experts, depth, width) * 0.05
+        if quant == "mxfp4":
+            return ops.prepare(formats.Mxfp4Blocks(*codecs.quantize_mxfp4(w)))
+        if quant == "bf16":
+            return ops.prepare(formats.Bf16(w.to(torch.bfloat16)))
+        return ops.prepare({"fp8_block": formats.Fp8Blocks, "fp8_channel": formats.Fp8Channels, "nvfp4": formats.NvFp4}[quant].quantized(w))
+
+    gate, up = bank(depth, width), bank(depth, width)
+    x = normal(40, depth).to(torch.bfloat16)
+    gather = torch.randint(0, 40, (rows,), generator=generator, device="cuda", dtype=torch.int32)
+    scatter = torch.randperm(rows, generator=generator, device="cuda").to(torch.int32)
+    sizes = torch.tensor(sizes, dtype=torch.int32, device="cuda")
+    offsets = ops.group_offsets(sizes)
+    bias = normal(experts, width)
+    calls = {"paired": lambda: ops.gateup_swiglu(x, gate, up, offsets, gather=gather),
+             "paired, clamped": lambda: ops.gateup_swiglu(x, gate, up, None, sizes=sizes, gather=gather, activation="geglu", limit=1.0),
+             "plain": lambda: ops.grouped_gemm(x, gate, offsets, gather=gather, scatter=scatter),
+             "biased": lambda: ops.grouped_gemm(x, gate, None, sizes=sizes, gather=gather, scatter=scatter, bias=bias, round_bias=True),
+             "interleaved": lambda: ops.gateup_interleaved(x, gate, offsets, bias=bias, gather=gather)}
+    for name, call in calls.items():
+        got = call()
+        with ops.tile_rows(32):
+            want = call()
+        assert torch.equal(got, want) and bool(got.any()), name
