@@ -1175,7 +1175,7 @@ static int tile_rows(const GemmParams& p, bool cheap) {
 // tokens: 73 -> 69 us). It reads a tile's rows again for every 32 columns: tiles of more than some 12 rows take it only
 // where they are under a hundred blocks (8 experts of 1024 x 512, bf16, 384 rows: 17.2 -> 8.7 us; at 160 blocks no faster).
 static bool few_tiles(const GemmParams& p, bool unquantized) {
-  const long long touched = p.rows < p.experts ? p.rows : p.experts, spread = p.rows / 32 + p.experts / 2;
+  const long long touched = p.rows < p.experts ? p.rows : p.experts, spread = p.rows / 32 + touched / 2;
   const long long blocks = (touched > spread ? touched : spread) * ((p.width + 127) / 128);
   return blocks <= 96 || (blocks <= (unquantized ? 512 : 256) && p.rows <= 12 * touched);
 }

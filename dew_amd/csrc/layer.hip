@@ -4,6 +4,7 @@
 // Measured on one token of 128 experts of 2048 x 768 (FP8 blocks), where the launches' own time is 51 us: 123 us a pass
 // through the separate entry points, each with its own checks, allocations and foreign call.
 #include "common.h"
+#include "sort.h"
 
 namespace dew {
 
@@ -37,7 +38,7 @@ static LayerWorkspace layer_workspace(const dew_moe_layer* layer, const dew_moe_
     at += (static_cast<size_t>(bytes) + 255) / 256 * 256;
     return here;
   };
-  w.logits = take(tokens * layer->router.experts * 4);
+  w.logits = take(tokens * layer->router.experts * 4 * (tokens <= kShareTokens ? kLogitShares : 1));
   w.weights = take(slots * 4);
   w.indices = take(slots * 4);
   w.sizes = take(groups * 4);
@@ -114,12 +115,24 @@ extern "C" int dew_moe_layer_forward(const dew_moe_layer* layer, const void* x, 
   float* logits = reinterpret_cast<float*>(base + w.logits);
   float* weights = reinterpret_cast<float*>(base + w.weights);
   int32_t *indices = words(w.indices), *sizes = words(w.sizes), *offsets = words(w.offsets), *order = words(w.order), *gather = words(w.rows);
-  if (int rc = dew_moe_router_logits(x, gate_kernel, gate_bias, logits, tokens, gate->depth, experts, stream)) return rc;
-  if (int rc = dew_moe_route_with(&layer->router, logits, selection_bias, tokens, weights, indices, nullptr, nullptr, stream)) return rc;
-  if (int rc = layer->shared ? dew_moe_permute_shared(indices, tokens, top_k, experts, tokens, sizes, offsets, order, gather, base + w.sort,
-                                                      w.sort_bytes, stream)
-                             : dew_moe_permute(indices, tokens, top_k, experts, sizes, offsets, order, gather, base + w.sort, w.sort_bytes, stream))
+  // a decode step's gate leaves its logits in shares, which spread over more CUs and which its router adds up
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool in_shares = tokens <= kShareTokens && gate->depth % 16 == 0 && aligned16(x);
+  if (int rc = in_shares ? router_logit_shares(x, gate_kernel, logits, tokens, gate->depth, experts, s)
+                         : dew_moe_router_logits(x, gate_kernel, gate_bias, logits, tokens, gate->depth, experts, stream))
     return rc;
+  if (in_shares && tokens <= kRouteAndSortTokens && rows <= kSmallSlots) {
+    if (int rc = route_and_sort(&layer->router, logits, gate_bias, selection_bias, tokens, layer->shared != 0, weights, sizes, offsets, order, gather, s))
+      return rc;
+  } else {
+    if (int rc = in_shares ? route_shares(&layer->router, logits, gate_bias, selection_bias, tokens, weights, indices, s)
+                           : dew_moe_route_with(&layer->router, logits, selection_bias, tokens, weights, indices, nullptr, nullptr, stream))
+      return rc;
+    if (int rc = layer->shared ? dew_moe_permute_shared(indices, tokens, top_k, experts, tokens, sizes, offsets, order, gather, base + w.sort,
+                                                        w.sort_bytes, stream)
+                               : dew_moe_permute(indices, tokens, top_k, experts, sizes, offsets, order, gather, base + w.sort, w.sort_bytes, stream))
+      return rc;
+  }
   uint8_t* slots = base + w.slots;
   if (form == kRowsSplit) {
     if (int rc = dew_moe_gated_mlp_split(x, tokens, gather, offsets, nullptr, gate, up, down, layer->gating, layer->limit, order, slots, rows,

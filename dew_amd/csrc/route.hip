@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "sort.h"
 
 #pragma clang fp contract(off)
 
@@ -105,6 +106,8 @@ struct RouteParams {
   uint32_t* block_keys;    // [rows x (length + 1), E]: a block's best selection for every expert, as ordered keys (0: none yet)
   const uint8_t* allowed;  // [rows x (length + 1), 64]: bit i of byte `lane` set where expert lane + 64 i is on the block's shortlist
   int gather_blocks;       // this launch only gathers the blocks' best selections into block_keys
+  int shares;              // `logits` are kLogitShares partial sums of them, [share][T][E] (logits.hip), to which `gate_bias` is still due
+  const float* gate_bias;  // nullable [E]
 };
 
 // A float as an unsigned key of the same order (-inf lowest of the non-NaN), never 0.
@@ -127,23 +130,43 @@ __device__ __forceinline__ size_t block_of(const RouteParams& p, int token) {
 // Laguna's capped gate logit (`capped_logits`, src/dew/nn/precision.py:2086-2092): cap * tanh(logit / cap) in fp32.
 __device__ __forceinline__ float capped(float logit, float cap) { return cap > 0.0f ? cap * tanhf(logit / cap) : logit; }
 
-template <int kPerLane>  // experts <= 64 * kPerLane
-__global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p) {
-  extern __shared__ float shared[];  // [kRouteWaves][experts] selections, for the group scores
+// A token's logits, expert lane + 64 i in logit[i]: as they are, or added up from the gate's shares of the depth in the order the
+// gate's own launch adds them.
+template <int kPerLane>
+__device__ __forceinline__ void read_logits(const RouteParams& p, int token, float (&logit)[kPerLane]) {
   const int lane = threadIdx.x % kWave;
-  const int wave = threadIdx.x / kWave;
-  const int token_raw = blockIdx.x * kRouteWaves + wave;
-  const bool active = token_raw < p.tokens;
-  const int token = active ? token_raw : p.tokens - 1;
   const float* row = p.logits + static_cast<size_t>(token) * p.experts;
-  const float ninf = -__builtin_inff();
-
-  float logit[kPerLane], score[kPerLane], select[kPerLane];
 #pragma unroll
   for (int i = 0; i < kPerLane; ++i) {
-    const int e = lane + kWave * i;
-    logit[i] = e < p.experts ? row[e] : ninf;
+    const int e = lane + kWave * i, at = min(e, p.experts - 1);
+    float value;
+    if (p.shares) {
+      float share[kLogitShares];
+#pragma unroll
+      for (int s = 0; s < kLogitShares; ++s) share[s] = row[static_cast<size_t>(s) * p.tokens * p.experts + at];
+      __builtin_amdgcn_sched_barrier(0);  // (all of them asked for before the first is waited for)
+      value = share[0];
+#pragma unroll
+      for (int s = 1; s < kLogitShares; ++s) value += share[s];
+      if (p.gate_bias != nullptr) value = value + p.gate_bias[at];
+    } else {
+      value = row[at];
+    }
+    logit[i] = e < p.experts ? value : -__builtin_inff();
   }
+}
+
+// One token of a wavefront, from its logits (expert lane + 64 i in logit[i], -inf past the experts) to its experts and weights:
+// lane j < top_k returns the j-th. `mine`: the wavefront's own LDS, p.experts floats, where there are expert groups.
+struct Chosen {
+  float weight;
+  int expert;
+};
+template <int kPerLane>  // experts <= 64 * kPerLane
+__device__ __forceinline__ Chosen routed_token(const RouteParams& p, int token, bool active, float (&logit)[kPerLane], float* mine) {
+  const int lane = threadIdx.x % kWave;
+  const float ninf = -__builtin_inff();
+  float score[kPerLane], select[kPerLane];
   if (p.softcap > 0.0f) {  // (a branch of its own: the cap's hyperbolic tangent stays out of the routers that have none)
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i)
@@ -219,7 +242,7 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
           if (e < p.experts) atomicMax(p.block_keys + block * p.experts + e, ordered_key(select[i]));
         }
       }
-      return;
+      return Chosen{0.0f, 0};
     }
     const unsigned shortlist = p.allowed[block * kWave + lane];
 #pragma unroll
@@ -228,13 +251,15 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
   }
 
   if (p.expert_groups > 1) {
-    float* mine = shared + wave * p.experts;
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) {
       const int e = lane + kWave * i;
       if (e < p.experts) mine[e] = select[i];
     }
-    __syncthreads();
+    // (the selections are the wavefront's own: an order between its lanes is all the reads below need)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     const int per_group = p.experts / p.expert_groups;
     // lane g scores group g: the sum of its two best selections
     float group_score = ninf;
@@ -305,8 +330,12 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
 
   // gate weights: lane j < k owns the j-th choice
   const bool owner = lane < p.top_k && in_range;
-  float chosen_logit = owner ? row[my_choice] : ninf;
-  if (p.softcap > 0.0f && owner) chosen_logit = capped(chosen_logit, p.softcap);
+  float chosen_logit = ninf;  // (read from the lane that holds it: no round trip to the logits)
+#pragma unroll
+  for (int i = 0; i < kPerLane; ++i) {
+    const float held = __shfl(logit[i], my_choice % kWave, kWave);
+    if (owner && my_choice / kWave == i) chosen_logit = held;
+  }
   float weight = 0.0f;
   if (p.score_function == DEW_MOE_SCORE_SOFTMAX && p.normalize && !p.bias_in_weights && !(p.sum_min != 0.0f)) {
     const float m = wave_max(chosen_logit);
@@ -328,10 +357,48 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
     }
   }
   weight = weight * p.scaling;
+  return Chosen{in_range ? weight : 0.0f, replayed ? given_id : my_choice};
+}
+
+template <int kPerLane>
+__global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p) {
+  extern __shared__ float shared[];  // [kRouteWaves][experts] selections, for the group scores
+  const int lane = threadIdx.x % kWave;
+  const int wave = threadIdx.x / kWave;
+  const int token_raw = blockIdx.x * kRouteWaves + wave;
+  const bool active = token_raw < p.tokens;
+  const int token = active ? token_raw : p.tokens - 1;
+  float logit[kPerLane];
+  read_logits<kPerLane>(p, token, logit);
+  const Chosen chosen = routed_token<kPerLane>(p, token, active, logit, shared + wave * p.experts);
+  if (p.gather_blocks) return;
   if (active && lane < p.top_k) {
-    p.weights[static_cast<size_t>(token) * p.top_k + lane] = in_range ? weight : 0.0f;
-    p.indices[static_cast<size_t>(token) * p.top_k + lane] = replayed ? given_id : my_choice;
+    p.weights[static_cast<size_t>(token) * p.top_k + lane] = chosen.weight;
+    p.indices[static_cast<size_t>(token) * p.top_k + lane] = chosen.expert;
   }
+}
+
+// The router and the sort of up to sixteen tokens in one block: a wavefront routes a token and leaves its experts in the LDS,
+// where the whole block then sorts them. They are two launches of 4 to 5 us otherwise, most of either its own latency. (More
+// tokens, several a wavefront, are slower than two launches: some 750 instructions a token on one CU's four SIMDs.)
+// Measured, one token of 128 experts, top 8: 8.3 us, the two launches and the gap between them 9.5.
+constexpr int kSortWaves = kSmallThreads / kWave;
+template <int kPerLane>
+__global__ __launch_bounds__(kSmallThreads) void route_and_sort_kernel(RouteParams p, PermuteParams sort) {
+  extern __shared__ int32_t scratch[];  // the sort's counters (before them the group scores' selections), then the slots' experts
+  int32_t* ids = scratch + max(kSortWaves * p.experts, (kSortWaves + 1) * sort.buckets + 1);
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  if (wave < p.tokens) {  // a wavefront a token; the others wait for the sort
+    float logit[kPerLane];
+    read_logits<kPerLane>(p, wave, logit);
+    const Chosen chosen = routed_token<kPerLane>(p, wave, true, logit, reinterpret_cast<float*>(scratch) + wave * p.experts);
+    if (lane < p.top_k) {
+      p.weights[wave * p.top_k + lane] = chosen.weight;
+      ids[wave * p.top_k + lane] = chosen.expert;
+    }
+  }
+  __syncthreads();
+  sort_small<kSmallThreads>(sort, scratch, [ids](int slot) { return ids[slot]; });
 }
 
 // Each block's shortlist: the `count` best of its best selections (ties to the lower index), one wavefront a block.
@@ -414,16 +481,13 @@ extern "C" int dew_moe_route_call(const dew_moe_router* router, const float* log
                            scores, log_z, stream);
 }
 
-int dew::route_launch(const dew_moe_router* router, const float* logits, const float* bias, const float* media_bias,
-                             const uint8_t* media, const int32_t* given, const uint8_t* covered, const BlockRouting& by_block,
-                             int32_t tokens, float* weights, int32_t* indices, float* scores, float* log_z, void* stream) {
-  DEW_REQUIRE(given || !covered, "dew_moe_route: a coverage without the experts it covers");
-  DEW_REQUIRE((media == nullptr) == (media_bias == nullptr), "dew_moe_route: the media tokens and the bias that chooses for them come together");
+namespace dew {
+
+static int check_router(const dew_moe_router* router, const float* bias, int32_t tokens) {
   DEW_REQUIRE(router, "dew_moe_route: the router's description must not be null");
   const int experts = router->experts, top_k = router->top_k, score_function = router->score_function;
   const int expert_groups = router->expert_groups, groups_per_token = router->groups_per_token;
   DEW_REQUIRE(tokens >= 0 && experts >= 1, "dew_moe_route: tokens %d experts %d", tokens, experts);
-  DEW_REQUIRE(tokens == 0 || (logits && weights && indices), "dew_moe_route: logits, weights and indices must not be null");
   DEW_REQUIRE(experts <= kWave * kMaxPerLane, "dew_moe_route: at most %d experts, got %d", kWave * kMaxPerLane,
               experts);
   DEW_REQUIRE(top_k >= 1 && top_k <= experts && top_k <= kWave, "dew_moe_route: top_k %d of %d experts (at most %d)",
@@ -449,26 +513,83 @@ int dew::route_launch(const dew_moe_router* router, const float* logits, const f
               static_cast<double>(router->weight_sum_epsilon), static_cast<double>(router->weight_sum_min));
   DEW_REQUIRE(router->logit_softcap >= 0.0f, "dew_moe_route: logit_softcap %g is a positive cap, or 0 for none",
               static_cast<double>(router->logit_softcap));
-  if (tokens == 0) return DEW_MOE_OK;
-  RouteParams p{logits, bias, weights, indices, tokens, experts, top_k, score_function, router->normalize ? 1 : 0,
-                expert_groups, groups_per_token, router->group_score == DEW_MOE_GROUP_MAX ? 1 : 0, router->scaling, scores, log_z,
+  return DEW_MOE_OK;
+}
+
+static RouteParams route_params(const dew_moe_router* router, const float* logits, const float* bias, const float* media_bias, const uint8_t* media,
+                                const int32_t* given, const uint8_t* covered, const BlockRouting& by_block, int32_t tokens, float* weights,
+                                int32_t* indices, float* scores, float* log_z) {
+  return RouteParams{logits, bias, weights, indices, tokens, router->experts, router->top_k, router->score_function, router->normalize ? 1 : 0,
+                router->expert_groups, router->groups_per_token, router->group_score == DEW_MOE_GROUP_MAX ? 1 : 0, router->scaling, scores, log_z,
                 router->bias_in_weights ? 1 : 0, router->weight_sum_epsilon, router->weight_sum_min,
                 router->fill_excluded ? 1 : 0, router->excluded_group_score, router->logit_softcap, given, covered, media_bias, media,
-                by_block.blocks, by_block.length, by_block.keys, by_block.allowed, by_block.gather};
-  const int blocks = (tokens + kRouteWaves - 1) / kRouteWaves;
-  const size_t shared = expert_groups > 1 ? sizeof(float) * kRouteWaves * experts : 0;
-  const dim3 grid(blocks), block(kWave * kRouteWaves);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (experts <= 64) {
+                by_block.blocks, by_block.length, by_block.keys, by_block.allowed, by_block.gather, 0, nullptr};
+}
+
+static int launch_route(const RouteParams& p, hipStream_t s) {
+  const size_t shared = p.expert_groups > 1 ? sizeof(float) * kRouteWaves * p.experts : 0;
+  const dim3 grid((p.tokens + kRouteWaves - 1) / kRouteWaves), block(kWave * kRouteWaves);
+  if (p.experts <= 64) {
     hipLaunchKernelGGL(route_kernel<1>, grid, block, shared, s, p);
-  } else if (experts <= 128) {
+  } else if (p.experts <= 128) {
     hipLaunchKernelGGL(route_kernel<2>, grid, block, shared, s, p);
-  } else if (experts <= 256) {
+  } else if (p.experts <= 256) {
     hipLaunchKernelGGL(route_kernel<4>, grid, block, shared, s, p);
   } else {
     hipLaunchKernelGGL(route_kernel<kMaxPerLane>, grid, block, shared, s, p);
   }
   return launched("route_kernel");
+}
+
+}  // namespace dew
+
+int dew::route_launch(const dew_moe_router* router, const float* logits, const float* bias, const float* media_bias,
+                             const uint8_t* media, const int32_t* given, const uint8_t* covered, const BlockRouting& by_block,
+                             int32_t tokens, float* weights, int32_t* indices, float* scores, float* log_z, void* stream) {
+  DEW_REQUIRE(given || !covered, "dew_moe_route: a coverage without the experts it covers");
+  DEW_REQUIRE((media == nullptr) == (media_bias == nullptr), "dew_moe_route: the media tokens and the bias that chooses for them come together");
+  if (int rc = check_router(router, bias, tokens)) return rc;
+  DEW_REQUIRE(tokens == 0 || (logits && weights && indices), "dew_moe_route: logits, weights and indices must not be null");
+  if (tokens == 0) return DEW_MOE_OK;
+  const RouteParams p = route_params(router, logits, bias, media_bias, media, given, covered, by_block, tokens, weights, indices, scores, log_z);
+  return launch_route(p, static_cast<hipStream_t>(stream));
+}
+
+int dew::route_shares(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
+                      float* weights, int32_t* indices, hipStream_t stream) {
+  if (int rc = check_router(router, selection_bias, tokens)) return rc;
+  RouteParams p = route_params(router, partial, selection_bias, nullptr, nullptr, nullptr, nullptr, BlockRouting{}, tokens, weights, indices, nullptr,
+                               nullptr);
+  p.shares = 1;
+  p.gate_bias = gate_bias;
+  return launch_route(p, stream);
+}
+
+int dew::route_and_sort(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
+                        bool shared, float* weights, int32_t* sizes, int32_t* offsets, int32_t* order, int32_t* rows, hipStream_t stream) {
+  if (int rc = check_router(router, selection_bias, tokens)) return rc;
+  const int experts = router->experts, slots = tokens * router->top_k + (shared ? tokens : 0);
+  DEW_REQUIRE(tokens >= 1 && tokens <= kRouteAndSortTokens && slots <= kSmallSlots, "route_and_sort: %d tokens, %d slots", tokens, slots);
+  RouteParams p = route_params(router, partial, selection_bias, nullptr, nullptr, nullptr, nullptr, BlockRouting{}, tokens, weights, nullptr, nullptr,
+                               nullptr);
+  p.shares = 1;
+  p.gate_bias = gate_bias;
+  const int groups = experts + (shared ? 1 : 0);
+  const PermuteParams sort{nullptr, sizes, offsets, order, rows, nullptr, nullptr, slots, tokens * router->top_k, experts, groups, router->top_k, 1,
+                           groups + 1};
+  const size_t lds = sizeof(int32_t) * (static_cast<size_t>(std::max(kSortWaves * experts, (kSortWaves + 1) * sort.buckets + 1)) + sort.routed);
+  static_assert(sizeof(int32_t) * ((kSortWaves + 1) * (kWave * kMaxPerLane + 2) + 1 + kSmallSlots) <= 65536, "the block's LDS");
+  const dim3 grid(1), block(kSmallThreads);
+  if (experts <= 64) {
+    hipLaunchKernelGGL(route_and_sort_kernel<1>, grid, block, lds, stream, p, sort);
+  } else if (experts <= 128) {
+    hipLaunchKernelGGL(route_and_sort_kernel<2>, grid, block, lds, stream, p, sort);
+  } else if (experts <= 256) {
+    hipLaunchKernelGGL(route_and_sort_kernel<4>, grid, block, lds, stream, p, sort);
+  } else {
+    hipLaunchKernelGGL(route_and_sort_kernel<kMaxPerLane>, grid, block, lds, stream, p, sort);
+  }
+  return launched("route_and_sort_kernel");
 }
 
 extern "C" size_t dew_moe_route_blocks_workspace_bytes(int32_t rows, int32_t length, int32_t experts) {

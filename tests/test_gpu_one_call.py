@@ -16,6 +16,8 @@ CASES = {
     "mxfp4, split rows": dict(tokens=1600, experts=8, top_k=2, quant="mxfp4"),
     "groups, bias, shared": dict(tokens=33, experts=64, top_k=8, quant="fp8_block", score_function="sigmoid", routed_scaling_factor=2.5,
                                  expert_groups=8, groups_per_token=4, expert_bias=True, shared=256),
+    "groups, bias, shared, 16 tokens": dict(tokens=16, experts=64, top_k=8, quant="fp8_block", score_function="sigmoid",
+                                            expert_groups=8, groups_per_token=4, expert_bias=True, shared=256),
     "groups, bias, shared, 65 tokens": dict(tokens=65, experts=64, top_k=8, quant="fp8_block", score_function="sigmoid",
                                             expert_groups=8, groups_per_token=4, expert_bias=True, shared=256),
     "300 experts": dict(tokens=64, experts=300, top_k=6, quant="fp8_block"),
