@@ -184,6 +184,10 @@ def gemm(lhs: torch.Tensor, rhs, group_sizes, *, paired=None, gather: torch.Tens
     case = GroupedCase(lhs, rhs, paired, epilogue, out_dtype, compute, tuple(epilogue_operands))
     named = None if implementation in (None, "auto") else implementation
     selection.select(GROUPED, case, named)
+    if torch.is_tensor(rhs) and paired is None and epilogue is None:   # a plain operand's product alone: read where it lies
+        groups = GroupSizes.operands(group_sizes)
+        return ops.dense_gemm(lhs, rhs if rhs.is_contiguous() or rhs.transpose(1, 2).is_contiguous() else rhs.contiguous(), groups["offsets"],
+                              gather=gather, scatter=scatter, sizes=groups.get("sizes"))
     first = prepared(rhs)
     if epilogue == "gpt_oss_gated":
         if scatter is not None:
@@ -208,19 +212,11 @@ def gemm(lhs: torch.Tensor, rhs, group_sizes, *, paired=None, gather: torch.Tens
 def gemm_t(lhs: torch.Tensor, rhs: torch.Tensor, group_sizes, *, out_dtype=torch.bfloat16, whole_steps: bool = False) -> torch.Tensor:
     """Each group's rows of `lhs [rows, depth]` transposed times its rows of `rhs [rows, width]`: `[groups, depth,
     width]` in `out_dtype`, an empty group's zero, exact bf16 products summed in fp32 (the reference's `gemm_t`,
-    src/dew/nn/kernels/gemm.py:418-431: a grouped product's kernel gradient). Both operands are written transposed
-    first (one pass each) so that the contraction runs along contiguous tokens, each group from a whole 64-token step
-    on with zeros filling its last step, so the groups are of any sizes and rows past them add nothing. A caller whose
-    groups are whole 64-row steps and whose rows whole 128s (a recipe pads them so) says `whole_steps` and saves the
-    padding."""
-    groups = GroupSizes.of(group_sizes)
-    if whole_steps:
-        rows_t, _ = ops.transpose_columns(lhs.contiguous(), as_bank=False)
-        bank, _ = ops.transpose_columns(rhs.contiguous(), as_bank=True)
-        return ops.kernel_gradient_bf16(rows_t, bank, groups.offsets, out_dtype=out_dtype)
-    rows_t, padded = ops.transpose_groups(lhs.contiguous(), groups.offsets, as_bank=False)
-    bank, _ = ops.transpose_groups(rhs.contiguous(), groups.offsets, as_bank=True)
-    return ops.kernel_gradient_bf16(rows_t, bank, padded, out_dtype=out_dtype)
+    src/dew/nn/kernels/gemm.py:418-431: a grouped product's kernel gradient). Both operands are read where they lie; the groups
+    are of any sizes and rows past them add nothing. (`whole_steps`, a caller's word that its groups are whole 64-row steps,
+    changes nothing any more.)"""
+    groups = GroupSizes.operands(group_sizes)
+    return ops.dense_gradient(lhs.contiguous(), rhs.contiguous(), groups["offsets"], sizes=groups.get("sizes"), out_dtype=out_dtype)
 
 
 def swiglu_mlp_on_split_rows(lhs: torch.Tensor, gate, up, down, group_sizes, *, gather: torch.Tensor | None = None,

@@ -448,6 +448,46 @@ def grouped_gemm(x: torch.Tensor, bank: PreparedBank, offsets: torch.Tensor | No
     return out
 
 
+def dense_gemm(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor | None, *, gather: torch.Tensor | None = None,
+               scatter: torch.Tensor | None = None, sizes: torch.Tensor | None = None) -> torch.Tensor:
+    """`grouped_gemm` of plain bf16 matrices `w [E, K, N]` (contiguous, or the transpose of contiguous memory), read where they
+    lie: no bank is prepared."""
+    kmajor = not w.is_contiguous()
+    _device(x, "x", torch.bfloat16), _device(w.transpose(1, 2) if kmajor else w, "w", torch.bfloat16)
+    groups, depth, width = w.shape
+    if x.shape[-1] != depth:
+        raise KernelError(f"x rows are {x.shape[-1]} deep, the matrices {depth}")
+    rows = _product_rows(x, "x", offsets, groups, gather, scatter, None, sizes)
+    out = torch.empty((rows, width), dtype=torch.bfloat16, device=x.device)
+    _lib.check(_lib.library().dew_moe_dense_gemm(_ptr(x), _ptr(gather), _ptr(offsets), _ptr(None if offsets is not None else sizes), _ptr(w), int(kmajor),
+                                                 _ptr(scatter), _ptr(out), rows, groups, depth, width, _stream()), "dew_moe_dense_gemm")
+    return out
+
+
+def dense_gradient(lhs: torch.Tensor, rhs: torch.Tensor, offsets: torch.Tensor | None, *, sizes: torch.Tensor | None = None,
+                   lhs_scale: torch.Tensor | None = None, rhs_scale: torch.Tensor | None = None, out_dtype=torch.bfloat16) -> torch.Tensor:
+    """Each group's rows of `lhs [rows, K]` transposed times its rows of `rhs [rows, N]`, times the two scales (fp32, one element),
+    `[groups, K, N]` in bf16 or fp32; both read where they lie, groups of any sizes, an empty group's gradient zero."""
+    _device(lhs, "lhs", torch.bfloat16), _device(rhs, "rhs", torch.bfloat16)
+    if lhs.dim() != 2 or rhs.dim() != 2 or lhs.shape[0] != rhs.shape[0]:
+        raise KernelError(f"lhs {tuple(lhs.shape)} and rhs {tuple(rhs.shape)} do not share their rows")
+    if out_dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"a kernel gradient is written in bfloat16 or float32, not {out_dtype}")
+    for name, index in (("offsets", offsets), ("group_sizes", sizes)):
+        if index is not None:
+            _device(index, name, torch.int32)
+    for name, scale in (("lhs_scale", lhs_scale), ("rhs_scale", rhs_scale)):
+        if scale is not None:
+            _device(scale, name, torch.float32)
+    groups = offsets.numel() - 1 if offsets is not None else sizes.numel()
+    (rows, depth), width = lhs.shape, rhs.shape[1]
+    out = torch.empty((groups, depth, width), dtype=out_dtype, device=lhs.device)
+    _lib.check(_lib.library().dew_moe_dense_gradient(_ptr(lhs), _ptr(rhs), _ptr(offsets), _ptr(None if offsets is not None else sizes), _ptr(lhs_scale),
+                                                     _ptr(rhs_scale), _ptr(out), int(out_dtype == torch.float32), rows, groups, depth, width, _stream()),
+               "dew_moe_dense_gradient")
+    return out
+
+
 def gateup_interleaved(x: torch.Tensor, gate_up: PreparedBank, offsets: torch.Tensor, *, limit: float = 7.0,
                        bias: torch.Tensor | None = None, gather: torch.Tensor | None = None,
                        rows: int | None = None) -> torch.Tensor:

@@ -546,6 +546,19 @@ int dew_moe_combine(const void* slots /* bf16 [T,k,D] */, const float* weights /
                     const void* addend /* nullable */, void* out /* bf16 [T,D] */, int32_t tokens,
                     int32_t top_k, int32_t width, void* stream);
 
+/* ---- Grouped products of plain bf16 operands, read where they lie (a training step's unquantized matrices) --------------
+ * out[scatter[i]] = x[gather[i]] @ w[group of sorted position i] (the `ragged_dot` of src/dew/nn/kernels/gemm.py:84-198 on
+ * plain operands), w bf16 [E, K, N], or [E, N, K] where `kmajor`; K in whole 64s, N in whole 32s. And a kernel gradient
+ * (`gemm_t`, src/dew/nn/kernels/gemm.py:418-431): out[g] = lhs[rows of g]^T @ rhs[rows of g] times the two scales (each
+ * nullable), bf16 or fp32 [E, K, N], an empty group's zero; K and N in whole 8s. The groups are `offsets` [E + 1] or
+ * `group_sizes` [E], the other NULL.                                                                                          */
+int dew_moe_dense_gemm(const void* x /* bf16 [T,K] */, const int32_t* gather /* nullable */, const int32_t* offsets, const int32_t* group_sizes,
+                       const void* w, int32_t kmajor, const int32_t* scatter /* nullable */, void* out /* bf16 [rows,N] */, int32_t rows,
+                       int32_t groups, int32_t depth, int32_t width, void* stream);
+int dew_moe_dense_gradient(const void* lhs /* bf16 [rows,K] */, const void* rhs /* bf16 [rows,N] */, const int32_t* offsets,
+                           const int32_t* group_sizes, const float* lhs_scale, const float* rhs_scale, void* out, int32_t out_is_f32,
+                           int32_t rows, int32_t groups, int32_t depth, int32_t width, void* stream);
+
 /* ---- A sparse layer's forward pass as one call -------------------------------------------------------
  * SparseMLP.__call__ (src/dew/nn/moe.py:1488-1503) and GptOssMLP.__call__ (src/dew/nn/gpt_oss.py:129-171) from the tokens to
  * the layer's output: gate logits, routing, sort, expert products, combine. `gate`, `up`, `down` are prepared banks; an
