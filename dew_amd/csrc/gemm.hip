@@ -167,8 +167,11 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   // shorter lookahead.
   // Quantized rows on the full 256 x 256 tile: a step's weights are 64 registers a lane, of which two sets fit
   // beside the accumulators (a load then has most of a 2048-cycle step to land).
-  // (bf16 matrices: a step's raw data is twice FP8's, three sets of it fit beside the 256-row tile's accumulators)
-  constexpr int kSets = (kFp8A && BN == 256) ? 2 : (kSplit && !kFp8A && BM == 128) ? 2 : (kBf16 || (!kFp4 && BM == 128 && kMatrices * BN == 256)) ? 3 : 4;
+  // (bf16 matrices: a step's raw data is twice FP8's, three sets of it fit beside the 256-row tile's accumulators. On 32- and
+  // 64-row tiles the step's counted wait, which lets the loads behind the last A rows' stay in flight, does not cover the
+  // youngest of three sets where the next step multiplies it, and the compiler then drains the memory pipeline in two steps of
+  // three: four sets there. 1 111 tokens x 6 of 64 experts of 2048 x 1408: the layer 1.5 % shorter.)
+  constexpr int kSets = (kFp8A && BN == 256) ? 2 : (kSplit && !kFp8A && BM == 128) ? 2 : ((kBf16 && BM > 64) || (!kFp4 && !kBf16 && BM == 128 && kMatrices * BN == 256)) ? 3 : 4;
 
   extern __shared__ u32x4_t lds[];  // a ring of three stages of A: BM rows of 128 bytes each
   __shared__ int wave_tiles[4], wave_rows[4];
