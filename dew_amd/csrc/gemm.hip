@@ -165,8 +165,8 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   // MFMAs for each A fragment read from LDS) runs two blocks a CU (256 registers a lane each),
   // which FP8's 32 raw bytes a lane a tile a step only fit with three sets; two resident blocks cover the
   // shorter lookahead.
-  // Quantized rows on the full 256 x 256 tile: a step's weights are 64 registers a lane, of which two sets fit
-  // beside the accumulators (a load then has most of a 2048-cycle step to land).
+  // Quantized rows on the full 256 x 256 tile: two sets of 32 registers a lane beside the accumulators and two halves of eight
+  // row tiles' fragments (a load then has most of a 2048-cycle step to land).
   // (bf16 matrices: a step's raw data is twice FP8's, three sets of it fit beside the 256-row tile's accumulators. On 32- and
   // 64-row tiles the step's counted wait, which lets the loads behind the last A rows' stay in flight, does not cover the
   // youngest of three sets where the next step multiplies it, and the compiler then drains the memory pipeline in two steps of
@@ -454,20 +454,30 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   // is a first touch of its cache line, and the vmcnt wait of each step's barrier, which counts loads in order,
   // stalled on them.)
   const int a_pitch = block_scale_pitch(p.depth);
+  const int a_lds_pitch = a_pitch + (kFp8Rows ? 4 : 0);  // (quantized rows: a dword more, so that 32 rows' bytes of a step lie in 32 banks)
   uint8_t* block_scales = reinterpret_cast<uint8_t*>(lds + kStages * kStageChunks);
   if constexpr (kBlockScales) {
     static_assert(!kBlockScales || BM <= kThreads, "one thread copies one row's scales");
     if (tid < BM) {
       const u32x4_t* from = reinterpret_cast<const u32x4_t*>(p.a_scale + static_cast<size_t>(thread_source) * a_pitch);
-      u32x4_t* to = reinterpret_cast<u32x4_t*>(block_scales + tid * a_pitch);
-      for (int piece = 0; piece < a_pitch / 16; ++piece) to[piece] = from[piece];
+      if constexpr (kFp8Rows) {
+        uint32_t* to = reinterpret_cast<uint32_t*>(block_scales + tid * a_lds_pitch);
+        for (int piece = 0; piece < a_pitch / 16; ++piece) {
+          const u32x4_t words = from[piece];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) to[4 * piece + i] = words[i];
+        }
+      } else {
+        u32x4_t* to = reinterpret_cast<u32x4_t*>(block_scales + tid * a_lds_pitch);
+        for (int piece = 0; piece < a_pitch / 16; ++piece) to[piece] = from[piece];
+      }
     }
   }
   int a_block_word[2][kBlockScales ? TI : 1], a_block_byte[kBlockScales ? TI : 1];
   auto load_block_scales = [&](int block) __attribute__((always_inline)) {
     if constexpr (kBlockScales) {
 #pragma unroll
-      for (int i = 0; i < TI; ++i) a_block_byte[i] = block_scales[(wm0 + 32 * i + lane % 32) * a_pitch + block];
+      for (int i = 0; i < TI; ++i) a_block_byte[i] = block_scales[(wm0 + 32 * i + lane % 32) * a_lds_pitch + block];
     }
   };
   auto form_block_words = [&](auto buffer) __attribute__((always_inline)) {
@@ -491,28 +501,31 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
 #endif
   };
 
-  // MXFP8 rows: a step's four scale bytes of each row, one dword a row, ride the ring beside the A rows: thread t
-  // fetches row t's (one 4-byte LDS-DMA load a wavefront a step), into BM dwords a stage behind the ring.
+  // MXFP8 rows: a step takes four scale bytes of each row, one dword, and a row's dwords lie depth / 32 bytes apart: 64 lanes'
+  // loads touch 64 cache lines whatever they take of them. So thread t fetches row t's dwords of four steps at once, 16 bytes,
+  // four steps ahead into registers, and leaves them two steps later in one of two buffers of [row][4 steps] behind the ring.
+  // (Fetched a dword a step they filled the L1 with as many lines as the rows themselves: 32 KB a step, each for 256 bytes.)
+  // The last fetch of a row is moved back to end with the row, a step's place in it with it.
+  const int a_mx_last = max(p.depth / 128 - 4 - first_step, -first_step);  // the last fetch's first step
   uint32_t* a_mx_stage = reinterpret_cast<uint32_t*>(lds + kStages * kStageChunks);
   const uint8_t* a_mx_src = nullptr;
-  (void)a_mx_src;  // (the host pass compiles no load)
   if constexpr (kMxRows) {
     static_assert(!kMxRows || BM == kThreads, "one thread fetches one row's scales");
     a_mx_src = p.a_scale + static_cast<size_t>(thread_source) * (p.depth / 32) + first_step * 4;
   }
-  auto load_a_scales = [&](int stage_number, int step) __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    if constexpr (kMxRows)
-      __builtin_amdgcn_global_load_lds(a_mx_src + 4 * step, (__attribute__((address_space(3))) void*)(a_mx_stage + stage_number * BM + wave * 64),
-                                       4, 0, 0);
-#endif
+  u32x4_t a_mx_next = {0, 0, 0, 0};
+  auto load_a_scales = [&](int first) __attribute__((always_inline)) {  // the dwords of steps first .. first + 3 (rows of 4 steps or more)
+    if constexpr (kMxRows) __builtin_memcpy(&a_mx_next, a_mx_src + 4 * min(first, a_mx_last), sizeof(a_mx_next));
+  };
+  auto keep_a_scales = [&](int first) __attribute__((always_inline)) {
+    if constexpr (kMxRows) reinterpret_cast<u32x4_t*>(a_mx_stage)[(first / 4 % 2) * BM + tid] = a_mx_next;
   };
   uint32_t a_mx_word[2][kMxRows ? TI : 1];  // the lane's rows' scale dwords of a step, shifted so that byte 2 t is term t's
-  auto fetch_a_scales = [&](auto buffer, int stage_number) __attribute__((always_inline)) {
+  auto fetch_a_scales = [&](auto buffer, int step) __attribute__((always_inline)) {
     if constexpr (kMxRows) {
+      const uint32_t* from = a_mx_stage + ((step / 4 % 2) * BM + wm0 + lane % 32) * 4 + (step - min(step & ~3, a_mx_last));
 #pragma unroll
-      for (int i = 0; i < TI; ++i)
-        a_mx_word[buffer.value][i] = a_mx_stage[stage_number * BM + wm0 + 32 * i + lane % 32] >> (8 * (lane / 32));
+      for (int i = 0; i < TI; ++i) a_mx_word[buffer.value][i] = from[32 * i * 4] >> (8 * (lane / 32));
     }
   };
 
@@ -731,14 +744,16 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
       constexpr std::integral_constant<int, kWeightsFirst ? 0 : kRowLoads / 2> ah{};
       constexpr std::integral_constant<int, kWeightsFirst ? kTiles : kTiles / 2> bh{};
       constexpr int kSplitMfmas = kMatrices * TI * TJ;
-      constexpr int kSplitLoads = ah.value + bh.value * kLoadsPerTile + (kMxRows ? 1 : 0);  // the first phase's, the younger ones at the barrier
+      constexpr bool kScales = kMxRows && quarter.value == 0 && !last_steps.value;  // the rows' scales of the four steps after these
+      constexpr int kSplitLoads = ah.value + bh.value * kLoadsPerTile + (kScales ? 1 : 0);  // the first phase's, the younger ones at the barrier
       static_assert(kRowLoads % 2 == 0 && kTiles % 2 == 0, "two even halves of loads");
       // younger than the last A load of the step before: only this phase's loads are sure to be
       constexpr int kSplitWait = (kSplitLoads & 0xF) | (7 << 4) | (0 << 8) | ((kSplitLoads >> 4) << 14);
       fetch_term(current, c1);
       multiply_term(set, c0, step, scale_buffer);
       load_a(fill, ahead_a, c0, ah);
-      load_a_scales(fill_index, ahead_a);  // (MXFP8 rows: the step's scale dwords, with this phase's loads)
+      if constexpr (kScales) load_a_scales(step + 4);  // (with this phase's loads)
+      if constexpr (kMxRows && quarter.value == 2 && !last_steps.value) keep_a_scales(step + 2);  // (landed before step - 1's barrier)
       load_b(filling, ahead_b, c0, bh);
       schedule_phase<0, kSplitMfmas, 2 * TI, 0, 2 * kTiles + 2 * kSplitLoads, kSplitLoads>();
       __builtin_amdgcn_sched_barrier(0);
@@ -750,7 +765,7 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
       // block scales: the bytes of the next 128 depths are read from the LDS in the second phase of an even step
       // and formed into words in the second phase of the odd step that follows, one phase before they multiply
       if constexpr (kMxRows) {
-        fetch_a_scales(std::integral_constant<int, 1 - set.value % 2>{}, next_index);  // the next step's, landed before the barrier
+        fetch_a_scales(std::integral_constant<int, 1 - set.value % 2>{}, min(step + 1, steps - 1));  // the next step's, kept before the barrier
       } else if constexpr (kFp8Rows) {  // a step is the 128 depths of one scale: the next step's, into the other set
         load_block_scales(min(step + 1, steps - 1));
         form_block_words(std::integral_constant<int, 1 - set.value % 2>{});
@@ -827,8 +842,15 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   };
   load_a(lds, 0, c0, a4);
   load_a(lds + kStageChunks, min(1, steps - 1), c0, a4);
-  load_a_scales(0, 0);
-  load_a_scales(1, min(1, steps - 1));
+  if constexpr (kMxRows) {
+    if (p.depth >= 512) {
+      load_a_scales(0);
+    } else {  // rows of fewer than four steps: all of them, from the row's first on
+#pragma unroll
+      for (int i = 0; i < 4; ++i) __builtin_memcpy(reinterpret_cast<uint8_t*>(&a_mx_next) + 4 * i, a_mx_src + 4 * (min(i, p.depth / 128 - 1) - first_step), 4);
+    }
+    keep_a_scales(0);
+  }
   asm volatile("" ::: "memory");
   __builtin_amdgcn_s_waitcnt(kWaitAll);
   __builtin_amdgcn_s_barrier();
@@ -853,7 +875,7 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   constexpr bool kRaisePriority = BM < 256;
   if constexpr (kRaisePriority) __builtin_amdgcn_s_setprio(3);
   // unrolled so that the register sets, and the block scales' buffers (which turn every four steps), are constants
-  constexpr int kUnroll = (kBlockScales && !kFp8A && kSets < 4) ? 4 : kSets;
+  constexpr int kUnroll = (((kBlockScales && !kFp8A) || kMxRows) && kSets < 4) ? 4 : kSets;
   static_assert(kUnroll % kSets == 0, "whole rounds of the register sets");
   for (; step + kUnroll <= steps; step += kUnroll) {
     static_range<0>(std::make_integer_sequence<int, kUnroll>{}, [&](auto at) {
@@ -1119,8 +1141,8 @@ template <int FORMAT, int MODE, int BM, int BN, int WM, int WN>
 static int launch_tile(const char* who, GemmParams p, hipStream_t stream) {
   // block-scaled activations keep their tile's scales behind the ring (reserved at their largest: kMaxBlockScaleDepth)
   constexpr size_t kShared = shared_bytes<BM, BN, MODE>() +
-                             (FORMAT == kFormatMxSplitBlocks || FORMAT == kFormatFp8Rows ? static_cast<size_t>(BM) * block_scale_pitch(kMaxBlockScaleDepth) : 0) +
-                             (FORMAT == kFormatMxFp8Rows || FORMAT == kFormatMxFp8Window ? 3 * static_cast<size_t>(BM) * 4 : 0);  // MXFP8 rows: a dword a row a stage
+                             (FORMAT == kFormatMxSplitBlocks || FORMAT == kFormatFp8Rows ? static_cast<size_t>(BM) * (block_scale_pitch(kMaxBlockScaleDepth) + (FORMAT == kFormatFp8Rows ? 4 : 0)) : 0) +
+                             (FORMAT == kFormatMxFp8Rows || FORMAT == kFormatMxFp8Window ? 2 * static_cast<size_t>(BM) * 16 : 0);  // MXFP8 rows: four steps' dwords of each row, twice
   auto kernel = grouped_gemm_kernel<FORMAT, MODE, BM, BN, WM, WN>;
   static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel (whichever thread calls first)
   static hipError_t reserved = hipSuccess;
@@ -1413,7 +1435,13 @@ extern "C" int dew_moe_grouped_gemm_fp8_rows(const void* x_codes, const uint8_t*
   GemmParams p{};
   if (int rc = fill_single(who, p, x_codes, gather, offsets, w, bias, scatter, out, rows)) return rc;
   p.a_scale = x_scales;
-  if (p.width % 256 == 0) return launch_tile<kFormatFp8Rows, kPlain, 256, 256, 2, 2>(who, p, static_cast<hipStream_t>(stream));
+  // Quantized rows' 256 x 256 tile is bound by what reaches the CU from the L2, not by the LDS (10 % busy) nor, at two thirds of
+  // the matrix pipe, by that: 24 bytes a clock came in, of which half were two wavefronts' copies of the same weights and MXFP8
+  // rows' scales (see load_a_scales). Side by side along the columns no two wavefronts load the same weights; each reads all rows
+  // from the LDS, which has the time. [32 x 1024, 7168] x 2048 as 2 x 2 and as 1 x 4 (us): forward 476 -> 463, input's gradient 541
+  // -> 512; MXFP8 579 -> 519; kernel's gradient 780 -> 678; [8 x 4096, 4096] x 14336 in MXFP8, the three products: 1916 -> 1679,
+  // 1793 -> 1628, 1757 -> 1627 (2.0 to 2.2 -> 2.3 to 2.4 PFLOP/s).
+  if (p.width % 256 == 0) return launch_tile<kFormatFp8Rows, kPlain, 256, 256, 1, 4>(who, p, static_cast<hipStream_t>(stream));
   return launch_tile<kFormatFp8Rows, kPlain, 256, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
 }
 
@@ -1430,7 +1458,7 @@ extern "C" int dew_moe_grouped_gemm_mxfp8_rows(const void* x_codes, const uint8_
   GemmParams p{};
   if (int rc = fill_single(who, p, x_codes, gather, offsets, w, bias, scatter, out, rows)) return rc;
   p.a_scale = x_scales;
-  if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Rows, kPlain, 256, 256, 2, 2>(who, p, static_cast<hipStream_t>(stream));
+  if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Rows, kPlain, 256, 256, 1, 4>(who, p, static_cast<hipStream_t>(stream));
   return launch_tile<kFormatMxFp8Rows, kPlain, 256, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
 }
 
@@ -1468,10 +1496,10 @@ extern "C" int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint
   p.rows = groups * depth;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (out_is_f32) {
-    if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Window, kPlainF32, 256, 256, 2, 2>(who, p, s);
+    if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Window, kPlainF32, 256, 256, 1, 4>(who, p, s);
     return launch_tile<kFormatMxFp8Window, kPlainF32, 256, 128, 2, 2>(who, p, s);
   }
-  if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Window, kPlain, 256, 256, 2, 2>(who, p, s);
+  if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Window, kPlain, 256, 256, 1, 4>(who, p, s);
   return launch_tile<kFormatMxFp8Window, kPlain, 256, 128, 2, 2>(who, p, s);
 }
 

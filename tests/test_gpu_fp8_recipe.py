@@ -182,6 +182,33 @@ def test_the_mxfp8_product_matches_the_oracle(ops, label, sizes, depth, width):
         assert (got == want).mean() > 0.97
 
 
+@pytest.mark.parametrize("depth", [128, 256, 384, 512, 640, 896, 1152, 2048])
+def test_mxfp8_rows_scales_are_fetched_four_steps_at_a_time(ops, depth):
+    """A step is 128 depths; the tile of 256 columns fetches a row's scales for four at once, the last four moved back to end
+    with the row. Fewer than four steps, whole fours and each remainder, with scales that differ by row and 32-deep block, and
+    as windows of a kernel gradient's tokens that begin at any step. Against the oracle, in units of the same bars as above."""
+    from dew_amd import formats, projections
+
+    rng = np.random.default_rng(depth)
+    spread = lambda rows: np.exp2(rng.integers(-6, 7, size=(rows, depth // 32))).repeat(32, axis=1)
+    sizes, width = [70, 0, 300], 256
+    x = torch.from_numpy((rng.standard_normal((370, depth)) * spread(370)).astype(np.float32)).to(torch.bfloat16)
+    w = weights_case(3, depth, width, seed=depth)
+    bank = formats.MxFp8.quantized(torch.from_numpy(w)).to("cuda")
+    got = bf16_np(projections.mxfp8_product(projections.mxfp8_rows(x.cuda()), bank, torch.tensor(sizes, dtype=torch.int32).cuda()))
+    want = oracle.mxfp8_projection(bf16_np(x), w, sizes)
+    assert np.abs(got - want).max() <= 2.0 ** -7 * np.abs(want).max() and (got == want).mean() > 0.97
+    blocks, left = [], depth // 128
+    while left:
+        blocks.append(min(left, 1 + len(blocks) % 5))
+        left -= blocks[-1]
+    a = torch.from_numpy((rng.standard_normal((256, depth)) * spread(256)).T.astype(np.float32)).to(torch.bfloat16)
+    dy = torch.from_numpy(rng.standard_normal((depth, 256)).astype(np.float32)).to(torch.bfloat16)
+    _, want = oracle.mxfp8_gradients(bf16_np(a), np.zeros((len(blocks), 256, 256), np.float32), bf16_np(dy), blocks, dtype="float32")
+    got = projections.kernel_gradient(a.cuda(), dy.cuda(), blocks, mx=True, out_dtype=torch.float32).cpu().numpy()
+    assert np.abs(got - want).max() <= 2.0 ** -13 * np.abs(want).max()
+
+
 def test_mxfp8_gathered_rows_scattered_outputs_and_whole_blocks(ops):
     from dew_amd import formats, projections
 
