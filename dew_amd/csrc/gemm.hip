@@ -1173,19 +1173,41 @@ static int launch_tile(const char* who, GemmParams p, hipStream_t stream) {
 // what the shorter tile loses when full (it reads and converts the weights again for half the rows: 15 to 26 % on an
 // FP8 bank, 5 to 11 % on one whose codes cost the vector unit little) is less than what the taller one multiplies
 // of empty rows: 32-row tiles up to 26 rows a group (at 32, half the groups need a second, nearly empty one and
-// 64-row tiles are 15 to 25 % faster), 64-row tiles up to 72 rows on FP8 banks (and from 129 to 184, where three
-// of them cover what two 128-row tiles would, 5 to 10 % faster) and up to 384 on the cheap ones.
+// 64-row tiles are 15 to 25 % faster), 64-row tiles up to 72 rows on FP8 banks and up to 384 on the cheap ones.
+// (NVFP4 banks take them from 129 to 184 rows too, where three cover what two 128-row tiles would. FP8 banks did: 5 to 10 % faster on
+// sizes an eighth around their mean, but where a gate's preferences spread the sizes by half and more, 128-row tiles are the
+// faster ones there: 32 experts x 138 rows of 1792 x 2816 paired 160 -> 144 us, 16 x 173 of 3328 x 1152 60 -> 50, 128 x 169 of
+// 1664 x 1024 in one bank 120 -> 103; the few worse shapes lose up to 7 %.)
 // Occupancy: a launch of fewer tiles than CUs halves its tile until there are enough (8 experts x 512 rows x 512
 // columns: 144 tiles of 128 rows take 16.5 us, 272 tiles of 64 rows 11.7 us). 256-row tiles, which fill every
 // accumulator register, are kept to the cheap banks and to groups of 2048 rows or more. Decode-sized groups take the
 // 32-row tile, whose four wavefronts split the columns, so that thousands of wavefronts stream the weights at once.
 static thread_local int forced_tile_rows = 0;  // dew_moe_tile_rows, per calling thread: 0 leaves the choice to the rules below
 
-static int tile_rows(const GemmParams& p, bool cheap) {
+static int tile_rows(const GemmParams& p, bool cheap, int format, bool paired) {
   if (forced_tile_rows != 0) return forced_tile_rows;
   const int average = p.rows / p.experts;
   if (cheap && average >= 2048 && p.width % 256 == 0) return 256;  // below, two 128-row blocks a CU are 2 to 5 % faster
-  int rows = average <= 26 ? 32 : average <= (cheap ? 384 : 72) || (average > 128 && average <= 184) ? 64 : 128;
+  // Unquantized banks' weights are the bytes that their launches move, and a taller tile reads them for more rows; the matrix
+  // pipe waits for them, so that padding costs little. One bank: 128 rows from groups of 76 rows on, wherever that leaves 160
+  // blocks (16 experts x 77 rows of 3328 x 3072: 83 us in 64-row tiles, 72 in 128; 32 x 345 of 2304 x 1920: 161 -> 133; at 108
+  // blocks or on groups of 59 rows 20 to 50 % slower). A paired launch's 128-row block is alone on its CU, so it wants a depth
+  // that its start and end are small beside and several rounds of blocks (16 x 135 rows of 3456 x 3328: 217 -> 192 us, 64 x 291
+  // of 2304 x 1792: 446 -> 411; at 1.5 rounds or 1152 depths 5 to 25 % slower, 32 x 416 of 256 x 3200 15 %). Nor are 64-row tiles halved before they are very
+  // few: 8 x 57 rows of 3328 x 2176 in one bank 48 us in 32-row tiles and 32 in 64, 16 x 409 of 3200 x 256 paired 71 and 31,
+  // 8 x 45 of 896 x 768 paired 9 (a wavefront a strip: few_tiles) and 18.
+  const long long blocks = (p.rows / 128 + p.experts / 2) * static_cast<long long>(p.width / 128);
+  if (format == DEW_MOE_W_BF16 && average > 26 && average <= 512) {
+    const bool rounds = (p.depth >= 2048 && blocks >= 640) || (p.depth >= 1792 && blocks >= 900);
+    if (paired ? average >= 96 && rounds : average >= 76 && blocks >= 160) return 128;
+    const long long shorter = (p.rows / 64 + p.experts / 2) * static_cast<long long>(p.width / 128);
+    return shorter < (paired ? 140 : 100) && average <= 48 ? 32 : 64;
+  }
+  // (a general NVFP4 bank costs the vector unit what an FP8 one does: one-bank launches of many blocks from 212 rows a group on,
+  // 64 experts x 234 rows of 1280 x 2560: 130 us in 64-row tiles, 114 in 128; at 144 to 208 rows or under 900 blocks no faster)
+  if (format == DEW_MOE_W_NVFP4 && !paired && average > 212 && blocks >= 1000) cheap = false;
+  const bool fp8 = format == DEW_MOE_W_FP8_BLOCK || format == DEW_MOE_W_FP8_CHANNEL;
+  int rows = average <= 26 ? 32 : average <= (cheap ? 384 : 72) || (!fp8 && average > 128 && average <= 184) ? 64 : 128;
   const long long strips = p.width / 128;
   // (of 128-row tiles a launch wants one and a half a CU: at 288 and 376 of them, 8 experts x 512 and 700 rows x 1024
   // columns, 64-row tiles are 5 to 13 % faster on FP8 and NVFP4 banks; at 432 and 448, on deeper banks, 17 % slower)
@@ -1212,7 +1234,7 @@ static int launch_format(const char* who, const GemmParams& p, hipStream_t strea
   // than one 256-row block; a one-bank launch the same there and 4 to 7 % slower on 4096-row groups, so it keeps the taller tile)
   constexpr bool kPaired = MODE == kSwigluOfTwo;
   constexpr bool kFp4 = FORMAT == DEW_MOE_W_MXFP4 || FORMAT == DEW_MOE_W_BF16 || (FORMAT == DEW_MOE_W_NVFP4 && !kPaired);
-  switch (tile_rows(p, kFp4)) {
+  switch (tile_rows(p, kFp4, FORMAT, kPaired)) {
     case 32:
       if constexpr (FORMAT != kFormatNvF16) {
         if (forced_tile_rows == 0 && few_tiles(p, FORMAT == DEW_MOE_W_BF16)) return launch_few_tiles(who, p, FORMAT, MODE, stream);
@@ -1236,10 +1258,14 @@ static int launch_format(const char* who, const GemmParams& p, hipStream_t strea
       // it pays only where it fills the chip by itself and most groups have such a last tile: the average group just
       // over a whole number of tiles (256 groups of 256 +- 16 rows: 2.5 tiles a group become 2 and a 64-row one, 1.5
       // to 2.5 % faster; at 160 or 200 rows a group the same two launches are 5 to 15 % slower than one, a bank of 8
-      // experts, whose few last tiles run their whole depth alone, 20 to 35 % slower, and groups of 1024 rows 1 %).
+      // experts, whose few last tiles run their whole depth alone, 20 to 35 % slower, and groups of 1024 rows 1 %). Where a
+      // gate's preferences spread the sizes widely, half the groups have such a last tile whatever the average: 256 experts of
+      // 7168 x 2048 gain 2 %, 128 experts nothing, and 64 or 128 experts of 2048 to 4096 x 2048 lose 2 to 8 % (FP8 at 140 and 275
+      // rows a group 848 -> 777 and 1145 -> 1089 us a layer in one launch, NVFP4 at 256 918 -> 896, MXFP4 at 412 999 -> 939): from
+      // 3072 strips of tiles on.
       const int average = p.rows / p.experts;
-      const bool shared = forced_tile_rows == 0 && average >= 128 && average < 512 && average % 128 <= 40 &&
-                          static_cast<long long>(p.experts) * (p.width / 128) >= 512;
+      const bool shared = forced_tile_rows == 0 && FORMAT != DEW_MOE_W_BF16 && average >= 192 && average < 512 && average % 128 <= 40 &&
+                          static_cast<long long>(p.experts) * (p.width / 128) >= 3072;
       GemmParams taller = p;
       taller.skip_tails = shared ? 64 : 0;
       int status;
