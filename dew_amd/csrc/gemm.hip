@@ -1441,8 +1441,10 @@ extern "C" int dew_moe_grouped_gemm_split_blocks(const void* x_split, const uint
   GemmParams p{};
   if (int rc = fill_single(who, p, x_split, gather, offsets, w, bias, scatter, out, rows)) return rc;
   p.a_scale = x_scales;
-  if (forced_tile_rows == 128) return launch_tile<kFormatMxSplitBlocks, kPlain, 128, 256, 2, 2>(who, p, static_cast<hipStream_t>(stream));
-  return launch_tile<kFormatMxSplitBlocks, kPlain, 256, 256, 2, 2>(who, p, static_cast<hipStream_t>(stream));
+  // 128-row tiles, two blocks a CU: half the padding at a group's end, and a tile's start and epilogue under the other block's loop.
+  // Against 256 x 256 tiles, a layer of MXFP4 experts (us): 64 x 412 rows of 2048 x 3072 1008 -> 933, 8 x 1024 of 4096 x 4096 736 ->
+  // 706, 8 x 4096 of 2048 x 2048 741 -> 708, 16 x 4096 of 2048 x 7168 4308 -> 4162, 8 x 4096 of 14336 x 4096 7478 -> 7458.
+  return launch_tile<kFormatMxSplitBlocks, kPlain, 128, 256, 2, 2>(who, p, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int dew_moe_grouped_gemm_fp8_rows(const void* x_codes, const uint8_t* x_scales, const int32_t* gather,
