@@ -16,6 +16,7 @@
 // rules as whole-tensor operations and a re-layout of their result took 4.5 (FP8) and 8.5 ms (MXFP8); NVFP4 on [8, 2048, 4096]
 // 67 us and 26 us for the largest magnitude, against some 7 ms (its E2M1 choice is 30 vector instructions an element).
 #include "common.h"
+#include "nvfp4.h"
 
 namespace dew {
 
@@ -145,6 +146,8 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
     tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
     if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) tensor_scales[e] = tensor;
   }
+  const bool quick = kNv && sizeof(T) == 2 && nvfp4_in_range(tensor);  // (the same for the whole launch)
+  const float inverse_tensor = kNv ? 1.0f / tensor : 1.0f;
   auto magnitude = [](float value) { return __float_as_uint(value) & 0x7FFFFFFFu; };
   float inverse = 1.0f;  // FP8 blocks: the tile's one
   if constexpr (kBlocks) {
@@ -185,7 +188,8 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
       if constexpr (kNv) {
         const uint32_t byte = nvfp4_block_byte(__uint_as_float(maxima[block][column]), tensor);
         scale_bytes[block][column] = static_cast<uint8_t>(byte);
-        each_of[block][column] = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
+        const float each = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
+        each_of[block][column] = quick ? nvfp4_inverse(each) : each;
       } else {
         const uint32_t byte = mx_byte(max(maxima[2 * block][column], maxima[2 * block + 1][column]));
         scale_bytes[block][column] = static_cast<uint8_t>(byte);
@@ -206,8 +210,13 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
         const int quad = group * (kLoads / 4) + d;
         if constexpr (kNv) {
           uint32_t nibbles = 0;
+          if (quick) {
+            const Nvfp4Scales by{tensor, inverse_tensor, __builtin_amdgcn_cvt_f32_fp8(scale_bytes[block][column], 0), each};
+            nibbles = by.four(v[4 * d][i], v[4 * d + 1][i], v[4 * d + 2][i], v[4 * d + 3][i]);
+          } else {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) nibbles |= e2m1_code(v[4 * d + r][i], tensor, each) << (4 * r);
+            for (int r = 0; r < 4; ++r) nibbles |= e2m1_code(v[4 * d + r][i], tensor, each) << (4 * r);
+          }
           reinterpret_cast<uint16_t*>(staged)[quad * kMatrixTile + column] = static_cast<uint16_t>(nibbles);
         } else {
           float q[4];
@@ -238,8 +247,13 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
       for (int d = 0; d < kVec / 4; ++d) {
         if constexpr (kNv) {
           uint32_t nibbles = 0;
+          if (quick) {
+            const Nvfp4Scales by{tensor, inverse_tensor, each, nvfp4_inverse(each)};
+            nibbles = by.four(v[p][4 * d], v[p][4 * d + 1], v[p][4 * d + 2], v[p][4 * d + 3]);
+          } else {
 #pragma unroll
-          for (int r = 0; r < 4; ++r) nibbles |= e2m1_code(v[p][4 * d + r], tensor, each) << (4 * r);
+            for (int r = 0; r < 4; ++r) nibbles |= e2m1_code(v[p][4 * d + r], tensor, each) << (4 * r);
+          }
           *reinterpret_cast<uint16_t*>(staged + column * kPitch + k / 2 + 2 * d) = static_cast<uint16_t>(nibbles);
         } else {
           float q[4];

@@ -9,6 +9,7 @@
 // The scales are kept as their e8m0 bytes, block_scale_pitch(depth) a row (one byte per 128 depths, padded to 16).
 // HBM-bound: 2 bytes read and 1 written per element.
 #include "common.h"
+#include "nvfp4.h"
 
 namespace dew {
 
@@ -171,6 +172,8 @@ __global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_nvfp4_kerne
   // largest / (6 * 448), fp32's least normal at least; 1 for an operand of zeros
   const float tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
   if (blockIdx.x == 0 && threadIdx.x == 0) *tensor_scale = tensor;
+  const bool quick = nvfp4_in_range(tensor);  // (the same for the whole launch)
+  const float inverse_tensor = 1.0f / tensor;
   const int lane = threadIdx.x % 64;
   const int row = blockIdx.x * kQuantizeWaves + threadIdx.x / 64;
   if (row >= rows) return;
@@ -194,6 +197,13 @@ __global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_nvfp4_kerne
     if (__builtin_amdgcn_cvt_f32_fp8(byte, 0) < ratio) byte = min(byte + 1u, 0x7Eu);
     const float each = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
     u32x4_t packed;
+    if (quick) {
+      const Nvfp4Scales by{tensor, inverse_tensor, each, nvfp4_inverse(each)};
+#pragma unroll
+      for (int i = 0; i < 4; ++i) packed[i] = by.values(v[2 * i], v[2 * i + 1]);
+      *reinterpret_cast<u32x4_t*>(target + chunk * 8) = packed;
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       float pair[2];
@@ -385,6 +395,16 @@ __global__ __launch_bounds__(256) void transpose_columns_kernel(const bf16_t* __
       uint32_t byte = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(ratio, 448.0f), 0.0f, 0, false) & 0xFFu;
       if (__builtin_amdgcn_cvt_f32_fp8(byte, 0) < ratio) byte = min(byte + 1u, 0x7Eu);
       const float each = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
+      if (nvfp4_in_range(tensor)) {
+        const Nvfp4Scales by{tensor, 1.0f / tensor, each, nvfp4_inverse(each)};
+#pragma unroll
+        for (int i = 0; i < 16; i += 2) {
+          const uint32_t both = by.values(__uint_as_float(bits[16 * block + i] << 16), __uint_as_float(bits[16 * block + i + 1] << 16));
+          bits[16 * block + i] = both & 0xFFFFu;
+          bits[16 * block + i + 1] = both >> 16;
+        }
+        continue;
+      }
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
         const float value = __uint_as_float(bits[16 * block + i] << 16);

@@ -71,3 +71,37 @@ def test_what_cannot_be_quantized_is_refused(ops):
                       (torch.zeros((1, 128, 128), dtype=torch.bfloat16), "mxfp8")):
         with pytest.raises(ops.KernelError):
             ops.quantize_matrices(w, recipe)
+
+
+@pytest.mark.parametrize("exponent", [0, -79, 60, -100], ids=["ones", "least", "large", "past"])   # the tensor scale in and (2^-100) out of the range of the short form
+def test_every_significand_against_every_tensor_scale(ops, exponent):
+    """NVFP4's quotients of bf16 values come from reciprocals and a Newton step. Every significand of the largest magnitude (21 / 16
+    and its like, whose tensor scales make most thresholds exact ties) with every significand as a block's largest, and values of
+    every significand and a dozen binades below, in each of the four launches that choose codes."""
+    from dew_amd import codecs
+
+    e2m1 = torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, -0.0, -0.5, -1, -1.5, -2, -3, -4, -6], device="cuda")
+    generator = torch.Generator(device="cuda").manual_seed(exponent + 200)
+    significands = 1 + torch.arange(128, device="cuda") / 128
+    for first in range(0, 128, 8):
+        for largest in significands[first:first + 8].tolist():
+            tops = largest * torch.exp2(-torch.randint(0, 11, (64, 128), generator=generator, device="cuda").float())
+            tops = torch.minimum(tops * significands / 2, torch.tensor(largest, device="cuda"))
+            values = tops[:, :, None] * torch.exp2(-torch.randint(0, 12, (64, 128, 16), generator=generator, device="cuda").float())
+            values *= significands[torch.randint(0, 128, (64, 128, 16), generator=generator, device="cuda")] / 2
+            values *= torch.randint(0, 2, (64, 128, 16), generator=generator, device="cuda") * 2 - 1
+            values[:, :, 3] = tops
+            values[0, 0, 3] = largest
+            x = (values.reshape(256, 512) * 2.0 ** exponent).to(torch.bfloat16)     # [tokens or width, depth], blocks of 16 along the depth
+            w = x.t()[None]                                                         # [1, 512, 256], held K-major
+            want = ops.prepare(by_whole_tensors("nvfp4", w))
+            compared = x.numel() // 2 + x.numel() // 16
+            for held in (w, w.contiguous()):
+                got = ops.quantize_matrices(held, "nvfp4")
+                assert torch.equal(got.keep[0][:compared], want.keep[0][:compared]) and torch.equal(got.keep[2], want.keep[2])
+            codes, scales, _ = codecs.nvfp4_coded(w[0].float())
+            decoded = (e2m1[codes.long()] * scales.view(torch.float8_e4m3fn).float().repeat_interleave(16, 0)).t()
+            rows, scale = ops.quantize_rows_nvfp4(x.contiguous())
+            assert scale.item() == want.keep[2][0].item() and torch.equal(rows.float(), decoded)
+            columns, scale = ops.transpose_columns(x.t().contiguous(), nvfp4=True, as_bank=False)
+            assert scale.item() == want.keep[2][0].item() and torch.equal(columns.float(), decoded)
