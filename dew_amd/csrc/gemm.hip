@@ -401,8 +401,8 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   }
   int thread_source = 0;  // row tid of the tile, where one thread fetches one row's scales
   if constexpr (kNvF16 || kBlockScales || kMxRows) {
-    if (tid < BM) {
-      const int sorted = row0 + min(tid, valid_rows - 1);
+    if (kMxRows || tid < BM) {  // (MXFP8 rows: two threads the same row's where the tile is shorter, which leave the same bytes)
+      const int sorted = row0 + min(tid % BM, valid_rows - 1);
       thread_source = kWindow ? sorted - expert * p.window_rows : p.gather ? p.gather[sorted] : sorted;
     }
   }
@@ -510,7 +510,6 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   uint32_t* a_mx_stage = reinterpret_cast<uint32_t*>(lds + kStages * kStageChunks);
   const uint8_t* a_mx_src = nullptr;
   if constexpr (kMxRows) {
-    static_assert(!kMxRows || BM == kThreads, "one thread fetches one row's scales");
     a_mx_src = p.a_scale + static_cast<size_t>(thread_source) * (p.depth / 32) + first_step * 4;
   }
   u32x4_t a_mx_next = {0, 0, 0, 0};
@@ -518,7 +517,7 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
     if constexpr (kMxRows) __builtin_memcpy(&a_mx_next, a_mx_src + 4 * min(first, a_mx_last), sizeof(a_mx_next));
   };
   auto keep_a_scales = [&](int first) __attribute__((always_inline)) {
-    if constexpr (kMxRows) reinterpret_cast<u32x4_t*>(a_mx_stage)[(first / 4 % 2) * BM + tid] = a_mx_next;
+    if constexpr (kMxRows) reinterpret_cast<u32x4_t*>(a_mx_stage)[(first / 4 % 2) * BM + tid % BM] = a_mx_next;
   };
   uint32_t a_mx_word[2][kMxRows ? TI : 1];  // the lane's rows' scale dwords of a step, shifted so that byte 2 t is term t's
   auto fetch_a_scales = [&](auto buffer, int step) __attribute__((always_inline)) {
@@ -1320,6 +1319,20 @@ static int fill_single(const char* who, GemmParams& p, const void* x, const int3
   return DEW_MOE_OK;
 }
 
+// Whether a recipe's product runs on 128 x 128 tiles: where its 256 x 256 ones, half of each group's last one empty, would leave a
+// good part of the chip idle. At 18 to 128 of them four times as many blocks are up to twice as fast (us; 640 rows of 4 x 1024 x
+// 2048 21 -> 10, 2048 of 16 x 2048 x 2048 30 -> 21, 1024 of 2 x 4096 x 4096 49 -> 28); at 192 and 256 they are 5 to 14 % slower.
+static bool few_blocks(const GemmParams& p) {
+  if (forced_tile_rows != 0) return forced_tile_rows == 128;
+  return (p.rows / 256 + p.experts / 2) * static_cast<long long>((p.width + 255) / 256) <= 160;
+}
+
+// The same of a kernel's gradient, whose tiles are whole: at 128 tiles of 256 x 256, 1024 tokens a group.
+static bool few_gradient_blocks(const GemmParams& p) {
+  if (forced_tile_rows != 0) return forced_tile_rows == 128;
+  return static_cast<long long>(p.experts) * ((p.window_rows + 255) / 256) * ((p.width + 255) / 256) <= 128;
+}
+
 }  // namespace dew
 
 extern "C" int dew_moe_tile_rows(int32_t rows) {
@@ -1469,6 +1482,7 @@ extern "C" int dew_moe_grouped_gemm_fp8_rows(const void* x_codes, const uint8_t*
   // from the LDS, which has the time. [32 x 1024, 7168] x 2048 as 2 x 2 and as 1 x 4 (us): forward 476 -> 463, input's gradient 541
   // -> 512; MXFP8 579 -> 519; kernel's gradient 780 -> 678; [8 x 4096, 4096] x 14336 in MXFP8, the three products: 1916 -> 1679,
   // 1793 -> 1628, 1757 -> 1627 (2.0 to 2.2 -> 2.3 to 2.4 PFLOP/s).
+  if (few_blocks(p)) return launch_tile<kFormatFp8Rows, kPlain, 128, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
   if (p.width % 256 == 0) return launch_tile<kFormatFp8Rows, kPlain, 256, 256, 1, 4>(who, p, static_cast<hipStream_t>(stream));
   return launch_tile<kFormatFp8Rows, kPlain, 256, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
 }
@@ -1486,6 +1500,7 @@ extern "C" int dew_moe_grouped_gemm_mxfp8_rows(const void* x_codes, const uint8_
   GemmParams p{};
   if (int rc = fill_single(who, p, x_codes, gather, offsets, w, bias, scatter, out, rows)) return rc;
   p.a_scale = x_scales;
+  if (few_blocks(p)) return launch_tile<kFormatMxFp8Rows, kPlain, 128, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
   if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Rows, kPlain, 256, 256, 1, 4>(who, p, static_cast<hipStream_t>(stream));
   return launch_tile<kFormatMxFp8Rows, kPlain, 256, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
 }
@@ -1524,10 +1539,11 @@ extern "C" int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint
   p.rows = groups * depth;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (out_is_f32) {
-    if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Window, kPlainF32, 256, 256, 1, 4>(who, p, s);
+    if (p.width % 256 == 0 && !few_gradient_blocks(p)) return launch_tile<kFormatMxFp8Window, kPlainF32, 256, 256, 1, 4>(who, p, s);
     return launch_tile<kFormatMxFp8Window, kPlainF32, 256, 128, 2, 2>(who, p, s);
   }
-  if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Window, kPlain, 256, 256, 1, 4>(who, p, s);
+  // (few tiles: half as wide ones, 8 groups of 512 tokens x 1024 x 1024 19 -> 14 us; 128 x 128 take 17)
+  if (p.width % 256 == 0 && !few_gradient_blocks(p)) return launch_tile<kFormatMxFp8Window, kPlain, 256, 256, 1, 4>(who, p, s);
   return launch_tile<kFormatMxFp8Window, kPlain, 256, 128, 2, 2>(who, p, s);
 }
 
@@ -1565,9 +1581,12 @@ extern "C" int dew_moe_kernel_gradient_bf16(const void* lhs_t, const dew_moe_ban
   p.rows = groups * depth;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (out_is_f32) {
+    if (few_gradient_blocks(p)) return launch_tile<kFormatBf16Window, kPlainF32, 128, 128, 1, 4>(who, p, s);
     if (p.width % 256 == 0) return launch_tile<kFormatBf16Window, kPlainF32, 256, 256, 1, 4>(who, p, s);
     return launch_tile<kFormatBf16Window, kPlainF32, 256, 128, 1, 4>(who, p, s);
   }
+  // (one group of 2048 tokens x 512 x 2048: 42 us in 16 tiles, 20 in 64)
+  if (few_gradient_blocks(p)) return launch_tile<kFormatBf16Window, kPlain, 128, 128, 1, 4>(who, p, s);
   if (p.width % 256 == 0) return launch_tile<kFormatBf16Window, kPlain, 256, 256, 1, 4>(who, p, s);
   return launch_tile<kFormatBf16Window, kPlain, 256, 128, 1, 4>(who, p, s);
 }

@@ -195,9 +195,11 @@ def test_mxfp8_rows_scales_are_fetched_four_steps_at_a_time(ops, depth):
     x = torch.from_numpy((rng.standard_normal((370, depth)) * spread(370)).astype(np.float32)).to(torch.bfloat16)
     w = weights_case(3, depth, width, seed=depth)
     bank = formats.MxFp8.quantized(torch.from_numpy(w)).to("cuda")
-    got = bf16_np(projections.mxfp8_product(projections.mxfp8_rows(x.cuda()), bank, torch.tensor(sizes, dtype=torch.int32).cuda()))
     want = oracle.mxfp8_projection(bf16_np(x), w, sizes)
-    assert np.abs(got - want).max() <= 2.0 ** -7 * np.abs(want).max() and (got == want).mean() > 0.97
+    for tile in (256, 128):
+        with ops.tile_rows(tile):
+            got = bf16_np(projections.mxfp8_product(projections.mxfp8_rows(x.cuda()), bank, torch.tensor(sizes, dtype=torch.int32).cuda()))
+        assert np.abs(got - want).max() <= 2.0 ** -7 * np.abs(want).max() and (got == want).mean() > 0.97, tile
     blocks, left = [], depth // 128
     while left:
         blocks.append(min(left, 1 + len(blocks) % 5))
@@ -205,8 +207,36 @@ def test_mxfp8_rows_scales_are_fetched_four_steps_at_a_time(ops, depth):
     a = torch.from_numpy((rng.standard_normal((256, depth)) * spread(256)).T.astype(np.float32)).to(torch.bfloat16)
     dy = torch.from_numpy(rng.standard_normal((depth, 256)).astype(np.float32)).to(torch.bfloat16)
     _, want = oracle.mxfp8_gradients(bf16_np(a), np.zeros((len(blocks), 256, 256), np.float32), bf16_np(dy), blocks, dtype="float32")
-    got = projections.kernel_gradient(a.cuda(), dy.cuda(), blocks, mx=True, out_dtype=torch.float32).cpu().numpy()
-    assert np.abs(got - want).max() <= 2.0 ** -13 * np.abs(want).max()
+    for tile in (256, 128):
+        with ops.tile_rows(tile):
+            got = projections.kernel_gradient(a.cuda(), dy.cuda(), blocks, mx=True, out_dtype=torch.float32).cpu().numpy()
+        assert np.abs(got - want).max() <= 2.0 ** -13 * np.abs(want).max(), tile
+
+
+@pytest.mark.parametrize("recipe", ["blockwise_fp8", "mxfp8", "nvfp4"])
+@pytest.mark.parametrize("blocks,depth,width", [((1, 0, 3, 5), 384, 384), ((2, 1), 512, 1280), ((3,), 256, 256)])
+def test_a_recipes_short_tiles_return_the_tall_ones_bits(ops, recipe, blocks, depth, width):
+    """Few tiles run as 128 x 128 (a gradient's as half as wide ones): the same sums in the same order."""
+    from dew_amd import projections
+
+    if recipe == "nvfp4":
+        depth, width = (depth + 255) // 256 * 256, (width + 255) // 256 * 256
+    generator = torch.Generator(device="cuda").manual_seed(depth + width)
+    tokens = 128 * sum(blocks)
+    x = torch.randn((tokens, depth), generator=generator, device="cuda").to(torch.bfloat16)
+    dy = torch.randn((tokens, width), generator=generator, device="cuda").to(torch.bfloat16)
+    w = torch.randn((len(blocks), depth, width), generator=generator, device="cuda").to(torch.bfloat16)
+    forward = {"blockwise_fp8": projections.blockwise_fp8_projection, "mxfp8": projections.mxfp8_projection, "nvfp4": projections.nvfp4_projection}[recipe]
+    gradients = {"blockwise_fp8": projections.blockwise_fp8_gradients, "mxfp8": projections.mxfp8_gradients, "nvfp4": projections.nvfp4_gradients}[recipe]
+    results = {}
+    for tile in (0, 128, 256):
+        with ops.tile_rows(tile):
+            results[tile] = (forward(x, w, list(blocks)), *gradients(x, w, dy, list(blocks)),
+                             gradients(x, w, dy, list(blocks), out_dtype=torch.float32)[1])
+    assert all(r.isfinite().all() and r.abs().amax() > 0 for r in results[256])
+    for tile in (0, 128):
+        for got, want in zip(results[tile], results[256]):
+            assert torch.equal(got, want), tile
 
 
 def test_mxfp8_gathered_rows_scattered_outputs_and_whole_blocks(ops):
