@@ -12,14 +12,14 @@
 // A 256-thread block owns a BM x 256 tile and walks the contraction in steps of 32: operands global -> LDS by DMA into a ring of
 // three stages (24 KB each at BM = 128, so that two blocks share a CU and one's start and end run under the other's loop; a
 // contraction of a few hundred rows, a kernel gradient's, is otherwise half start and end), one barrier a step, wavefronts side
-// by side along the columns. Sums are taken along the contraction in the tiled launch's order: the same bits.
+// by side along the columns; where such tiles are few, smaller ones. Sums are taken along the contraction in the tiled launch's order: the same bits.
 #include <mutex>
 
 #include "gemm.h"
 
 namespace dew {
 
-constexpr int kDepthStep = 32, kColumns = 256, kRing = 3, kBlock = 256;
+constexpr int kDepthStep = 32, kRing = 3, kBlock = 256;
 
 struct DenseParams {
   const bf16_t* a;  // [rows, inner] (gathered), or, contracted over groups of rows, [rows, outer_m]
@@ -81,13 +81,13 @@ struct Staged {
 };
 
 // kAAcross: a kernel gradient (both operands' rows run across the contraction, which is a group's rows). kBAcross: w [.., depth, width].
-template <int BM, bool kAAcross, bool kBAcross, bool kOutF32>
+template <int BM, int kColumns, bool kAAcross, bool kBAcross, bool kOutF32>
 __global__ __launch_bounds__(kBlock, 2) void dense_kernel(DenseParams p) {
   using A = Staged<BM, kAAcross>;
   using B = Staged<kColumns, kBAcross>;
   static_assert(!kAAcross || kBAcross, "a kernel gradient's operands both run across");
   constexpr int kStageBytes = A::kBytes + B::kBytes, kLoads = A::kLoads + B::kLoads;
-  constexpr int TI = BM / 32, TJ = 2;
+  constexpr int TI = BM / 32, TJ = kColumns / 128;
   extern __shared__ uint8_t stages[];  // the ring; then the finished tile's rows
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
 
@@ -221,7 +221,7 @@ __global__ __launch_bounds__(kBlock, 2) void dense_kernel(DenseParams p) {
   auto fetch = [&](int stage, auto slice) __attribute__((always_inline)) {
     const uint8_t* from = stages + stage * kStageBytes;
 #pragma unroll
-    for (int j = 0; j < TJ; ++j) b_frag[slice.value][j] = B::template fragment<decltype(slice)::value>(from + A::kBytes, 2 * wave + j, lane);
+    for (int j = 0; j < TJ; ++j) b_frag[slice.value][j] = B::template fragment<decltype(slice)::value>(from + A::kBytes, TJ * wave + j, lane);
 #pragma unroll
     for (int i = 0; i < TI; ++i) a_frag[slice.value][i] = A::template fragment<decltype(slice)::value>(from, i, lane);
   };
@@ -294,7 +294,7 @@ __global__ __launch_bounds__(kBlock, 2) void dense_kernel(DenseParams p) {
         const int row = 32 * i + 8 * (q / 4) + 4 * (lane / 32) + q % 4;
 #pragma unroll
         for (int j = 0; j < TJ; ++j) {
-          const int column = n0 + 64 * wave + 32 * j + lane % 32;
+          const int column = n0 + 32 * (TJ * wave + j) + lane % 32;
           if (row < valid_rows && column < p.outer_n) out[static_cast<size_t>(row) * p.outer_n + column] = acc[i][j][q] * factor;
         }
       }
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kBlock, 2) void dense_kernel(DenseParams p) {
         for (int j = 0; j < TJ; ++j) {
           const uint32_t mine = pack_bf16(acc[i][j][q] * factor, acc[i][j][q + 1] * factor);
           const uint32_t other = __builtin_amdgcn_mov_dpp(mine, 0xB1, 0xF, 0xF, true);
-          staged[row * kRowDwords + (64 * wave + 32 * j + (lane % 32 & ~1)) / 2] = __builtin_amdgcn_perm(other, mine, select);
+          staged[row * kRowDwords + (32 * (TJ * wave + j) + (lane % 32 & ~1)) / 2] = __builtin_amdgcn_perm(other, mine, select);
         }
       }
     __syncthreads();
@@ -329,12 +329,12 @@ __global__ __launch_bounds__(kBlock, 2) void dense_kernel(DenseParams p) {
   }
 }
 
-template <int BM, bool kAAcross, bool kBAcross, bool kOutF32>
+template <int BM, int kColumns, bool kAAcross, bool kBAcross, bool kOutF32>
 static int launch_dense(const char* who, DenseParams p, hipStream_t stream) {
   constexpr size_t kRingBytes = kRing * (Staged<BM, kAAcross>::kBytes + Staged<kColumns, kBAcross>::kBytes);
   constexpr size_t kStagedBytes = static_cast<size_t>(BM) * (kColumns / 2 + 4) * 4;
   constexpr size_t kShared = kRingBytes > kStagedBytes ? kRingBytes : kStagedBytes;
-  auto kernel = dense_kernel<BM, kAAcross, kBAcross, kOutF32>;
+  auto kernel = dense_kernel<BM, kColumns, kAAcross, kBAcross, kOutF32>;
   static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
   static hipError_t reserved = hipSuccess;
   std::call_once(configured, [&] {
@@ -350,6 +350,11 @@ static int launch_dense(const char* who, DenseParams p, hipStream_t stream) {
   const int blocks = static_cast<int>((total + round - 1) / round * round);
   hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kBlock), kShared, stream, p);
   return launched(who);
+}
+
+constexpr int kFewTiles = 128;
+static bool few_tiles(int rows, int groups, int width) {  // about so many of 128 x 256, the groups' last ones half empty
+  return (rows / 128 + groups / 2 + 1) * static_cast<long long>((width + 255) / 256) <= kFewTiles;
 }
 
 }  // namespace dew
@@ -378,9 +383,14 @@ extern "C" int dew_moe_dense_gemm(const void* x, const int32_t* gather, const in
   p.inner = depth;
   p.outer_n = width;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  // Where 128 x 256 tiles would leave half of the chip idle, a quarter of one each: a block's walk down the contraction is what the
+  // launch takes then (us: 640 rows of 4 x 1024 x 2048 22 -> 14 and its input's gradient 38 -> 22, 1000 of 8 x 3072 x 1024 57 -> 31, 3000
+  // of 8 x 2048 x 1024, 112 tiles, 42 -> 32; at 160 to 220 tiles 3 to 30 % slower).
+  if (few_tiles(rows, groups, width))
+    return kmajor ? launch_dense<64, 128, false, false, false>(who, p, s) : launch_dense<64, 128, false, true, false>(who, p, s);
   if (rows / groups <= 64)
-    return kmajor ? launch_dense<64, false, false, false>(who, p, s) : launch_dense<64, false, true, false>(who, p, s);
-  return kmajor ? launch_dense<128, false, false, false>(who, p, s) : launch_dense<128, false, true, false>(who, p, s);
+    return kmajor ? launch_dense<64, 256, false, false, false>(who, p, s) : launch_dense<64, 256, false, true, false>(who, p, s);
+  return kmajor ? launch_dense<128, 256, false, false, false>(who, p, s) : launch_dense<128, 256, false, true, false>(who, p, s);
 }
 
 extern "C" int dew_moe_dense_gradient(const void* lhs, const void* rhs, const int32_t* offsets, const int32_t* group_sizes, const float* lhs_scale,
@@ -405,5 +415,9 @@ extern "C" int dew_moe_dense_gradient(const void* lhs, const void* rhs, const in
   p.outer_m = depth;
   p.outer_n = width;
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  return out_is_f32 ? launch_dense<128, true, true, true>(who, p, s) : launch_dense<128, true, true, false>(who, p, s);
+  // (few tiles: half as wide, 4 groups of 4096 rows, 1024 x 1024, 128 tiles, 96 -> 77 us; 3333 rows, 2 x 640 x 4096, 39 -> 34; at 512
+  // tiles 8 to 10 % slower)
+  if (static_cast<long long>(groups) * ((depth + 127) / 128) * ((width + 255) / 256) <= 2 * kFewTiles)
+    return out_is_f32 ? launch_dense<128, 128, true, true, true>(who, p, s) : launch_dense<128, 128, true, true, false>(who, p, s);
+  return out_is_f32 ? launch_dense<128, 256, true, true, true>(who, p, s) : launch_dense<128, 256, true, true, false>(who, p, s);
 }

@@ -63,3 +63,15 @@ def test_kernel_gradients_of_plain_rows(name, depth, width, out_dtype):
         begin += size
     scale = torch.tensor([0.5], device="cuda")
     assert torch.equal(ops.dense_gradient(x, dy, None, sizes=sizes, lhs_scale=scale, out_dtype=out_dtype), got * 0.5)
+
+
+# (a launch of few tiles takes a quarter of one each, a gradient's half: these are many, the last one's columns past the width)
+@pytest.mark.parametrize("name", ("ragged", "tall", "many"))
+def test_products_of_many_tiles(name):
+    test_products_of_plain_matrices(name, 192, 5152)
+
+
+@pytest.mark.parametrize("name", ("ragged", "many"))
+@pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
+def test_kernel_gradients_of_many_tiles(name, out_dtype):
+    test_kernel_gradients_of_plain_rows(name, 264, 5152, out_dtype)
