@@ -38,7 +38,7 @@ static LayerWorkspace layer_workspace(const dew_moe_layer* layer, const dew_moe_
     at += (static_cast<size_t>(bytes) + 255) / 256 * 256;
     return here;
   };
-  w.logits = take(tokens * layer->router.experts * 4 * (tokens <= kShareTokens ? kLogitShares : 1));
+  w.logits = take(tokens * layer->router.experts * 4 * (logit_shares(static_cast<int>(tokens), gate->depth, layer->router.experts) ? kLogitShares : 1));
   w.weights = take(slots * 4);
   w.indices = take(slots * 4);
   w.sizes = take(groups * 4);
@@ -115,9 +115,9 @@ extern "C" int dew_moe_layer_forward(const dew_moe_layer* layer, const void* x, 
   float* logits = reinterpret_cast<float*>(base + w.logits);
   float* weights = reinterpret_cast<float*>(base + w.weights);
   int32_t *indices = words(w.indices), *sizes = words(w.sizes), *offsets = words(w.offsets), *order = words(w.order), *gather = words(w.rows);
-  // a decode step's gate leaves its logits in shares, which spread over more CUs and which its router adds up
+  // a decode step's or a short prompt's gate leaves its logits in shares, which spread over more CUs and which its router adds up
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const bool in_shares = tokens <= kShareTokens && gate->depth % 16 == 0 && aligned16(x);
+  const bool in_shares = logit_shares(tokens, gate->depth, experts) != kNoShares && aligned16(x);
   if (int rc = in_shares ? router_logit_shares(x, gate_kernel, logits, tokens, gate->depth, experts, s)
                          : dew_moe_router_logits(x, gate_kernel, gate_bias, logits, tokens, gate->depth, experts, stream))
     return rc;

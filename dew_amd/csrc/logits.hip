@@ -201,7 +201,67 @@ __global__ __launch_bounds__(64) void router_logit_shares_kernel(const bf16_t* _
   }
 }
 
+// The shares of router_logits_mfma_kernel<1, 16> the same way: 32 tokens x 32 experts of one share of the depth a wavefront, for
+// the few hundred tokens whose tiles with sixteen wavefronts each leave CUs without one. The partial sums are that kernel's and are
+// added in its order: the same bits.
+__global__ __launch_bounds__(64) void router_logit_tile_shares_kernel(const bf16_t* __restrict__ x, const float* __restrict__ kernel,
+                                                                      float* __restrict__ partial, int tokens, int depth, int experts) {
+  const int lane = threadIdx.x, t0 = blockIdx.x * 32, e0 = blockIdx.y * 32, share = blockIdx.z;
+  const int chunks = depth / 16;
+  const int first = static_cast<int>(static_cast<long long>(chunks) * share / kShares);
+  const int last = static_cast<int>(static_cast<long long>(chunks) * (share + 1) / kShares);
+  const bf16_t* a_src = x + static_cast<size_t>(min(t0 + lane % 32, tokens - 1)) * depth + 8 * (lane / 32);
+  const float* b_src = kernel + static_cast<size_t>(8 * (lane / 32)) * experts + min(e0 + lane % 32, experts - 1);
+  f32x16 acc;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
+  u32x4 words[2];
+  float b[2][8];
+  auto load = [&](int set, int chunk) __attribute__((always_inline)) {
+    words[set] = *reinterpret_cast<const u32x4*>(a_src + chunk * 16);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[set][j] = b_src[static_cast<size_t>(chunk * 16 + j) * experts];
+  };
+  auto multiply = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const uint32_t word = words[set][j / 2];
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(j % 2 ? word & 0xFFFF0000u : word << 16), b[set][j], acc, 0, 0, 0);
+    }
+  };
+  if (first < last) load(0, first);
+  for (int chunk = first; chunk < last; chunk += 2) {  // (past the share: the last chunk again, which multiplies nothing)
+    load(1, min(chunk + 1, last - 1));
+    multiply(0);
+    load(0, min(chunk + 2, last - 1));
+    if (chunk + 1 < last) multiply(1);
+  }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int t = t0 + 8 * (i / 4) + 4 * (lane / 32) + i % 4, e = e0 + lane % 32;
+    if (t < tokens && e < experts) partial[(static_cast<size_t>(share) * tokens + t) * experts + e] = acc[i];
+  }
+}
+
+// How a layer's gate leaves its logits: in shares, by 16 x 16 tiles as the fine launch's (up to kShareTokens tokens, and wherever
+// dew_moe_router_logits takes that launch) or by 32 x 32 tiles as its sixteen wavefronts', or finished. Past some hundred such tiles
+// the shares' sixteen times the bytes cost more than the idle CUs do. A layer's pass (us): 200 tokens of a 2048 x 8 gate 85.0 -> 81.4,
+// 100 of 7168 x 256 (32 tiles) 393 -> 381, 2048 of 512 x 8 (64) 52.0 -> 50.3, 1111 of 2048 x 64 (70) 134.5 -> 131.9, 1000 of 7168 x 128
+// (128) 489.5 and 490.4, 600 of 2048 x 256 (152) 284.6 and 288.
+LogitShares logit_shares(int tokens, int depth, int experts) {
+  if (depth % 16 != 0) return kNoShares;
+  if (tokens <= kShareTokens) return kFineShares;
+  const long long blocks = static_cast<long long>((tokens + 31) / 32) * ((experts + 31) / 32);
+  if (depth < 64 || tokens > 2048 || blocks >= 112) return kNoShares;
+  return blocks < 64 ? kFineShares : kTileShares;
+}
+
 int router_logit_shares(const void* x, const float* kernel, float* partial, int tokens, int depth, int experts, hipStream_t stream) {
+  if (logit_shares(tokens, depth, experts) == kTileShares) {
+    hipLaunchKernelGGL(router_logit_tile_shares_kernel, dim3((tokens + 31) / 32, (experts + 31) / 32, kShares), dim3(64), 0, stream,
+                       static_cast<const bf16_t*>(x), kernel, partial, tokens, depth, experts);
+    return launched("router_logit_tile_shares_kernel");
+  }
   hipLaunchKernelGGL(router_logit_shares_kernel, dim3((tokens + 15) / 16, (experts + 15) / 16, kShares), dim3(64), 0, stream,
                      static_cast<const bf16_t*>(x), kernel, partial, tokens, depth, experts);
   return launched("router_logit_shares_kernel");

@@ -140,11 +140,13 @@ __device__ __forceinline__ void sort_small(const PermuteParams& p, int32_t* runn
 }
 
 // A decode step's gate and dispatch (layer.hip): the gate's logits as kLogitShares partial sums of the depth,
-// [share][token][expert] (logits.hip), for at most kShareTokens tokens; a router that adds them (route.hip); and, for at most
+// [share][token][expert] (logits.hip), where logit_shares says so; a router that adds them (route.hip); and, for at most
 // kRouteAndSortTokens tokens, that router and the sort as one launch.
 constexpr int kLogitShares = 16;
 constexpr int kShareTokens = 64;
 constexpr int kRouteAndSortTokens = 16;
+enum LogitShares { kNoShares = 0, kFineShares = 1, kTileShares = 2 };
+LogitShares logit_shares(int tokens, int depth, int experts);
 int router_logit_shares(const void* x, const float* kernel, float* partial, int tokens, int depth, int experts, hipStream_t stream);
 int route_shares(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
                  float* weights, int32_t* indices, hipStream_t stream);

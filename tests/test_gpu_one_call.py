@@ -20,6 +20,11 @@ CASES = {
                                             expert_groups=8, groups_per_token=4, expert_bias=True, shared=256),
     "groups, bias, shared, 65 tokens": dict(tokens=65, experts=64, top_k=8, quant="fp8_block", score_function="sigmoid",
                                             expert_groups=8, groups_per_token=4, expert_bias=True, shared=256),
+    # the gate's shares by tiles: 105 of 32 x 32, neither extent whole; and one tile short of, at and past the lines at 64 and 112
+    "shares by tiles": dict(tokens=1111, experts=70, top_k=2, quant="fp8_block"),
+    "shares, 63 tiles": dict(tokens=2016, experts=32, top_k=2, quant="fp8_block"),
+    "shares, 111 tiles": dict(tokens=1184, experts=96, top_k=1, quant="fp8_block"),
+    "no shares, 112 tiles": dict(tokens=1792, experts=64, top_k=1, quant="fp8_block"),
     "300 experts": dict(tokens=64, experts=300, top_k=6, quant="fp8_block"),
 }
 DEPTH, HIDDEN = 512, 256
