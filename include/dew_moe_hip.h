@@ -425,7 +425,7 @@ int dew_moe_grouped_gemm_mxfp8_rows(const void* x_codes, const uint8_t* x_scales
  * dew_moe_kernel_gradient_mxfp8: out [groups, depth, width] (bf16, or fp32 where out_is_f32) from the lhs_t operand
  * [depth, tokens] and the rhs_t bank [width, tokens]; group g contracts tokens offsets[g] .. offsets[g + 1], whole
  * 128-token blocks (device int32 [groups + 1]); an empty group's matrix is zero. Both operands enter
- * v_mfma_scale_f32_32x32x64_f8f6f4 as stored, 256 x 256 tiles.                                                    */
+ * v_mfma_scale_f32_32x32x64_f8f6f4 as stored, 256 x 256 tiles (128 x 128 where those are few).                    */
 int dew_moe_quantize_columns_fp8(const void* x /* bf16 [tokens, dim] */, void* codes, void* scales, int32_t tokens,
                                  int32_t dim, int32_t as_bank, void* stream);
 int dew_moe_quantize_columns_mxfp8(const void* x /* bf16 [tokens, dim] */, void* codes, void* scales, int32_t tokens,
@@ -444,7 +444,8 @@ int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint8_t* lhs_t_
  * arithmetic along the tokens) and *tensor_scale written; workspace is 4 bytes of device memory.
  * dew_moe_kernel_gradient_bf16: out [groups, depth, width] (bf16, or fp32 where out_is_f32) = lhs_t[:, tokens of g] x
  * rhs_t[:, tokens of g]^T, exact products, fp32 sums, times *lhs_scale x *rhs_scale (device floats, each may be null),
- * one rounding. Group g contracts tokens offsets[g] .. offsets[g + 1], whole 64-token steps. 256 x 256 tiles.        */
+ * one rounding. Group g contracts tokens offsets[g] .. offsets[g + 1], whole 64-token steps. 256 x 256 tiles, or
+ * 128 x 128 where those are few.                                                                                     */
 int dew_moe_transpose_columns(const void* x /* bf16 [tokens, dim] */, void* out, int32_t tokens, int32_t dim,
                               int32_t as_bank, void* stream);
 /* dew_moe_transpose_groups: dew_moe_transpose_columns for ragged groups (`gemm_t`'s `group_sizes` are any sizes): x bf16
