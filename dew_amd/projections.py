@@ -1,4 +1,4 @@
-"""The blockwise FP8 recipe's projection, forward only, shaped as the reference's
+"""The blockwise FP8 recipe's projection, shaped as the reference's
 (`src/dew/nn/kernels/projections.py:50-60,96-204`: `blockwise_fp8_projection`, `recipe_projection`,
 `rows_quantized`, `blocks_quantized`; product `gemm.blockwise_fp8_product` `src/dew/nn/kernels/gemm.py:764-793`).
 
@@ -9,7 +9,7 @@ row's and its block's scale, summed in fp32, rounded once. On gfx950 both operan
 (`ops.quantize_rows_fp8`) and the product one grouped launch (`ops.grouped_gemm_fp8_rows`). A group's rows need
 no padding to whole 128-row blocks here (the launch finds its tiles from the group offsets), so
 `recipe_projection` takes ragged groups as they are; the zero rows the reference pads with add nothing there.
-The recipe's gradients (its own FP8 products of requantized operands) are not part of this package.
+The MXFP8 and NVFP4 recipes and all three recipes' gradients follow below.
 """
 
 import dataclasses
