@@ -185,9 +185,12 @@ def gemm(lhs: torch.Tensor, rhs, group_sizes, *, paired=None, gather: torch.Tens
     named = None if implementation in (None, "auto") else implementation
     selection.select(GROUPED, case, named)
     if torch.is_tensor(rhs) and paired is None and epilogue is None:   # a plain operand's product alone: read where it lies
+        if not (rhs.is_contiguous() or rhs.transpose(1, 2).is_contiguous()):
+            rhs = rhs.contiguous()
+        elif rhs.data_ptr() % 16:    # (a view into a flat buffer of parameters begins anywhere; the launch loads 16 bytes at a time)
+            rhs = rhs.clone()        # (which keeps the strides)
         groups = GroupSizes.operands(group_sizes)
-        return ops.dense_gemm(lhs, rhs if rhs.is_contiguous() or rhs.transpose(1, 2).is_contiguous() else rhs.contiguous(), groups["offsets"],
-                              gather=gather, scatter=scatter, sizes=groups.get("sizes"))
+        return ops.dense_gemm(lhs, rhs, groups["offsets"], gather=gather, scatter=scatter, sizes=groups.get("sizes"))
     first = prepared(rhs)
     if epilogue == "gpt_oss_gated":
         if scatter is not None:

@@ -75,3 +75,18 @@ def test_products_of_many_tiles(name):
 @pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
 def test_kernel_gradients_of_many_tiles(name, out_dtype):
     test_kernel_gradients_of_plain_rows(name, 264, 5152, out_dtype)
+
+
+@pytest.mark.parametrize("turned", (False, True), ids=("natural", "kmajor"))
+@pytest.mark.parametrize("offset", (1, 4))                # elements: off by two bytes, and by eight
+def test_matrices_that_begin_anywhere(offset, turned):
+    """A view into a flat buffer of parameters need not begin on 16 bytes."""
+    from dew_amd import gemm
+
+    x, w, _, sizes = inputs(SIZES["ragged"], 192, 288)
+    held = w.transpose(1, 2).contiguous() if turned else w
+    flat = torch.empty(w.numel() + 8, dtype=torch.bfloat16, device="cuda")
+    view = flat[offset:offset + w.numel()].view(held.shape)
+    view.copy_(held)
+    assert view.data_ptr() % 16 == 2 * offset and view.is_contiguous()
+    assert torch.equal(gemm.gemm(x, view.transpose(1, 2) if turned else view, sizes), gemm.gemm(x, w, sizes))
