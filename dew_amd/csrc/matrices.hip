@@ -141,12 +141,13 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
     values_of<T>(*reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch), v[p]);
 
   float tensor = 1.0f;
+  bool quick = false;  // (the same for the whole launch)
   if constexpr (kNv) {
     const float top = __uint_as_float(*largest);
     tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
+    quick = sizeof(T) == 2 && nvfp4_in_range(top, tensor);
     if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) tensor_scales[e] = tensor;
   }
-  const bool quick = kNv && sizeof(T) == 2 && nvfp4_in_range(tensor);  // (the same for the whole launch)
   const float inverse_tensor = kNv ? 1.0f / tensor : 1.0f;
   auto magnitude = [](float value) { return __float_as_uint(value) & 0x7FFFFFFFu; };
   float inverse = 1.0f;  // FP8 blocks: the tile's one

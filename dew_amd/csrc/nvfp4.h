@@ -6,15 +6,19 @@
 // multiply-adds (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000 processor", 1990): the IEEE
 // quotient. Checked for every pair that comes here: values of eight significant bits over tensor scales fl(amax / 2688) of bf16
 // amax, all 128 x 128 significands, and all 2^23 significands over the eight of e4m3. Tensor scales near the ends of fp32's range,
-// where a step's remainder could be subnormal, keep the division; so does a weight held in fp32. The conversion instruction
-// rounds as the rule does.
+// where a step's remainder could be subnormal, keep the division; so do a weight held in fp32 and every operand that holds an
+// infinity or a NaN, wherever it stands: a step from an infinity ends in inf - inf, and the conversion instruction has no code
+// for a NaN, which the comparisons read as a zero. The instruction rounds as the rule does.
 #pragma once
 
 #include "common.h"
 
 namespace dew {
 
-__device__ __forceinline__ bool nvfp4_in_range(float tensor) { return tensor >= 0x1p-80f && tensor <= 0x1p+117f; }
+// Whether an operand of this largest magnitude (a NaN where it holds one) and tensor scale takes the short form.
+__device__ __forceinline__ bool nvfp4_in_range(float largest, float tensor) {
+  return largest < __builtin_inff() && tensor >= 0x1p-80f && tensor <= 0x1p+117f;
+}
 
 // The reciprocal of a block's scale: 0 where the block has none (zeros, or a NaN), whose codes are all 0.
 __device__ __forceinline__ float nvfp4_inverse(float each) { return each > 0.0f ? 1.0f / each : 0.0f; }

@@ -172,7 +172,7 @@ __global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_nvfp4_kerne
   // largest / (6 * 448), fp32's least normal at least; 1 for an operand of zeros
   const float tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
   if (blockIdx.x == 0 && threadIdx.x == 0) *tensor_scale = tensor;
-  const bool quick = nvfp4_in_range(tensor);  // (the same for the whole launch)
+  const bool quick = nvfp4_in_range(top, tensor);  // (the same for the whole launch)
   const float inverse_tensor = 1.0f / tensor;
   const int lane = threadIdx.x % 64;
   const int row = blockIdx.x * kQuantizeWaves + threadIdx.x / 64;
@@ -363,9 +363,11 @@ __global__ __launch_bounds__(256) void transpose_columns_kernel(const bf16_t* __
   }
   __syncthreads();
   float tensor = 1.0f;
+  bool quick = false;  // (the same for the whole launch)
   if constexpr (NVFP4) {
     const float top = __uint_as_float(*largest << 16);
     tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
+    quick = nvfp4_in_range(top, tensor);
     if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *tensor_scale = tensor;
   }
 #pragma unroll
@@ -395,7 +397,7 @@ __global__ __launch_bounds__(256) void transpose_columns_kernel(const bf16_t* __
       uint32_t byte = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(ratio, 448.0f), 0.0f, 0, false) & 0xFFu;
       if (__builtin_amdgcn_cvt_f32_fp8(byte, 0) < ratio) byte = min(byte + 1u, 0x7Eu);
       const float each = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
-      if (nvfp4_in_range(tensor)) {
+      if (quick) {
         const Nvfp4Scales by{tensor, 1.0f / tensor, each, nvfp4_inverse(each)};
 #pragma unroll
         for (int i = 0; i < 16; i += 2) {

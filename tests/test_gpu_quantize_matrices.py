@@ -105,3 +105,31 @@ def test_every_significand_against_every_tensor_scale(ops, exponent):
             assert scale.item() == want.keep[2][0].item() and torch.equal(rows.float(), decoded)
             columns, scale = ops.transpose_columns(x.t().contiguous(), nvfp4=True, as_bank=False)
             assert scale.item() == want.keep[2][0].item() and torch.equal(columns.float(), decoded)
+
+
+def test_nans_and_infinities_among_nvfp4_operands(ops):
+    """An operand that holds a NaN has the tensor scale 1. In the rows' and columns' blocks the NaN itself reads as a zero and the rest
+    as ever, an infinity as the block's largest code under the largest scale; a block of matrices with a NaN has no scale."""
+    from dew_amd import codecs
+
+    nan, inf, e2m1 = float("nan"), float("inf"), torch.tensor([0, 0.5, 1, 1.5, 2, 3, 4, 6, -0.0, -0.5, -1, -1.5, -2, -3, -4, -6], device="cuda")
+    generator = torch.Generator(device="cuda").manual_seed(11)
+    x = torch.randn((128, 256), generator=generator, device="cuda").to(torch.bfloat16)
+    x[0, 160], x[5, 16:32], x[7, 3], x[7, 4], x[9, 40], x[11, 50] = nan, nan, inf, nan, -inf, inf
+    finite = torch.where(x.isnan(), 0.0, x.float()).clamp(-1e30, 1e30)
+    blocks = finite.reshape(-1, 16).t()                                            # the rule on finite values, under the scale 1
+    ratio = blocks.abs().amax(dim=0) / 6
+    nearest = codecs.e4m3_bytes(ratio.clamp(max=448.0)).to(torch.int32)
+    each = codecs.e4m3_values(torch.where(codecs.e4m3_values(nearest.to(torch.uint8)) < ratio, (nearest + 1).clamp(max=0x7E), nearest).to(torch.uint8))
+    codes = codecs._e2m1_rne(torch.where(each > 0, blocks / torch.where(each > 0, each, 1.0), 0.0))
+    want = (e2m1[codes.long()] * each).t().reshape(x.shape)
+    rows, scale = ops.quantize_rows_nvfp4(x)
+    assert scale.item() == 1.0 and torch.equal(rows.float(), want)
+    columns, scale = ops.transpose_columns(x.t().contiguous(), nvfp4=True, as_bank=False)
+    assert scale.item() == 1.0 and torch.equal(columns.float(), want)
+    w = x.t()[None]
+    prepared = ops.prepare(by_whole_tensors("nvfp4", w))
+    compared = x.numel() // 2 + x.numel() // 16
+    for held in (w, w.contiguous()):
+        got = ops.quantize_matrices(held, "nvfp4")
+        assert torch.equal(got.keep[0][:compared], prepared.keep[0][:compared]) and torch.equal(got.keep[2], prepared.keep[2])
