@@ -95,7 +95,10 @@ class GptOssMLP(_Module):
 
     @functools.cached_property
     def _one_call(self):
-        """The layer's fixed part for `layer_call.forward`, or None where its options are not among those the one call covers."""
+        """The layer's fixed part for `layer_call.forward`, or None where its options are not among those the one call covers, or its
+        class overrides what that call computes."""
+        if not layer_call.computes(self, GptOssMLP, ("__call__", "_bound", "logits", "experts")):
+            return None
         if self.implementation != "auto" or self.dispatch not in ("auto", "global") or self.capacity_factor is not None or self.dtype not in (
                 None, torch.bfloat16):
             return None

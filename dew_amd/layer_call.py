@@ -17,6 +17,12 @@ def described(router: _lib.Router, gating: int, limit: float, shared: bool) -> _
     return _lib.Layer(router, gating, limit, int(shared))
 
 
+def computes(layer, of: type, names: tuple) -> bool:
+    """Whether `layer` computes with `of`'s own methods and properties `names`, the ones that the call stands for: a subclass that
+    overrides one of them is run through it."""
+    return all(getattr(type(layer), name) is getattr(of, name) for name in names)
+
+
 def _parameter(tensor, shape: tuple) -> bool:
     return (torch.is_tensor(tensor) and tensor.is_cuda and tensor.dtype == torch.float32 and tensor.is_contiguous()
             and tuple(tensor.shape) == shape)

@@ -525,7 +525,10 @@ class SparseMLP(_Module):
 
     @functools.cached_property
     def _one_call(self):
-        """The layer's fixed part for `layer_call.forward`, or None where its options are not among those the one call covers."""
+        """The layer's fixed part for `layer_call.forward`, or None where its options are not among those the one call covers, or its
+        class overrides what that call computes."""
+        if not layer_call.computes(self, SparseMLP, ("__call__", "_bound", "gate", "experts", "shared_experts")):
+            return None
         plain = (self.activation in ops.GATES and self.implementation == "auto" and self.dispatch in ("auto", "global")
                  and self.dtype in (None, torch.bfloat16) and self.fused and self.capacity_factor is None and not self.shared_gate
                  and self.latent_features is None and not self.scale_inputs and self.hash_vocab is None and not self.media_bias
