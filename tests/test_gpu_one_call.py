@@ -62,7 +62,12 @@ def test_one_call_returns_the_separate_calls_bits(name):
     assert got is not None and torch.equal(got, want) and bool(got.any())
     shaped = x[None].expand(2, -1, -1)                                     # (not contiguous: the separate calls answer)
     assert layer._applied(variables, shaped) is None
-    assert torch.equal(layer.apply(variables, shaped), torch.stack((want, want))) or tokens * top_k // experts > 12   # (tile heights differ)
+    separate = layer._bound(variables, ())
+    assert torch.equal(layer.apply(variables, shaped), separate(torch.stack((x, x))))
+    # twice the tokens take other tiles, which sum alike: the same bits from the same logits (whose own sums' order, in the gate, goes by
+    # the number of tokens)
+    logits = separate.gate.logits(x)
+    assert torch.equal(layer.apply(variables, shaped, logits=torch.stack((logits, logits))), torch.stack((want, want)))
 
 
 @pytest.mark.parametrize("tokens", (1, 24, 700))
