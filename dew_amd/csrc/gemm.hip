@@ -1175,8 +1175,8 @@ static int launch_tile(const char* who, GemmParams p, hipStream_t stream) {
 // 64-row tiles are 15 to 25 % faster), 64-row tiles up to 72 rows on FP8 banks and up to 384 on the cheap ones.
 // (NVFP4 banks take them from 129 to 184 rows too, where three cover what two 128-row tiles would. FP8 banks did: 5 to 10 % faster on
 // sizes an eighth around their mean, but where a gate's preferences spread the sizes by half and more, 128-row tiles are the
-// faster ones there: 32 experts x 138 rows of 1792 x 2816 paired 160 -> 144 us, 16 x 173 of 3328 x 1152 60 -> 50, 128 x 169 of
-// 1664 x 1024 in one bank 120 -> 103; the few worse shapes lose up to 7 %.)
+// faster ones there: 32 experts x 138 rows of 1792 x 2816 paired 156 -> 141 us, 128 x 169 of 1664 x 1024 in one bank
+// 124 -> 105; the few worse shapes, 16 x 173 of 3328 x 2304 paired, 128 -> 132, lose up to 7 %.)
 // Occupancy: a launch of fewer tiles than CUs halves its tile until there are enough (8 experts x 512 rows x 512
 // columns: 144 tiles of 128 rows take 16.5 us, 272 tiles of 64 rows 11.7 us). 256-row tiles, which fill every
 // accumulator register, are kept to the cheap banks and to groups of 2048 rows or more. Decode-sized groups take the
@@ -1191,8 +1191,11 @@ static int tile_rows(const GemmParams& p, bool cheap, int format, bool paired) {
   // pipe waits for them, so that padding costs little. One bank: 128 rows from groups of 76 rows on, wherever that leaves 160
   // blocks (16 experts x 77 rows of 3328 x 3072: 83 us in 64-row tiles, 72 in 128; 32 x 345 of 2304 x 1920: 161 -> 133; at 108
   // blocks or on groups of 59 rows 20 to 50 % slower). A paired launch's 128-row block is alone on its CU, so it wants a depth
-  // that its start and end are small beside and several rounds of blocks (16 x 135 rows of 3456 x 3328: 217 -> 192 us, 64 x 291
-  // of 2304 x 1792: 446 -> 411; at 1.5 rounds or 1152 depths 5 to 25 % slower, 32 x 416 of 256 x 3200 15 %). Nor are 64-row tiles halved before they are very
+  // that its start and end are small beside and several rounds of blocks (64 x 291 rows of 2304 x 1792, 2478 blocks: 451 -> 413 us,
+  // 16 x 150 of 3456 x 3328, 676: 210 -> 195, 32 x 120 of 2560 x 2048, 736: 177 -> 162; at the line, 32 x 97 of 2048 x 2048, 130
+  // either way; at 1.5 rounds or 1152 depths 5 to 25 % slower, 32 x 416 of 256 x 3200 15 %. A line by blocks alone leaves out
+  // deep products just below it: 16 x 135 of 3456 x 3328, 624 blocks, 213 us in 64-row tiles and 196 in 128, 8 x 200 of 4096 x
+  // 4096, 512 blocks, 189 and 170). Nor are 64-row tiles halved before they are very
   // few: 8 x 57 rows of 3328 x 2176 in one bank 48 us in 32-row tiles and 32 in 64, 16 x 409 of 3200 x 256 paired 71 and 31,
   // 8 x 45 of 896 x 768 paired 9 (a wavefront a strip: few_tiles) and 18.
   const long long blocks = (p.rows / 128 + p.experts / 2) * static_cast<long long>(p.width / 128);
@@ -1215,11 +1218,14 @@ static int tile_rows(const GemmParams& p, bool cheap, int format, bool paired) {
 }
 
 // Whether 32-row tiles run as a wavefront a strip of 32 columns (decode.hip) rather than a block of four over 128. Counted in
-// blocks of the latter: up to one a CU the finer launch is the faster one (128 experts of 2048 x 768 in FP8, one token: 48
-// blocks, 21.7 -> 13.1 us, down product 10.6 -> 5.9; eight tokens, 306 blocks: 37.9 -> 36.6 and 21.3 -> 22.4; at 1500 blocks 5 to
-// 20 % slower), on unquantized banks, whose every 32 columns are twice the bytes, up to two (64 experts of 2048 x 1408, eight
-// tokens: 73 -> 69 us). It reads a tile's rows again for every 32 columns: tiles of more than some 12 rows take it only
-// where they are under a hundred blocks (8 experts of 1024 x 512, bf16, 384 rows: 17.2 -> 8.7 us; at 160 blocks no faster).
+// blocks of the latter, as many as the host cannot rule out (each row on an expert of its own): up to one a CU the finer launch
+// is the faster one (us, 128 experts of 2048 x 768 in FP8, top 8: one token, 48 blocks, 21.5 -> 13.6, its down product, 128,
+// 11.2 -> 6.7; five, 240 blocks, 24.6 -> 20.4; the down product at 512 blocks 12.9 either way, the paired at 576 38.5 and 38.9),
+// on unquantized banks, whose every 32 columns are twice the bytes, up to two (64 experts of 2048 x 1408, top 6: four tokens,
+// 264 blocks, 46.0 -> 39.1, seven, 462 blocks, 67.7 -> 54.5). Some launches past the lines would gain too: FP8 paired at 288 and
+// 384 blocks 25.2 -> 23.3 and 34.1 -> 30.5, bf16 paired at 528 and 704 70.3 -> 58.0 and 78.0 -> 68.9. It reads a tile's rows
+// again for every 32 columns: tiles of more than some 12 rows take it only where they are under a hundred blocks (8 experts of
+// 1024 x 512, bf16, 384 rows: 17.2 -> 8.7 us; at 160 blocks no faster).
 static bool few_tiles(const GemmParams& p, bool unquantized) {
   const long long touched = p.rows < p.experts ? p.rows : p.experts, spread = p.rows / 32 + touched / 2;
   const long long blocks = (touched > spread ? touched : spread) * ((p.width + 127) / 128);
