@@ -13,7 +13,10 @@ the dominant kernel alone (the paired gate/up launch: two thirds of the FLOPs), 
 the launch stream around every one of its launches in the timed region. `cpu_baseline` is the CPU oracle on a
 bounded sample of the same workload, on this box's host cores. `configs` holds the same measurement for each of
 the five workloads c1 .. c5 (step time, the dominant kernel against its roofline, parity of a full-size sample
-against the CPU oracle, and the least top-k margin of the routing); `--only` leaves it out.
+against the CPU oracle, and the least top-k margin of the routing) but the one at the top level; `--only` leaves it out.
+
+The line holds figures, some six thousand characters of them, so that whoever keeps only the end of the output keeps all of it;
+`--full PATH` writes the record with its notes, and the narrower formats' fractions of every workload, to a file.
 """
 
 import argparse
@@ -38,6 +41,27 @@ GRAPHED = ("c1", "c3")
 """The launch-bound workloads: their step is replayed as one captured HIP graph."""
 DECODE = ("c3",)
 """The workloads whose dominant kernel is bound by HBM bandwidth, not by the matrix cores."""
+
+
+NOTE_KEYS = ("note", "peak_note", "issue_time_note", "rows_note", "traffic_source")
+TOP_ONLY = ("kernel", "algorithmic_flops", "hbm_view", "frac_of_fp8_peak", "frac_of_fp4_peak", "executed", "algorithmic", "sustained", "bar",
+            "launch", "routed_rows", "fp32_spacings", "token")
+"""What the line's `configs` leave out beside the notes: it is the top level's too, or follows from what they hold."""
+
+
+def figures(record, without=NOTE_KEYS):
+    """A measurement's figures: the record without the keys `without`, at any depth."""
+    if isinstance(record, dict):
+        return {key: figures(value, without) for key, value in record.items() if key not in without}
+    return record
+
+
+def line(result, config):
+    """The one line that is printed of a run whose top level is `config`."""
+    printed = figures({key: value for key, value in result.items() if key != "configs"})
+    if "configs" in result:
+        printed["configs"] = {name: figures(measured, NOTE_KEYS + TOP_ONLY) for name, measured in result["configs"].items() if name != config}
+    return json.dumps(printed)
 
 
 def build_workload(case, device, seed=0):
@@ -536,6 +560,7 @@ def main():
                              "of as group #E of the routed launches")
     parser.add_argument("--graph", choices=["auto", "on", "off"], default="auto",
                         help="replay the step as one captured HIP graph (auto: for the launch-bound configs c1 and c3)")
+    parser.add_argument("--full", type=Path, default=None, help="also write the whole record, with its notes, to this file")
     args = parser.parse_args()
     if args.gpus != 1:
         sys.exit("bench.py measures one GPU: this build has no multi-GPU path (the path would shard by expert over "
@@ -586,7 +611,9 @@ def main():
                 finally:
                     gemm.SPLIT_SECOND_TERM = held
         result["configs"] = per_config
-    print(json.dumps(result))
+    if args.full is not None:
+        args.full.write_text(json.dumps(result, indent=1) + "\n")
+    print(line(result, args.config))
 
 
 if __name__ == "__main__":
