@@ -1,10 +1,10 @@
 """Times the training recipes' products on synthetic operands of a model's expert shapes: for the blockwise FP8, MXFP8
 and NVFP4 recipes and for plain bf16 matrices, the forward product, the input's gradient and the matrices' gradient
-(each with the passes that quantize or transpose its operands timed beside it). One JSON line a product.
+(each with the passes that quantize its operands timed beside it). One JSON line a product.
 
     python bench_recipes.py [--shape mixtral|deepseek] [--steps 5]
 
-`tflops` counts 2 x rows x depth x width for the product alone; `prepare_us` is the operands' quantizing / transposing
+`tflops` counts 2 x rows x depth x width for the product alone; `prepare_us` is the operands' quantizing
 passes of that product (the matrices' own quantization, done once a step for all three products, is not timed)."""
 
 import argparse
@@ -37,13 +37,9 @@ def products(recipe: str, x, w, dy, blocks, offsets):
     """(name, prepare call, product call) for the recipe's three products, operands prepared once outside the timing."""
     sizes = offsets[1:] - offsets[:-1]
     if recipe == "bf16":
-        bank, bank_t = ops.prepare(formats.Bf16(w)), ops.prepare(formats.Bf16(w).T)
-        rows_t, _ = ops.transpose_columns(x, as_bank=False)
-        dy_bank, _ = ops.transpose_columns(dy, as_bank=True)
-        return [("forward", None, lambda: ops.grouped_gemm(x, bank, offsets)),
-                ("d_x", None, lambda: ops.grouped_gemm(dy, bank_t, offsets)),
-                ("d_w", lambda: (ops.transpose_columns(x, as_bank=False), ops.transpose_columns(dy, as_bank=True)),
-                 lambda: ops.kernel_gradient_bf16(rows_t, dy_bank, offsets))]
+        return [("forward", None, lambda: ops.dense_gemm(x, w, offsets)),      # (every operand read where it lies)
+                ("d_x", None, lambda: ops.dense_gemm(dy, w.transpose(1, 2), offsets)),
+                ("d_w", None, lambda: ops.dense_gradient(x, dy, offsets))]
     if recipe == "nvfp4":
         bank, bank_t = projections.nvfp4_matrices(w), projections.nvfp4_matrices(w.transpose(1, 2).contiguous())
         rows, cotangents = projections.nvfp4_rows(x), projections.nvfp4_rows(dy)

@@ -448,7 +448,8 @@ int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint8_t* lhs_t_
  * 128 x 128 where those are few.                                                                                     */
 int dew_moe_transpose_columns(const void* x /* bf16 [tokens, dim] */, void* out, int32_t tokens, int32_t dim,
                               int32_t as_bank, void* stream);
-/* dew_moe_transpose_groups: dew_moe_transpose_columns for ragged groups (`gemm_t`'s `group_sizes` are any sizes): x bf16
+/* dew_moe_transpose_groups: dew_moe_transpose_columns for ragged groups, for a caller that holds its operands transposed (one
+ * that does not reads them where they lie: dew_moe_dense_gradient, which takes groups of any sizes): x bf16
  * [rows, dim], group g its rows offsets[g] .. offsets[g + 1] (device int32 [groups + 1]); each group is written from a
  * whole 64-token step on and its last step filled with zeros, into padded_tokens tokens (whole 128s, at least rows +
  * 64 * groups; the rest zeros); padded_offsets [groups + 1] receives the groups' offsets in the written order, which
