@@ -90,3 +90,22 @@ def test_matrices_that_begin_anywhere(offset, turned):
     view.copy_(held)
     assert view.data_ptr() % 16 == 2 * offset and view.is_contiguous()
     assert torch.equal(gemm.gemm(x, view.transpose(1, 2) if turned else view, sizes), gemm.gemm(x, w, sizes))
+
+
+# (groups, rows a group, depth, width, turned): on the lines from which the matrices are laid out first, and just short of each
+LINES = [(1, 8192, 2048, 1536, False), (1, 8191, 2048, 1536, False), (1, 4096, 2048, 3072, True), (1, 4095, 2048, 3072, True), (1, 4096, 1984, 3072, True),
+         (2, 3000, 4096, 2048, True), (2, 2999, 4096, 2048, True), (2, 3000, 4096, 1920, True), (1, 8192, 2048, 1312, False), (1, 8192, 2048, 1568, True)]
+
+
+@pytest.mark.parametrize("groups,rows,depth,width,turned", LINES)
+def test_matrices_laid_out_first_return_the_same_bits(groups, rows, depth, width, turned):
+    from dew_amd import gemm, ops
+
+    x, w, _, sizes = inputs([rows + 5 * (1 - 2 * (g % 2)) * (groups > 1) for g in range(groups)], depth, width, extra=0)
+    if turned:
+        w = w.transpose(1, 2).contiguous().transpose(1, 2)
+    average, tiles = rows, (groups * rows // 128 + groups // 2 + 1) * -(-width // 256)
+    laid = tiles >= 384 and depth >= 2048 and average >= (8192 if not turned else 3000 if depth >= 4096 else 4096) and (not turned or width % 128 == 0)
+    assert gemm._relaid_first(w, x.shape[0]) == laid
+    scatter = torch.randperm(x.shape[0], device="cuda").to(torch.int32)
+    assert torch.equal(gemm.gemm(x, w, sizes, scatter=scatter), ops.dense_gemm(x, w, ops.group_offsets(sizes), scatter=scatter))
