@@ -37,9 +37,9 @@ def products(recipe: str, x, w, dy, blocks, offsets):
     """(name, prepare call, product call) for the recipe's three products, operands prepared once outside the timing."""
     sizes = offsets[1:] - offsets[:-1]
     if recipe == "bf16":
-        return [("forward", None, lambda: ops.dense_gemm(x, w, offsets)),      # (every operand read where it lies)
-                ("d_x", None, lambda: ops.dense_gemm(dy, w.transpose(1, 2), offsets)),
-                ("d_w", None, lambda: ops.dense_gradient(x, dy, offsets))]
+        return [("forward", None, lambda: gemm.gemm(x, w, sizes)),      # (whatever their matrices' way to the launch is)
+                ("d_x", None, lambda: gemm.gemm(dy, w.transpose(1, 2), sizes)),
+                ("d_w", None, lambda: gemm.gemm_t(x, dy, sizes))]
     if recipe == "nvfp4":
         bank, bank_t = projections.nvfp4_matrices(w), projections.nvfp4_matrices(w.transpose(1, 2).contiguous())
         rows, cotangents = projections.nvfp4_rows(x), projections.nvfp4_rows(dy)
