@@ -7,8 +7,8 @@
 // quotient. Checked for every pair that comes here: values of eight significant bits over tensor scales fl(amax / 2688) of bf16
 // amax, all 128 x 128 significands, and all 2^23 significands over the eight of e4m3. Tensor scales near the ends of fp32's range,
 // where a step's remainder could be subnormal, keep the division; so do a weight held in fp32 and every operand that holds an
-// infinity or a NaN, wherever it stands: a step from an infinity ends in inf - inf, and the conversion instruction has no code
-// for a NaN, which the comparisons read as a zero. The instruction rounds as the rule does.
+// infinity or a NaN, wherever it stands: the conversion instruction makes a NaN the largest code, where the comparisons read a
+// zero, and a step from an infinity ends in inf - inf, a NaN. The instruction rounds as the rule does.
 #pragma once
 
 #include "common.h"
