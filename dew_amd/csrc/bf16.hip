@@ -13,26 +13,20 @@
 // three stages (24 KB each at BM = 128, so that two blocks share a CU and one's start and end run under the other's loop; a
 // contraction of a few hundred rows, a kernel gradient's, is otherwise half start and end), one barrier a step, wavefronts side
 // by side along the columns; where such tiles are few, smaller ones. Sums are taken along the contraction in the tiled launch's order: the same bits.
-// From groups of some thousands of rows on the weights' pass is the smaller price: an operand whose rows run along the contraction
+// Launches that fill the chip with 256 x 256 tiles take those (wide.hip); rows that are gathered or scattered stay here. For them, from
+// groups of some thousands of rows on, the weights' pass is the smaller price: an operand whose rows run along the contraction
 // gives a step 64 bytes of each of its cache lines, so that K-major matrices cost 10 to 17 % more than natural ones, and the tiled
 // launch's 256-row tiles fetch half as much. The caller (gemm.py, with the sizes measured) brings such matrices to order first.
+#include <math.h>
+
 #include <mutex>
 
+#include "dense.h"
 #include "gemm.h"
 
 namespace dew {
 
 constexpr int kDepthStep = 32, kRing = 3, kBlock = 256;
-
-struct DenseParams {
-  const bf16_t* a;  // [rows, inner] (gathered), or, contracted over groups of rows, [rows, outer_m]
-  const bf16_t* b;  // [groups, inner, outer_n], or [groups, outer_n, inner], or [rows, outer_n]
-  const int32_t *gather, *scatter;
-  const int32_t *offsets, *sizes;  // the groups of rows: their exclusive prefix [groups + 1], or their sizes
-  void* out;
-  const float *factor0, *factor1;  // a kernel gradient's sums times *factor0 * *factor1 (each may be null)
-  int groups, rows, inner, outer_m, outer_n, m_tiles, group_m;
-};
 
 __device__ const u32x4_t zero_rows[1] = {u32x4_t{0, 0, 0, 0}};  // what a step reads past a group's last row
 
@@ -360,6 +354,33 @@ static bool few_tiles(int rows, int groups, int width) {  // about so many of 12
   return (rows / 128 + groups / 2 + 1) * static_cast<long long>((width + 255) / 256) <= kFewTiles;
 }
 
+// Whether about `tiles` 256 x 256 tiles keep `percent` of the 256 CUs busy over the rounds they take (one tile a CU and round; groups
+// end where they end, so that a round's last few tiles may not be there).
+static bool fills_rounds(double tiles, int percent) {
+  const double rounds = tiles <= 264 ? 1 : ceil(tiles / 256 - 0.03);
+  return tiles * 100 >= rounds * 256 * percent;
+}
+
+static bool wide_extents(int groups, int a, int b) { return groups <= kWideGroups && a <= (1 << 20) && b <= (1 << 20); }  // (offsets within a tile are 32-bit)
+
+// 256 x 256 tiles (wide.hip) where they fill the CUs over the rounds that they take, on groups of at least about half a tile's rows.
+// Measured against the tiles below on 105 shapes (512 to 65 536 rows, 1 to 60 groups, extents 512 to 14 336; us, there and here):
+// 14 134 rows of 15 x 2048 x 1024 65.7 and 57.0, 32 768 of 8 x 4096 x 4096 992 and 886, 24 000 of 8 x 7168 x 7168 2203 and 1918; at
+// rounds filled to 0.56 .. 0.74 between 0.93 and 1.07 times as fast, under half 0.4 to 0.75 times; groups of 64 to 97 rows 0.82 to 0.98
+// times. K-major matrices, which the tiles below read half a cache line at a step, gain from 0.55 on: 4807 of 7 x 2688 x 3968 as its
+// input's gradient at 0.96 1.37 times, 1981 of 1 x 5120 x 10 240 at 0.64 1.33, 9569 of 4 x 1920 x 1792 at 0.62 1.10.
+static bool wide_product(int rows, int groups, int depth, int width, bool kmajor) {
+  const double tiles = (rows / 256.0 + groups / 2.0) * ((width + 255) / 256);
+  return wide_extents(groups, depth, width) && rows / groups >= 112 && fills_rounds(tiles, kmajor ? 55 : 75);
+}
+
+// A kernel's gradient, whose tiles are whole: 27 097 rows of 10 x 5376 x 768 at rounds filled to 0.82 243 and 213, 28 140 of 10 x 4352 x
+// 3200 782 and 657; groups of fewer than 256 rows, four steps, are all start and end either way (0.91 to 1.18 times as fast).
+static bool wide_gradient(int rows, int groups, int depth, int width) {
+  const double tiles = static_cast<double>(groups) * ((depth + 255) / 256) * ((width + 255) / 256);
+  return wide_extents(groups, depth, width) && rows / groups >= 256 && fills_rounds(tiles, 75);
+}
+
 }  // namespace dew
 
 extern "C" int dew_moe_dense_gemm(const void* x, const int32_t* gather, const int32_t* offsets, const int32_t* group_sizes, const void* w,
@@ -386,6 +407,7 @@ extern "C" int dew_moe_dense_gemm(const void* x, const int32_t* gather, const in
   p.inner = depth;
   p.outer_n = width;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (!gather && !scatter && wide_product(rows, groups, depth, width, kmajor != 0)) return launch_wide(who, p, false, kmajor != 0, false, s);
   // Where 128 x 256 tiles would leave half of the chip idle, a quarter of one each: a block's walk down the contraction is what the
   // launch takes then (us: 640 rows of 4 x 1024 x 2048 22 -> 14 and its input's gradient 38 -> 22, 1000 of 8 x 3072 x 1024 57 -> 31, 3000
   // of 8 x 2048 x 1024, 112 tiles, 42 -> 32; at 160 to 220 tiles 3 to 30 % slower).
@@ -418,6 +440,7 @@ extern "C" int dew_moe_dense_gradient(const void* lhs, const void* rhs, const in
   p.outer_m = depth;
   p.outer_n = width;
   const hipStream_t s = static_cast<hipStream_t>(stream);
+  if (wide_gradient(rows, groups, depth, width)) return launch_wide(who, p, true, false, out_is_f32 != 0, s);
   // (few tiles: half as wide, 4 groups of 4096 rows, 1024 x 1024, 128 tiles, 96 -> 77 us; 3333 rows, 2 x 640 x 4096, 39 -> 34; at 512
   // tiles 8 to 10 % slower)
   if (static_cast<long long>(groups) * ((depth + 127) / 128) * ((width + 255) / 256) <= 2 * kFewTiles)

@@ -1,0 +1,460 @@
+// Grouped products of plain bf16 operands in 256 x 256 tiles: the operands and results of bf16.hip, in rows as they lie, with the same
+// bits (the sums run along the contraction in the same order).
+//
+// A 128 x 256 tile of 32-deep steps asks its CU for 48 bytes a clock at the matrix pipe's rate and the L1 gives 64 at best: those launches
+// ran the pipe 38 to 43 % busy. Here a step is 64 KB for 2048 cycles of the pipe, 32 a clock, and whole cache lines either way round.
+//  * 256 blocks of 4 wavefronts, one a CU, that stay and take tile after tile: the loads run on into the next tile while one leaves.
+//    2 x 2 wavefronts of 128 x 128, their 256 sums a lane in the accumulation registers: 8 fragments read from the LDS for 16 matrix
+//    instructions (8 wavefronts of 128 x 64 read half as much again, and were 5 to 10 % slower).
+//  * All 160 KB of the LDS: a ring of three stages of the first operand and two of the second, so that of a step's sixteen loads a
+//    wavefront one goes out every fourth matrix instruction. In bursts they filled the L1's queue, and the wavefront behind them
+//    stopped: 16 384 x 4096 x 4096 515 us against 409.
+//  * Loads through a buffer descriptor a step, whose end is the tile's last row (a gradient's: the group's): what lies past it arrives as
+//    zeros, without a compare a lane.
+//  * Everything between two matrix instructions is placed by hand (`phase`): one wavefront a SIMD issues an instruction every four
+//    cycles, eight a matrix instruction, and what stood between the phases was time the pipe lost.
+//  * The operands enter the instruction the other way round, so that a lane holds four neighbouring columns of a row; two exchanges
+//    between lane groups make them 64 bytes a row, and the tile leaves from registers, without the LDS and without a barrier.
+//
+// us, in 128 x 256 tiles and here: 16 384 x 4096 x 4096 forward 468 and 409 (1.34 PFLOP/s; the pipe 74 % busy at 1.66 GHz, the power
+// limit, without the loads 1.62), input's gradient 534 and 395, kernel's gradient 491 and 393; 10 007 rows of 16 x 2048 x 4096 223
+// and 161, 230 and 190 (1.5 rounds of tiles), 216 and 191 (268 MB written).
+#include <mutex>
+
+#include "dense.h"
+#include "gemm.h"
+
+namespace dew {
+
+constexpr int kWideThreads = 256, kWideTile = 256, kWideStep = 64;
+constexpr int kWideLoads = 8;                                      // 1 KiB loads of each operand that a wavefront makes a step
+constexpr int kOperandBytes = kWideTile * kWideStep * 2;           // 32 KB: one operand's stage
+constexpr int kFirstStages = 3, kSecondStages = 2;                 // of the first operand's ring and the second's
+constexpr int kWideShared = (kFirstStages + kSecondStages) * kOperandBytes;  // all of the LDS
+
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// One operand as it is staged. kAcross false: 256 rows of 64 depths (128 bytes, chunk index xor-swizzled as in the tiled launch);
+// kAcross true: 64 rows of 256 columns in units of 32 columns (64 bytes) whose index is xor-ed with the row mod 4.
+template <bool kAcross>
+struct WideOperand {
+  static __device__ __forceinline__ int row(int load, int lane) { return kAcross ? 2 * load + lane / 32 : 8 * load + lane / 8; }
+  static __device__ __forceinline__ int chunk(int row, int lane) {  // the 16 bytes of the row that the lane fetches
+    if (kAcross) return ((lane % 32 / 4) ^ (row & 3)) * 4 + lane % 4;
+    return (lane % 8) ^ (((row >> 1) & 7) ^ ((row & 1) << 2));
+  }
+  // Address `which` of a lane: of slice `which` (rows along the contraction; the tiles are then constants apart), or of tile
+  // `which` (across; the slices are).
+  static __device__ __forceinline__ uint32_t address(uint32_t base, int first_tile, int which, int lane) {
+    if (kAcross) {
+      const int piece = lane % 16;
+      return base + (8 * (lane / 32) + piece / 4) * 512 + (((first_tile + which) ^ (piece / 4)) * 64) + (lane / 16 % 2) * 32 + (piece % 4) * 8;
+    }
+    const int row = 32 * first_tile + lane % 32;
+    return base + row * 128 + (((2 * which + lane / 32) ^ (((row >> 1) & 7) ^ ((row & 1) << 2))) * 16);
+  }
+};
+
+// (Written out: the compiler takes any LDS-DMA load in flight for a write these reads may depend on, and would drain the
+// memory pipeline in front of them. What they return is used behind an explicit wait: `arrived`.)
+template <bool kAcross, int kSlice, int kTile>
+__device__ __forceinline__ bf16x8_t wide_fragment(const uint32_t (&at)[4]) {
+  if constexpr (kAcross) {
+    u32x2_t low, high;
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(low) : "v"(at[kTile]), "n"(kSlice * 16 * 512));
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(high) : "v"(at[kTile]), "n"((kSlice * 16 + 4) * 512));
+    return __builtin_bit_cast(bf16x8_t, u32x4_t{low[0], low[1], high[0], high[1]});
+  } else {
+    u32x4_t words;
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(words) : "v"(at[kSlice]), "n"(kTile * 32 * 128));
+    return __builtin_bit_cast(bf16x8_t, words);
+  }
+}
+
+template <bool kAAcross, bool kBAcross, bool kOutF32>
+__global__ __launch_bounds__(kWideThreads, 1) void wide_kernel(DenseParams p) {
+  using A = WideOperand<kAAcross>;
+  using B = WideOperand<kBAcross>;
+  extern __shared__ uint8_t lds[];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int wave_row = wave / 2, wave_column = wave % 2;  // 2 x 2 wavefronts of 128 x 128
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)lds));
+
+  // ---- the groups' tiles and rows, a lane a group, 64 groups a register ----
+  const int m_tiles_of_gradient = (p.outer_m + kWideTile - 1) / kWideTile;
+  constexpr int kRounds = kWideGroups / 64;
+  int first_tile[kRounds], first_row[kRounds], group_size[kRounds];
+  int m_tiles = 0, held = 0;
+  {
+    auto scanned = [lane](int value) {
+#pragma unroll
+      for (int offset = 1; offset < 64; offset <<= 1) {
+        const int other = __shfl_up(value, offset, 64);
+        if (lane >= offset) value += other;
+      }
+      return value;
+    };
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round) {
+      const int g = 64 * round + lane;
+      first_tile[round] = 0x7FFFFFFF;
+      first_row[round] = group_size[round] = 0;
+      if (64 * round < p.groups) {
+        const int size = g >= p.groups ? 0 : p.sizes ? max(p.sizes[g], 0) : max(p.offsets[g + 1] - p.offsets[g], 0);
+        const int tiles = g >= p.groups ? 0 : kAAcross ? m_tiles_of_gradient : (size + kWideTile - 1) / kWideTile;
+        const int rows = scanned(size), inclusive = scanned(tiles);
+        if (g < p.groups) {
+          first_tile[round] = m_tiles + inclusive - tiles;
+          first_row[round] = p.sizes ? held + rows - size : p.offsets[g];
+          group_size[round] = size;
+        }
+        m_tiles += __builtin_amdgcn_readlane(inclusive, 63);
+        held += __builtin_amdgcn_readlane(rows, 63);
+      }
+    }
+    if (!p.sizes) held = p.offsets[p.groups];
+  }
+  const int strips = (p.outer_n + kWideTile - 1) / kWideTile, total = __builtin_amdgcn_readfirstlane(m_tiles * strips);
+
+  if constexpr (!kAAcross) {  // the rows of no group are zero
+    const int pieces = p.outer_n / 8;
+    const long long items = static_cast<long long>(max(p.rows - held, 0)) * pieces;
+    for (long long item = static_cast<long long>(blockIdx.x) * kWideThreads + threadIdx.x; item < items; item += static_cast<long long>(gridDim.x) * kWideThreads) {
+      const int row = held + static_cast<int>(item / pieces);
+      *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(p.out) + static_cast<size_t>(row) * p.outer_n + item % pieces * 8) = u32x4_t{0, 0, 0, 0};
+    }
+  }
+
+  // ---- tile number `order` of this block's: chunks of group_m row tiles x 8 strips, dealt round-robin to the XCDs ----
+  struct Tile {
+    int group, row0, valid_rows, n0, m0, depth, steps;
+  };
+  const int chunk_tiles = 32, slots = gridDim.x / 8;
+  auto tile_at = [&](int turn, Tile& tile) {
+    const int place = turn * slots + blockIdx.x / 8;
+    const int order = __builtin_amdgcn_readfirstlane(((place / chunk_tiles) * 8 + blockIdx.x % 8) * chunk_tiles + place % chunk_tiles);
+    if (order >= total) return false;
+    const int across = order / strips;  // (the tiles of a group are in a row: this many before it at most)
+    int group = -1;
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round) group += __builtin_popcountll(__ballot(first_tile[round] <= across));
+    int before = 0, start = 0, size = 0;
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round)
+      if (group / 64 == round) {
+        before = __builtin_amdgcn_readlane(first_tile[round], group % 64);
+        start = __builtin_amdgcn_readlane(first_row[round], group % 64);
+        size = __builtin_amdgcn_readlane(group_size[round], group % 64);
+      }
+    const int tiles = kAAcross ? m_tiles_of_gradient : (size + kWideTile - 1) / kWideTile;
+    const int place_in_group = order - before * strips;
+    const int band = place_in_group / (p.group_m * strips), band_tiles = min(p.group_m, tiles - band * p.group_m), within = place_in_group % (p.group_m * strips);
+    const int within_group = band * p.group_m + within % band_tiles;
+    tile.n0 = (within / band_tiles) * kWideTile;
+    tile.group = group;
+    if constexpr (kAAcross) {
+      tile.m0 = within_group * kWideTile;
+      tile.row0 = min(max(start, 0), p.rows);
+      tile.depth = min(max(start + size, tile.row0), p.rows) - tile.row0;
+      tile.valid_rows = min(kWideTile, p.outer_m - tile.m0);
+      tile.steps = max((tile.depth + kWideStep - 1) / kWideStep, 1);
+    } else {
+      tile.m0 = 0;
+      tile.row0 = start + within_group * kWideTile;
+      tile.valid_rows = min(kWideTile, size - within_group * kWideTile);
+      tile.depth = p.inner;
+      tile.steps = p.inner / kWideStep;
+    }
+    return true;
+  };
+
+  // ---- what fetches: the first operand two steps ahead of what multiplies, the second one. A step's bytes are a buffer: what lies
+  // past its end (the rows past a tile's last, those past a group's last) reads as zero ----
+  Tile fetched;
+  if (!tile_at(0, fetched)) return;  // (the same for the whole block)
+  Tile tile = fetched;
+  int fetched_turn = 0, fetched_step = 0, first_slot = 0, second_slot = 0;
+  bool moved = false;
+  const uint8_t *a_next = nullptr, *b_next = nullptr;  // the next step's bytes
+  int a_bytes = 0, b_bytes = 0, a_rows = 0, b_rows = 0;
+  uint32_t a_offset[kWideLoads], b_offset[kWideLoads];  // of the lane's 16 bytes of each load
+  const uint32_t a_pitch = (kAAcross ? p.outer_m : p.inner) * 2, b_pitch = (kBAcross ? p.outer_n : p.inner) * 2;
+  size_t a_stride = kAAcross ? static_cast<size_t>(kWideStep) * a_pitch : kWideStep * 2;
+  size_t b_stride = kBAcross ? static_cast<size_t>(kWideStep) * b_pitch : kWideStep * 2;
+#pragma unroll
+  for (int i = 0; i < kWideLoads; ++i) {
+    const int a_row = A::row(kWideLoads * wave + i, lane), b_row = B::row(kWideLoads * wave + i, lane);
+    a_offset[i] = a_row * a_pitch + 16 * A::chunk(a_row, lane);
+    b_offset[i] = b_row * b_pitch + 16 * B::chunk(b_row, lane);
+  }
+  __amdgpu_buffer_rsrc_t a_buffer, b_buffer;
+  auto buffer = [](const uint8_t* at, int bytes) __attribute__((always_inline)) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(at), 0, bytes, 0x00027000); };
+  auto aim_first = [&]() __attribute__((always_inline)) {
+    if constexpr (kAAcross) {
+      a_next = reinterpret_cast<const uint8_t*>(p.a) + static_cast<size_t>(fetched.row0) * a_pitch + fetched.m0 * 2;
+      a_rows = fetched.depth;
+    } else {
+      a_next = reinterpret_cast<const uint8_t*>(p.a) + static_cast<size_t>(fetched.row0) * a_pitch;
+      a_bytes = fetched.valid_rows * a_pitch;
+    }
+  };
+  auto aim_second = [&]() __attribute__((always_inline)) {
+    if constexpr (kAAcross) {
+      b_next = reinterpret_cast<const uint8_t*>(p.b) + static_cast<size_t>(fetched.row0) * b_pitch + fetched.n0 * 2;
+      b_rows = fetched.depth;
+    } else {
+      const uint8_t* matrix = reinterpret_cast<const uint8_t*>(p.b + static_cast<size_t>(fetched.group) * p.inner * p.outer_n);
+      b_next = kBAcross ? matrix + fetched.n0 * 2 : matrix + static_cast<size_t>(fetched.n0) * b_pitch;
+      b_bytes = kBAcross ? kWideStep * b_pitch - fetched.n0 * 2 : min(kWideTile, p.outer_n - fetched.n0) * b_pitch;
+    }
+  };
+  auto next_first = [&]() __attribute__((always_inline)) {  // ahead of a step's loads of the first operand
+    if (fetched_step == fetched.steps) {
+      if (!tile_at(++fetched_turn, fetched)) a_stride = b_stride = 0;  // (none left: the last one's first step, again and again)
+      fetched_step = 0;
+      moved = true;
+      aim_first();
+    }
+    ++fetched_step;
+  };
+  auto next_second = [&]() __attribute__((always_inline)) {  // of the second, which follows the first
+    if (moved) {
+      moved = false;
+      aim_second();
+    }
+  };
+  auto begin_first = [&]() __attribute__((always_inline)) {
+    if constexpr (kAAcross) {
+      a_bytes = max(min(a_rows, kWideStep) * static_cast<int>(a_pitch) - fetched.m0 * 2, 0);
+      a_rows -= kWideStep;
+    }
+    a_buffer = buffer(a_next, a_bytes);
+    a_next += a_stride;
+    first_slot = first_slot == kFirstStages - 1 ? 0 : first_slot + 1;
+  };
+  auto begin_second = [&]() __attribute__((always_inline)) {
+    if constexpr (kAAcross) {
+      b_bytes = max(min(b_rows, kWideStep) * static_cast<int>(b_pitch) - fetched.n0 * 2, 0);
+      b_rows -= kWideStep;
+    }
+    b_buffer = buffer(b_next, b_bytes);
+    b_next += b_stride;
+    second_slot ^= 1;
+  };
+  auto load_first = [&](auto piece) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(3))) void* lds_t;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buffer, (lds_t)(lds + first_slot * kOperandBytes + (wave * kWideLoads + piece.value) * 1024), 16, a_offset[piece.value], 0, 0, 0);
+#endif
+  };
+  auto load_second = [&](auto piece) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __attribute__((address_space(3))) void* lds_t;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(b_buffer, (lds_t)(lds + (kFirstStages + second_slot) * kOperandBytes + (wave * kWideLoads + piece.value) * 1024), 16,
+                                             b_offset[piece.value], 0, 0, 0);
+#endif
+  };
+
+  // ---- what multiplies ----
+  uint32_t a_at[4], b_at[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    a_at[i] = A::address(lds_base, 4 * wave_row, i, lane);
+    b_at[i] = B::address(lds_base + kFirstStages * kOperandBytes, 4 * wave_column, i, lane);
+  }
+  f32x16_t acc[4][4];
+  bf16x8_t a_frag[2][4], b_frag[2][4];
+  auto clear = [&]() __attribute__((always_inline)) {  // (half the time of as many moves)
+    bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0, 0, 0, 0});
+    f32x16_t none;
+#pragma unroll
+    for (int q = 0; q < 16; ++q) none[q] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(zero, zero, none, 0, 0, 0);
+  };
+  auto read_piece = [&](auto slice, auto set, auto piece) __attribute__((always_inline)) {
+    constexpr int s = decltype(slice)::value, i = decltype(piece)::value;
+    if constexpr (i < 4) b_frag[set.value][i] = wide_fragment<kBAcross, s, i>(b_at);
+    else if constexpr (i < 4 + 4) a_frag[set.value][i - 4] = wide_fragment<kAAcross, s, i - 4>(a_at);
+  };
+  // one phase: a slice multiplied, and in the shadows of its matrix instructions the next one's fragments read and `beside` done
+  auto phase = [&](auto from, auto slice, auto into, auto&& beside) __attribute__((always_inline)) {
+    static_for<16>([&](auto m) __attribute__((always_inline)) {
+      constexpr int t = decltype(m)::value;
+      read_piece(slice, into, m);
+      acc[t / 4][t % 4] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b_frag[from.value][t % 4], a_frag[from.value][t / 4], acc[t / 4][t % 4], 0, 0, 0);
+      beside(m);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  auto arrived = [&](auto set) __attribute__((always_inline)) {  // this wavefront's reads are back
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_waitcnt(0xF | (7 << 4) | (3 << 14));  // lgkmcnt(0)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(a_frag[set.value][i]));
+#pragma unroll
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+v"(b_frag[set.value][j]));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  constexpr std::integral_constant<int, 0> c0{};
+  constexpr std::integral_constant<int, 1> c1{};
+  constexpr std::integral_constant<int, 2> c2{};
+  constexpr std::integral_constant<int, 3> c3{};
+  // every wavefront's loads but its `younger` last memory operations are done, and so are its reads of the other stage
+  auto landed = [&](auto younger) __attribute__((always_inline)) {
+    constexpr int n = decltype(younger)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4));  // vmcnt(n) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the loads go out one every four matrix instructions (the L1 takes them at half its rate; in bursts they held up the wavefront
+  // that issued them, and its matrix instructions behind them)
+  auto second_half = [&](auto m) __attribute__((always_inline)) {
+    if constexpr (decltype(m)::value % 4 == 3) load_second(std::integral_constant<int, 4 + decltype(m)::value / 4>{});
+  };
+  clear();
+  aim_first();
+  aim_second();
+  first_slot = kFirstStages - 1, second_slot = 1;  // (they turn ahead of each step)
+  next_first();
+  begin_first();
+  static_for<8>(load_first);
+  begin_second();
+  static_for<8>(load_second);
+  next_first();
+  begin_first();
+  static_for<8>(load_first);
+  next_second();
+  begin_second();
+  static_for<4>(load_second);
+  landed(c0);
+  static_for<8>([&](auto piece) __attribute__((always_inline)) { read_piece(c0, c0, piece); });
+  arrived(c0);
+  int read_slot = 0, turn = 0;
+  uint32_t a_move = 0, b_move = 0;
+  constexpr std::integral_constant<int, 8> younger{};  // the first operand's loads of the step after the next
+  for (;;) {
+    for (int step = 0; step < tile.steps; ++step) {
+      phase(c0, c1, c1, second_half);
+      next_first();
+      arrived(c1);
+      phase(c1, c2, c0, [&](auto m) __attribute__((always_inline)) {
+        if constexpr (decltype(m)::value == 1) begin_first();
+        if constexpr (decltype(m)::value % 4 == 3) load_first(std::integral_constant<int, decltype(m)::value / 4>{});
+      });
+      arrived(c0);
+      phase(c0, c3, c1, [&](auto m) __attribute__((always_inline)) {
+        constexpr int t = decltype(m)::value;
+        if constexpr (t == 1) {
+          a_move = read_slot % kFirstStages == kFirstStages - 1 ? -(kFirstStages - 1) * kOperandBytes : kOperandBytes;
+          b_move = read_slot % 2 == 1 ? -kOperandBytes : kOperandBytes;
+          read_slot = read_slot == 5 ? 0 : read_slot + 1;
+        }
+        if constexpr (t % 4 == 3) load_first(std::integral_constant<int, 4 + t / 4>{});
+        if constexpr (t >= 8 && t < 12) a_at[t % 4] += a_move;  // (behind the last reads of this step)
+        if constexpr (t >= 12) b_at[t % 4] += b_move;
+      });
+      landed(younger);
+      arrived(c1);
+      next_second();
+      phase(c1, c0, c0, [&](auto m) __attribute__((always_inline)) {  // (reads the next step's first slice; nothing's behind the last)
+        if constexpr (decltype(m)::value == 1) begin_second();
+        if constexpr (decltype(m)::value % 4 == 3) load_second(std::integral_constant<int, decltype(m)::value / 4>{});
+      });
+      arrived(c0);
+    }
+
+    // ---- the tile leaves: acc[i][j][q] is row 8 (q / 4) + 4 (lane / 32) + q % 4, column lane % 32 of its 32 x 32 tile ----
+    int lane = threadIdx.x % 64;
+    asm volatile("" : "+v"(lane));
+    float factor = 1.0f;
+    if constexpr (kAAcross) factor = (p.factor0 ? *p.factor0 : 1.0f) * (p.factor1 ? *p.factor1 : 1.0f);
+    // (what lies past the buffer's end, the rows past the tile's last, and the columns sent there are not stored)
+    constexpr int kOutBytes = kOutF32 ? 4 : 2;
+    const int column0 = tile.n0 + 128 * wave_column, tile_row = 128 * wave_row;
+    const size_t out_row0 = kAAcross ? static_cast<size_t>(tile.group) * p.outer_m + tile.m0 : tile.row0;
+    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(static_cast<uint8_t*>(p.out) + out_row0 * p.outer_n * kOutBytes, 0,
+                                                                         tile.valid_rows * p.outer_n * kOutBytes, 0x00027000);
+    constexpr uint32_t kNowhere = 0xFFFFFFF0u;
+    // (row tile i's sums are in accumulation registers up to here: moved at the loop's end, all 256 at once took every other register)
+    auto stay = [&](int i) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[i][j]));
+#endif
+    };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      stay(i);
+      const int row = tile_row + 32 * i;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if constexpr (kOutF32) {
+          const int column = column0 + 32 * j + 4 * (lane / 32);
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const uint32_t to = column + 8 * g < p.outer_n ? ((row + lane % 32) * p.outer_n + column + 8 * g) * 4 : kNowhere;
+            __builtin_amdgcn_raw_buffer_store_b128(
+                __builtin_bit_cast(u32x4_t, f32x4_t{acc[i][j][4 * g] * factor, acc[i][j][4 * g + 1] * factor, acc[i][j][4 * g + 2] * factor, acc[i][j][4 * g + 3] * factor}),
+                out, to, 0, 0);
+          }
+        } else {
+          uint32_t words[2][4];  // after the first exchange: [k][..] is columns 8 (2 k + lane / 32) .. + 7 of row lane % 32
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+              const int q = 8 * k + 2 * h;
+              const auto swapped = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[i][j][q] * factor, acc[i][j][q + 1] * factor),
+                                                                    pack_bf16(acc[i][j][q + 4] * factor, acc[i][j][q + 5] * factor), false, false);
+              words[k][h] = swapped[0];
+              words[k][2 + h] = swapped[1];
+            }
+#pragma unroll
+          for (int d = 0; d < 4; ++d) {  // after the second: row 16 k + lane % 16, columns 8 ((lane >> 4 & 1) * 2 + lane / 32) .. + 7
+            const auto swapped = __builtin_amdgcn_permlane16_swap(words[0][d], words[1][d], false, false);
+            words[0][d] = swapped[0];
+            words[1][d] = swapped[1];
+          }
+          const int column = column0 + 32 * j + 8 * ((lane >> 4 & 1) * 2 + lane / 32);
+          const uint32_t to = column < p.outer_n ? ((row + lane % 16) * p.outer_n + column) * 2 : kNowhere;
+          const uint32_t sixteen_rows = column < p.outer_n ? 16 * p.outer_n * 2 : 0;
+#pragma unroll
+          for (int k = 0; k < 2; ++k)
+            __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{words[k][0], words[k][1], words[k][2], words[k][3]}, out, to + k * sixteen_rows, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (!tile_at(++turn, tile)) return;
+    clear();
+  }
+}
+
+template <bool kAAcross, bool kBAcross, bool kOutF32>
+static int launch_wide_kernel(const char* who, const DenseParams& p, hipStream_t stream) {
+  auto kernel = wide_kernel<kAAcross, kBAcross, kOutF32>;
+  static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
+  static hipError_t reserved = hipSuccess;
+  std::call_once(configured, [&] {
+    reserved = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kWideShared);
+  });
+  if (reserved != hipSuccess) return fail(DEW_MOE_ELAUNCH, "%s: cannot reserve %d bytes of LDS", who, kWideShared);
+  hipLaunchKernelGGL(kernel, dim3(256), dim3(kWideThreads), kWideShared, stream, p);  // one block a CU
+  return launched(who);
+}
+
+int launch_wide(const char* who, const DenseParams& params, bool across, bool kmajor, bool out_f32, hipStream_t stream) {
+  DenseParams p = params;
+  p.group_m = 4;  // (4 row tiles x 8 strips are what an XCD's 32 CUs hold at once; 6 or 8 were 0 to 3 % slower)
+  if (across) return out_f32 ? launch_wide_kernel<true, true, true>(who, p, stream) : launch_wide_kernel<true, true, false>(who, p, stream);
+  return kmajor ? launch_wide_kernel<false, false, false>(who, p, stream) : launch_wide_kernel<false, true, false>(who, p, stream);
+}
+
+}  // namespace dew

@@ -173,7 +173,7 @@ def prepared(bank) -> ops.PreparedBank:
 
 
 def _relaid_first(matrices: torch.Tensor, rows: int) -> bool:
-    """Whether `rows` rows times plain matrices are the faster product on matrices brought to the matrix instruction's order at the
+    """Whether `rows` gathered or scattered rows times plain matrices are the faster product on matrices brought to the matrix instruction's order at the
     call (`prepared`) than on matrices read where they lie (`ops.dense_gemm`); the bits are the same. The pass over the matrices is
     small beside the work of groups of thousands of rows, and the launch on prepared matrices then runs in 256-row tiles that fetch
     half the bytes from the L2; K-major matrices lose the more by lying where they are, since a step reads half of each cache line.
@@ -208,7 +208,8 @@ def gemm(lhs: torch.Tensor, rhs, group_sizes, *, paired=None, gather: torch.Tens
             rhs = rhs.contiguous()
         elif rhs.data_ptr() % 16:    # (a view into a flat buffer of parameters begins anywhere; the launch loads 16 bytes at a time)
             rhs = rhs.clone()        # (which keeps the strides)
-        if not _relaid_first(rhs, lhs.shape[0] if gather is None else gather.numel()):
+        # (rows as they lie: the launch takes tiles of its own that need no order, see wide.hip)
+        if (gather is None and scatter is None) or not _relaid_first(rhs, lhs.shape[0] if gather is None else gather.numel()):
             groups = GroupSizes.operands(group_sizes)
             return ops.dense_gemm(lhs, rhs, groups["offsets"], gather=gather, scatter=scatter, sizes=groups.get("sizes"))
     first = prepared(rhs)
