@@ -17,8 +17,6 @@
 // groups of some thousands of rows on, the weights' pass is the smaller price: an operand whose rows run along the contraction
 // gives a step 64 bytes of each of its cache lines, so that K-major matrices cost 10 to 17 % more than natural ones, and the tiled
 // launch's 256-row tiles fetch half as much. The caller (gemm.py, with the sizes measured) brings such matrices to order first.
-#include <math.h>
-
 #include <mutex>
 
 #include "dense.h"
@@ -353,15 +351,6 @@ constexpr int kFewTiles = 128;
 static bool few_tiles(int rows, int groups, int width) {  // about so many of 128 x 256, the groups' last ones half empty
   return (rows / 128 + groups / 2 + 1) * static_cast<long long>((width + 255) / 256) <= kFewTiles;
 }
-
-// Whether about `tiles` 256 x 256 tiles keep `percent` of the 256 CUs busy over the rounds they take (one tile a CU and round; groups
-// end where they end, so that a round's last few tiles may not be there).
-static bool fills_rounds(double tiles, int percent) {
-  const double rounds = tiles <= 264 ? 1 : ceil(tiles / 256 - 0.03);
-  return tiles * 100 >= rounds * 256 * percent;
-}
-
-static bool wide_extents(int groups, int a, int b) { return groups <= kWideGroups && a <= (1 << 20) && b <= (1 << 20); }  // (offsets within a tile are 32-bit)
 
 // 256 x 256 tiles (wide.hip) where they fill the CUs over the rounds that they take, on groups of at least about half a tile's rows.
 // Measured against the tiles below on 105 shapes (512 to 65 536 rows, 1 to 60 groups, extents 512 to 14 336; us, there and here):

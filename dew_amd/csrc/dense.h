@@ -2,6 +2,7 @@
 #pragma once
 
 #include "common.h"
+#include "wide.h"
 
 namespace dew {
 
@@ -14,8 +15,6 @@ struct DenseParams {
   const float *factor0, *factor1;  // a kernel gradient's sums times *factor0 * *factor1 (each may be null)
   int groups, rows, inner, outer_m, outer_n, m_tiles, group_m;
 };
-
-constexpr int kWideGroups = 256;  // groups that a 256 x 256 launch keeps the tiles of in the LDS
 
 // 256 x 256 tiles on blocks that stay (wide.hip), of rows that are neither gathered nor scattered; `across`: a kernel gradient; `kmajor`:
 // w [groups, width, depth].

@@ -30,6 +30,7 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "wide_fp8.h"
 
 namespace dew {
 
@@ -1339,6 +1340,31 @@ static bool few_gradient_blocks(const GemmParams& p) {
   return static_cast<long long>(p.experts) * ((p.window_rows + 255) / 256) * ((p.width + 255) / 256) <= 128;
 }
 
+// The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered: where such
+// tiles keep the CUs busy over the rounds they take. Measured against the launches below on 70 shapes (512 to 32 768 rows, 1 to 51 groups,
+// extents 512 to 14 336; us, there and here): [32 768, 7168] x 2048 of 32 groups, blockwise, forward 470 and 424, input's gradient 520 and
+// 444, kernel's gradient 692 and 565; [32 768, 4096] x 14336 of 8, MXFP8, 1636 and 1500, 1600 and 1470, 1637 and 1470; [12 672, 512] x 3456
+// of 21 70 and 39; [4608, 896] x 7552 of 33, kernel's gradient, 220 and 125. At rounds filled to 0.56 .. 0.7 1.02 to 1.2 times as fast, in one
+// round from 0.66 on 1.1 to 1.7; at 260 tiles, two rounds, 0.77 to 0.89.
+static bool fills_wide_rounds(double tiles, int percent_of_one, int percent_of_more) {
+  const double rounds = ceil(tiles / 256);
+  return tiles * 100 >= rounds * 256 * (rounds <= 1 ? percent_of_one : percent_of_more);
+}
+
+static WideFp8Params wide_fp8_params(const GemmParams& p, int a_scale_pitch) {
+  return WideFp8Params{reinterpret_cast<const uint8_t*>(p.x), p.a_scale, p.w0.codes, p.w0.scales, p.offsets, p.out, p.experts, p.rows, p.depth, p.width, a_scale_pitch};
+}
+
+static bool wide_fp8_product(const GemmParams& p) {
+  const double tiles = (p.rows / 256.0 + p.experts / 2.0) * ((p.width + 255) / 256);
+  return forced_tile_rows == 0 && !p.gather && !p.scatter && !p.bias && wide_extents(p.experts, p.depth, p.width) && p.depth >= 512 &&
+         p.rows / p.experts >= 112 && fills_wide_rounds(tiles, 62, 56);
+}
+
+static bool wide_fp8_gradient_extents(int tokens, int depth, int width, int groups) {
+  return tokens >= 512 && tokens <= (1 << 20) && wide_extents(groups, depth, width);
+}
+
 }  // namespace dew
 
 extern "C" int dew_moe_tile_rows(int32_t rows) {
@@ -1488,6 +1514,8 @@ extern "C" int dew_moe_grouped_gemm_fp8_rows(const void* x_codes, const uint8_t*
   // from the LDS, which has the time. [32 x 1024, 7168] x 2048 as 2 x 2 and as 1 x 4 (us): forward 476 -> 463, input's gradient 541
   // -> 512; MXFP8 579 -> 519; kernel's gradient 780 -> 678; [8 x 4096, 4096] x 14336 in MXFP8, the three products: 1916 -> 1679,
   // 1793 -> 1628, 1757 -> 1627 (2.0 to 2.2 -> 2.3 to 2.4 PFLOP/s).
+  if (wide_fp8_product(p))
+    return launch_wide_fp8(who, wide_fp8_params(p, block_scale_pitch(p.depth)), false, false, false, static_cast<hipStream_t>(stream));
   if (few_blocks(p)) return launch_tile<kFormatFp8Rows, kPlain, 128, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
   if (p.width % 256 == 0) return launch_tile<kFormatFp8Rows, kPlain, 256, 256, 1, 4>(who, p, static_cast<hipStream_t>(stream));
   return launch_tile<kFormatFp8Rows, kPlain, 256, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
@@ -1506,6 +1534,8 @@ extern "C" int dew_moe_grouped_gemm_mxfp8_rows(const void* x_codes, const uint8_
   GemmParams p{};
   if (int rc = fill_single(who, p, x_codes, gather, offsets, w, bias, scatter, out, rows)) return rc;
   p.a_scale = x_scales;
+  if (wide_fp8_product(p))
+    return launch_wide_fp8(who, wide_fp8_params(p, p.depth / 32), true, false, false, static_cast<hipStream_t>(stream));
   if (few_blocks(p)) return launch_tile<kFormatMxFp8Rows, kPlain, 128, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
   if (p.width % 256 == 0) return launch_tile<kFormatMxFp8Rows, kPlain, 256, 256, 1, 4>(who, p, static_cast<hipStream_t>(stream));
   return launch_tile<kFormatMxFp8Rows, kPlain, 256, 128, 2, 2>(who, p, static_cast<hipStream_t>(stream));
@@ -1551,6 +1581,35 @@ extern "C" int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint
   // (few tiles: half as wide ones, 8 groups of 512 tokens x 1024 x 1024 19 -> 14 us; 128 x 128 take 17)
   if (p.width % 256 == 0 && !few_gradient_blocks(p)) return launch_tile<kFormatMxFp8Window, kPlain, 256, 256, 1, 4>(who, p, s);
   return launch_tile<kFormatMxFp8Window, kPlain, 256, 128, 2, 2>(who, p, s);
+}
+
+extern "C" int dew_moe_kernel_gradient_takes_banks(int32_t tokens, int32_t depth, int32_t width, int32_t groups) {
+  using namespace dew;
+  const double tiles = static_cast<double>(groups) * ((depth + 255) / 256) * ((width + 255) / 256);
+  // (its tiles are whole, and those of the launch of one tile a block start and end worse: 270 tiles 49.5 and 33.4 us. One round of long
+  // tiles, which few blocks fetch from the memory and not from each other's L2, is slower here: 168 of 18 steps 40 and 49)
+  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && fills_wide_rounds(tiles, 70, 53);
+}
+
+extern "C" int dew_moe_kernel_gradient_mxfp8_banks(const dew_moe_bank* lhs_t, const dew_moe_bank* rhs_t, const int32_t* offsets, void* out,
+                                                   int32_t out_is_f32, int32_t groups, void* stream) {
+  using namespace dew;
+  const char* who = "dew_moe_kernel_gradient_mxfp8_banks";
+  for (const dew_moe_bank* bank : {lhs_t, rhs_t}) {
+    DEW_REQUIRE(bank, "%s: the banks must not be null", who);
+    DEW_REQUIRE(bank->format == DEW_MOE_W_MXFP8 && bank->layout == DEW_MOE_LAYOUT_PREPARED && bank->experts == 1,
+                "%s: an operand is one prepared MXFP8 matrix [extent, tokens] (dew_moe_quantize_columns_*, as a bank), not format %d, layout %d, %d experts",
+                who, bank->format, bank->layout, bank->experts);
+    DEW_REQUIRE(bank->depth % 128 == 0 && bank->width >= 128 && bank->width % 128 == 0, "%s: %d tokens of %d are not whole 128s", who, bank->depth, bank->width);
+    DEW_REQUIRE(bank->codes && bank->scales && aligned16(bank->codes) && aligned16(bank->scales), "%s: the banks must not be null and must be 16-byte aligned", who);
+  }
+  DEW_REQUIRE(lhs_t->depth == rhs_t->depth, "%s: %d and %d tokens", who, lhs_t->depth, rhs_t->depth);
+  DEW_REQUIRE(groups >= 1 && wide_fp8_gradient_extents(lhs_t->depth, lhs_t->width, rhs_t->width, groups),
+              "%s: %d groups, %d tokens, %d x %d (at most 256 groups, 512 to 2^20 tokens, extents to 2^20)", who, groups, lhs_t->depth, lhs_t->width, rhs_t->width);
+  DEW_REQUIRE(offsets && out && aligned16(out), "%s: offsets and out must not be null, out 16-byte aligned", who);
+  const WideFp8Params p{static_cast<const uint8_t*>(lhs_t->codes), static_cast<const uint8_t*>(lhs_t->scales), static_cast<const uint8_t*>(rhs_t->codes),
+                        rhs_t->scales, offsets, out, groups, lhs_t->width, lhs_t->depth, rhs_t->width, lhs_t->depth / 32};
+  return launch_wide_fp8(who, p, true, true, out_is_f32 != 0, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int dew_moe_kernel_gradient_bf16(const void* lhs_t, const dew_moe_bank* rhs_t, const int32_t* offsets, const float* lhs_scale,

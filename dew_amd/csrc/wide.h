@@ -1,0 +1,189 @@
+// What the launches of 256 x 256 tiles on blocks that stay share (wide.hip: plain bf16 operands; wide_fp8.hip: the recipes' e4m3 ones):
+// a block's tiles, one after another, and a finished tile's way out.
+#pragma once
+
+#include <math.h>
+
+#include "common.h"
+#include "gemm.h"
+
+namespace dew {
+
+constexpr int kWideThreads = 256, kWideTile = 256;
+constexpr int kWideGroups = 256;  // groups that such a launch keeps the tiles of in registers
+
+// Whether about `tiles` 256 x 256 tiles keep `percent` of the 256 CUs busy over the rounds they take (one tile a CU and round; groups
+// end where they end, so that a round's last few tiles may not be there).
+inline bool fills_rounds(double tiles, int percent) {
+  const double rounds = tiles <= 264 ? 1 : ceil(tiles / 256 - 0.03);
+  return tiles * 100 >= rounds * 256 * percent;
+}
+
+inline bool wide_extents(int groups, int a, int b) { return groups <= kWideGroups && a <= (1 << 20) && b <= (1 << 20); }  // (offsets within a tile are 32-bit)
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+struct WidePlace {
+  int group, start, size;  // the tile's group: its first row and its rows
+  int within, strip;       // row tile of the group, column strip
+};
+
+// The groups' tiles and rows, a lane a group, 64 groups a register. kGradient: every group has the same row tiles, of `outer_m` rows.
+template <bool kGradient>
+struct WideTiles {
+  static constexpr int kRounds = kWideGroups / 64;
+  int first_tile[kRounds], first_row[kRounds], group_size[kRounds];
+  int gradient_tiles, strips, total, held;  // `held`: rows in all groups
+
+  __device__ __forceinline__ void find(const int32_t* offsets, const int32_t* sizes, int groups, int outer_m, int outer_n) {
+    const int lane = threadIdx.x % 64;
+    auto scanned = [lane](int value) {
+#pragma unroll
+      for (int offset = 1; offset < 64; offset <<= 1) {
+        const int other = __shfl_up(value, offset, 64);
+        if (lane >= offset) value += other;
+      }
+      return value;
+    };
+    gradient_tiles = (outer_m + kWideTile - 1) / kWideTile;
+    int m_tiles = 0;
+    held = 0;
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round) {
+      const int g = 64 * round + lane;
+      first_tile[round] = 0x7FFFFFFF;
+      first_row[round] = group_size[round] = 0;
+      if (64 * round < groups) {
+        const int size = g >= groups ? 0 : sizes ? max(sizes[g], 0) : max(offsets[g + 1] - offsets[g], 0);
+        const int tiles = g >= groups ? 0 : kGradient ? gradient_tiles : (size + kWideTile - 1) / kWideTile;
+        const int rows = scanned(size), inclusive = scanned(tiles);
+        if (g < groups) {
+          first_tile[round] = m_tiles + inclusive - tiles;
+          first_row[round] = sizes ? held + rows - size : offsets[g];
+          group_size[round] = size;
+        }
+        m_tiles += __builtin_amdgcn_readlane(inclusive, 63);
+        held += __builtin_amdgcn_readlane(rows, 63);
+      }
+    }
+    if (!sizes) held = offsets[groups];
+    strips = (outer_n + kWideTile - 1) / kWideTile;
+    total = __builtin_amdgcn_readfirstlane(m_tiles * strips);
+  }
+
+  // The block's tile number `turn`, false past its last: chunks of group_m row tiles x 8 strips, dealt round-robin to the XCDs.
+  __device__ __forceinline__ bool at(int turn, int group_m, WidePlace& out) const {
+    const int chunk_tiles = 32, slots = gridDim.x / 8;
+    const int place = turn * slots + blockIdx.x / 8;
+    const int order = __builtin_amdgcn_readfirstlane(((place / chunk_tiles) * 8 + blockIdx.x % 8) * chunk_tiles + place % chunk_tiles);
+    if (order >= total) return false;
+    const int across = order / strips;  // (the tiles of a group are in a row: this many before it at most)
+    int group = -1;
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round) group += __builtin_popcountll(__ballot(first_tile[round] <= across));
+    int before = 0, start = 0, size = 0;
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round)
+      if (group / 64 == round) {
+        before = __builtin_amdgcn_readlane(first_tile[round], group % 64);
+        start = __builtin_amdgcn_readlane(first_row[round], group % 64);
+        size = __builtin_amdgcn_readlane(group_size[round], group % 64);
+      }
+    const int tiles = kGradient ? gradient_tiles : (size + kWideTile - 1) / kWideTile;
+    const int place_in_group = order - before * strips;
+    const int band = place_in_group / (group_m * strips), band_tiles = min(group_m, tiles - band * group_m), within = place_in_group % (group_m * strips);
+    out = WidePlace{group, start, size, band * group_m + within % band_tiles, within / band_tiles};
+    return true;
+  }
+};
+
+// The rows of no group are zero: rows held .. rows of `out`, `width` wide (a multiple of 8), by all of the launch's threads.
+__device__ __forceinline__ void clear_unowned(bf16_t* out, int held, int rows, int width) {
+  const int pieces = width / 8;
+  const long long items = static_cast<long long>(max(rows - held, 0)) * pieces;
+  for (long long item = static_cast<long long>(blockIdx.x) * kWideThreads + threadIdx.x; item < items; item += static_cast<long long>(gridDim.x) * kWideThreads) {
+    const int row = held + static_cast<int>(item / pieces);
+    *reinterpret_cast<u32x4_t*>(out + static_cast<size_t>(row) * width + item % pieces * 8) = u32x4_t{0, 0, 0, 0};
+  }
+}
+
+// The sums are zero: sixteen products of zeros, in half the time of as many moves (each of its own, or the compiler makes one and copies it).
+__device__ __forceinline__ void clear_sums(f32x16_t (&acc)[4][4]) {
+  bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0, 0, 0, 0});
+  f32x16_t none;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) none[q] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      asm volatile("" : "+v"(zero));
+      acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(zero, zero, none, 0, 0, 0);
+    }
+}
+
+// A wavefront's 128 x 128 sums leave from registers, without the LDS and without a barrier. The operands entered the instruction the
+// other way round: acc[i][j][q] is row lane % 32, column 8 (q / 4) + 4 (lane / 32) + q % 4 of its 32 x 32 tile, and two exchanges between
+// lane groups make a lane's sums 16 bytes of a row. `out_row0`, `valid_rows`: the block's tile (what lies past the buffer's end, the rows
+// past its last, and the columns sent there are not stored); `tile_row`, `column0`: the wavefront's place in it and in the row.
+template <bool kOutF32>
+__device__ __forceinline__ void leave(f32x16_t (&acc)[4][4], void* to_rows, size_t out_row0, int valid_rows, int width, int tile_row, int column0, float factor) {
+  int lane = threadIdx.x % 64;
+  asm volatile("" : "+v"(lane));
+  constexpr int kOutBytes = kOutF32 ? 4 : 2;
+  const __amdgpu_buffer_rsrc_t out =
+      __builtin_amdgcn_make_buffer_rsrc(static_cast<uint8_t*>(to_rows) + out_row0 * width * kOutBytes, 0, valid_rows * width * kOutBytes, 0x00027000);
+  constexpr uint32_t kNowhere = 0xFFFFFFF0u;
+  // (row tile i's sums are in accumulation registers up to here: moved at the loop's end, all 256 at once took every other register)
+  auto stay = [&](int i) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[i][j]));
+#endif
+  };
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    stay(i);
+    const int row = tile_row + 32 * i;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if constexpr (kOutF32) {
+        const int column = column0 + 32 * j + 4 * (lane / 32);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const uint32_t to = column + 8 * g < width ? ((row + lane % 32) * width + column + 8 * g) * 4 : kNowhere;
+          __builtin_amdgcn_raw_buffer_store_b128(
+              __builtin_bit_cast(u32x4_t, f32x4_t{acc[i][j][4 * g] * factor, acc[i][j][4 * g + 1] * factor, acc[i][j][4 * g + 2] * factor, acc[i][j][4 * g + 3] * factor}),
+              out, to, 0, 0);
+        }
+      } else {
+        uint32_t words[2][4];  // after the first exchange: [k][..] is columns 8 (2 k + lane / 32) .. + 7 of row lane % 32
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int q = 8 * k + 2 * h;
+            const auto swapped = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[i][j][q] * factor, acc[i][j][q + 1] * factor),
+                                                                  pack_bf16(acc[i][j][q + 4] * factor, acc[i][j][q + 5] * factor), false, false);
+            words[k][h] = swapped[0];
+            words[k][2 + h] = swapped[1];
+          }
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {  // after the second: row 16 k + lane % 16, columns 8 ((lane >> 4 & 1) * 2 + lane / 32) .. + 7
+          const auto swapped = __builtin_amdgcn_permlane16_swap(words[0][d], words[1][d], false, false);
+          words[0][d] = swapped[0];
+          words[1][d] = swapped[1];
+        }
+        const int column = column0 + 32 * j + 8 * ((lane >> 4 & 1) * 2 + lane / 32);
+        const uint32_t to = column < width ? ((row + lane % 16) * width + column) * 2 : kNowhere;
+        const uint32_t sixteen_rows = column < width ? 16 * width * 2 : 0;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{words[k][0], words[k][1], words[k][2], words[k][3]}, out, to + k * sixteen_rows, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+}  // namespace dew

@@ -23,17 +23,17 @@
 
 #include "dense.h"
 #include "gemm.h"
+#include "wide.h"
 
 namespace dew {
 
-constexpr int kWideThreads = 256, kWideTile = 256, kWideStep = 64;
+constexpr int kWideStep = 64;
 constexpr int kWideLoads = 8;                                      // 1 KiB loads of each operand that a wavefront makes a step
 constexpr int kOperandBytes = kWideTile * kWideStep * 2;           // 32 KB: one operand's stage
 constexpr int kFirstStages = 3, kSecondStages = 2;                 // of the first operand's ring and the second's
 constexpr int kWideShared = (kFirstStages + kSecondStages) * kOperandBytes;  // all of the LDS
 
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // One operand as it is staged. kAcross false: 256 rows of 64 depths (128 bytes, chunk index xor-swizzled as in the tiled launch);
 // kAcross true: 64 rows of 256 columns in units of 32 columns (64 bytes) whose index is xor-ed with the row mod 4.
@@ -81,88 +81,29 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_kernel(DenseParams p) {
   const int wave_row = wave / 2, wave_column = wave % 2;  // 2 x 2 wavefronts of 128 x 128
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)lds));
 
-  // ---- the groups' tiles and rows, a lane a group, 64 groups a register ----
-  const int m_tiles_of_gradient = (p.outer_m + kWideTile - 1) / kWideTile;
-  constexpr int kRounds = kWideGroups / 64;
-  int first_tile[kRounds], first_row[kRounds], group_size[kRounds];
-  int m_tiles = 0, held = 0;
-  {
-    auto scanned = [lane](int value) {
-#pragma unroll
-      for (int offset = 1; offset < 64; offset <<= 1) {
-        const int other = __shfl_up(value, offset, 64);
-        if (lane >= offset) value += other;
-      }
-      return value;
-    };
-#pragma unroll
-    for (int round = 0; round < kRounds; ++round) {
-      const int g = 64 * round + lane;
-      first_tile[round] = 0x7FFFFFFF;
-      first_row[round] = group_size[round] = 0;
-      if (64 * round < p.groups) {
-        const int size = g >= p.groups ? 0 : p.sizes ? max(p.sizes[g], 0) : max(p.offsets[g + 1] - p.offsets[g], 0);
-        const int tiles = g >= p.groups ? 0 : kAAcross ? m_tiles_of_gradient : (size + kWideTile - 1) / kWideTile;
-        const int rows = scanned(size), inclusive = scanned(tiles);
-        if (g < p.groups) {
-          first_tile[round] = m_tiles + inclusive - tiles;
-          first_row[round] = p.sizes ? held + rows - size : p.offsets[g];
-          group_size[round] = size;
-        }
-        m_tiles += __builtin_amdgcn_readlane(inclusive, 63);
-        held += __builtin_amdgcn_readlane(rows, 63);
-      }
-    }
-    if (!p.sizes) held = p.offsets[p.groups];
-  }
-  const int strips = (p.outer_n + kWideTile - 1) / kWideTile, total = __builtin_amdgcn_readfirstlane(m_tiles * strips);
+  WideTiles<kAAcross> tiles;
+  tiles.find(p.offsets, p.sizes, p.groups, p.outer_m, p.outer_n);
 
-  if constexpr (!kAAcross) {  // the rows of no group are zero
-    const int pieces = p.outer_n / 8;
-    const long long items = static_cast<long long>(max(p.rows - held, 0)) * pieces;
-    for (long long item = static_cast<long long>(blockIdx.x) * kWideThreads + threadIdx.x; item < items; item += static_cast<long long>(gridDim.x) * kWideThreads) {
-      const int row = held + static_cast<int>(item / pieces);
-      *reinterpret_cast<u32x4_t*>(static_cast<bf16_t*>(p.out) + static_cast<size_t>(row) * p.outer_n + item % pieces * 8) = u32x4_t{0, 0, 0, 0};
-    }
-  }
+  if constexpr (!kAAcross) clear_unowned(static_cast<bf16_t*>(p.out), tiles.held, p.rows, p.outer_n);
 
-  // ---- tile number `order` of this block's: chunks of group_m row tiles x 8 strips, dealt round-robin to the XCDs ----
   struct Tile {
     int group, row0, valid_rows, n0, m0, depth, steps;
   };
-  const int chunk_tiles = 32, slots = gridDim.x / 8;
   auto tile_at = [&](int turn, Tile& tile) {
-    const int place = turn * slots + blockIdx.x / 8;
-    const int order = __builtin_amdgcn_readfirstlane(((place / chunk_tiles) * 8 + blockIdx.x % 8) * chunk_tiles + place % chunk_tiles);
-    if (order >= total) return false;
-    const int across = order / strips;  // (the tiles of a group are in a row: this many before it at most)
-    int group = -1;
-#pragma unroll
-    for (int round = 0; round < kRounds; ++round) group += __builtin_popcountll(__ballot(first_tile[round] <= across));
-    int before = 0, start = 0, size = 0;
-#pragma unroll
-    for (int round = 0; round < kRounds; ++round)
-      if (group / 64 == round) {
-        before = __builtin_amdgcn_readlane(first_tile[round], group % 64);
-        start = __builtin_amdgcn_readlane(first_row[round], group % 64);
-        size = __builtin_amdgcn_readlane(group_size[round], group % 64);
-      }
-    const int tiles = kAAcross ? m_tiles_of_gradient : (size + kWideTile - 1) / kWideTile;
-    const int place_in_group = order - before * strips;
-    const int band = place_in_group / (p.group_m * strips), band_tiles = min(p.group_m, tiles - band * p.group_m), within = place_in_group % (p.group_m * strips);
-    const int within_group = band * p.group_m + within % band_tiles;
-    tile.n0 = (within / band_tiles) * kWideTile;
-    tile.group = group;
+    WidePlace place;
+    if (!tiles.at(turn, p.group_m, place)) return false;
+    tile.group = place.group;
+    tile.n0 = place.strip * kWideTile;
     if constexpr (kAAcross) {
-      tile.m0 = within_group * kWideTile;
-      tile.row0 = min(max(start, 0), p.rows);
-      tile.depth = min(max(start + size, tile.row0), p.rows) - tile.row0;
+      tile.m0 = place.within * kWideTile;
+      tile.row0 = min(max(place.start, 0), p.rows);
+      tile.depth = min(max(place.start + place.size, tile.row0), p.rows) - tile.row0;
       tile.valid_rows = min(kWideTile, p.outer_m - tile.m0);
       tile.steps = max((tile.depth + kWideStep - 1) / kWideStep, 1);
     } else {
       tile.m0 = 0;
-      tile.row0 = start + within_group * kWideTile;
-      tile.valid_rows = min(kWideTile, size - within_group * kWideTile);
+      tile.row0 = place.start + place.within * kWideTile;
+      tile.valid_rows = min(kWideTile, place.size - place.within * kWideTile);
       tile.depth = p.inner;
       tile.steps = p.inner / kWideStep;
     }
@@ -265,16 +206,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_kernel(DenseParams p) {
   }
   f32x16_t acc[4][4];
   bf16x8_t a_frag[2][4], b_frag[2][4];
-  auto clear = [&]() __attribute__((always_inline)) {  // (half the time of as many moves)
-    bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0, 0, 0, 0});
-    f32x16_t none;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) none[q] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(zero, zero, none, 0, 0, 0);
-  };
+  auto clear = [&]() __attribute__((always_inline)) { clear_sums(acc); };
   auto read_piece = [&](auto slice, auto set, auto piece) __attribute__((always_inline)) {
     constexpr int s = decltype(slice)::value, i = decltype(piece)::value;
     if constexpr (i < 4) b_frag[set.value][i] = wide_fragment<kBAcross, s, i>(b_at);
@@ -370,68 +302,10 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_kernel(DenseParams p) {
       arrived(c0);
     }
 
-    // ---- the tile leaves: acc[i][j][q] is row 8 (q / 4) + 4 (lane / 32) + q % 4, column lane % 32 of its 32 x 32 tile ----
-    int lane = threadIdx.x % 64;
-    asm volatile("" : "+v"(lane));
     float factor = 1.0f;
     if constexpr (kAAcross) factor = (p.factor0 ? *p.factor0 : 1.0f) * (p.factor1 ? *p.factor1 : 1.0f);
-    // (what lies past the buffer's end, the rows past the tile's last, and the columns sent there are not stored)
-    constexpr int kOutBytes = kOutF32 ? 4 : 2;
-    const int column0 = tile.n0 + 128 * wave_column, tile_row = 128 * wave_row;
     const size_t out_row0 = kAAcross ? static_cast<size_t>(tile.group) * p.outer_m + tile.m0 : tile.row0;
-    const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(static_cast<uint8_t*>(p.out) + out_row0 * p.outer_n * kOutBytes, 0,
-                                                                         tile.valid_rows * p.outer_n * kOutBytes, 0x00027000);
-    constexpr uint32_t kNowhere = 0xFFFFFFF0u;
-    // (row tile i's sums are in accumulation registers up to here: moved at the loop's end, all 256 at once took every other register)
-    auto stay = [&](int i) __attribute__((always_inline)) {
-#if defined(__HIP_DEVICE_COMPILE__)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[i][j]));
-#endif
-    };
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      stay(i);
-      const int row = tile_row + 32 * i;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (kOutF32) {
-          const int column = column0 + 32 * j + 4 * (lane / 32);
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const uint32_t to = column + 8 * g < p.outer_n ? ((row + lane % 32) * p.outer_n + column + 8 * g) * 4 : kNowhere;
-            __builtin_amdgcn_raw_buffer_store_b128(
-                __builtin_bit_cast(u32x4_t, f32x4_t{acc[i][j][4 * g] * factor, acc[i][j][4 * g + 1] * factor, acc[i][j][4 * g + 2] * factor, acc[i][j][4 * g + 3] * factor}),
-                out, to, 0, 0);
-          }
-        } else {
-          uint32_t words[2][4];  // after the first exchange: [k][..] is columns 8 (2 k + lane / 32) .. + 7 of row lane % 32
-#pragma unroll
-          for (int k = 0; k < 2; ++k)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-              const int q = 8 * k + 2 * h;
-              const auto swapped = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[i][j][q] * factor, acc[i][j][q + 1] * factor),
-                                                                    pack_bf16(acc[i][j][q + 4] * factor, acc[i][j][q + 5] * factor), false, false);
-              words[k][h] = swapped[0];
-              words[k][2 + h] = swapped[1];
-            }
-#pragma unroll
-          for (int d = 0; d < 4; ++d) {  // after the second: row 16 k + lane % 16, columns 8 ((lane >> 4 & 1) * 2 + lane / 32) .. + 7
-            const auto swapped = __builtin_amdgcn_permlane16_swap(words[0][d], words[1][d], false, false);
-            words[0][d] = swapped[0];
-            words[1][d] = swapped[1];
-          }
-          const int column = column0 + 32 * j + 8 * ((lane >> 4 & 1) * 2 + lane / 32);
-          const uint32_t to = column < p.outer_n ? ((row + lane % 16) * p.outer_n + column) * 2 : kNowhere;
-          const uint32_t sixteen_rows = column < p.outer_n ? 16 * p.outer_n * 2 : 0;
-#pragma unroll
-          for (int k = 0; k < 2; ++k)
-            __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{words[k][0], words[k][1], words[k][2], words[k][3]}, out, to + k * sixteen_rows, 0, 0);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
+    leave<kOutF32>(acc, p.out, out_row0, tile.valid_rows, p.outer_n, 128 * wave_row, tile.n0 + 128 * wave_column, factor);
     if (!tile_at(++turn, tile)) return;
     clear();
   }

@@ -980,6 +980,24 @@ def kernel_gradient_mxfp8(codes: torch.Tensor, scales: torch.Tensor, rhs_t: Prep
     return out
 
 
+def kernel_gradient_mxfp8_banks(lhs_t: PreparedBank, rhs_t: PreparedBank, offsets: torch.Tensor, *, out_dtype=torch.bfloat16) -> torch.Tensor:
+    """`kernel_gradient_mxfp8` from both of `quantize_columns`' operands as banks (`[depth, tokens]` and `[width, tokens]`): the same
+    bits, and the faster form where `kernel_gradient_takes_banks`."""
+    if out_dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"a kernel gradient is written in bfloat16 or float32, not {out_dtype}")
+    _device(offsets, "offsets", torch.int32)
+    groups = offsets.numel() - 1
+    out = torch.empty((groups, lhs_t.shape[2], rhs_t.shape[2]), dtype=out_dtype, device=offsets.device)
+    _lib.check(_lib.library().dew_moe_kernel_gradient_mxfp8_banks(lhs_t.descriptor, rhs_t.descriptor, _ptr(offsets), _ptr(out),
+                                                                  int(out_dtype == torch.float32), groups, _stream()),
+               "dew_moe_kernel_gradient_mxfp8_banks")
+    return out
+
+
+def kernel_gradient_takes_banks(tokens: int, depth: int, width: int, groups: int) -> bool:
+    return bool(_lib.library().dew_moe_kernel_gradient_takes_banks(tokens, depth, width, groups))
+
+
 def transpose_columns(x: torch.Tensor, *, nvfp4: bool = False, as_bank: bool):
     """bf16 `[tokens, dim]` written transposed, a bf16 kernel gradient's operand (`dew_moe_transpose_columns`), or, `nvfp4`,
     its NVFP4 values along the tokens short of the tensor scale (`dew_moe_quantize_columns_nvfp4`). The lhs_t operand

@@ -264,9 +264,12 @@ def kernel_gradient(x: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, m
     1 x 128 tiles (`rows_quantized(x.T)`, `blockwise_fp8_kernel_gradient`, src/dew/nn/kernels/projections.py:220-223)
     or, `mx`, MXFP8's blocks of 32 tokens (src/dew/nn/kernels/projections.py:268-274). Group `g` holds
     `group_blocks[g]` whole 128-token blocks; an empty group's gradient is zero."""
-    codes, scales = ops.quantize_columns(x.contiguous(), mx=mx, as_bank=False)
+    offsets = _groups(group_blocks, x.device).offsets
     bank = ops.quantize_columns(cotangent.contiguous(), mx=mx, as_bank=True)
-    return ops.kernel_gradient_mxfp8(codes, scales, bank, _groups(group_blocks, x.device).offsets, out_dtype=out_dtype)
+    if out_dtype in (torch.bfloat16, torch.float32) and ops.kernel_gradient_takes_banks(x.shape[0], x.shape[1], cotangent.shape[1], offsets.numel() - 1):
+        return ops.kernel_gradient_mxfp8_banks(ops.quantize_columns(x.contiguous(), mx=mx, as_bank=True), bank, offsets, out_dtype=out_dtype)
+    codes, scales = ops.quantize_columns(x.contiguous(), mx=mx, as_bank=False)
+    return ops.kernel_gradient_mxfp8(codes, scales, bank, offsets, out_dtype=out_dtype)
 
 
 def blockwise_fp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):

@@ -425,7 +425,9 @@ int dew_moe_grouped_gemm_mxfp8_rows(const void* x_codes, const uint8_t* x_scales
  * dew_moe_kernel_gradient_mxfp8: out [groups, depth, width] (bf16, or fp32 where out_is_f32) from the lhs_t operand
  * [depth, tokens] and the rhs_t bank [width, tokens]; group g contracts tokens offsets[g] .. offsets[g + 1], whole
  * 128-token blocks (device int32 [groups + 1]); an empty group's matrix is zero. Both operands enter
- * v_mfma_scale_f32_32x32x64_f8f6f4 as stored, 256 x 256 tiles (128 x 128 where those are few).                    */
+ * v_mfma_scale_f32_32x32x64_f8f6f4 as stored, 256 x 256 tiles (256 x 128 where those are few).
+ * dew_moe_kernel_gradient_mxfp8_banks: the same bits from both operands as banks (as_bank 1), in 256 x 256 tiles on blocks that
+ * stay: the faster form where dew_moe_kernel_gradient_takes_banks is not 0. At most 256 groups, 512 to 2^20 tokens, and extents to 2^20.   */
 int dew_moe_quantize_columns_fp8(const void* x /* bf16 [tokens, dim] */, void* codes, void* scales, int32_t tokens,
                                  int32_t dim, int32_t as_bank, void* stream);
 int dew_moe_quantize_columns_mxfp8(const void* x /* bf16 [tokens, dim] */, void* codes, void* scales, int32_t tokens,
@@ -433,6 +435,9 @@ int dew_moe_quantize_columns_mxfp8(const void* x /* bf16 [tokens, dim] */, void*
 int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint8_t* lhs_t_scales, const dew_moe_bank* rhs_t,
                                   const int32_t* offsets, void* out, int32_t out_is_f32, int32_t depth, int32_t groups,
                                   void* stream);
+int dew_moe_kernel_gradient_takes_banks(int32_t tokens, int32_t depth, int32_t width, int32_t groups);
+int dew_moe_kernel_gradient_mxfp8_banks(const dew_moe_bank* lhs_t, const dew_moe_bank* rhs_t, const int32_t* offsets, void* out,
+                                        int32_t out_is_f32, int32_t groups, void* stream);
 /* The kernel gradient of bf16 operands: the reference's `gemm_t` src/dew/nn/kernels/gemm.py:418-431 (each group's rows
  * of lhs transposed times its rows of rhs, fp32 sums), and with it the NVFP4 recipe's `_nvfp4_backward`
  * src/dew/nn/kernels/projections.py:322-337 (both operands quantized along the tokens, every 16 a scale, decoded, the
