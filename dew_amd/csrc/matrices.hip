@@ -40,44 +40,6 @@ __device__ __forceinline__ void values_of(const u32x4_t& words, float (&v)[16 / 
   }
 }
 
-// The largest magnitude's bits (magnitudes order as their bit patterns do; a NaN's are the largest) of all of w, for the
-// NVFP4 tensor scale. One atomic a block, and none where the word already holds as much: on one address they are served one
-// after another, some 10 ns each.
-template <typename T>
-__global__ __launch_bounds__(256) void matrices_absmax_kernel(const T* __restrict__ w, long long chunks, uint32_t* __restrict__ largest) {
-  uint32_t mine = 0;
-  const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
-  auto take = [&](const u32x4_t& words) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (sizeof(T) == 2)
-        mine = max(mine, max((words[i] << 16) & 0x7FFF0000u, words[i] & 0x7FFF0000u));
-      else
-        mine = max(mine, words[i] & 0x7FFFFFFFu);
-    }
-  };
-  long long chunk = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
-  for (; chunk + 7 * stride < chunks; chunk += 8 * stride) {  // eight loads in flight a lane
-    u32x4_t words[8];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) words[k] = reinterpret_cast<const u32x4_t*>(w)[chunk + k * stride];
-#pragma unroll
-    for (int k = 0; k < 8; ++k) take(words[k]);
-  }
-  for (; chunk < chunks; chunk += stride) take(reinterpret_cast<const u32x4_t*>(w)[chunk]);
-#pragma unroll
-  for (int offset = 32; offset >= 1; offset >>= 1) mine = max(mine, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), offset, 64)));
-  __shared__ uint32_t waves[4];
-  if (threadIdx.x % 64 == 0) waves[threadIdx.x / 64] = mine;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    mine = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
-    if (mine > __hip_atomic_load(largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(largest, mine);
-  }
-}
-
-__global__ void matrices_clear_kernel(uint32_t* __restrict__ largest) { *largest = 0u; }
-
 // The e4m3 scale byte of a 16-deep NVFP4 block whose largest magnitude is `block`, under the tensor scale: the nearest e4m3
 // to block / tensor / 6 and the next one where that lies below (quantize_rows_nvfp4_kernel's rule); a NaN stays one.
 __device__ __forceinline__ uint32_t nvfp4_block_byte(float block, float tensor) {
@@ -89,7 +51,7 @@ __device__ __forceinline__ uint32_t nvfp4_block_byte(float block, float tensor) 
 }
 
 // The E2M1 code (sign in bit 3) of value / tensor / each, ties to the even code; zero under a zero (or NaN) scale. The
-// thresholds are multiplied by `each` instead of the quotient divided: exact, see e2m1_scaled in quantize.hip.
+// thresholds are multiplied by `each` instead of the quotient divided: exact, see e2m1_scaled in nvfp4.h.
 __device__ __forceinline__ uint32_t e2m1_code(float value, float tensor, float each) {
   if (!(each > 0.0f)) return 0u;
   const float y = value / tensor, m = fabsf(y);
@@ -136,19 +98,22 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
   // natural: a thread's rows are consecutive depths; K-major: rows are columns, dealt group by group
   auto row_of = [&](int p) { return KMAJOR ? p * kGroups + group : group * kLoads + p; };
   const T* source = w + e * depth * width + static_cast<size_t>(KMAJOR ? n0 : k0) * pitch + (KMAJOR ? k0 : n0) + piece * kVec;
-  float v[kLoads][kVec];
+  const uint32_t share = kNv ? nvfp4_share(largest, kNvfp4Partials) : 0u;
+  u32x4_t words[kLoads];
 #pragma unroll
-  for (int p = 0; p < kLoads; ++p)
-    values_of<T>(*reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch), v[p]);
+  for (int p = 0; p < kLoads; ++p) words[p] = *reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch);
 
   float tensor = 1.0f;
   bool quick = false;  // (the same for the whole launch)
   if constexpr (kNv) {
-    const float top = __uint_as_float(*largest);
-    tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
+    const float top = nvfp4_top(share);
+    tensor = nvfp4_tensor_scale(top);
     quick = sizeof(T) == 2 && nvfp4_in_range(top, tensor);
     if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) tensor_scales[e] = tensor;
   }
+  float v[kLoads][kVec];
+#pragma unroll
+  for (int p = 0; p < kLoads; ++p) values_of<T>(words[p], v[p]);
   const float inverse_tensor = kNv ? 1.0f / tensor : 1.0f;
   auto magnitude = [](float value) { return __float_as_uint(value) & 0x7FFFFFFFu; };
   float inverse = 1.0f;  // FP8 blocks: the tile's one
@@ -314,7 +279,7 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
   }
 }
 
-// An NVFP4 bank's buffer: codes, block scales, then a word for the largest magnitude (256 bytes) and the tensor scales.
+// An NVFP4 bank's buffer: codes, block scales, then the partial largest magnitudes and the tensor scales.
 static size_t nvfp4_scales_at(size_t elements) { return elements / 2; }
 static size_t nvfp4_largest_at(size_t elements) { return elements / 2 + elements / 16; }
 
@@ -323,15 +288,10 @@ static int quantize_matrices(const T* w, bool kmajor, int experts, int depth, in
   const size_t elements = static_cast<size_t>(experts) * depth * width;
   uint8_t* scales = prepared + (FORMAT == DEW_MOE_W_NVFP4 ? nvfp4_scales_at(elements) : elements);
   uint32_t* largest = reinterpret_cast<uint32_t*>(prepared + nvfp4_largest_at(elements));
-  float* tensor_scales = reinterpret_cast<float*>(largest + 64);
+  float* tensor_scales = reinterpret_cast<float*>(largest + kNvfp4Partials);
   *out = dew_moe_bank{FORMAT, DEW_MOE_LAYOUT_PREPARED, experts, depth, width, prepared, scales, FORMAT == DEW_MOE_W_NVFP4 ? tensor_scales : nullptr};
   if (FORMAT == DEW_MOE_W_NVFP4) {
-    hipLaunchKernelGGL(matrices_clear_kernel, dim3(1), dim3(1), 0, s, largest);
-    if (int rc = launched("matrices_clear_kernel")) return rc;
-    const long long chunks = static_cast<long long>(elements / (16 / sizeof(T)));
-    const int blocks = static_cast<int>(min((chunks + 255) / 256, 256ll * 2));
-    hipLaunchKernelGGL(matrices_absmax_kernel<T>, dim3(blocks), dim3(256), 0, s, w, chunks, largest);
-    if (int rc = launched("matrices_absmax_kernel")) return rc;
+    if (int rc = dew_moe_nvfp4_largest(w, static_cast<int64_t>(elements), sizeof(T) == 4, largest, s)) return rc;
   }
   const dim3 grid = kmajor ? dim3(depth / 128, width / 128, experts) : dim3(width / 128, depth / 128, experts);
   if (kmajor)
@@ -346,7 +306,7 @@ static int quantize_matrices(const T* w, bool kmajor, int experts, int depth, in
 extern "C" size_t dew_moe_quantized_matrices_bytes(int32_t format, int32_t experts, int32_t depth, int32_t width) {
   if (experts <= 0 || depth <= 0 || width <= 0) return 0;
   const size_t elements = static_cast<size_t>(experts) * depth * width;
-  if (format == DEW_MOE_W_NVFP4) return dew::nvfp4_largest_at(elements) + 256 + (static_cast<size_t>(experts) * 4 + 255) / 256 * 256;
+  if (format == DEW_MOE_W_NVFP4) return dew::nvfp4_largest_at(elements) + 4 * dew::kNvfp4Partials + (static_cast<size_t>(experts) * 4 + 255) / 256 * 256;
   return dew_moe_prepared_bytes(format, experts, depth, width);
 }
 

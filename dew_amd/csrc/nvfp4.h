@@ -53,4 +53,54 @@ struct Nvfp4Scales {
   }
 };
 
+// An operand's largest magnitude as fp32 bits (magnitudes order as their bit patterns do; a NaN's are the largest), from the `count` partial
+// ones that a launch left, one a block: some hundred words for every wavefront that wants it, where one word would take a launch that clears
+// it. In two parts, so that a wavefront's other loads go out between them: a lane's share, and the whole.
+constexpr int kNvfp4Partials = 512;
+__device__ __forceinline__ uint32_t nvfp4_share(const uint32_t* __restrict__ partials, int count) {
+  uint32_t mine = 0;
+  if (count == 1) return *partials;
+#pragma unroll
+  for (int i = 0; i < kNvfp4Partials / 64; ++i) mine = max(mine, partials[64 * i + threadIdx.x % 64]);
+  return mine;
+}
+__device__ __forceinline__ float nvfp4_top(uint32_t mine) {
+#pragma unroll
+  for (int offset = 32; offset >= 1; offset >>= 1) mine = max(mine, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), offset, 64)));
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(mine));
+}
+
+// largest / (6 * 448), fp32's least normal at least; 1 for an operand of zeros
+__device__ __forceinline__ float nvfp4_tensor_scale(float top) { return top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f; }
+
+// A block's scale: the least e4m3 at or above blockmax / tensor / 6, the nearest one and the next where that lies below.
+__device__ __forceinline__ float nvfp4_block_scale(float block, float tensor) {
+  const float ratio = (block / tensor) / 6.0f;
+  uint32_t byte = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(ratio, 448.0f), 0.0f, 0, false) & 0xFFu;
+  if (__builtin_amdgcn_cvt_f32_fp8(byte, 0) < ratio) byte = min(byte + 1u, 0x7Eu);
+  return __builtin_amdgcn_cvt_f32_fp8(byte, 0);
+}
+
+// The nearest E2M1 to a quotient by the block scale (ties to the even code) times that scale, without the quotient: for y = x / tensor and the block scale `each` (an e4m3
+// value, four significant bits), fl(y / each) > t exactly where y > t each, and >= likewise, for each of the seven
+// thresholds t (at most three significant bits, so t each is exact): a y above t each lies at least one ulp of t each
+// above it, which is more than half an ulp of t above t in the quotient (their ratio is 1 / m or 2 / m for each's
+// significand m < 2), so the quotient rounds past t; at or below, it cannot round above. One IEEE division an element
+// instead of two.
+__device__ __forceinline__ float e2m1_scaled(float magnitude, float each) {
+  float value = magnitude > 0.25f * each ? 0.5f * each : 0.0f;
+  value = magnitude >= 0.75f * each ? each : value;
+  value = magnitude > 1.25f * each ? 1.5f * each : value;
+  value = magnitude >= 1.75f * each ? 2.0f * each : value;
+  value = magnitude > 2.5f * each ? 3.0f * each : value;
+  value = magnitude >= 3.5f * each ? 4.0f * each : value;
+  return magnitude > 5.0f * each ? 6.0f * each : value;
+}
+
+// Two values' codes times the block scale as bf16 patterns, the first below, by divisions: exact in bf16.
+__device__ __forceinline__ uint32_t nvfp4_values_divided(float first, float second, float tensor, float each) {
+  const float a = each > 0.0f ? first / tensor : 0.0f, b = each > 0.0f ? second / tensor : 0.0f;
+  return (__float_as_uint(copysignf(e2m1_scaled(fabsf(a), each), a)) >> 16) | (__float_as_uint(copysignf(e2m1_scaled(fabsf(b), each), b)) & 0xFFFF0000u);
+}
+
 }  // namespace dew

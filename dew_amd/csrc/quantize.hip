@@ -16,6 +16,7 @@ namespace dew {
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
+typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 constexpr int kQuantizeWaves = 4;  // rows per 256-thread block
 
 __global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_fp8_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes,
@@ -133,90 +134,174 @@ __global__ __launch_bounds__(256) void absmax_kernel(const bf16_t* __restrict__ 
   if (threadIdx.x % 64 == 0) waves[threadIdx.x / 64] = mine;
   __syncthreads();
   if (threadIdx.x == 0) {
-    mine = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
+    mine = max(max(waves[0], waves[1]), max(waves[2], waves[3])) << 16;  // (as fp32 bits)
     if (mine > __hip_atomic_load(largest, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(largest, mine);
   }
 }
 
-__device__ __forceinline__ float e2m1_nearest(float magnitude) {
-  // ties to the even code: 0.25 -> 0, 0.75 -> 1, 1.25 -> 1, 1.75 -> 2, 2.5 -> 2, 3.5 -> 4, 5 -> 4
-  float value = magnitude > 0.25f ? 0.5f : 0.0f;
-  value = magnitude >= 0.75f ? 1.0f : value;
-  value = magnitude > 1.25f ? 1.5f : value;
-  value = magnitude >= 1.75f ? 2.0f : value;
-  value = magnitude > 2.5f ? 3.0f : value;
-  value = magnitude >= 3.5f ? 4.0f : value;
-  return magnitude > 5.0f ? 6.0f : value;
-}
-
-// The same choice times the block scale, without the quotient: for y = x / tensor and the block scale `each` (an e4m3
-// value, four significant bits), fl(y / each) > t exactly where y > t each, and >= likewise, for each of the seven
-// thresholds t (at most three significant bits, so t each is exact): a y above t each lies at least one ulp of t each
-// above it, which is more than half an ulp of t above t in the quotient (their ratio is 1 / m or 2 / m for each's
-// significand m < 2), so the quotient rounds past t; at or below, it cannot round above. One IEEE division an element
-// instead of two.
-__device__ __forceinline__ float e2m1_scaled(float magnitude, float each) {
-  float value = magnitude > 0.25f * each ? 0.5f * each : 0.0f;
-  value = magnitude >= 0.75f * each ? each : value;
-  value = magnitude > 1.25f * each ? 1.5f * each : value;
-  value = magnitude >= 1.75f * each ? 2.0f * each : value;
-  value = magnitude > 2.5f * each ? 3.0f * each : value;
-  value = magnitude >= 3.5f * each ? 4.0f * each : value;
-  return magnitude > 5.0f * each ? 6.0f * each : value;
-}
-
-__global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_nvfp4_kernel(const bf16_t* __restrict__ x, const uint32_t* __restrict__ largest,
+// `count` partial magnitudes; `bank_scales` (or null): the `experts` tensor scales of the bank these rows will multiply, which leave times
+// the rows' own as `products`. The blocks stay for row after row: what each first makes of the partials it makes once.
+__global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_nvfp4_kernel(const bf16_t* __restrict__ x, const uint32_t* __restrict__ largest, int count,
                                                                                 bf16_t* __restrict__ out, float* __restrict__ tensor_scale,
-                                                                                int rows, int depth) {
-  const float top = __uint_as_float(*largest << 16);
-  // largest / (6 * 448), fp32's least normal at least; 1 for an operand of zeros
-  const float tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
-  if (blockIdx.x == 0 && threadIdx.x == 0) *tensor_scale = tensor;
+                                                                                const float* __restrict__ bank_scales, float* __restrict__ products,
+                                                                                int experts, int rows, int depth) {
+  const float top = nvfp4_top(nvfp4_share(largest, count));
+  const float tensor = nvfp4_tensor_scale(top);
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) *tensor_scale = tensor;
+    if (bank_scales)
+      for (int e = threadIdx.x; e < experts; e += blockDim.x) products[e] = bank_scales[e] * tensor;
+  }
   const bool quick = nvfp4_in_range(top, tensor);  // (the same for the whole launch)
   const float inverse_tensor = 1.0f / tensor;
   const int lane = threadIdx.x % 64;
-  const int row = blockIdx.x * kQuantizeWaves + threadIdx.x / 64;
-  if (row >= rows) return;
-  const bf16_t* source = x + static_cast<size_t>(row) * depth;
-  bf16_t* target = out + static_cast<size_t>(row) * depth;
-  for (int chunk = lane; chunk < depth / 8; chunk += 64) {  // 8 depths a lane, 2 lanes a block of 16
-    const u32x4_t words = *reinterpret_cast<const u32x4_t*>(source + chunk * 8);
-    float v[8];
+  for (int row = blockIdx.x * kQuantizeWaves + threadIdx.x / 64; row < rows; row += gridDim.x * kQuantizeWaves) {
+    const bf16_t* source = x + static_cast<size_t>(row) * depth;
+    bf16_t* target = out + static_cast<size_t>(row) * depth;
+    for (int chunk = lane; chunk < depth / 8; chunk += 64) {  // 8 depths a lane, 2 lanes a block of 16
+      const u32x4_t words = *reinterpret_cast<const u32x4_t*>(source + chunk * 8);
+      float v[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = __uint_as_float(words[i] << 16);
-      v[2 * i + 1] = __uint_as_float(words[i] & 0xFFFF0000u);
-    }
-    float block = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) block = fmaxf(block, fabsf(v[i]));
-    block = fmaxf(block, __shfl_xor(block, 1, 64));
-    // the least e4m3 at or above blockmax / tensor / 6: the nearest one, and the next where that lies below
-    const float ratio = (block / tensor) / 6.0f;
-    uint32_t byte = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(ratio, 448.0f), 0.0f, 0, false) & 0xFFu;
-    if (__builtin_amdgcn_cvt_f32_fp8(byte, 0) < ratio) byte = min(byte + 1u, 0x7Eu);
-    const float each = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
-    u32x4_t packed;
-    if (quick) {
-      const Nvfp4Scales by{tensor, inverse_tensor, each, nvfp4_inverse(each)};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) packed[i] = by.values(v[2 * i], v[2 * i + 1]);
-      *reinterpret_cast<u32x4_t*>(target + chunk * 8) = packed;
-      continue;
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float pair[2];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const float source_value = v[2 * i + h];
-        const float over_tensor = each > 0.0f ? source_value / tensor : 0.0f;
-        pair[h] = copysignf(e2m1_scaled(fabsf(over_tensor), each), over_tensor);  // code x block scale: exact in bf16
+      for (int i = 0; i < 4; ++i) {
+        v[2 * i] = __uint_as_float(words[i] << 16);
+        v[2 * i + 1] = __uint_as_float(words[i] & 0xFFFF0000u);
       }
-      packed[i] = (__float_as_uint(pair[0]) >> 16) | (__float_as_uint(pair[1]) & 0xFFFF0000u);
+      float block = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) block = fmaxf(block, fabsf(v[i]));
+      block = fmaxf(block, __shfl_xor(block, 1, 64));
+      const float each = nvfp4_block_scale(block, tensor);
+      u32x4_t packed;
+      if (quick) {
+        const Nvfp4Scales by{tensor, inverse_tensor, each, nvfp4_inverse(each)};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) packed[i] = by.values(v[2 * i], v[2 * i + 1]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) packed[i] = nvfp4_values_divided(v[2 * i], v[2 * i + 1], tensor, each);
+      }
+      *reinterpret_cast<u32x4_t*>(target + chunk * 8) = packed;
     }
-    *reinterpret_cast<u32x4_t*>(target + chunk * 8) = packed;
   }
+}
+
+// The operands of a step's gradients, x [tokens, dim] quantized ALONG THE TOKENS where it lies (the kernel gradient of dense operands
+// contracts the tokens of both as they are: no transposed copy), and, ROWS, along its rows too from the same read, which the cotangent's
+// other product takes. A thread owns 16 tokens x 4 columns: a block of each column, and a quarter of a block of each row, the others three
+// neighbouring lanes' (8 columns a thread took
+// 256 registers, one wavefront a SIMD: 34 M elements 139 us, 47 here; tokens alone, 17 M, 29 and 17). The arithmetic of quantize_rows_nvfp4_kernel.
+// Bound by memory: 2 bytes read and 2 (ROWS: 4) written an element.
+template <bool ROWS>
+__global__ __launch_bounds__(256) void quantize_tokens_nvfp4_kernel(const bf16_t* __restrict__ x, const uint32_t* __restrict__ largest,
+                                                                    bf16_t* __restrict__ rows_out, bf16_t* __restrict__ tokens_out,
+                                                                    float* __restrict__ tensor_scale, const float* __restrict__ bank_scales,
+                                                                    float* __restrict__ products, int experts, int tokens, int dim) {
+  const uint32_t share = nvfp4_share(largest, kNvfp4Partials);
+  const long long item = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x, items = static_cast<long long>(tokens / 16) * (dim / 4);
+  const long long mine = item < items ? item : items - 4 + item % 4;  // (past the end: the last four's again, which store the same)
+  const int chunks = dim / 4;  // (whole 32s: four lanes are of the same tokens)
+  const size_t at = static_cast<size_t>(mine / chunks) * 16 * dim + mine % chunks * 4;
+  u32x2_t words[16];
+#pragma unroll
+  for (int t = 0; t < 16; ++t) words[t] = *reinterpret_cast<const u32x2_t*>(x + at + static_cast<size_t>(t) * dim);
+  const float top = nvfp4_top(share);
+  const float tensor = nvfp4_tensor_scale(top), inverse_tensor = 1.0f / tensor;
+  const bool quick = nvfp4_in_range(top, tensor);  // (the same for the whole launch)
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) *tensor_scale = tensor;
+    if (ROWS && bank_scales)
+      for (int e = threadIdx.x; e < experts; e += 256) products[e] = bank_scales[e] * tensor;
+  }
+  auto low = [](uint32_t word) { return __uint_as_float(word << 16); };
+  auto high = [](uint32_t word) { return __uint_as_float(word & 0xFFFF0000u); };
+  auto scales = [&](float block) {
+    const float each = nvfp4_block_scale(block, tensor);
+    return Nvfp4Scales{tensor, inverse_tensor, each, nvfp4_inverse(each)};
+  };
+  if (!quick) {  // an operand with a NaN, an infinity or a scale out of range: read again, value by value
+    if constexpr (ROWS) {
+#pragma unroll 1
+      for (int t = 0; t < 16; ++t) {
+        const u32x2_t word = *reinterpret_cast<const u32x2_t*>(x + at + static_cast<size_t>(t) * dim);
+        float block = fmaxf(fmaxf(fabsf(low(word[0])), fabsf(high(word[0]))), fmaxf(fabsf(low(word[1])), fabsf(high(word[1]))));
+        block = fmaxf(block, __shfl_xor(block, 1, 64));
+        block = fmaxf(block, __shfl_xor(block, 2, 64));
+        const float each = nvfp4_block_scale(block, tensor);
+        *reinterpret_cast<u32x2_t*>(rows_out + at + static_cast<size_t>(t) * dim) =
+            u32x2_t{nvfp4_values_divided(low(word[0]), high(word[0]), tensor, each), nvfp4_values_divided(low(word[1]), high(word[1]), tensor, each)};
+      }
+    }
+#pragma unroll 1
+    for (int c = 0; c < 4; ++c) {
+      float block = 0.0f;
+#pragma unroll 1
+      for (int t = 0; t < 16; ++t) block = fmaxf(block, fabsf(bf16_to_f32(x[at + static_cast<size_t>(t) * dim + c])));
+      const float each = nvfp4_block_scale(block, tensor);
+#pragma unroll 1
+      for (int t = 0; t < 16; ++t) {
+        const size_t place = at + static_cast<size_t>(t) * dim + c;
+        tokens_out[place] = static_cast<bf16_t>(nvfp4_values_divided(bf16_to_f32(x[place]), 0.0f, tensor, each));
+      }
+    }
+    return;
+  }
+  if constexpr (ROWS) {
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float block = fmaxf(fmaxf(fabsf(low(words[t][0])), fabsf(high(words[t][0]))), fmaxf(fabsf(low(words[t][1])), fabsf(high(words[t][1]))));
+      block = fmaxf(block, __shfl_xor(block, 1, 64));
+      block = fmaxf(block, __shfl_xor(block, 2, 64));
+      const Nvfp4Scales by = scales(block);
+      const u32x2_t packed = {by.values(low(words[t][0]), high(words[t][0])), by.values(low(words[t][1]), high(words[t][1]))};
+      *reinterpret_cast<u32x2_t*>(rows_out + at + static_cast<size_t>(t) * dim) = packed;
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // two columns
+    float first = 0.0f, second = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      first = fmaxf(first, fabsf(low(words[t][i])));
+      second = fmaxf(second, fabsf(high(words[t][i])));
+    }
+    const Nvfp4Scales by_first = scales(first), by_second = scales(second);
+#pragma unroll
+    for (int t = 0; t < 16; t += 2) {
+      const uint32_t a = by_first.values(low(words[t][i]), low(words[t + 1][i])), b = by_second.values(high(words[t][i]), high(words[t + 1][i]));
+      words[t][i] = __builtin_amdgcn_perm(b, a, 0x05040100u);
+      words[t + 1][i] = __builtin_amdgcn_perm(b, a, 0x07060302u);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int t = 0; t < 16; ++t) *reinterpret_cast<u32x2_t*>(tokens_out + at + static_cast<size_t>(t) * dim) = words[t];
+}
+
+// An operand's partial largest magnitudes, bf16 or fp32, a partial a block.
+template <bool F32>
+__global__ __launch_bounds__(256) void nvfp4_largest_kernel(const u32x4_t* __restrict__ x, long long chunks, uint32_t* __restrict__ partials) {
+  uint32_t mine = 0;
+  auto take = [&](const u32x4_t& words) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mine = F32 ? max(mine, words[i] & 0x7FFFFFFFu) : max(mine, max((words[i] << 16) & 0x7FFF0000u, words[i] & 0x7FFF0000u));
+  };
+  const long long stride = static_cast<long long>(gridDim.x) * 256;
+  long long chunk = static_cast<long long>(blockIdx.x) * 256 + threadIdx.x;
+  for (; chunk + 7 * stride < chunks; chunk += 8 * stride) {  // eight loads in flight a lane
+    u32x4_t words[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) words[k] = x[chunk + k * stride];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) take(words[k]);
+  }
+  for (; chunk < chunks; chunk += stride) take(x[chunk]);
+#pragma unroll
+  for (int offset = 32; offset >= 1; offset >>= 1) mine = max(mine, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), offset, 64)));
+  __shared__ uint32_t waves[4];
+  if (threadIdx.x % 64 == 0) waves[threadIdx.x / 64] = mine;
+  __syncthreads();
+  if (threadIdx.x == 0) partials[blockIdx.x] = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
 }
 
 // A kernel gradient's operands: x [tokens, dim] quantized ALONG THE TOKENS and written transposed, for the product
@@ -365,8 +450,8 @@ __global__ __launch_bounds__(256) void transpose_columns_kernel(const bf16_t* __
   float tensor = 1.0f;
   bool quick = false;  // (the same for the whole launch)
   if constexpr (NVFP4) {
-    const float top = __uint_as_float(*largest << 16);
-    tensor = top > 0.0f ? fmaxf(top / 2688.0f, 1.17549435e-38f) : 1.0f;
+    const float top = __uint_as_float(*largest);
+    tensor = nvfp4_tensor_scale(top);
     quick = nvfp4_in_range(top, tensor);
     if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *tensor_scale = tensor;
   }
@@ -393,10 +478,7 @@ __global__ __launch_bounds__(256) void transpose_columns_kernel(const bf16_t* __
       float largest_of_block = 0.0f;
 #pragma unroll
       for (int i = 0; i < 16; ++i) largest_of_block = fmaxf(largest_of_block, fabsf(__uint_as_float(bits[16 * block + i] << 16)));
-      const float ratio = (largest_of_block / tensor) / 6.0f;
-      uint32_t byte = __builtin_amdgcn_cvt_pk_fp8_f32(fminf(ratio, 448.0f), 0.0f, 0, false) & 0xFFu;
-      if (__builtin_amdgcn_cvt_f32_fp8(byte, 0) < ratio) byte = min(byte + 1u, 0x7Eu);
-      const float each = __builtin_amdgcn_cvt_f32_fp8(byte, 0);
+      const float each = nvfp4_block_scale(largest_of_block, tensor);
       if (quick) {
         const Nvfp4Scales by{tensor, 1.0f / tensor, each, nvfp4_inverse(each)};
 #pragma unroll
@@ -438,6 +520,8 @@ __global__ __launch_bounds__(256) void transpose_columns_kernel(const bf16_t* __
   }
 }
 
+static int rows_nvfp4_blocks(int rows) { return max(1, min((rows + kQuantizeWaves - 1) / kQuantizeWaves, 2048)); }  // (eight blocks a CU)
+
 static int transpose_columns(const char* who, bool nvfp4, const void* x, void* out, float* tensor_scale, uint32_t* workspace, int tokens,
                              int dim, int as_bank, void* stream, int rows = -1, const int32_t* offsets = nullptr, int groups = 0,
                              int32_t* padded = nullptr) {
@@ -457,8 +541,8 @@ static int transpose_columns(const char* who, bool nvfp4, const void* x, void* o
   }
   if (tokens == 0) {
     if (nvfp4) {  // an operand of no tokens: the unit scale
-      hipLaunchKernelGGL(quantize_rows_nvfp4_kernel, dim3(1), dim3(64 * kQuantizeWaves), 0, s, static_cast<const bf16_t*>(nullptr), workspace,
-                         static_cast<bf16_t*>(nullptr), tensor_scale, 0, 0);
+      hipLaunchKernelGGL(quantize_rows_nvfp4_kernel, dim3(1), dim3(64 * kQuantizeWaves), 0, s, static_cast<const bf16_t*>(nullptr), workspace, 1,
+                         static_cast<bf16_t*>(nullptr), tensor_scale, static_cast<const float*>(nullptr), static_cast<float*>(nullptr), 0, 0, 0);
       return launched("quantize_rows_nvfp4_kernel");
     }
     return DEW_MOE_OK;
@@ -549,9 +633,54 @@ extern "C" int dew_moe_quantize_rows_nvfp4(const void* x, void* values, float* t
     hipLaunchKernelGGL(absmax_kernel, dim3(blocks), dim3(256), 0, s, static_cast<const bf16_t*>(x), chunks, workspace);
     if (int rc = launched("absmax_kernel")) return rc;
   }
-  hipLaunchKernelGGL(quantize_rows_nvfp4_kernel, dim3(max(1, (rows + kQuantizeWaves - 1) / kQuantizeWaves)), dim3(64 * kQuantizeWaves), 0, s,
-                     static_cast<const bf16_t*>(x), workspace, static_cast<bf16_t*>(values), tensor_scale, rows, depth);
+  hipLaunchKernelGGL(quantize_rows_nvfp4_kernel, dim3(dew::rows_nvfp4_blocks(rows)), dim3(64 * kQuantizeWaves), 0, s, static_cast<const bf16_t*>(x), workspace,
+                     1, static_cast<bf16_t*>(values), tensor_scale, static_cast<const float*>(nullptr), static_cast<float*>(nullptr), 0, rows, depth);
   return launched("quantize_rows_nvfp4_kernel");
+}
+
+extern "C" int dew_moe_nvfp4_partials(void) { return dew::kNvfp4Partials; }
+
+extern "C" int dew_moe_nvfp4_largest(const void* operand, int64_t elements, int32_t is_f32, uint32_t* partials, void* stream) {
+  using namespace dew;
+  const char* who = "dew_moe_nvfp4_largest";
+  DEW_REQUIRE(partials, "%s: the partials must not be null", who);
+  DEW_REQUIRE(elements >= 0 && elements % 8 == 0, "%s: an operand of %lld elements (whole 8s)", who, static_cast<long long>(elements));
+  DEW_REQUIRE(elements == 0 || (operand && aligned16(operand)), "%s: the operand must not be null and must be 16-byte aligned", who);
+  const u32x4_t* x = static_cast<const u32x4_t*>(operand);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (is_f32)
+    hipLaunchKernelGGL(nvfp4_largest_kernel<true>, dim3(kNvfp4Partials), dim3(256), 0, s, x, elements / 4, partials);
+  else
+    hipLaunchKernelGGL(nvfp4_largest_kernel<false>, dim3(kNvfp4Partials), dim3(256), 0, s, x, elements / 8, partials);
+  return launched("nvfp4_largest_kernel");
+}
+
+extern "C" int dew_moe_quantize_nvfp4(const void* x, const uint32_t* largest, void* row_values, void* token_values, float* tensor_scale,
+                                      const float* bank_scales, float* products, int32_t experts, int32_t rows, int32_t depth, void* stream) {
+  using namespace dew;
+  const char* who = "dew_moe_quantize_nvfp4";
+  DEW_REQUIRE(rows >= 0 && depth >= 16 && depth % 16 == 0, "%s: rows %d, depth %d (whole 16s)", who, rows, depth);
+  DEW_REQUIRE(!token_values || (rows >= 1 && rows % 128 == 0 && depth % 128 == 0), "%s: %d tokens of %d columns are not whole 128s", who, rows, depth);
+  DEW_REQUIRE(largest && tensor_scale && (row_values || token_values), "%s: largest, tensor_scale and the values must not be null", who);
+  DEW_REQUIRE(!bank_scales || (products && experts >= 1 && row_values), "%s: %d products of a bank's tensor scales and the rows'", who, experts);
+  DEW_REQUIRE(rows == 0 || (x && aligned16(x) && aligned16(row_values) && aligned16(token_values)), "%s: x and the values must be 16-byte aligned", who);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bf16_t* from = static_cast<const bf16_t*>(x);
+  bf16_t *by_row = static_cast<bf16_t*>(row_values), *by_token = static_cast<bf16_t*>(token_values);
+  if (!token_values) {
+    hipLaunchKernelGGL(quantize_rows_nvfp4_kernel, dim3(rows_nvfp4_blocks(rows)), dim3(64 * kQuantizeWaves), 0, s, from, largest, kNvfp4Partials, by_row,
+                       tensor_scale, bank_scales, products, experts, rows, depth);
+    return launched("quantize_rows_nvfp4_kernel");
+  }
+  const long long blocks = (static_cast<long long>(rows / 16) * (depth / 4) + 255) / 256;
+  DEW_REQUIRE(blocks < (1ll << 31), "%s: %d tokens of %d columns", who, rows, depth);
+  if (row_values)
+    hipLaunchKernelGGL(quantize_tokens_nvfp4_kernel<true>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, from, largest, by_row, by_token,
+                       tensor_scale, bank_scales, products, experts, rows, depth);
+  else
+    hipLaunchKernelGGL(quantize_tokens_nvfp4_kernel<false>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, from, largest, by_row, by_token,
+                       tensor_scale, bank_scales, products, experts, rows, depth);
+  return launched("quantize_tokens_nvfp4_kernel");
 }
 
 extern "C" int dew_moe_quantize_rows_mxfp8(const void* x, void* codes, uint8_t* scales, int32_t rows, int32_t depth, void* stream) {

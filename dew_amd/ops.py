@@ -271,11 +271,14 @@ class PreparedBank:
     def scaled(self, by: torch.Tensor) -> "PreparedBank":
         """The same NVFP4 bank with every expert's tensor scale times `by` (a one-element device tensor): how a
         product of two NVFP4 operands owes both tensor scales to its fp32 sums."""
-        held = self.descriptor
-        if held.format not in (_lib.W_NVFP4, _lib.W_MXFP4):
+        if self.descriptor.format not in (_lib.W_NVFP4, _lib.W_MXFP4):
             raise KernelError("only an NVFP4 bank carries tensor scales")
         own = self.keep[2].reshape(-1)[self.first:self.first + self.experts]  # a layer's experts within its stack's scales
-        scales = (own.to(torch.float32) * by.to(torch.float32)).contiguous()
+        return self.under((own.to(torch.float32) * by.to(torch.float32)).contiguous())
+
+    def under(self, scales: torch.Tensor) -> "PreparedBank":
+        """The same NVFP4 bank under other tensor scales, fp32 `[experts]`."""
+        held = self.descriptor
         view = _lib.Bank(held.format, held.layout, held.experts, held.depth, held.width, held.codes, held.scales, _ptr(scales))
         return PreparedBank(view, self.shape, (self.keep[0], self.keep[1], scales), 0)
 
@@ -901,6 +904,31 @@ def quantize_rows_nvfp4(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     _lib.check(_lib.library().dew_moe_quantize_rows_nvfp4(_ptr(x), _ptr(values), _ptr(scale), _ptr(workspace), rows, depth, _stream()),
                "dew_moe_quantize_rows_nvfp4")
     return values, scale
+
+
+def nvfp4_largest(x: torch.Tensor) -> torch.Tensor:
+    """The partial largest magnitudes (words) of `x`, bf16 or fp32, that `quantize_nvfp4` takes its tensor scale from."""
+    _device(x, "x")
+    if x.dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"x must be torch.bfloat16 or torch.float32, got {x.dtype}")
+    partials = torch.empty(_lib.library().dew_moe_nvfp4_partials(), dtype=torch.int32, device=x.device)
+    _lib.check(_lib.library().dew_moe_nvfp4_largest(_ptr(x), x.numel(), int(x.dtype == torch.float32), _ptr(partials), _stream()), "dew_moe_nvfp4_largest")
+    return partials
+
+
+def quantize_nvfp4(x: torch.Tensor, largest: torch.Tensor, *, rows: bool, tokens: bool, bank: PreparedBank | None = None):
+    """`x [R, K]` bf16 in NVFP4 along its rows (`quantize_rows_nvfp4`'s values) and, or, along its tokens where they lie (a scale every
+    16 rows of a column), from one read of it and `nvfp4_largest`'s `largest`: (row values or None, token values or None, tensor scale
+    fp32 `[1]`, the tensor scales of `bank`, which the rows will multiply, times it, or None)."""
+    _device(x, "x", torch.bfloat16), _device(largest, "largest", torch.int32)
+    by_row, by_token = (torch.empty_like(x) if wanted else None for wanted in (rows, tokens))
+    scale = torch.empty(1, dtype=torch.float32, device=x.device)
+    experts = 0 if bank is None else bank.shape[0]
+    products = None if bank is None else torch.empty(experts, dtype=torch.float32, device=x.device)
+    _lib.check(_lib.library().dew_moe_quantize_nvfp4(_ptr(x), _ptr(largest), _ptr(by_row), _ptr(by_token), _ptr(scale),
+                                                     None if bank is None else bank.descriptor.tensor_scale, _ptr(products), experts, x.shape[0],
+                                                     x.shape[1], _stream()), "dew_moe_quantize_nvfp4")
+    return by_row, by_token, scale, products
 
 
 def quantize_rows_mxfp8(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:

@@ -77,14 +77,20 @@ def _bank(w, recipe: str, bank_types: tuple, quantized):
     else by `quantized`, which also refuses the extents that no bank has."""
     if isinstance(w, bank_types):
         return w
+    matrices = _read_by_the_quantizer(w, recipe)
+    return quantized(w) if matrices is None else ops.quantize_matrices(matrices, recipe)
+
+
+def _read_by_the_quantizer(w: torch.Tensor, recipe: str):
+    """`w` as the device's quantizer of matrices reads it (as it lies, or a copy), None where its extents do not fit."""
     whole = SCALE_DEPTH * (2 if recipe == "nvfp4" else 1)    # (an NVFP4 bank's depth is whole 256s)
-    if w.is_cuda and w.dim() == 3 and w.shape[0] >= 1 and w.shape[1] and w.shape[2] and w.shape[1] % whole == 0 and w.shape[2] % SCALE_DEPTH == 0:
-        if w.dtype not in (torch.bfloat16, torch.float32):
-            w = w.to(torch.float32)
-        if not (w.is_contiguous() or w.transpose(1, 2).is_contiguous()) or w.data_ptr() % 16:
-            w = w.clone(memory_format=torch.contiguous_format)
-        return ops.quantize_matrices(w, recipe)
-    return quantized(w)
+    if not (w.is_cuda and w.dim() == 3 and w.shape[0] >= 1 and w.shape[1] and w.shape[2] and w.shape[1] % whole == 0 and w.shape[2] % SCALE_DEPTH == 0):
+        return None
+    if w.dtype not in (torch.bfloat16, torch.float32):
+        w = w.to(torch.float32)
+    if not (w.is_contiguous() or w.transpose(1, 2).is_contiguous()) or w.data_ptr() % 16:
+        w = w.clone(memory_format=torch.contiguous_format)
+    return w
 
 
 def _offsets(group_sizes, rows: int, device) -> torch.Tensor:
@@ -251,8 +257,27 @@ def nvfp4_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torch.bfloat
     """Each group's rows of `x [rows, depth]` times its matrix of `w [groups, depth, width]` in the NVFP4 recipe, both
     quantized along the depth (src/dew/nn/kernels/projections.py:261-275); group `g` holds `group_blocks[g]` whole
     128-row blocks. `w` is the weights (quantized here, `nvfp4_matrices`) or an NVFP4 bank already quantized."""
-    bank = _bank(w, "nvfp4", (formats.NvFp4, ops.PreparedBank), nvfp4_matrices)
-    return nvfp4_block_product(nvfp4_rows(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
+    matrices = None if isinstance(w, (formats.NvFp4, ops.PreparedBank)) else _read_by_the_quantizer(w, "nvfp4")
+    if matrices is None or not _quantized_in_place(x):
+        bank = _bank(w, "nvfp4", (formats.NvFp4, ops.PreparedBank), nvfp4_matrices)
+        return nvfp4_block_product(nvfp4_rows(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
+    x = x.contiguous()
+    bank = ops.quantize_matrices(matrices, "nvfp4")
+    values, _, _, scales = ops.quantize_nvfp4(x, ops.nvfp4_largest(x), rows=True, tokens=False, bank=bank)
+    return _nvfp4_product(values, bank.under(scales), _groups(group_blocks, x.device), out_dtype)
+
+
+def _quantized_in_place(x: torch.Tensor) -> bool:
+    """Whether rows are ones that `ops.quantize_nvfp4` takes; the others are quantized by the launches of one operand, which refuse what
+    no launch takes."""
+    return x.is_cuda and x.dtype == torch.bfloat16 and x.dim() == 2 and x.shape[0] > 0 and x.shape[1] > 0 and x.shape[1] % 16 == 0 and x.data_ptr() % 16 == 0
+
+
+def _nvfp4_product(values: torch.Tensor, bank: ops.PreparedBank, groups: gemm.GroupSizes, out_dtype):
+    """`nvfp4_block_product` of rows and a bank that carries both tensor scales."""
+    if out_dtype != torch.bfloat16:
+        raise ValueError(f"the launch writes bfloat16, not {out_dtype}")
+    return ops.grouped_gemm(values, bank, groups.offsets)
 
 
 # ---- the recipes' gradients ------------------------------------------------------------------------------
@@ -290,16 +315,38 @@ def mxfp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, g
     return d_x, kernel_gradient(x, cotangent, group_blocks, mx=True, out_dtype=out_dtype)
 
 
+def _contracted_in_place(tokens: int, depth: int, width: int, groups: int) -> bool:
+    """Whether an NVFP4 kernel gradient contracts the tokens of its operands where they lie (`ops.dense_gradient`) rather than of transposed
+    copies. Without the copies, and their reads of the operands for the largest magnitude, a step is the shorter: 8192 tokens of 8 x 2048 x
+    4096 655 and 597 us, 640 of 16 x 1536 x 1024 165 and 120. Only few tiles that each walk many tokens are slower so (32 384 tokens of one
+    768 x 768 517 and 652, of one 1024 x 1536 788 and 825, of four 768 x 768 383 and 400; 8192 of one 1024 x 1536 256 and 239)."""
+    return tokens <= 6144 * groups or groups * -(-depth // 256) * -(-width // 256) >= 128
+
+
+def _nvfp4_transposed_gradient(x: torch.Tensor, cotangent: torch.Tensor, groups: gemm.GroupSizes, out_dtype) -> torch.Tensor:
+    rows, rows_scale = ops.transpose_columns(x, nvfp4=True, as_bank=False)
+    columns, columns_scale = ops.transpose_columns(cotangent, nvfp4=True, as_bank=True)
+    return ops.kernel_gradient_bf16(rows, columns, groups.offsets, lhs_scale=rows_scale, rhs_scale=columns_scale, out_dtype=out_dtype)
+
+
 def nvfp4_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):
     """`_nvfp4_backward` (src/dew/nn/kernels/projections.py:322-337) -> (d_x, d_w): the NVFP4 product of the cotangent
     and the matrices, both quantized along the width; and each group's tokens contracted over `x` and the cotangent
     quantized along the tokens, every 16 a scale. The decoded operands short of their tensor scales are exact in bf16,
     so the contraction is the bf16 kernel gradient with both tensor scales applied to its fp32 sums."""
     group_blocks = _groups(group_blocks, x.device)    # once for both products
-    d_x = nvfp4_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
-    rows, rows_scale = ops.transpose_columns(x.contiguous(), nvfp4=True, as_bank=False)
-    bank, bank_scale = ops.transpose_columns(cotangent.contiguous(), nvfp4=True, as_bank=True)
-    d_w = ops.kernel_gradient_bf16(rows, bank, _groups(group_blocks, x.device).offsets, lhs_scale=rows_scale, rhs_scale=bank_scale,
-                                   out_dtype=out_dtype)
+    matrices = None if isinstance(w, (formats.NvFp4, ops.PreparedBank)) else _read_by_the_quantizer(w.transpose(1, 2), "nvfp4")
+    if matrices is None or not (_quantized_in_place(x) and _quantized_in_place(cotangent)):
+        d_x = nvfp4_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
+        return d_x, _nvfp4_transposed_gradient(x.contiguous(), cotangent.contiguous(), group_blocks, out_dtype)
+    x, cotangent = x.contiguous(), cotangent.contiguous()
+    bank = ops.quantize_matrices(matrices, "nvfp4")
+    in_place = _contracted_in_place(x.shape[0], x.shape[1], cotangent.shape[1], group_blocks.offsets.numel() - 1)
+    # the cotangent's two quantizations from one read
+    values, columns, columns_scale, scales = ops.quantize_nvfp4(cotangent, ops.nvfp4_largest(cotangent), rows=True, tokens=in_place, bank=bank)
+    d_x = _nvfp4_product(values, bank.under(scales), group_blocks, x.dtype)
+    if not in_place:
+        return d_x, _nvfp4_transposed_gradient(x, cotangent, group_blocks, out_dtype)
+    _, rows, rows_scale, _ = ops.quantize_nvfp4(x, ops.nvfp4_largest(x), rows=False, tokens=True)
+    d_w = ops.dense_gradient(rows, columns, group_blocks.offsets, lhs_scale=rows_scale, rhs_scale=columns_scale, out_dtype=out_dtype)
     return d_x, d_w
-

@@ -476,6 +476,16 @@ int dew_moe_kernel_gradient_bf16(const void* lhs_t, const dew_moe_bank* rhs_t, c
  * memory; tensor_scale: one device float, written.                                                               */
 int dew_moe_quantize_rows_nvfp4(const void* x /* bf16 [rows, K] */, void* values /* bf16 [rows, K] */,
                                 float* tensor_scale, uint32_t* workspace, int32_t rows, int32_t depth, void* stream);
+/* The same quantizer for an operand that a step quantizes along its rows and its tokens. dew_moe_nvfp4_largest: an operand's partial
+ * largest magnitudes (bf16, or fp32 where is_f32; whole 8 elements, 16-byte aligned), dew_moe_nvfp4_partials() words, every one written.
+ * dew_moe_quantize_nvfp4: x bf16 [rows, K] under the tensor scale of such partials, along its rows
+ * (row_values bf16 [rows, K], or null) and along its tokens where they lie (token_values bf16 [rows, K], or null: a scale every 16 rows
+ * of a column; rows and K whole 128s): the operands of dew_moe_dense_gradient with the tensor scales as its factors. bank_scales (or null):
+ * the [experts] tensor scales of the bank that the rows will multiply; products [experts] receives them times the rows'.      */
+int dew_moe_nvfp4_partials(void);
+int dew_moe_nvfp4_largest(const void* operand, int64_t elements, int32_t is_f32, uint32_t* partials, void* stream);
+int dew_moe_quantize_nvfp4(const void* x, const uint32_t* largest, void* row_values, void* token_values, float* tensor_scale,
+                           const float* bank_scales, float* products, int32_t experts, int32_t rows, int32_t depth, void* stream);
 int dew_moe_quantize_rows_fp8(const void* x /* bf16 [rows, K] */, void* codes /* [rows, K] bytes */,
                               uint8_t* scales /* [rows, P] e8m0 */, int32_t rows, int32_t depth, void* stream);
 int dew_moe_grouped_gemm_fp8_rows(const void* x_codes, const uint8_t* x_scales, const int32_t* gather,
