@@ -381,7 +381,7 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
 // The router and the sort of up to sixteen tokens in one block: a wavefront routes a token and leaves its experts in the LDS,
 // where the whole block then sorts them. They are two launches of 4 to 5 us otherwise, most of either its own latency. (More
 // tokens, several a wavefront, are slower than two launches: some 750 instructions a token on one CU's four SIMDs.)
-// Measured, one token of 128 experts, top 8: 8.3 us, the two launches and the gap between them 9.5.
+// Measured, one token of 128 experts, top 8: 8.8 us with the sort that counts, 6.8 with the one of few slots.
 constexpr int kSortWaves = kSmallThreads / kWave;
 template <int kPerLane>
 __global__ __launch_bounds__(kSmallThreads) void route_and_sort_kernel(RouteParams p, PermuteParams sort) {
@@ -398,7 +398,11 @@ __global__ __launch_bounds__(kSmallThreads) void route_and_sort_kernel(RoutePara
     }
   }
   __syncthreads();
-  sort_small<kSmallThreads>(sort, scratch, [ids](int slot) { return ids[slot]; });
+  auto id_of = [ids](int slot) { return ids[slot]; };
+  if (sort.slots <= kFewSlots)
+    sort_few(sort, id_of);
+  else
+    sort_small<kSmallThreads>(sort, scratch, id_of);
 }
 
 // Each block's shortlist: the `count` best of its best selections (ties to the lower index), one wavefront a block.
@@ -579,7 +583,8 @@ int dew::route_and_sort(const dew_moe_router* router, const float* partial, cons
                            groups + 1};
   const size_t lds = sizeof(int32_t) * (static_cast<size_t>(std::max(kSortWaves * experts, (kSortWaves + 1) * sort.buckets + 1)) + sort.routed);
   static_assert(sizeof(int32_t) * ((kSortWaves + 1) * (kWave * kMaxPerLane + 2) + 1 + kSmallSlots) <= 65536, "the block's LDS");
-  const dim3 grid(1), block(kSmallThreads);
+  // (few slots are sorted by any block: a wavefront a token, and four at least for the offsets)
+  const dim3 grid(1), block(slots <= kFewSlots ? kWave * std::max(tokens, 4) : kSmallThreads);
   if (experts <= 64) {
     hipLaunchKernelGGL(route_and_sort_kernel<1>, grid, block, lds, stream, p, sort);
   } else if (experts <= 128) {

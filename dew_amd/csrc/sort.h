@@ -139,6 +139,36 @@ __device__ __forceinline__ void sort_small(const PermuteParams& p, int32_t* runn
   }
 }
 
+// The same sort of a few slots, a lane a slot, by a block of any size: no counters, no barrier. A slot's place is the number of slots
+// before it in (bucket, slot) order, an offset the number of slots in lower buckets.
+constexpr int kFewSlots = 16;  // (at 45 to 60 slots the walks over them take longer than the counting)
+template <class IdOf>
+__device__ __forceinline__ void sort_few(const PermuteParams& p, IdOf id_of) {
+  const int lane = threadIdx.x % 64;
+  const int bucket = lane >= p.slots ? p.buckets : lane < p.routed ? bucket_of_id(p, id_of(lane)) : p.experts;
+  if (threadIdx.x < 64) {
+    int place = 0;
+    for (int slot = 0; slot < p.slots; ++slot) {
+      const int other = __builtin_amdgcn_readlane(bucket, slot);
+      place += other < bucket || (other == bucket && slot < lane) ? 1 : 0;
+    }
+    if (lane < p.slots) {
+      p.order[place] = lane;
+      p.rows[place] = row_of(p, lane);
+    }
+  }
+  for (int b = threadIdx.x; b - lane <= p.groups; b += blockDim.x) {  // (whole wavefronts: every lane's slot is read)
+    int below = 0, held = 0;
+    for (int slot = 0; slot < p.slots; ++slot) {
+      const int other = __builtin_amdgcn_readlane(bucket, slot);
+      below += other < b ? 1 : 0;
+      held += other == b ? 1 : 0;
+    }
+    if (b <= p.groups) p.offsets[b] = below;
+    if (b < p.groups) p.sizes[b] = held;
+  }
+}
+
 // A decode step's gate and dispatch (layer.hip): the gate's logits as kLogitShares partial sums of the depth,
 // [share][token][expert] (logits.hip), where logit_shares says so; a router that adds them (route.hip); and, for at most
 // kRouteAndSortTokens tokens, that router and the sort as one launch.
