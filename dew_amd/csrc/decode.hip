@@ -7,9 +7,71 @@
 // few, so their fragments come straight from global memory (the lanes past a group's rows read its last row again, the
 // same cache lines). The depth is not split between wavefronts: every sum is taken in the tiled launches' order, so a
 // product's bits do not depend on which of them ran.
+#include <mutex>
+
 #include "gemm.h"
+#include "wide.h"
 
 namespace dew {
+
+constexpr int kFewRows = 32;
+
+// An inclusive sum over the lanes, by lane moves of the vector unit (a sixth of the time of as many trips through the LDS).
+__device__ __forceinline__ int lanes_scanned(int value) {
+  value += __builtin_amdgcn_update_dpp(0, value, 0x111, 0xF, 0xF, false);  // row_shr:1
+  value += __builtin_amdgcn_update_dpp(0, value, 0x112, 0xF, 0xF, false);  // row_shr:2
+  value += __builtin_amdgcn_update_dpp(0, value, 0x114, 0xF, 0xF, false);  // row_shr:4
+  value += __builtin_amdgcn_update_dpp(0, value, 0x118, 0xF, 0xF, false);  // row_shr:8
+  value += __builtin_amdgcn_update_dpp(0, value, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  value += __builtin_amdgcn_update_dpp(0, value, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
+  return value;
+}
+
+// Which expert owns row tile `m_tile` (-1: past the last tile)? Every wavefront scans the groups for itself, 64 a round, without a barrier.
+struct FewTile {
+  int expert, row0, end;      // the tile's first row, its group's end
+  int carried, carried_rows;  // past the last tile: the tiles and (of group sizes) the rows of all groups
+};
+__device__ __forceinline__ FewTile few_tile(const GemmParams& p, int m_tile) {
+  const int lane = threadIdx.x % 64;
+  auto size_of = [&p](int e) { return e >= p.experts ? 0 : p.sizes ? max(p.sizes[e], 0) : p.offsets[e + 1] - p.offsets[e]; };
+  auto first_row_of = [&p](int e) { return e >= p.experts || p.sizes ? 0 : p.offsets[e]; };
+  FewTile tile{-1, 0, 0, 0, 0};
+  int next_size = size_of(lane), next_first = first_row_of(lane);
+  for (int base = 0; base < p.experts; base += 64) {
+    const int size = next_size;
+    int start = next_first;
+    next_size = size_of(base + 64 + lane);
+    next_first = first_row_of(base + 64 + lane);
+    if (p.sizes) {
+      const int rows = lanes_scanned(size);
+      start = tile.carried_rows + rows - size;
+      tile.carried_rows += __builtin_amdgcn_readlane(rows, 63);
+    }
+    const int tiles = (size + kFewRows - 1) / kFewRows, inclusive = lanes_scanned(tiles), first = tile.carried + inclusive - tiles;
+    const unsigned long long hit = __ballot(m_tile >= first && m_tile < first + tiles);
+    if (hit != 0ull) {
+      const int owner = __builtin_ctzll(hit);
+      tile.expert = base + owner;
+      tile.row0 = __builtin_amdgcn_readlane(start + (m_tile - first) * kFewRows, owner);
+      tile.end = __builtin_amdgcn_readlane(start + size, owner);
+      break;
+    }
+    tile.carried += __builtin_amdgcn_readlane(inclusive, 63);
+  }
+  return tile;
+}
+
+// Past the last tile: the rows that no expert owns are zero.
+template <int kOutColumns>
+__device__ __forceinline__ void clear_past_last(const GemmParams& p, int m_tile, const FewTile& tile, int strip, int out_width) {
+  const int tail_begin = (p.sizes ? tile.carried_rows : p.offsets[p.experts]) + (m_tile - tile.carried) * kFewRows;
+  const int tail_end = min(tail_begin + kFewRows, p.rows);
+  for (int item = threadIdx.x; item < (tail_end - tail_begin) * (kOutColumns / 8); item += blockDim.x) {
+    const int sorted = tail_begin + item / (kOutColumns / 8), row = p.scatter ? p.scatter[sorted] : sorted;
+    *reinterpret_cast<u32x4_t*>(p.out + static_cast<size_t>(row) * out_width + strip * kOutColumns + item % (kOutColumns / 8) * 8) = u32x4_t{0, 0, 0, 0};
+  }
+}
 
 template <int FORMAT, int MODE>
 __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
@@ -18,56 +80,18 @@ __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
   constexpr int kMatrices = kPaired ? 2 : 1;
   constexpr int kAtomK = kFp4 ? 64 : kBf16 ? 16 : 32, kAtoms = 64 / kAtomK;  // 16-byte loads a lane makes per matrix and 64 depths
   constexpr int kAhead = kMatrices * kAtoms >= 8 ? 4 : kMatrices * kAtoms >= 4 ? 6 : 8;  // steps of 64 depths in flight
-  constexpr int kRows = 32;
   const int lane = threadIdx.x;
   const int strips = p.width / 32, m_tile = blockIdx.x / strips, strip = blockIdx.x % strips;
 
-  // ---- which expert owns row tile `m_tile`? Every wavefront scans the groups for itself, 64 a round, without a barrier ----
-  auto scanned = [lane](int value) {
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-      const int other = __shfl_up(value, offset, 64);
-      if (lane >= offset) value += other;
-    }
-    return value;
-  };
-  auto size_of = [&p](int e) { return e >= p.experts ? 0 : p.sizes ? max(p.sizes[e], 0) : p.offsets[e + 1] - p.offsets[e]; };
-  auto first_row_of = [&p](int e) { return e >= p.experts || p.sizes ? 0 : p.offsets[e]; };
-  int expert = -1, row0 = 0, end = 0, carried = 0, carried_rows = 0;
-  int next_size = size_of(lane), next_first = first_row_of(lane);
-  for (int base = 0; base < p.experts; base += 64) {
-    const int size = next_size;
-    int start = next_first;
-    next_size = size_of(base + 64 + lane);
-    next_first = first_row_of(base + 64 + lane);
-    if (p.sizes) {
-      const int rows = scanned(size);
-      start = carried_rows + rows - size;
-      carried_rows += __builtin_amdgcn_readlane(rows, 63);
-    }
-    const int tiles = (size + kRows - 1) / kRows, inclusive = scanned(tiles), first = carried + inclusive - tiles;
-    const unsigned long long hit = __ballot(m_tile >= first && m_tile < first + tiles);
-    if (hit != 0ull) {
-      const int owner = __builtin_ctzll(hit);
-      expert = base + owner;
-      row0 = __builtin_amdgcn_readlane(start + (m_tile - first) * kRows, owner);
-      end = __builtin_amdgcn_readlane(start + size, owner);
-      break;
-    }
-    carried += __builtin_amdgcn_readlane(inclusive, 63);
-  }
+  const FewTile tile = few_tile(p, m_tile);
+  const int expert = tile.expert, row0 = tile.row0;
   const int out_width = kGated ? p.width / 2 : p.width;
   constexpr int kOutColumns = kGated ? 16 : 32;
-  if (expert < 0) {  // past the last tile: zero the rows that no expert owns
-    const int tail_begin = (p.sizes ? carried_rows : p.offsets[p.experts]) + (m_tile - carried) * kRows;
-    const int tail_end = min(tail_begin + kRows, p.rows);
-    for (int item = threadIdx.x; item < (tail_end - tail_begin) * (kOutColumns / 8); item += 64) {
-      const int sorted = tail_begin + item / (kOutColumns / 8), row = p.scatter ? p.scatter[sorted] : sorted;
-      *reinterpret_cast<u32x4_t*>(p.out + static_cast<size_t>(row) * out_width + strip * kOutColumns + item % (kOutColumns / 8) * 8) = u32x4_t{0, 0, 0, 0};
-    }
+  if (expert < 0) {
+    clear_past_last<kOutColumns>(p, m_tile, tile, strip, out_width);
     return;
   }
-  const int valid_rows = min(kRows, end - row0);
+  const int valid_rows = min(kFewRows, tile.end - row0);
 
   const int steps = p.depth / 64;
   const int k_atoms = p.depth / kAtomK;
@@ -174,10 +198,218 @@ __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
   }
 }
 
+// Where strips are so few that most CUs have none, a block owns the 32 columns: of a pair each matrix has wavefronts of its own, and
+// kShares wavefronts share a matrix's depth in chunks of four steps, dealt round. Each has its chunks' weights fetched and brought to bf16
+// while the others multiply; what it multiplies it adds to the one before's sums, handed on through the LDS: every sum is still taken in
+// the tiled launches' order. The rows, which are few, are in the LDS.
+// One wavefront for a strip of both matrices spent 19 000 of its 28 000 cycles (2048 deep, FP8 blocks) on what is here 8 turns of 1000, half
+// of them matrix instructions: one token's 8 experts of 2048 x 768 15.0 -> 11.5 us.
+constexpr int kShares = 4, kMostShared = 131072;  // bytes of rows that a block may keep
+constexpr int shared_pitch(int depth) { return depth * 2 + 16; }  // (a row's LDS bytes: 32 rows' pieces on different banks)
+
+template <int FORMAT, int MODE>
+__global__ __launch_bounds__(64 * kShares * (MODE == kSwigluOfTwo ? 2 : 1)) void shared_strips_kernel(GemmParams p) {
+  constexpr bool kPaired = MODE == kSwigluOfTwo, kGated = MODE == kInterleavedGated;
+  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4 || FORMAT == DEW_MOE_W_MXFP4, kBf16 = FORMAT == DEW_MOE_W_BF16;
+  constexpr int kMatrices = kPaired ? 2 : 1;
+  constexpr int kAtomK = kFp4 ? 64 : kBf16 ? 16 : 32, kAtoms = 64 / kAtomK;  // 16-byte loads a lane makes per matrix and 64 depths
+  constexpr int kChunk = 4, kSets = kFp4 ? 3 : 2;  // steps of 64 depths a turn; chunks of weights in flight
+  constexpr int kWaves = kMatrices * kShares;
+  __shared__ f32x4_t handed[kMatrices][4 * 64];  // a matrix's sums on their way from one wavefront to the next, [quad][lane]
+  __shared__ int turn[kMatrices];                // the chunk that they are for
+  extern __shared__ u32x4_t shared_rows[];
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), matrix = wave % kMatrices, share = wave / kMatrices;
+  const int strips = p.width / 32, m_tile = blockIdx.x / strips, strip = blockIdx.x % strips;
+
+  const FewTile tile = few_tile(p, m_tile);
+  const int expert = tile.expert, row0 = tile.row0;
+  const int out_width = kGated ? p.width / 2 : p.width;
+  constexpr int kOutColumns = kGated ? 16 : 32;
+  if (expert < 0) {
+    clear_past_last<kOutColumns>(p, m_tile, tile, strip, out_width);
+    return;
+  }
+  const int valid_rows = min(kFewRows, tile.end - row0);
+
+  const int steps = p.depth / 64, chunks = (steps + kChunk - 1) / kChunk;
+  const int k_atoms = p.depth / kAtomK;
+  const size_t first_atom = (static_cast<size_t>(expert) * strips + strip) * k_atoms;
+  const BankView bank = matrix == 0 ? p.w0 : p.w1;
+  const uint8_t* b_src = bank.codes + first_atom * kAtomBytes + lane * 16;
+  const uint8_t* b_scale_src = kFp4 ? static_cast<const uint8_t*>(bank.scales) + first_atom * 128 + lane * 2 : nullptr;
+  const float* block_scales =
+      FORMAT == DEW_MOE_W_FP8_BLOCK ? static_cast<const float*>(bank.scales) + static_cast<size_t>(expert) * (p.depth / 128) * (p.width / 128) + strip / 4 : nullptr;
+  const int sorted_row = row0 + min(lane % 32, valid_rows - 1);
+  // The tile's rows, 16 bytes a thread at a time: a thread's first piece is asked for behind its weights, the row's index ahead of them
+  // (loads return in order).
+  const int pieces = p.depth / 8, pitch = shared_pitch(p.depth) / 16, row_pieces = valid_rows * pieces;
+  const int first_row = row0 + min(static_cast<int>(threadIdx.x) / pieces, valid_rows - 1), first_source = p.gather ? p.gather[first_row] : first_row;
+  u32x4_t b[kSets][kChunk][kAtoms];
+  uint32_t fp4_bytes[kSets][kChunk];
+  float scale[kSets][kChunk];
+  bf16x8_t fragment[kBf16 ? 1 : kChunk][4];
+  auto load_weights = [&](auto set, int chunk) __attribute__((always_inline)) {
+    constexpr int s = decltype(set)::value;
+    if (chunk >= chunks) return;  // (the same for the wavefront)
+#pragma unroll
+    for (int c = 0; c < kChunk; ++c) {
+      const int step = min(chunk * kChunk + c, steps - 1);  // (past the depth: the last step's again, which multiplies nothing)
+#pragma unroll
+      for (int i = 0; i < kAtoms; ++i)
+        b[s][c][i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(b_src + (static_cast<size_t>(step) * kAtoms + i) * kAtomBytes));
+      if constexpr (kFp4) fp4_bytes[s][c] = *reinterpret_cast<const uint16_t*>(b_scale_src + static_cast<size_t>(step) * 128);
+      if constexpr (FORMAT == DEW_MOE_W_FP8_BLOCK) scale[s][c] = block_scales[static_cast<size_t>(step / 2) * (p.width / 128)];
+    }
+  };
+  static_for<kSets>([&](auto set) { load_weights(set, share + decltype(set)::value * kShares); });
+  const float channel_scale = FORMAT == DEW_MOE_W_FP8_CHANNEL ? static_cast<const float*>(bank.scales)[static_cast<size_t>(expert) * p.width + strip * 32 + lane % 32] : 1.0f;
+  const u32x4_t first_piece = *reinterpret_cast<const u32x4_t*>(p.x + static_cast<size_t>(first_source) * p.depth + threadIdx.x % pieces * 8);
+  // where the rows' results go, asked for behind the first loads
+  const int out_row = p.scatter ? p.scatter[sorted_row] : sorted_row;
+  const float factor0 = kFp4 ? 256.0f * p.w0.tensor_scale[expert] : 1.0f, factor1 = kFp4 && kPaired ? 256.0f * p.w1.tensor_scale[expert] : 1.0f;
+  const int column = strip * 32 + lane % 32;
+  float bias = (!kPaired && p.bias) ? p.bias[static_cast<size_t>(expert) * p.width + column] : 0.0f;
+  if (p.round_bias) bias = bf16_round(bias);
+  auto convert = [&](auto set) __attribute__((always_inline)) {
+    constexpr int s = decltype(set)::value;
+    if constexpr (!kBf16) {
+#pragma unroll
+      for (int c = 0; c < kChunk; ++c)
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+          if constexpr (kFp4) {
+            const float half = (kk < 2 ? __builtin_amdgcn_cvt_f32_fp8(fp4_bytes[s][c], 0) : __builtin_amdgcn_cvt_f32_fp8(fp4_bytes[s][c], 1)) * 0.00390625f;
+            const uint32_t word = b[s][c][0][kk];
+            fragment[c][kk] = FORMAT == DEW_MOE_W_MXFP4 ? fragment_fp4_pow2(word, half) : fragment_fp4(word, half);
+          } else {
+            const u32x4_t& raw = b[s][c][kk / 2 % kAtoms];
+            fragment[c][kk] = fragment_fp8(raw[2 * (kk % 2)], raw[2 * (kk % 2) + 1], FORMAT == DEW_MOE_W_FP8_BLOCK ? scale[s][c] : channel_scale);
+          }
+          asm volatile("" : "+v"(fragment[c][kk]));  // (here, and not where it is multiplied)
+        }
+    }
+  };
+  if (!kBf16 && share < chunks) convert(std::integral_constant<int, 0>{});
+  if (threadIdx.x < kMatrices) turn[threadIdx.x] = 0;
+  if (static_cast<int>(threadIdx.x) < row_pieces) shared_rows[threadIdx.x / pieces * pitch + threadIdx.x % pieces] = first_piece;
+  for (int item = threadIdx.x + 64 * kWaves; item < row_pieces; item += 64 * kWaves) {
+    const int row = item / pieces, piece = item % pieces, source = p.gather ? p.gather[row0 + row] : row0 + row;
+    shared_rows[row * pitch + piece] = *reinterpret_cast<const u32x4_t*>(p.x + static_cast<size_t>(source) * p.depth + piece * 8);
+  }
+  asm volatile("" ::: "memory");  // (a barrier that leaves the loads in flight)
+  __builtin_amdgcn_s_waitcnt(0xF | (3 << 14) | (7 << 4));  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  // slice kk of a step: the 8 depths that the lane's weight bytes of that slice cover
+  const u32x4_t* a_row = shared_rows + min(lane % 32, valid_rows - 1) * pitch;
+  u32x4_t a[2][4];
+  auto fetch = [&](auto into, int step) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kk = 0; kk < 4; ++kk) {
+      const int piece = kFp4 ? 4 * (lane / 32) + kk : kBf16 ? 2 * kk + lane / 32 : 4 * (kk / 2) + 2 * (lane / 32) + kk % 2;
+      a[decltype(into)::value][kk] = a_row[min(step, steps - 1) * 8 + piece];
+    }
+  };
+  f32x16_t acc;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) acc[q] = 0.0f;
+  // the sums of the chunks before, once they are there (the wavefronts of a block run together: each turn comes)
+  auto take = [&](int chunk) __attribute__((always_inline)) {
+    if (chunk == 0) return;
+    while (__hip_atomic_load(&turn[matrix], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != chunk) {
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (8 * i >= valid_rows) break;  // (the same for the wavefront: sums of no row)
+      const f32x4_t quad = handed[matrix][i * 64 + lane];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[4 * i + q] = quad[q];
+    }
+  };
+  auto hand_on = [&](int chunk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (8 * i < valid_rows) handed[matrix][i * 64 + lane] = f32x4_t{acc[4 * i], acc[4 * i + 1], acc[4 * i + 2], acc[4 * i + 3]};
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    if (lane == 0) __hip_atomic_store(&turn[matrix], chunk + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  };
+  auto multiply = [&](auto set, int chunk) __attribute__((always_inline)) {  // (its first rows are fetched)
+    constexpr int s = decltype(set)::value;
+    static_for<kChunk>([&](auto of) __attribute__((always_inline)) {
+      constexpr int c = decltype(of)::value;
+      if (chunk * kChunk + c >= steps) return;
+      if constexpr (c + 1 < kChunk) fetch(std::integral_constant<int, (c + 1) % 2>{}, chunk * kChunk + c + 1);
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) {
+        bf16x8_t weights;
+        if constexpr (kBf16) weights = __builtin_bit_cast(bf16x8_t, b[s][c][kk]);
+        else weights = fragment[c][kk];
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[c % 2][kk]), weights, acc, 0, 0, 0);
+      }
+    });
+  };
+  for (int chunk = share; chunk < chunks;) {
+    static_for<kSets>([&](auto set) __attribute__((always_inline)) {
+      constexpr int s = decltype(set)::value;
+      if (chunk >= chunks) return;
+      if constexpr (!kBf16) load_weights(set, chunk + kSets * kShares);  // (the set's weights are fragments now)
+      fetch(std::integral_constant<int, 0>{}, chunk * kChunk);
+      take(chunk);
+      multiply(set, chunk);
+      hand_on(chunk);
+      if constexpr (kBf16) load_weights(set, chunk + kSets * kShares);
+      chunk += kShares;
+      if (!kBf16 && chunk < chunks) convert(std::integral_constant<int, (s + 1) % kSets>{});
+    });
+  }
+  __syncthreads();
+
+  // ---- a wavefront leaves every kWaves'th of the sixteen sums a lane ----
+#pragma unroll
+  for (int i = 0; i < 16 / kWaves; ++i) {
+    const int q = i * kWaves + wave;
+    if (8 * (q / 4) >= valid_rows) continue;  // (the same for every lane)
+    const int row = 8 * (q / 4) + 4 * (lane / 32) + q % 4;
+    const int to = __shfl(out_row, row, 64);
+    const float sum = handed[0][q / 4 * 64 + lane][q % 4];
+    bf16_t value;
+    if constexpr (kPaired) {
+      value = gated_rounded(sum * factor0, handed[kMatrices - 1][q / 4 * 64 + lane][q % 4] * factor1, p.limit, p.gating);
+    } else if constexpr (kGated) {  // an even lane holds a gate column, the odd one beside it its up column
+      const float mine = bf16_round(sum * factor0 + bias);
+      const float other = __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, mine), 0xB1, 0xF, 0xF, true));
+      value = gated_pair_rounded(mine, other, p.limit);
+    } else {
+      value = f32_to_bf16(sum * factor0 + bias);
+    }
+    if (row < valid_rows && (!kGated || lane % 2 == 0)) p.out[static_cast<size_t>(to) * out_width + (kGated ? column / 2 : column)] = value;
+  }
+}
+
 template <int FORMAT, int MODE>
 static int launch_few(const char* who, const GemmParams& p, hipStream_t stream) {
   // every expert with rows ends in one partial tile, and the rows no expert owns fill tiles behind them
   const int tiles = min(p.rows, p.rows / 32 + p.experts + 1), blocks = tiles * (p.width / 32);
+  // Shared strips: formats whose conversion costs more than the product, deep enough that the hand-overs are few beside it, and one round
+  // of blocks (us of a layer's pass, a wavefront a strip and shared: FP8 blocks, one token's 8 experts of 2048 x 768 31.5 and 28.2, 7 tokens
+  // on 8 experts of 1792 x 768 28.2 and 24.0; NVFP4, 2 tokens, 4 experts of 1792 x 5120 42.3 and 39.9; 640 deep 25.6 and 26.9; one
+  // matrix, 1536 deep 25.9 and 27.2; MXFP4,
+  // whose conversion is one instruction for two codes, 1408 deep 37.7 and 40.5; bf16, which has none, 1152 deep 23.6 and 25.7).
+  if constexpr (FORMAT == DEW_MOE_W_FP8_BLOCK || FORMAT == DEW_MOE_W_FP8_CHANNEL || FORMAT == DEW_MOE_W_NVFP4) {
+    constexpr int kMatrices = MODE == kSwigluOfTwo ? 2 : 1;
+    const int touched = min(p.rows, p.experts) + p.rows / 32;  // the tiles that have rows, at most
+    const size_t rows_bytes = static_cast<size_t>(min(p.rows, 32)) * shared_pitch(p.depth);
+    if (p.depth >= (kMatrices == 2 ? 1024 : 4096) && touched * static_cast<long long>(p.width / 32) * kMatrices <= 512 && rows_bytes <= kMostShared) {
+      auto kernel = shared_strips_kernel<FORMAT, MODE>;
+      static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
+      static hipError_t reserved = hipSuccess;
+      std::call_once(configured, [&] { reserved = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kMostShared); });
+      if (reserved != hipSuccess) return fail(DEW_MOE_ELAUNCH, "%s: cannot reserve %d bytes of LDS", who, kMostShared);
+      hipLaunchKernelGGL(kernel, dim3(blocks), dim3(64 * kMatrices * kShares), rows_bytes, stream, p);
+      return launched(who);
+    }
+  }
   hipLaunchKernelGGL((few_tiles_kernel<FORMAT, MODE>), dim3(blocks), dim3(64), 0, stream, p);
   return launched(who);
 }
