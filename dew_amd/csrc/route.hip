@@ -579,8 +579,7 @@ int dew::route_and_sort(const dew_moe_router* router, const float* partial, cons
   p.shares = 1;
   p.gate_bias = gate_bias;
   const int groups = experts + (shared ? 1 : 0);
-  const PermuteParams sort{nullptr, sizes, offsets, order, rows, nullptr, nullptr, slots, tokens * router->top_k, experts, groups, router->top_k, 1,
-                           groups + 1};
+  const PermuteParams sort{nullptr, sizes, offsets, order, rows, nullptr, slots, tokens * router->top_k, experts, groups, router->top_k, 1, groups + 1, slots};
   const size_t lds = sizeof(int32_t) * (static_cast<size_t>(std::max(kSortWaves * experts, (kSortWaves + 1) * sort.buckets + 1)) + sort.routed);
   static_assert(sizeof(int32_t) * ((kSortWaves + 1) * (kWave * kMaxPerLane + 2) + 1 + kSmallSlots) <= 65536, "the block's LDS");
   // (few slots are sorted by any block: a wavefront a token, and four at least for the offsets)

@@ -13,11 +13,10 @@ struct PermuteParams {
   int32_t* order;      // [slots]
   int32_t* rows;       // [slots]
   int32_t* counts;     // workspace [blocks][buckets]
-  int32_t* bases;      // workspace [blocks][buckets]
   // `slots` sorted positions: the `routed` = tokens * top_k slots of `ids`, then `slots - routed` rows that every token
   // sends to one always-on (shared) expert, which sorts as group `experts`. `groups` = the groups written (experts, or
   // experts + 1 with a shared one); bucket `groups` collects the dropped slots (an id outside [0, experts)), last.
-  int slots, routed, experts, groups, top_k, blocks, buckets;
+  int slots, routed, experts, groups, top_k, blocks, buckets, slots_a_block;
 };
 
 __device__ __forceinline__ int bucket_of_id(const PermuteParams& p, int id) { return (id < 0 || id >= p.experts) ? p.groups : id; }
@@ -31,12 +30,63 @@ __device__ __forceinline__ int row_of(const PermuteParams& p, int slot) {
   return slot < p.routed ? slot / p.top_k : slot - p.routed;
 }
 
+// The exclusive scan of `buckets` totals by one wavefront, 64 a round; totals[buckets] is their sum.
+__device__ __forceinline__ void scan_buckets(int32_t* totals, int buckets) {
+  const int lane = threadIdx.x % 64;
+  int carried = 0;
+  for (int base = 0; base < buckets; base += 64) {
+    const int b = base + lane;
+    const int size = b < buckets ? totals[b] : 0;
+    int inclusive = size;
+#pragma unroll
+    for (int offset = 1; offset < 64; offset <<= 1) {
+      const int other = __shfl_up(inclusive, offset, 64);
+      if (lane >= offset) inclusive += other;
+    }
+    if (b < buckets) totals[b] = carried + inclusive - size;
+    carried += __shfl(inclusive, 63, 64);
+  }
+  if (lane == 0) totals[buckets] = carried;
+}
+
+// A wavefront's 64 slots to their places: ranked among themselves, behind the wavefront's running positions `mine`. A lane without a slot
+// has bucket `buckets`.
+__device__ __forceinline__ void place_round(const PermuteParams& p, int slot, int bucket, int bits, int32_t* mine) {
+  const int lane = threadIdx.x % 64;
+  const bool valid = bucket < p.buckets;
+  unsigned long long same = __ballot(valid);
+  for (int bit = 0; bit < bits; ++bit) {
+    const bool set = (bucket >> bit) & 1;
+    const unsigned long long vote = __ballot(set);
+    same &= set ? vote : ~vote;
+  }
+  const int rank = __popcll(same & ((1ull << lane) - 1ull));
+  const int count = __popcll(same);
+  int position = 0;
+  if (valid) position = mine[bucket] + rank;
+  // The running positions are the wavefront's own (no other wavefront touches them), so no block barrier is needed,
+  // only an order between this wavefront's lanes: every lane's read above before the one lane's write below, and that
+  // write before the next round's reads. The wavefront-scope fences state that order to the compiler and the memory
+  // model (they cost no instruction: a wavefront's LDS operations are issued and served in order).
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (valid && rank == count - 1) mine[bucket] = position + 1;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  if (valid) {
+    p.order[position] = slot;
+    p.rows[position] = row_of(p, slot);
+  }
+}
+
 // The whole sort in one block for at most kSmallSlots slots (a decode step, a small prefill): the block
 // counts, scans and scatters, each wavefront a contiguous run of the slots, with the LDS histogram as the only
 // intermediate.
 // Measured under graph replay, sixteen wavefronts: 2048 slots 5.1 to 6.8 us (four wavefronts: 7.9 to 10.0), 4096 slots
-// 7.5 us against 11.4 us for the three launches, 8192 slots the same either way.
-constexpr int kSmallSlots = 4096;      // beyond this three launches over many blocks are as fast or faster
+// 7.5 us.
+constexpr int kSmallSlots = 4096;      // beyond this two launches over many blocks are as fast or faster
 constexpr int kSmallThreads = 1024;    // sixteen wavefronts, where their counters fit the LDS a launch may take unasked
 constexpr int kNarrowSmallSlots = 2048;  // the four-wavefront form's reach, for more buckets than that
 // `running`: LDS, [THREADS / 64][buckets] then [buckets + 1] totals. `id_of(slot)`: a routed slot's expert.
@@ -70,22 +120,7 @@ __device__ __forceinline__ void sort_small(const PermuteParams& p, int32_t* runn
     totals[b] = sum;
   }
   __syncthreads();
-  if (threadIdx.x < 64) {  // exclusive scan of the bucket totals by one wavefront, 64 buckets a round
-    int carried = 0;
-    for (int base = 0; base < p.buckets; base += 64) {
-      const int b = base + lane;
-      const int size = b < p.buckets ? totals[b] : 0;
-      int inclusive = size;
-#pragma unroll
-      for (int offset = 1; offset < 64; offset <<= 1) {
-        const int other = __shfl_up(inclusive, offset, 64);
-        if (lane >= offset) inclusive += other;
-      }
-      if (b < p.buckets) totals[b] = carried + inclusive - size;
-      carried += __shfl(inclusive, 63, 64);
-    }
-    if (lane == 0) totals[p.buckets] = carried;
-  }
+  if (threadIdx.x < 64) scan_buckets(totals, p.buckets);
   __syncthreads();
   for (int b = threadIdx.x; b < p.buckets; b += THREADS) {
     const int start = totals[b];
@@ -109,33 +144,7 @@ __device__ __forceinline__ void sort_small(const PermuteParams& p, int32_t* runn
   for (int round = 0; round < kMaxRounds; ++round) {
     if (round >= rounds) continue;  // (the same for the whole block)
     const int slot = wave_begin + round * 64 + lane;
-    const int bucket = kept[round];
-    const bool valid = bucket < p.buckets;
-    unsigned long long same = __ballot(valid);
-    for (int bit = 0; bit < bits; ++bit) {
-      const bool set = (bucket >> bit) & 1;
-      const unsigned long long vote = __ballot(set);
-      same &= set ? vote : ~vote;
-    }
-    const int rank = __popcll(same & ((1ull << lane) - 1ull));
-    const int count = __popcll(same);
-    int position = 0;
-    if (valid) position = mine[bucket] + rank;
-    // The running positions are the wavefront's own (no other wavefront touches them), so no block barrier is needed,
-    // only an order between this wavefront's lanes: every lane's read above before the one lane's write below, and that
-    // write before the next round's reads. The wavefront-scope fences state that order to the compiler and the memory
-    // model (they cost no instruction: a wavefront's LDS operations are issued and served in order).
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (valid && rank == count - 1) mine[bucket] = position + 1;
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    if (valid) {
-      p.order[position] = slot;
-      p.rows[position] = row_of(p, slot);
-    }
+    place_round(p, slot, kept[round], bits, mine);
   }
 }
 
