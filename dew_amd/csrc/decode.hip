@@ -16,17 +16,6 @@ namespace dew {
 
 constexpr int kFewRows = 32;
 
-// An inclusive sum over the lanes, by lane moves of the vector unit (a sixth of the time of as many trips through the LDS).
-__device__ __forceinline__ int lanes_scanned(int value) {
-  value += __builtin_amdgcn_update_dpp(0, value, 0x111, 0xF, 0xF, false);  // row_shr:1
-  value += __builtin_amdgcn_update_dpp(0, value, 0x112, 0xF, 0xF, false);  // row_shr:2
-  value += __builtin_amdgcn_update_dpp(0, value, 0x114, 0xF, 0xF, false);  // row_shr:4
-  value += __builtin_amdgcn_update_dpp(0, value, 0x118, 0xF, 0xF, false);  // row_shr:8
-  value += __builtin_amdgcn_update_dpp(0, value, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
-  value += __builtin_amdgcn_update_dpp(0, value, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
-  return value;
-}
-
 // Which expert owns row tile `m_tile` (-1: past the last tile)? Every wavefront scans the groups for itself, 64 a round, without a barrier.
 struct FewTile {
   int expert, row0, end;      // the tile's first row, its group's end

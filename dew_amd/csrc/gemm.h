@@ -112,6 +112,17 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_each(std::make_integer_sequence<int, N>{}, f);
 }
 
+// An inclusive sum over the lanes, by lane moves of the vector unit (a sixth of the time of as many trips through the LDS).
+__device__ __forceinline__ int lanes_scanned(int value) {
+  value += __builtin_amdgcn_update_dpp(0, value, 0x111, 0xF, 0xF, false);  // row_shr:1
+  value += __builtin_amdgcn_update_dpp(0, value, 0x112, 0xF, 0xF, false);  // row_shr:2
+  value += __builtin_amdgcn_update_dpp(0, value, 0x114, 0xF, 0xF, false);  // row_shr:4
+  value += __builtin_amdgcn_update_dpp(0, value, 0x118, 0xF, 0xF, false);  // row_shr:8
+  value += __builtin_amdgcn_update_dpp(0, value, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1, 3
+  value += __builtin_amdgcn_update_dpp(0, value, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2, 3
+  return value;
+}
+
 // The launch for few tiles of few rows (decode.hip); `mode`: kPlain, kSwigluOfTwo or kInterleavedGated.
 int launch_few_tiles(const char* who, const GemmParams& p, int format, int mode, hipStream_t stream);
 

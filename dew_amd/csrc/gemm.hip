@@ -175,8 +175,6 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   constexpr int kSets = (kFp8A && BN == 256) ? 2 : (kSplit && !kFp8A && BM == 128) ? 2 : ((kBf16 && BM > 64) || (!kFp4 && !kBf16 && BM == 128 && kMatrices * BN == 256)) ? 3 : 4;
 
   extern __shared__ u32x4_t lds[];  // a ring of three stages of A: BM rows of 128 bytes each
-  __shared__ int wave_tiles[4], wave_rows[4];
-  __shared__ int found[5];  // expert, first sorted row of the tile, total m-tiles, the expert's last row + 1, rows in all groups
   // FP8 128 x 128 blocks: the scales of the block's column blocks down the whole depth, read once
   constexpr int kScaleColumns = kBlockBank ? kMatrices * (BN / 128) : 1;
   __shared__ float depth_scales[kScaleColumns][kBlockBank ? kMaxDepthBlocks : 1];
@@ -203,38 +201,24 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   const int m_tile = group * kGroupM + within % group_m;
   const int n0 = (within / group_m) * BN;
 
-  // ---- which expert owns m-tile `m_tile`? inclusive scan of ceil(size / BM) over the experts (and, where the caller
-  // gave group sizes instead of their prefix, of the sizes themselves: an expert's first row) ----
-  if (tid == 0) found[0] = -1;
-  int carried = 0, carried_rows = 0;
-  // (a round's sizes and first rows are asked for one round ahead: past 256 experts the rounds' loads then overlap, instead
-  // of one memory round trip a round in front of every tile)
+  // ---- which expert owns m-tile `m_tile`? inclusive scan of ceil(size / BM) over the experts (and, where the caller gave group sizes
+  // instead of their prefix, of the sizes themselves: an expert's first row), by every wavefront for itself, 64 experts a round, without
+  // the LDS and its barriers. A round's sizes and first rows are asked for one round ahead ----
   auto size_of = [&](int e) { return e >= p.experts ? 0 : kWindow ? p.window_rows : p.sizes ? max(p.sizes[e], 0) : p.offsets[e + 1] - p.offsets[e]; };
   auto first_row_of = [&](int e) { return e >= p.experts || (p.sizes && !kWindow) ? 0 : kWindow ? e * p.window_rows : p.offsets[e]; };
-  int next_size = size_of(tid), next_first_row = first_row_of(tid);
-  for (int base = 0; base < p.experts; base += kThreads) {
-    const int e = base + tid;
-    int start = 0, tiles = 0;
-    const int size = next_size, first_row = next_first_row;
-    next_size = size_of(e + kThreads);
-    next_first_row = first_row_of(e + kThreads);
+  int expert = -1, row0 = 0, group_end = 0, carried = 0, carried_rows = 0;  // past the last tile: the tiles and (of sizes) the rows of all groups
+  int next_size = size_of(lane), next_first_row = first_row_of(lane);
+  for (int base = 0; base < p.experts; base += 64) {
+    const int size = next_size, e = base + lane;
+    int start = next_first_row, tiles = 0;
+    next_size = size_of(e + 64);
+    next_first_row = first_row_of(e + 64);
     if (p.sizes && !kWindow) {  // (uniform) exclusive prefix of the sizes
-      int inclusive_rows = size;
-#pragma unroll
-      for (int offset = 1; offset < 64; offset <<= 1) {
-        const int other = __shfl_up(inclusive_rows, offset, 64);
-        if (lane >= offset) inclusive_rows += other;
-      }
-      __syncthreads();
-      if (lane == 63) wave_rows[wave] = inclusive_rows;
-      __syncthreads();
-      start = carried_rows + inclusive_rows - size;
-      for (int w = 0; w < wave; ++w) start += wave_rows[w];
-      carried_rows += wave_rows[0] + wave_rows[1] + wave_rows[2] + wave_rows[3];
-    } else {
-      start = first_row;
+      const int rows = lanes_scanned(size);
+      start = carried_rows + rows - size;
+      carried_rows += __builtin_amdgcn_readlane(rows, 63);
     }
-    const int group_end = start + size;
+    const int end = start + size;
     if (e < p.experts) {
       if (p.tail_of > 0) {
         const int rest = size % p.tail_of;
@@ -244,36 +228,22 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
         tiles = size / BM + (size % BM > p.skip_tails ? 1 : 0);
       }
     }
-    int inclusive = tiles;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-      const int other = __shfl_up(inclusive, offset, 64);
-      if (lane >= offset) inclusive += other;
+    const int inclusive = lanes_scanned(tiles), first = carried + inclusive - tiles;
+    const unsigned long long hit = __ballot(m_tile >= first && m_tile < first + tiles);
+    if (hit != 0ull) {
+      const int owner = __builtin_ctzll(hit);
+      expert = base + owner;
+      row0 = __builtin_amdgcn_readlane(start + (m_tile - first) * BM, owner);
+      group_end = __builtin_amdgcn_readlane(end, owner);
+      break;
     }
-    __syncthreads();
-    if (lane == 63) wave_tiles[wave] = inclusive;
-    __syncthreads();
-    int before = carried;
-    for (int w = 0; w < wave; ++w) before += wave_tiles[w];
-    const int first = before + inclusive - tiles;
-    if (tiles > 0 && m_tile >= first && m_tile < first + tiles) {
-      found[0] = e;
-      found[1] = start + (m_tile - first) * BM;
-      found[3] = group_end;
-    }
-    carried += wave_tiles[0] + wave_tiles[1] + wave_tiles[2] + wave_tiles[3];
+    carried += __builtin_amdgcn_readlane(inclusive, 63);
   }
-  if (tid == 0) {
-    found[2] = carried;
-    found[4] = p.sizes ? carried_rows : 0;  // the rows the groups hold (read from the prefix's last entry otherwise)
-  }
-  __syncthreads();
-  const int expert = found[0];
 
   if (expert < 0) {
     if (kWindow || p.tail_of > 0) return;  // (the taller tiles' launch zeroes them; a kernel gradient has no rows past its groups)
     // Past the last real tile: zero the rows no expert owns (sorted positions offsets[E] .. rows).
-    const int tail_begin = (p.sizes ? found[4] : p.offsets[p.experts]) + (m_tile - found[2]) * BM;
+    const int tail_begin = (p.sizes ? carried_rows : p.offsets[p.experts]) + (m_tile - carried) * BM;
     const int tail_end = min(tail_begin + BM, p.rows);
     const int out_width = kGated ? p.width / 2 : p.width, out_n0 = kGated ? n0 / 2 : n0;
     for (int item = tid; item < (tail_end - tail_begin) * (kOutBN / 8); item += kThreads) {
@@ -288,8 +258,7 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
     return;
   }
 
-  const int row0 = found[1];
-  const int valid_rows = min(BM, found[3] - row0);
+  const int valid_rows = min(BM, group_end - row0);
   // a kernel gradient's group contracts its own whole steps of the depth (128 tokens of e4m3 codes, 64 of bf16)
   const int first_step = kWindow ? min(max(p.windows[expert], 0), p.depth) / kStepDepth : 0;
   const int steps = kWindow ? max(min(max(p.windows[expert + 1], 0), p.depth) / kStepDepth - first_step, 0) : p.depth / kStepDepth;

@@ -37,14 +37,6 @@ struct WideTiles {
 
   __device__ __forceinline__ void find(const int32_t* offsets, const int32_t* sizes, int groups, int outer_m, int outer_n) {
     const int lane = threadIdx.x % 64;
-    auto scanned = [lane](int value) {
-#pragma unroll
-      for (int offset = 1; offset < 64; offset <<= 1) {
-        const int other = __shfl_up(value, offset, 64);
-        if (lane >= offset) value += other;
-      }
-      return value;
-    };
     gradient_tiles = (outer_m + kWideTile - 1) / kWideTile;
     int m_tiles = 0;
     held = 0;
@@ -56,7 +48,7 @@ struct WideTiles {
       if (64 * round < groups) {
         const int size = g >= groups ? 0 : sizes ? max(sizes[g], 0) : max(offsets[g + 1] - offsets[g], 0);
         const int tiles = g >= groups ? 0 : kGradient ? gradient_tiles : (size + kWideTile - 1) / kWideTile;
-        const int rows = scanned(size), inclusive = scanned(tiles);
+        const int rows = lanes_scanned(size), inclusive = lanes_scanned(tiles);
         if (g < groups) {
           first_tile[round] = m_tiles + inclusive - tiles;
           first_row[round] = sizes ? held + rows - size : offsets[g];
