@@ -117,9 +117,32 @@ __device__ __forceinline__ void clear_sums(f32x16_t (&acc)[4][4]) {
     }
 }
 
+// v[g] of lane 4 m + l becomes v[l] of lane 4 m + g.
+__device__ __forceinline__ void across_quads(uint32_t (&v)[4]) {
+  const int lane = threadIdx.x;
+#pragma unroll
+  for (int g = 0; g < 4; g += 2) {
+    const uint32_t a = v[g], b = v[g + 1];
+    const uint32_t a_beside = __builtin_amdgcn_mov_dpp(a, 0xB1, 0xF, 0xF, true), b_beside = __builtin_amdgcn_mov_dpp(b, 0xB1, 0xF, 0xF, true);  // quad_perm 1 0 3 2
+    v[g] = lane & 1 ? b_beside : a;
+    v[g + 1] = lane & 1 ? b : a_beside;
+  }
+#pragma unroll
+  for (int g = 0; g < 2; ++g) {
+    const uint32_t a = v[g], b = v[g + 2];
+    const uint32_t a_beside = __builtin_amdgcn_mov_dpp(a, 0x4E, 0xF, 0xF, true), b_beside = __builtin_amdgcn_mov_dpp(b, 0x4E, 0xF, 0xF, true);  // quad_perm 2 3 0 1
+    v[g] = lane & 2 ? b_beside : a;
+    v[g + 2] = lane & 2 ? b : a_beside;
+  }
+}
+
 // A wavefront's 128 x 128 sums leave from registers, without the LDS and without a barrier. The operands entered the instruction the
-// other way round: acc[i][j][q] is row lane % 32, column 8 (q / 4) + 4 (lane / 32) + q % 4 of its 32 x 32 tile, and two exchanges between
-// lane groups make a lane's sums 16 bytes of a row. `out_row0`, `valid_rows`: the block's tile (what lies past the buffer's end, the rows
+// other way round: acc[i][j][q] is row lane % 32, column 8 (q / 4) + 4 (lane / 32) + q % 4 of its 32 x 32 tile. One exchange between the
+// halves of the wavefront makes a lane's sums whole pieces of 16 bytes of its row, in the left or the right of two tiles, and another within
+// four lanes puts four such pieces of a row into neighbours: a store is sixteen runs of 64 bytes, both halves of eight 128-byte lines (f32:
+// halves of sixteen). Stores of a row a lane, 16 bytes 64 apart, cost the L2 more than these exchanges do: us of a kernel gradient, eight
+// steps and a store a tile, FP8, 32 768 tokens of 32 x 7168 x 2048, 561 -> 526 (396 without any store), of 8 x 4096 x 14 336 1510 -> 1487;
+// of products, deeper, 1 to 2 % less. `out_row0`, `valid_rows`: the block's tile (what lies past the buffer's end, the rows
 // past its last, and the columns sent there are not stored); `tile_row`, `column0`: the wavefront's place in it and in the row.
 template <bool kOutF32>
 __device__ __forceinline__ void leave(f32x16_t (&acc)[4][4], void* to_rows, size_t out_row0, int valid_rows, int width, int tile_row, int column0, float factor) {
@@ -139,42 +162,41 @@ __device__ __forceinline__ void leave(f32x16_t (&acc)[4][4], void* to_rows, size
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     stay(i);
-    const int row = tile_row + 32 * i;
+    const uint32_t row = tile_row + 32 * i + lane % 32 / 4 * 4;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if constexpr (kOutF32) {
-        const int column = column0 + 32 * j + 4 * (lane / 32);
+    for (int pair = 0; pair < 2; ++pair) {
+      // the lane's row of tile 2 pair + lane / 32, in pieces of 16 bytes
+      constexpr int kPieces = kOutF32 ? 8 : 4;
+      uint32_t pieces[kPieces][4];
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const uint32_t to = column + 8 * g < width ? ((row + lane % 32) * width + column + 8 * g) * 4 : kNowhere;
-          __builtin_amdgcn_raw_buffer_store_b128(
-              __builtin_bit_cast(u32x4_t, f32x4_t{acc[i][j][4 * g] * factor, acc[i][j][4 * g + 1] * factor, acc[i][j][4 * g + 2] * factor, acc[i][j][4 * g + 3] * factor}),
-              out, to, 0, 0);
+      for (int q = 0; q < 16; q += kOutF32 ? 1 : 2) {
+        uint32_t words[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const f32x16_t& sums = acc[i][2 * pair + t];
+          words[t] = kOutF32 ? __float_as_uint(sums[q] * factor) : pack_bf16(sums[q] * factor, sums[q + (kOutF32 ? 0 : 1)] * factor);
         }
-      } else {
-        uint32_t words[2][4];  // after the first exchange: [k][..] is columns 8 (2 k + lane / 32) .. + 7 of row lane % 32
+        const auto swapped = __builtin_amdgcn_permlane32_swap(words[0], words[1], false, false);
+        const int piece = kOutF32 ? q / 4 * 2 : q / 4, word = kOutF32 ? q % 4 : q % 4 / 2;
+        pieces[piece][word] = swapped[0];
+        pieces[piece + (kOutF32 ? 1 : 0)][word + (kOutF32 ? 0 : 2)] = swapped[1];
+      }
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
+      for (int four = 0; four < kPieces; four += 4) {
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const int q = 8 * k + 2 * h;
-            const auto swapped = __builtin_amdgcn_permlane32_swap(pack_bf16(acc[i][j][q] * factor, acc[i][j][q + 1] * factor),
-                                                                  pack_bf16(acc[i][j][q + 4] * factor, acc[i][j][q + 5] * factor), false, false);
-            words[k][h] = swapped[0];
-            words[k][2 + h] = swapped[1];
-          }
+        for (int word = 0; word < 4; ++word) {
+          uint32_t v[4];
 #pragma unroll
-        for (int d = 0; d < 4; ++d) {  // after the second: row 16 k + lane % 16, columns 8 ((lane >> 4 & 1) * 2 + lane / 32) .. + 7
-          const auto swapped = __builtin_amdgcn_permlane16_swap(words[0][d], words[1][d], false, false);
-          words[0][d] = swapped[0];
-          words[1][d] = swapped[1];
+          for (int g = 0; g < 4; ++g) v[g] = pieces[four + g][word];
+          across_quads(v);
+#pragma unroll
+          for (int g = 0; g < 4; ++g) pieces[four + g][word] = v[g];
         }
-        const int column = column0 + 32 * j + 8 * ((lane >> 4 & 1) * 2 + lane / 32);
-        const uint32_t to = column < width ? ((row + lane % 16) * width + column) * 2 : kNowhere;
-        const uint32_t sixteen_rows = column < width ? 16 * width * 2 : 0;
+        const int column = column0 + 64 * pair + 32 * (lane / 32) + (16 / kOutBytes) * (four + lane % 4);
+        const uint32_t to = column < width ? (row * width + column) * kOutBytes : kNowhere, next_row = column < width ? width * kOutBytes : 0;
 #pragma unroll
-        for (int k = 0; k < 2; ++k)
-          __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{words[k][0], words[k][1], words[k][2], words[k][3]}, out, to + k * sixteen_rows, 0, 0);
+        for (int g = 0; g < 4; ++g)
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{pieces[four + g][0], pieces[four + g][1], pieces[four + g][2], pieces[four + g][3]}, out, to + g * next_row, 0, 0);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
