@@ -1314,7 +1314,7 @@ static bool few_gradient_blocks(const GemmParams& p) {
 // The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered: where such
 // tiles keep the CUs busy over the rounds they take. Measured against the launches below on 70 shapes (512 to 32 768 rows, 1 to 51 groups,
 // extents 512 to 14 336; us, there and here): [32 768, 7168] x 2048 of 32 groups, blockwise, forward 470 and 424, input's gradient 520 and
-// 444, kernel's gradient 692 and 565; [32 768, 4096] x 14336 of 8, MXFP8, 1636 and 1500, 1600 and 1470, 1637 and 1470; [12 672, 512] x 3456
+// 444, kernel's gradient 692 and 530; [32 768, 4096] x 14336 of 8, MXFP8, 1636 and 1490, 1600 and 1460, 1637 and 1450; [12 672, 512] x 3456
 // of 21 70 and 39; [4608, 896] x 7552 of 33, kernel's gradient, 220 and 125. At rounds filled to 0.56 .. 0.7 1.02 to 1.2 times as fast, in one
 // round from 0.66 on 1.1 to 1.7; at 260 tiles, two rounds, 0.77 to 0.89.
 static bool fills_wide_rounds(double tiles, int percent_of_one, int percent_of_more) {

@@ -14,11 +14,11 @@
 //  * Everything between two matrix instructions is placed by hand (`phase`): one wavefront a SIMD issues an instruction every four
 //    cycles, eight a matrix instruction, and what stood between the phases was time the pipe lost.
 //  * The operands enter the instruction the other way round, so that a lane holds four neighbouring columns of a row; two exchanges
-//    between lane groups make them 64 bytes a row, and the tile leaves from registers, without the LDS and without a barrier.
+//    between lanes make them runs of 64 bytes, and the tile leaves from registers, without the LDS and without a barrier (wide.h).
 //
-// us, in 128 x 256 tiles and here: 16 384 x 4096 x 4096 forward 468 and 409 (1.34 PFLOP/s; the pipe 74 % busy at 1.66 GHz, the power
-// limit, without the loads 1.62), input's gradient 534 and 395, kernel's gradient 491 and 393; 10 007 rows of 16 x 2048 x 4096 223
-// and 161, 230 and 190 (1.5 rounds of tiles), 216 and 191 (268 MB written).
+// us, in 128 x 256 tiles and here: 16 384 x 4096 x 4096 forward 517 and 445 (on another box 468 and 409, 1.34 PFLOP/s; the pipe 74 % busy
+// at 1.66 GHz, the power limit, without the loads 1.62), input's gradient 543 and 404, kernel's gradient 498 and 403; 10 007 rows of 16 x
+// 2048 x 4096 187 and 165, 235 and 183 (1.5 rounds of tiles), 215 and 178 (268 MB written).
 #include <mutex>
 
 #include "dense.h"
