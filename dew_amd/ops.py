@@ -268,16 +268,23 @@ class PreparedBank:
     def experts(self):
         return self.shape[0]
 
+    def _carries_tensor_scales(self):
+        if self.descriptor.format not in (_lib.W_NVFP4, _lib.W_MXFP4):
+            raise KernelError("only an NVFP4 bank carries tensor scales")
+
     def scaled(self, by: torch.Tensor) -> "PreparedBank":
         """The same NVFP4 bank with every expert's tensor scale times `by` (a one-element device tensor): how a
         product of two NVFP4 operands owes both tensor scales to its fp32 sums."""
-        if self.descriptor.format not in (_lib.W_NVFP4, _lib.W_MXFP4):
-            raise KernelError("only an NVFP4 bank carries tensor scales")
+        self._carries_tensor_scales()
         own = self.keep[2].reshape(-1)[self.first:self.first + self.experts]  # a layer's experts within its stack's scales
         return self.under((own.to(torch.float32) * by.to(torch.float32)).contiguous())
 
     def under(self, scales: torch.Tensor) -> "PreparedBank":
         """The same NVFP4 bank under other tensor scales, fp32 `[experts]`."""
+        self._carries_tensor_scales()
+        if scales.numel() != self.experts:    # (a launch reads one for each of the bank's experts)
+            raise KernelError(f"{scales.numel()} tensor scales for the bank's {self.experts} experts")
+        _device(scales, "scales", torch.float32)
         held = self.descriptor
         view = _lib.Bank(held.format, held.layout, held.experts, held.depth, held.width, held.codes, held.scales, _ptr(scales))
         return PreparedBank(view, self.shape, (self.keep[0], self.keep[1], scales), 0)
@@ -920,6 +927,13 @@ def quantize_nvfp4(x: torch.Tensor, largest: torch.Tensor, *, rows: bool, tokens
     """`x [R, K]` bf16 in NVFP4 along its rows (`quantize_rows_nvfp4`'s values) and, or, along its tokens where they lie (a scale every
     16 rows of a column), from one read of it and `nvfp4_largest`'s `largest`: (row values or None, token values or None, tensor scale
     fp32 `[1]`, the tensor scales of `bank`, which the rows will multiply, times it, or None)."""
+    if x.dim() != 2:
+        raise KernelError(f"x is {tuple(x.shape)}, not [rows, depth]")
+    words = _lib.library().dew_moe_nvfp4_partials()
+    if largest.numel() != words:    # (every one of them is read)
+        raise KernelError(f"largest has {largest.numel()} words, not nvfp4_largest's {words}")
+    if bank is not None:
+        bank._carries_tensor_scales()
     _device(x, "x", torch.bfloat16), _device(largest, "largest", torch.int32)
     by_row, by_token = (torch.empty_like(x) if wanted else None for wanted in (rows, tokens))
     scale = torch.empty(1, dtype=torch.float32, device=x.device)

@@ -98,3 +98,44 @@ def test_the_float32_gate_and_a_latent_layers_projections_refuse_on_the_host():
         layer._bound(variables, ())._dense(x, "routed_expert_down_proj", 64, 16)
     with pytest.raises(KeyError, match="routed_expert_up_proj"):
         layer._bound(variables, ())._dense(x, "routed_expert_up_proj", 32, 64)
+
+
+@pytest.mark.parametrize("words", [0, 1, 511, 513])
+def test_nvfp4_magnitudes_of_another_length_are_refused(words):
+    """The quantizer reads every partial magnitude that `nvfp4_largest` writes, and so no shorter tensor."""
+    assert _lib.library().dew_moe_nvfp4_partials() == 512
+    with pytest.raises(KernelError, match=f"largest has {words} words, not nvfp4_largest's 512"):
+        ops.quantize_nvfp4(torch.zeros((128, 128), dtype=torch.bfloat16), torch.zeros(words, dtype=torch.int32), rows=True, tokens=False)
+
+
+@pytest.mark.parametrize("shape", [(128,), (2, 128, 128), ()])
+def test_an_nvfp4_operand_that_is_no_matrix_is_refused(shape):
+    with pytest.raises(KernelError, match=r"not \[rows, depth\]"):
+        ops.quantize_nvfp4(torch.zeros(shape, dtype=torch.bfloat16), torch.zeros(512, dtype=torch.int32), rows=True, tokens=False)
+
+
+def test_tensor_scales_go_to_banks_that_carry_them_one_an_expert():
+    nvfp4 = fake_bank(_lib.W_NVFP4, experts=3)
+    for count in (0, 1, 2, 4):
+        with pytest.raises(KernelError, match=f"{count} tensor scales for the bank's 3 experts"):
+            nvfp4.under(torch.zeros(count))
+    with pytest.raises(KernelError, match="must be on the GPU"):
+        nvfp4.under(torch.zeros(3))
+    x, largest = torch.zeros((128, 128), dtype=torch.bfloat16), torch.zeros(512, dtype=torch.int32)
+    for fmt in (_lib.W_FP8_BLOCK, _lib.W_FP8_CHANNEL, _lib.W_MXFP8, _lib.W_BF16):
+        bank = fake_bank(fmt, experts=3)
+        with pytest.raises(KernelError, match="only an NVFP4 bank carries tensor scales"):
+            bank.under(torch.zeros(3))
+        with pytest.raises(KernelError, match="only an NVFP4 bank carries tensor scales"):
+            ops.quantize_nvfp4(x, largest, rows=True, tokens=False, bank=bank)
+
+
+@pytest.mark.gpu
+def test_tensor_scales_of_another_dtype_or_spacing_are_refused_on_the_device_too():
+    nvfp4 = fake_bank(_lib.W_NVFP4, experts=3)
+    with pytest.raises(KernelError, match="scales must be torch.float32"):
+        nvfp4.under(torch.zeros(3, dtype=torch.float64, device="cuda"))
+    with pytest.raises(KernelError, match="scales must be contiguous"):
+        nvfp4.under(torch.zeros(6, device="cuda")[::2])
+    with pytest.raises(KernelError, match="largest must be torch.int32"):
+        ops.quantize_nvfp4(torch.zeros((128, 128), dtype=torch.bfloat16, device="cuda"), torch.zeros(512, device="cuda"), rows=True, tokens=False)
