@@ -352,22 +352,20 @@ static bool few_tiles(int rows, int groups, int width) {  // about so many of 12
   return (rows / 128 + groups / 2 + 1) * static_cast<long long>((width + 255) / 256) <= kFewTiles;
 }
 
-// 256 x 256 tiles (wide.hip) where they fill the CUs over the rounds that they take, on groups of at least about half a tile's rows.
-// Measured against the tiles below on 105 shapes (512 to 65 536 rows, 1 to 60 groups, extents 512 to 14 336; us, there and here):
-// 14 134 rows of 15 x 2048 x 1024 65.7 and 57.0, 32 768 of 8 x 4096 x 4096 992 and 886, 24 000 of 8 x 7168 x 7168 2203 and 1918; at
-// rounds filled to 0.56 .. 0.74 between 0.93 and 1.07 times as fast, under half 0.4 to 0.75 times; groups of 64 to 97 rows 0.82 to 0.98
-// times. K-major matrices, which the tiles below read half a cache line at a step, gain from 0.55 on: 4807 of 7 x 2688 x 3968 as its
-// input's gradient at 0.96 1.37 times, 1981 of 1 x 5120 x 10 240 at 0.64 1.33, 9569 of 4 x 1920 x 1792 at 0.62 1.10.
+// 256 x 256 tiles (wide.hip) where they fill the CUs over the rounds that they take, on groups of at least about half a tile's rows
+// (of 64 to 97 rows 0.82 to 0.98 times as fast). Measured against the tiles below on some 250 shapes (64 to 7168 deep, 1 to 64 groups; us,
+// there and here). Natural order, from 0.57 on: 4608 rows of 1 x 1024 x 2048, 148 tiles, 32.1 and 25.5, 4300 of 4 x 4096 x 2048 97.4 and 77.3,
+// 10 000 of 4 x 512 x 2048, 328 tiles, 33.7 and 30.9, 8192 of 8 x 4096 x 2048, 288, 159 and 162, 9000 of 1 x 4096 x 4096, 570, 290 and 262; below it 4096
+// of 1 x 4096 x 2048, 132, 67.5 and 80.3, 8300 of 4 x 4096 x 2048, 275, 158 and 164. K-major matrices, which the tiles below read half a cache line
+// at a step, from 0.51 on: 4608 of 1 x 4096 x 2048 121 and 78, 8300 of 4 x 4096 x 2048 184 and 162, 8448 of 1 x 7168 x 2048, 268 tiles, 318 and 278;
+// 4096 of 1 x 4096 x 2048, 132 tiles, 75.6 and 79.9, 3300 of 4, 119, 72.3 and 72.9.
 static bool wide_product(int rows, int groups, int depth, int width, bool kmajor) {
-  const double tiles = (rows / 256.0 + groups / 2.0) * ((width + 255) / 256);
-  return wide_extents(groups, depth, width) && rows / groups >= 112 && fills_rounds(tiles, kmajor ? 55 : 75);
+  return wide_extents(groups, depth, width) && rows / groups >= 112 && fills_rounds(product_tiles(rows, groups, width), kmajor ? 51 : 57, kGuessed);
 }
 
-// A kernel's gradient, whose tiles are whole: 27 097 rows of 10 x 5376 x 768 at rounds filled to 0.82 243 and 213, 28 140 of 10 x 4352 x
-// 3200 782 and 657; groups of fewer than 256 rows, four steps, are all start and end either way (0.91 to 1.18 times as fast).
+// A kernel's gradient; groups of fewer than 256 rows, four steps, are all start and end either way (0.91 to 1.18 times as fast).
 static bool wide_gradient(int rows, int groups, int depth, int width) {
-  const double tiles = static_cast<double>(groups) * ((depth + 255) / 256) * ((width + 255) / 256);
-  return wide_extents(groups, depth, width) && rows / groups >= 256 && fills_rounds(tiles, 75);
+  return wide_extents(groups, depth, width) && rows / groups >= 256 && fills_rounds(gradient_tiles(groups, depth, width), kGradientRounds);
 }
 
 }  // namespace dew

@@ -1311,25 +1311,20 @@ static bool few_gradient_blocks(const GemmParams& p) {
   return static_cast<long long>(p.experts) * ((p.window_rows + 255) / 256) * ((p.width + 255) / 256) <= 128;
 }
 
-// The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered: where such
-// tiles keep the CUs busy over the rounds they take. Measured against the launches below on 70 shapes (512 to 32 768 rows, 1 to 51 groups,
-// extents 512 to 14 336; us, there and here): [32 768, 7168] x 2048 of 32 groups, blockwise, forward 470 and 424, input's gradient 520 and
-// 444, kernel's gradient 692 and 530; [32 768, 4096] x 14336 of 8, MXFP8, 1636 and 1490, 1600 and 1460, 1637 and 1450; [12 672, 512] x 3456
-// of 21 70 and 39; [4608, 896] x 7552 of 33, kernel's gradient, 220 and 125. At rounds filled to 0.56 .. 0.7 1.02 to 1.2 times as fast, in one
-// round from 0.66 on 1.1 to 1.7; at 260 tiles, two rounds, 0.77 to 0.89.
-static bool fills_wide_rounds(double tiles, int percent_of_one, int percent_of_more) {
-  const double rounds = ceil(tiles / 256);
-  return tiles * 100 >= rounds * 256 * (rounds <= 1 ? percent_of_one : percent_of_more);
-}
+// The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered: on groups of half
+// a tile's rows, wherever such tiles are enough to measure, from three eighths of a round on. Against the launches below (us, there and
+// here, 160 shapes of 512 to 32 768 rows, 1 to 51 groups, depths from 512): blockwise, [2560, 512] x 2048 of 4 groups, 96 tiles, 14.2 and 12.7, 4096
+// deep 46.5 and 42.3; [4608, 1024] x 2048, 148, 26.0 and 18.3; [8192, 4096] x 2048 of 2, 264 tiles of two rounds, 92.2 and 87.7; [32 768, 7168] x 2048 of
+// 32, forward 470 and 424, input's gradient 520 and 444; MXFP8, [32 768, 4096] x 14336 of 8 1636 and 1490. Least: [3584, 1024] x 2048, 116, blockwise, 18.5 and 18.3.
+constexpr int kFp8ProductRounds = 37;
 
 static WideFp8Params wide_fp8_params(const GemmParams& p, int a_scale_pitch) {
   return WideFp8Params{reinterpret_cast<const uint8_t*>(p.x), p.a_scale, p.w0.codes, p.w0.scales, p.offsets, p.out, p.experts, p.rows, p.depth, p.width, a_scale_pitch};
 }
 
 static bool wide_fp8_product(const GemmParams& p) {
-  const double tiles = (p.rows / 256.0 + p.experts / 2.0) * ((p.width + 255) / 256);
   return forced_tile_rows == 0 && !p.gather && !p.scatter && !p.bias && wide_extents(p.experts, p.depth, p.width) && p.depth >= 512 &&
-         p.rows / p.experts >= 112 && fills_wide_rounds(tiles, 62, 56);
+         p.rows / p.experts >= 112 && fills_rounds(product_tiles(p.rows, p.experts, p.width), kFp8ProductRounds, kGuessed);
 }
 
 static bool wide_fp8_gradient_extents(int tokens, int depth, int width, int groups) {
@@ -1556,10 +1551,7 @@ extern "C" int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint
 
 extern "C" int dew_moe_kernel_gradient_takes_banks(int32_t tokens, int32_t depth, int32_t width, int32_t groups) {
   using namespace dew;
-  const double tiles = static_cast<double>(groups) * ((depth + 255) / 256) * ((width + 255) / 256);
-  // (its tiles are whole, and those of the launch of one tile a block start and end worse: 270 tiles 49.5 and 33.4 us. One round of long
-  // tiles, which few blocks fetch from the memory and not from each other's L2, is slower here: 168 of 18 steps 40 and 49)
-  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && fills_wide_rounds(tiles, 70, 53);
+  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && fills_rounds(gradient_tiles(groups, depth, width), kGradientRounds);
 }
 
 extern "C" int dew_moe_kernel_gradient_mxfp8_banks(const dew_moe_bank* lhs_t, const dew_moe_bank* rhs_t, const int32_t* offsets, void* out,

@@ -1,0 +1,38 @@
+"""256 x 256 tiles on the lines from which they are taken: so few that half of the blocks have none, and a second round just begun. The
+comparisons are those of test_gpu_wide.py and test_gpu_wide_fp8.py, with the launches of smaller tiles (the same bits)."""
+
+import pytest
+import test_gpu_wide
+import test_gpu_wide_fp8
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+# (those files add 300 rows of no group: 148, 266 and 292 tiles by the launch's guess, of which K-major matrices take all and natural ones
+# the first and the last; blocks without a tile clear rows all the same)
+@pytest.mark.parametrize("sizes,width", (([940, 1000, 1100, 900], 2048), ([1900, 2050, 2000, 1750], 2048), ([1900, 1850, 2000, 1750], 2304)))
+def test_products(monkeypatch, sizes, width):
+    monkeypatch.setitem(test_gpu_wide.SIZES, "lines", sizes)
+    monkeypatch.setitem(test_gpu_wide.WIDTHS, "lines", width)
+    test_gpu_wide.test_products("lines", 320)
+
+
+@pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("sizes,depth,width", (([257, 300, 700, 0, 500, 299, 301, 302, 400], 1032, 1000), ([300] * 9, 1024, 2048)))     # 180 tiles, 288
+def test_gradients(sizes, depth, width, out_dtype):
+    test_gpu_wide.test_gradients(sizes, depth, width, out_dtype)
+
+
+@pytest.mark.parametrize("sizes", ([480, 600, 700, 500], [1900, 2050, 2100, 1950]))     # 97 tiles by the launch's guess, 275
+@pytest.mark.parametrize("recipe", ("blockwise_fp8", "mxfp8"))
+def test_recipes_products(monkeypatch, recipe, sizes):
+    monkeypatch.setitem(test_gpu_wide_fp8.SIZES, "lines", (sizes, 2048))
+    test_gpu_wide_fp8.test_products(recipe, "lines", 640)
+
+
+@pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("mx", (True, False))
+@pytest.mark.parametrize("blocks,depth,width", (([1, 2, 0, 3, 1, 1, 2, 1, 4], 1024, 1024), ([1] * 9, 1024, 2048)))     # 144 tiles, 288
+def test_recipes_gradients(blocks, depth, width, mx, out_dtype):
+    test_gpu_wide_fp8.test_gradients(blocks, depth, width, mx, out_dtype)
