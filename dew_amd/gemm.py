@@ -172,9 +172,17 @@ def prepared(bank) -> ops.PreparedBank:
     return held
 
 
-def _relaid_first(matrices: torch.Tensor, rows: int) -> bool:
-    """Whether `rows` gathered or scattered rows times plain matrices are the faster product on matrices brought to the matrix instruction's order at the
-    call (`prepared`) than on matrices read where they lie (`ops.dense_gemm`); the bits are the same. The pass over the matrices is
+MOST_WIDE_GROUPS = 256
+"""The most groups whose tiles a launch of 256 x 256 tiles holds (`kWideGroups`, csrc/wide.h)."""
+
+
+def _relaid_first(matrices: torch.Tensor, rows: int, as_they_lie: bool = False) -> bool:
+    """Whether `rows` rows (`as_they_lie`, or gathered or scattered) times plain matrices are the faster product on matrices brought to the matrix
+    instruction's order at the call (`prepared`) than on matrices read where they lie (`ops.dense_gemm`); the bits are the same. Rows as they lie
+    of at most 256 groups are multiplied in 256 x 256 tiles, which need no order (us there, in smaller tiles and laid out first: K-major, 1 x 8448
+    of 4096 x 2048 164, 185 and 172, 4 x 4250 of 7168 x 1024 281, 337 and 321; natural order, 1 x 9000 of 4096 x 4096 262, 290 and 280, 1 x 12 032
+    of 2048 x 2048 92, 93 and 101). No such tiles are for more groups: 257 x 3000 of 4096 x 512, K-major, 3703 in smaller ones and 3251 laid out
+    first, 300 x 3000 of 4096 x 256 2488 and 2267, natural 257 x 8300 of 2048 x 256 2668 and 2576. The pass over the matrices is
     small beside the work of groups of thousands of rows, and the launch on prepared matrices then runs in 256-row tiles that fetch
     half the bytes from the L2; K-major matrices lose the more by lying where they are, since a step reads half of each cache line.
     Measured on 237 shapes of 1 to 16 groups, us where they lie and laid out first: K-major, 8 x 4096 rows of 4096 x 4096 1172 and
@@ -183,7 +191,7 @@ def _relaid_first(matrices: torch.Tensor, rows: int) -> bool:
     8192 of 4096 x 14336 3305 and 3113 (8 x 4096 of 4096 x 4096 991 and 989, 2 x 4096 of 2048 x 4096 138 and 159)."""
     groups, depth, width = matrices.shape
     kmajor = not matrices.is_contiguous()
-    if groups == 0 or depth > 32768 or (kmajor and (depth % 128 or width % 128)):     # (what no prepared bank holds)
+    if (as_they_lie and groups <= MOST_WIDE_GROUPS) or groups == 0 or depth > 32768 or (kmajor and (depth % 128 or width % 128)):     # (what no prepared bank holds)
         return False
     average, tiles = rows // groups, (rows // 128 + groups // 2 + 1) * ((width + 255) // 256)
     if tiles < 384 or depth < 2048:
@@ -208,8 +216,7 @@ def gemm(lhs: torch.Tensor, rhs, group_sizes, *, paired=None, gather: torch.Tens
             rhs = rhs.contiguous()
         elif rhs.data_ptr() % 16:    # (a view into a flat buffer of parameters begins anywhere; the launch loads 16 bytes at a time)
             rhs = rhs.clone()        # (which keeps the strides)
-        # (rows as they lie: the launch takes tiles of its own that need no order, see wide.hip)
-        if (gather is None and scatter is None) or not _relaid_first(rhs, lhs.shape[0] if gather is None else gather.numel()):
+        if not _relaid_first(rhs, lhs.shape[0] if gather is None else gather.numel(), gather is None and scatter is None):
             groups = GroupSizes.operands(group_sizes)
             return ops.dense_gemm(lhs, rhs, groups["offsets"], gather=gather, scatter=scatter, sizes=groups.get("sizes"))
     first = prepared(rhs)
