@@ -66,13 +66,14 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_fp8_kernel(WideFp8Params
     if (!tiles.at(turn, 4, place)) return false;  // (4 row tiles x 8 strips are what an XCD's 32 CUs hold at once)
     tile.group = place.group;
     tile.n0 = place.strip * kWideTile;
-    if constexpr (kGradient) {  // (an empty window: one step of zeros)
+    if constexpr (kGradient) {  // (an empty window: one step of zeros, the first: where it stands may be behind the last, whose scales are the last read)
       tile.row0 = place.within * kWideTile;
       tile.valid_rows = min(kWideTile, p.rows - tile.row0);
-      tile.first_step = min(max(place.start, 0), p.depth) / kFp8Step;
+      const int first_step = min(max(place.start, 0), p.depth) / kFp8Step;
       // (said to be the same in every lane: as conditions of each lane they made a loop over the lanes of every load)
-      const int steps = __builtin_amdgcn_readfirstlane(min(max(place.start + place.size, 0), p.depth) / kFp8Step - tile.first_step);
+      const int steps = __builtin_amdgcn_readfirstlane(min(max(place.start + place.size, 0), p.depth) / kFp8Step - first_step);
       tile.empty = __builtin_amdgcn_readfirstlane(steps <= 0);
+      tile.first_step = tile.empty ? 0 : first_step;
       tile.steps = max(steps, 1);
     } else {
       tile.row0 = place.start + place.within * kWideTile;

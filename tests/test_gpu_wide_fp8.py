@@ -78,3 +78,30 @@ def test_gradients(blocks, depth, width, mx, out_dtype):
     assert torch.equal(got, want) and got.dtype == out_dtype
     for g, count in enumerate(blocks):
         assert bool(got[g].any()) == (count > 0)
+
+
+@pytest.mark.parametrize("blocks", ([9, 2, 0], [4, 7, 0, 0], [11] + [0] * 5))
+@pytest.mark.parametrize("not_a_number", (False, True))
+def test_gradients_of_empty_groups_behind_the_last_token(blocks, not_a_number):
+    """Such a group has no step and no scales of its own: its gradient is zero, also beside other groups' scales that are NaN."""
+    from dew_amd import ops
+
+    depth, width = 896, 4096
+    x, _, _ = operands([128 * sum(blocks)], depth, 128, extra=0)
+    dy, _, _ = operands([128 * sum(blocks)], width, 128, extra=0)
+    offsets, tokens = ops.block_offsets(torch.tensor(blocks, dtype=torch.int32, device="cuda"), 128), x.shape[0]
+    lhs, rhs = (ops.quantize_columns(operand, mx=True, as_bank=True) for operand in (x, dy))
+    codes, scales = ops.quantize_columns(x, mx=True, as_bank=False)
+    want = ops.kernel_gradient_mxfp8(codes, scales, rhs, offsets)
+    if not_a_number:     # the last 128 tokens' scale bytes, in every column of both operands
+        for bank, columns in ((lhs, depth), (rhs, width)):
+            bank.keep[0][tokens * columns:][:tokens // 32 * columns].view(columns // 32, tokens // 128, 128)[:, -1] = 0xFF
+    got = ops.kernel_gradient_mxfp8_banks(lhs, rhs, offsets)
+    last = max(g for g, count in enumerate(blocks) if count)
+    for g, count in enumerate(blocks):
+        if not count:
+            assert not bool(got[g].any())
+        elif not_a_number and g == last:
+            assert bool(torch.isnan(got[g]).all())
+        else:
+            assert torch.equal(got[g], want[g]) and bool(got[g].any())
