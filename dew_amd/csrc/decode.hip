@@ -380,16 +380,19 @@ template <int FORMAT, int MODE>
 static int launch_few(const char* who, const GemmParams& p, hipStream_t stream) {
   // every expert with rows ends in one partial tile, and the rows no expert owns fill tiles behind them
   const int tiles = min(p.rows, p.rows / 32 + p.experts + 1), blocks = tiles * (p.width / 32);
-  // Shared strips: formats whose conversion costs more than the product, deep enough that the hand-overs are few beside it, and one round
-  // of blocks (us of a layer's pass, a wavefront a strip and shared: FP8 blocks, one token's 8 experts of 2048 x 768 31.5 and 28.2, 7 tokens
-  // on 8 experts of 1792 x 768 28.2 and 24.0; NVFP4, 2 tokens, 4 experts of 1792 x 5120 42.3 and 39.9; 640 deep 25.6 and 26.9; one
-  // matrix, 1536 deep 25.9 and 27.2; MXFP4,
-  // whose conversion is one instruction for two codes, 1408 deep 37.7 and 40.5; bf16, which has none, 1152 deep 23.6 and 25.7).
+  // Shared strips: formats whose conversion costs more than the product, deep enough that the hand-overs are few beside it, and at most one
+  // block a CU (us, a wavefront a strip and shared). Pairs, whose blocks hold twice the wavefronts, gain from 1024 deep on: FP8 blocks, 1024 x 2048
+  // of one row 7.5 and 6.2, of four 8.2 and 7.9, 4096 x 512 of one 21.5 and 12.4 (640 deep a layer's pass 25.6 and 26.9). One matrix, whose every turn
+  // waits for the one before: FP8 blocks, 3072 deep 10.2 and 10.2 to 10.9 and 12.0; 4096, 128 strips, 12.9 and 12.5, 256 13.5 and 14.2; 6144, 256, 18.9
+  // and 18.4; NVFP4, 4096, 256 strips, 14.3 and 13.9. At 512 strips, two blocks a CU where their rows leave room, else two rounds, FP8 4096 deep 16.4
+  // and 19.9, 6144 deep of eight rows 23.1 and 34.6, NVFP4 22.5 and 33.6. (MXFP4, whose conversion is one instruction for two codes, 1408
+  // deep 37.7 and 40.5 a layer's pass; bf16, which has none, 1152 deep 23.6 and 25.7.)
   if constexpr (FORMAT == DEW_MOE_W_FP8_BLOCK || FORMAT == DEW_MOE_W_FP8_CHANNEL || FORMAT == DEW_MOE_W_NVFP4) {
     constexpr int kMatrices = MODE == kSwigluOfTwo ? 2 : 1;
-    const int touched = min(p.rows, p.experts) + p.rows / 32;  // the tiles that have rows, at most
+    const long long strips = (min(p.rows, p.experts) + p.rows / 32) * static_cast<long long>(p.width / 32);  // of the tiles that have rows, at most
+    const int least_depth = kMatrices == 2 ? 1024 : FORMAT == DEW_MOE_W_NVFP4 || strips <= 128 ? 4096 : 6144;
     const size_t rows_bytes = static_cast<size_t>(min(p.rows, 32)) * shared_pitch(p.depth);
-    if (p.depth >= (kMatrices == 2 ? 1024 : 4096) && touched * static_cast<long long>(p.width / 32) * kMatrices <= 512 && rows_bytes <= kMostShared) {
+    if (p.depth >= least_depth && strips <= 256 && rows_bytes <= kMostShared) {
       auto kernel = shared_strips_kernel<FORMAT, MODE>;
       static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
       static hipError_t reserved = hipSuccess;

@@ -38,6 +38,24 @@ def test_shared_strips_return_the_tiled_launchs_bits(quant, depth, sizes):
         assert torch.equal(call(), want), name
 
 
+# one matrix on each side of the lines from which its strips are shared: 128 and 256 strips of 4096 and 6144 deep, and of rows that fill the LDS
+@pytest.mark.parametrize("quant", ("fp8_block", "fp8_channel", "nvfp4"))
+@pytest.mark.parametrize("depth,width,rows", ((4096, 1024, 4), (4096, 1280, 4), (4096, 2048, 4), (6144, 2048, 4), (6144, 2176, 4), (6144, 1024, 8), (6144, 2048, 8),
+                                              (8192, 1024, 7), (8192, 1024, 8)))
+def test_one_matrix_on_the_lines_of_shared_strips(quant, depth, width, rows):
+    from dew_amd import ops
+
+    generator = torch.Generator("cuda").manual_seed(width)
+    matrices = ops.prepare(bank(rows, depth, width, quant, generator))
+    x = torch.randn((rows, depth), generator=generator, device="cuda").to(torch.bfloat16)
+    for sizes in ([1] * rows, [0, rows - 1] + [0] * (rows - 2)):     # (the last row is no group's)
+        offsets = ops.group_offsets(torch.tensor(sizes, dtype=torch.int32, device="cuda"))
+        got = ops.grouped_gemm(x, matrices, offsets)
+        with ops.tile_rows(32):
+            want = ops.grouped_gemm(x, matrices, offsets)
+        assert torch.equal(got, want) and bool(got[0].any())
+
+
 @pytest.mark.parametrize("tokens,experts,top_k,shared", ((1, 8, 8, None), (1, 128, 8, None), (2, 8, 8, None), (16, 5, 1, None), (5, 300, 3, None),
                                                          (4, 64, 3, 256), (8, 16, 1, 256), (1, 20, 17, None), (17, 8, 1, None)))     # the last two: 17 slots
 def test_a_few_slots_sort_as_many_do(tokens, experts, top_k, shared):
