@@ -317,10 +317,14 @@ def mxfp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, g
 
 def _contracted_in_place(tokens: int, depth: int, width: int, groups: int) -> bool:
     """Whether an NVFP4 kernel gradient contracts the tokens of its operands where they lie (`ops.dense_gradient`) rather than of transposed
-    copies. Without the copies, and their reads of the operands for the largest magnitude, a step is the shorter: 8192 tokens of 8 x 2048 x
-    4096 655 and 597 us, 640 of 16 x 1536 x 1024 165 and 120. Only few tiles that each walk many tokens are slower so (32 384 tokens of one
-    768 x 768 517 and 652, of one 1024 x 1536 788 and 825, of four 768 x 768 383 and 400; 8192 of one 1024 x 1536 256 and 239)."""
-    return tokens <= 6144 * groups or groups * -(-depth // 256) * -(-width // 256) >= 128
+    copies (the same bits). Without the copies, and their reads of the operands for the largest magnitude, a step is the shorter, by the more the
+    larger the operands are, the cotangent (`width`) above all; but its tiles walk a group's tokens more slowly, which few tiles of many tokens do not
+    hide. Measured on 235 shapes of 2048 to 32 768 tokens, 1 to 8 groups (us of both gradients, transposed and where they lie): 8192 tokens of 8 x 1024 x
+    1024 115 and 96, 32 768 of 4 x 1024 x 1024 315 and 287, of one 2048 x 3328 1164 and 1128, of one 512 x 8192 1290 and 1083; on either side of the line of
+    tokens one 768 x 768 of 4096 115 and 116, of 6144 138 and 145, of 32 768 403 and 501, one 1024 x 1536 of 8192 175 and 186; of the line of columns
+    32 768 of one 2048 x 2560 997 and 1009, of one 2048 x 3072 1123 and 1128, of 2 x 1024 x 1536 455 and 457, of 2 x 512 x 2048 447 and 445. Furthest off: 32 768 of
+    3 x 768 x 1024, taken where they lie, 308 and 318; 16 384 of one 2048 x 2048, taken transposed, 426 and 411."""
+    return tokens <= 4096 * groups or groups * (depth + 3 * width) >= 11000
 
 
 def _nvfp4_transposed_gradient(x: torch.Tensor, cotangent: torch.Tensor, groups: gemm.GroupSizes, out_dtype) -> torch.Tensor:

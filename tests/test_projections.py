@@ -190,3 +190,17 @@ def test_rows_as_two_e2m3_terms_keep_what_their_bound_says():
     assert np.array_equal(held[4], x[4]) and not held[3].any() and (scales[3] == 1).all()
     first = np.ldexp(np.float32(1), scales[..., 0].astype(np.int32) - 127)[..., None]
     assert (largest <= 7.5 * first).all() and (largest[largest > 0] > 3.75 * first[largest > 0]).all()   # the least such power of two
+
+
+def test_an_nvfp4_gradient_takes_the_form_that_was_timed_to_be_the_faster():
+    """(tokens, depth, width, groups) of both forms' measurements, on both sides of both lines."""
+    from dew_amd import projections
+
+    lying = [(2048, 768, 768, 1), (4096, 1024, 1536, 1), (8192, 1024, 1024, 8), (32768, 1024, 1024, 4), (32768, 1536, 1024, 4), (24576, 2048, 1536, 2),
+             (16384, 512, 8192, 1), (32768, 2048, 3328, 1), (16384, 512, 3072, 2), (8192, 2048, 4096, 8)]
+    transposed = [(6144, 768, 768, 1), (6144, 1024, 1536, 1), (8192, 1024, 1536, 1), (32768, 768, 768, 1), (32768, 768, 768, 2), (12288, 768, 768, 2),
+                  (8192, 4096, 1536, 1), (8192, 4608, 512, 1), (12288, 2048, 2560, 1)]
+    for case in lying:
+        assert projections._contracted_in_place(*case), case
+    for case in transposed:
+        assert not projections._contracted_in_place(*case), case
