@@ -1,11 +1,13 @@
 // The grouped product for few tiles of few rows: a decode step of one or a few tokens.
 //
 // The tiled launch gives a tile of an expert's rows and 128 columns to a block of four wavefronts that share the rows in the
-// LDS. One token's eight experts of 768 columns are then 48 blocks, and 208 CUs idle. Here a wavefront is a block of its own
-// and owns 32 columns (of both matrices of a pair): the same wavefronts, but on as many CUs, each with the memory pipeline to
-// itself and, with no barrier and no LDS stage a step, as much of its weights in flight as the registers hold. The rows are
-// few, so their fragments come straight from global memory (the lanes past a group's rows read its last row again, the
-// same cache lines). The depth is not split between wavefronts: every sum is taken in the tiled launches' order, so a
+// LDS. One token's eight experts of 768 columns are then 48 blocks, and 208 CUs idle. Two launches of finer tiles stand in for it:
+//  * few_tiles_kernel: a wavefront is a block of its own and owns 32 columns (of both matrices of a pair): the same wavefronts, but on as
+//    many CUs, each with the memory pipeline to itself and, with no barrier and no LDS stage a step, as much of its weights in flight as the
+//    registers hold. The rows are few, so their fragments come straight from global memory (the lanes past a group's rows read its last
+//    row again, the same cache lines).
+//  * shared_strips_kernel, where even such strips are few: several wavefronts share a strip's depth and keep the rows in the LDS.
+// Every sum is taken in the tiled launches' order (a wavefront that shares a strip goes on from the sums of the one before), so a
 // product's bits do not depend on which of them ran.
 #include <mutex>
 
@@ -192,16 +194,16 @@ __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
 // while the others multiply; what it multiplies it adds to the one before's sums, handed on through the LDS: every sum is still taken in
 // the tiled launches' order. The rows, which are few, are in the LDS.
 // One wavefront for a strip of both matrices spent 19 000 of its 28 000 cycles (2048 deep, FP8 blocks) on what is here 8 turns of 1000, half
-// of them matrix instructions: one token's 8 experts of 2048 x 768 15.0 -> 11.5 us.
+// of them matrix instructions: one token's 8 experts of 2048 x 768 15.0 -> 11.5 us. FP8 and NVFP4 banks (`launch_few`).
 constexpr int kShares = 4, kMostShared = 131072;  // bytes of rows that a block may keep
 constexpr int shared_pitch(int depth) { return depth * 2 + 16; }  // (a row's LDS bytes: 32 rows' pieces on different banks)
 
 template <int FORMAT, int MODE>
 __global__ __launch_bounds__(64 * kShares * (MODE == kSwigluOfTwo ? 2 : 1)) void shared_strips_kernel(GemmParams p) {
   constexpr bool kPaired = MODE == kSwigluOfTwo, kGated = MODE == kInterleavedGated;
-  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4 || FORMAT == DEW_MOE_W_MXFP4, kBf16 = FORMAT == DEW_MOE_W_BF16;
+  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4;
   constexpr int kMatrices = kPaired ? 2 : 1;
-  constexpr int kAtomK = kFp4 ? 64 : kBf16 ? 16 : 32, kAtoms = 64 / kAtomK;  // 16-byte loads a lane makes per matrix and 64 depths
+  constexpr int kAtomK = kFp4 ? 64 : 32, kAtoms = 64 / kAtomK;  // 16-byte loads a lane makes per matrix and 64 depths
   constexpr int kChunk = 4, kSets = kFp4 ? 3 : 2;  // steps of 64 depths a turn; chunks of weights in flight
   constexpr int kWaves = kMatrices * kShares;
   __shared__ f32x4_t handed[kMatrices][4 * 64];  // a matrix's sums on their way from one wavefront to the next, [quad][lane]
@@ -236,7 +238,7 @@ __global__ __launch_bounds__(64 * kShares * (MODE == kSwigluOfTwo ? 2 : 1)) void
   u32x4_t b[kSets][kChunk][kAtoms];
   uint32_t fp4_bytes[kSets][kChunk];
   float scale[kSets][kChunk];
-  bf16x8_t fragment[kBf16 ? 1 : kChunk][4];
+  bf16x8_t fragment[kChunk][4];
   auto load_weights = [&](auto set, int chunk) __attribute__((always_inline)) {
     constexpr int s = decltype(set)::value;
     if (chunk >= chunks) return;  // (the same for the wavefront)
@@ -261,24 +263,21 @@ __global__ __launch_bounds__(64 * kShares * (MODE == kSwigluOfTwo ? 2 : 1)) void
   if (p.round_bias) bias = bf16_round(bias);
   auto convert = [&](auto set) __attribute__((always_inline)) {
     constexpr int s = decltype(set)::value;
-    if constexpr (!kBf16) {
 #pragma unroll
-      for (int c = 0; c < kChunk; ++c)
+    for (int c = 0; c < kChunk; ++c)
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-          if constexpr (kFp4) {
-            const float half = (kk < 2 ? __builtin_amdgcn_cvt_f32_fp8(fp4_bytes[s][c], 0) : __builtin_amdgcn_cvt_f32_fp8(fp4_bytes[s][c], 1)) * 0.00390625f;
-            const uint32_t word = b[s][c][0][kk];
-            fragment[c][kk] = FORMAT == DEW_MOE_W_MXFP4 ? fragment_fp4_pow2(word, half) : fragment_fp4(word, half);
-          } else {
-            const u32x4_t& raw = b[s][c][kk / 2 % kAtoms];
-            fragment[c][kk] = fragment_fp8(raw[2 * (kk % 2)], raw[2 * (kk % 2) + 1], FORMAT == DEW_MOE_W_FP8_BLOCK ? scale[s][c] : channel_scale);
-          }
-          asm volatile("" : "+v"(fragment[c][kk]));  // (here, and not where it is multiplied)
+      for (int kk = 0; kk < 4; ++kk) {
+        if constexpr (kFp4) {
+          const float half = (kk < 2 ? __builtin_amdgcn_cvt_f32_fp8(fp4_bytes[s][c], 0) : __builtin_amdgcn_cvt_f32_fp8(fp4_bytes[s][c], 1)) * 0.00390625f;
+          fragment[c][kk] = fragment_fp4(b[s][c][0][kk], half);
+        } else {
+          const u32x4_t& raw = b[s][c][kk / 2 % kAtoms];
+          fragment[c][kk] = fragment_fp8(raw[2 * (kk % 2)], raw[2 * (kk % 2) + 1], FORMAT == DEW_MOE_W_FP8_BLOCK ? scale[s][c] : channel_scale);
         }
-    }
+        asm volatile("" : "+v"(fragment[c][kk]));  // (here, and not where it is multiplied)
+      }
   };
-  if (!kBf16 && share < chunks) convert(std::integral_constant<int, 0>{});
+  if (share < chunks) convert(std::integral_constant<int, 0>{});
   if (threadIdx.x < kMatrices) turn[threadIdx.x] = 0;
   if (static_cast<int>(threadIdx.x) < row_pieces) shared_rows[threadIdx.x / pieces * pitch + threadIdx.x % pieces] = first_piece;
   for (int item = threadIdx.x + 64 * kWaves; item < row_pieces; item += 64 * kWaves) {
@@ -295,7 +294,7 @@ __global__ __launch_bounds__(64 * kShares * (MODE == kSwigluOfTwo ? 2 : 1)) void
   auto fetch = [&](auto into, int step) __attribute__((always_inline)) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk) {
-      const int piece = kFp4 ? 4 * (lane / 32) + kk : kBf16 ? 2 * kk + lane / 32 : 4 * (kk / 2) + 2 * (lane / 32) + kk % 2;
+      const int piece = kFp4 ? 4 * (lane / 32) + kk : 4 * (kk / 2) + 2 * (lane / 32) + kk % 2;
       a[decltype(into)::value][kk] = a_row[min(step, steps - 1) * 8 + piece];
     }
   };
@@ -323,33 +322,27 @@ __global__ __launch_bounds__(64 * kShares * (MODE == kSwigluOfTwo ? 2 : 1)) void
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     if (lane == 0) __hip_atomic_store(&turn[matrix], chunk + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
   };
-  auto multiply = [&](auto set, int chunk) __attribute__((always_inline)) {  // (its first rows are fetched)
-    constexpr int s = decltype(set)::value;
+  auto multiply = [&](int chunk) __attribute__((always_inline)) {  // (its first rows are fetched)
     static_for<kChunk>([&](auto of) __attribute__((always_inline)) {
       constexpr int c = decltype(of)::value;
       if (chunk * kChunk + c >= steps) return;
       if constexpr (c + 1 < kChunk) fetch(std::integral_constant<int, (c + 1) % 2>{}, chunk * kChunk + c + 1);
 #pragma unroll
-      for (int kk = 0; kk < 4; ++kk) {
-        bf16x8_t weights;
-        if constexpr (kBf16) weights = __builtin_bit_cast(bf16x8_t, b[s][c][kk]);
-        else weights = fragment[c][kk];
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[c % 2][kk]), weights, acc, 0, 0, 0);
-      }
+      for (int kk = 0; kk < 4; ++kk)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a[c % 2][kk]), fragment[c][kk], acc, 0, 0, 0);
     });
   };
   for (int chunk = share; chunk < chunks;) {
     static_for<kSets>([&](auto set) __attribute__((always_inline)) {
       constexpr int s = decltype(set)::value;
       if (chunk >= chunks) return;
-      if constexpr (!kBf16) load_weights(set, chunk + kSets * kShares);  // (the set's weights are fragments now)
+      load_weights(set, chunk + kSets * kShares);  // (the set's weights are fragments now)
       fetch(std::integral_constant<int, 0>{}, chunk * kChunk);
       take(chunk);
-      multiply(set, chunk);
+      multiply(chunk);
       hand_on(chunk);
-      if constexpr (kBf16) load_weights(set, chunk + kSets * kShares);
       chunk += kShares;
-      if (!kBf16 && chunk < chunks) convert(std::integral_constant<int, (s + 1) % kSets>{});
+      if (chunk < chunks) convert(std::integral_constant<int, (s + 1) % kSets>{});
     });
   }
   __syncthreads();

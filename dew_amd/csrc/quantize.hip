@@ -16,7 +16,6 @@ namespace dew {
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 constexpr int kQuantizeWaves = 4;  // rows per 256-thread block
 
 __global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_fp8_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes,
