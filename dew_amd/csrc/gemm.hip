@@ -204,8 +204,8 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
   // ---- which expert owns m-tile `m_tile`? inclusive scan of ceil(size / BM) over the experts (and, where the caller gave group sizes
   // instead of their prefix, of the sizes themselves: an expert's first row), by every wavefront for itself, 64 experts a round, without
   // the LDS and its barriers (two of them and a trip through the LDS a 256 experts before: us of a layer's pass, 64 tokens of 128 experts of
-  // 2048 x 768 114 -> 113, 1111 of 64 x 2048 x 1408 in bf16 318 -> 314, 552 of 32 x 768 x 896 in MXFP4 44.4 -> 43.2). A round's sizes and first
-  // rows are asked for one round ahead ----
+  // 2048 x 768 114 -> 113, 1111 of 64 x 2048 x 1408 in bf16 318 -> 314, 552 of 32 x 768 x 896 in MXFP4 44.4 -> 43.2: hardly more than two runs
+  // of one side differ by). A round's sizes and first rows are asked for one round ahead ----
   auto size_of = [&](int e) { return e >= p.experts ? 0 : kWindow ? p.window_rows : p.sizes ? max(p.sizes[e], 0) : p.offsets[e + 1] - p.offsets[e]; };
   auto first_row_of = [&](int e) { return e >= p.experts || (p.sizes && !kWindow) ? 0 : kWindow ? e * p.window_rows : p.offsets[e]; };
   int expert = -1, row0 = 0, group_end = 0, carried = 0, carried_rows = 0;  // past the last tile: the tiles and (of sizes) the rows of all groups

@@ -84,9 +84,10 @@ __device__ __forceinline__ void place_round(const PermuteParams& p, int slot, in
 // The whole sort in one block for at most kSmallSlots slots (a decode step, a small prefill): the block
 // counts, scans and scatters, each wavefront a contiguous run of the slots, with the LDS histogram as the only
 // intermediate.
-// Measured under graph replay, sixteen wavefronts: 2048 slots 5.1 to 6.8 us (four wavefronts: 7.9 to 10.0), 4096 slots
-// 7.5 us.
-constexpr int kSmallSlots = 4096;      // beyond this two launches over many blocks are as fast or faster
+// Measured under graph replay, sixteen wavefronts, of 8, 64 and 256 experts, and the two launches over many blocks beside it: 2048 slots 4.6,
+// 5.4 and 6.6 us (four wavefronts: 7.9 to 10.0) and 6.1, 6.8 and 7.9; 4096 slots 6.3, 7.2 and 8.8 and 6.7, 7.7 and 8.8; 5120 slots 7.4, 8.4 and
+// 10.3 and 6.7, 8.0 and 9.1; 8192 slots 10.0, 11.1 and 14.2 and 6.3, 7.1 and 8.6.
+constexpr int kSmallSlots = 4096;      // where the two meet
 constexpr int kSmallThreads = 1024;    // sixteen wavefronts, where their counters fit the LDS a launch may take unasked
 constexpr int kNarrowSmallSlots = 2048;  // the four-wavefront form's reach, for more buckets than that
 // `running`: LDS, [THREADS / 64][buckets] then [buckets + 1] totals. `id_of(slot)`: a routed slot's expert.

@@ -16,8 +16,8 @@
 //  * The operands enter the instruction the other way round, so that a lane holds four neighbouring columns of a row; two exchanges
 //    between lanes make them runs of 64 bytes, and the tile leaves from registers, without the LDS and without a barrier (wide.h).
 //
-// us, in 128 x 256 tiles and here: 16 384 x 4096 x 4096 forward 517 and 445 (on another box 468 and 409, 1.34 PFLOP/s; the pipe 74 % busy
-// at 1.66 GHz, the power limit, without the loads 1.62), input's gradient 543 and 404, kernel's gradient 498 and 403; 10 007 rows of 16 x
+// us, in 128 x 256 tiles and here: 16 384 x 4096 x 4096 forward 517 and 445 (on another box 468 and 409, 1.34 PFLOP/s; the pipe 75 % busy
+// at 1.55 to 1.8 GHz, profiles/wide_tiles_mfma_utilisation.txt), input's gradient 543 and 404, kernel's gradient 498 and 403; 10 007 rows of 16 x
 // 2048 x 4096 187 and 165, 235 and 183 (1.5 rounds of tiles), 215 and 178 (268 MB written).
 #include <mutex>
 

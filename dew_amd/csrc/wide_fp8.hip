@@ -10,7 +10,8 @@
 //    the bank's atoms of 64 depths, which lie in the instruction's order and are read as they were fetched, and two of scales.
 //  * A row's scale bytes are 16 at a time, those of 4 steps (a byte every 32 depths) or of 16 (one every 128): a dword a row a step
 //    filled the L1 with as many lines as the rows themselves.
-//  * The pipe is 68 to 70 % busy at 1.6 to 1.7 GHz, the power limit, over 32 steps a tile; 43 % over 8 at 2.1.
+//  * The pipe is 67 to 69 % busy at 1.9 GHz over 32 and more steps a tile of MXFP8 (2.6 to 2.7 PFLOP/s), 55 to 59 % at 2.0 to 2.3 over 16 and 56 of the blockwise
+//    recipe, 39 to 43 % over 8 at 2.1 to 2.4 (profiles/wide_tiles_mfma_utilisation.txt).
 //  * Before a phase a wavefront waits for the loads of the phase before the last, and all of them meet: every load has one to two phases.
 #include <mutex>
 
