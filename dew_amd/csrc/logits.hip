@@ -1,12 +1,10 @@
 // Router gate logits: logits[t, e] = sum_d f32(x[t, d]) * kernel[d, e] in IEEE fp32
 // (reference src/dew/nn/moe.py:526-534: tokens widened to fp32, Precision.HIGHEST), and group offsets.
-// Depths in whole 16s run on the fp32 matrix instruction (v_mfma_f32_32x32x2_f32: fp32 operands, exact products, fp32
-// sums): a block takes 32 (or 64) tokens and up to four 32-expert tiles, its wavefronts a share of the depth each; the
-// partial sums of a tile meet in LDS in wavefront order, so the result does not depend on timing. A decode step's few
-// tokens take 16 x 16 tiles (v_mfma_f32_16x16x4_f32), four times the blocks. Measured: 64 tokens of GPT-OSS's 2880 x 32
-// gate in about 5 us of kernel and 8192 tokens of a 7168 x 256 gate in 319 us (94 TFLOP/s), where the
-// plain kernel below (a 64-token x 64-expert tile, 16-deep LDS steps, fp32 FMA; depths in no whole 16s still take it)
-// needed 550 us and 1.3 ms.
+// Depths in whole 16s run on the matrix unit, the fp32 gate as three bf16 terms (below): a block takes 32 (or 64) tokens and up to
+// four 32-expert tiles, its wavefronts a share of the depth each; the partial sums of a tile meet in LDS in wavefront order, so the
+// result does not depend on timing. A decode step's few tokens take 16 x 16 tiles of the fp32 instruction (v_mfma_f32_16x16x4_f32),
+// four times the blocks: 64 tokens of GPT-OSS's 2880 x 32 gate in about 5 us. Depths in no whole 16s take the plain kernel below (a
+// 64-token x 64-expert tile, 16-deep LDS steps, fp32 FMA; 1.3 ms for 8192 tokens of a 7168 x 256 gate, where the terms take 99 us).
 #include "common.h"
 #include "sort.h"
 
@@ -15,99 +13,176 @@ namespace dew {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// WAVES wavefronts a block split the depth: 4 where the tokens alone fill the chip, 16 for the few tokens of a decode step
-// (64 tokens are two blocks: their latency is the depth a wavefront walks).
-template <int TILES, int WAVES, int ROWS = 1>
-__global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf16_t* __restrict__ x, const float* __restrict__ kernel,
-                                                                        const float* __restrict__ bias, float* __restrict__ logits,
-                                                                        int tokens, int depth, int experts) {
-  __shared__ float partial[WAVES][16][64];  // a tile's partial sums, [wavefront][register][lane]
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  const int t0 = blockIdx.x * 32 * ROWS;  // ROWS tiles of 32 tokens a block (2 where the tokens are many: a weight load serves both)
-  int row[ROWS];
-#pragma unroll
-  for (int r = 0; r < ROWS; ++r) row[r] = min(t0 + 32 * r + lane % 32, tokens - 1);  // (rows past the tokens repeat the last one; they are not stored)
-  const int chunks = depth / 16;                    // 16 depths a chunk: the lane's 8 are 8 (lane / 32) .. + 7 of them
-  const int first = static_cast<int>(static_cast<long long>(chunks) * wave / WAVES);
-  const int last = static_cast<int>(static_cast<long long>(chunks) * (wave + 1) / WAVES);
+// The exact split of the gate kernel: an fp32 value is the sum of three bf16 values, its upper 16 bits, the upper 16 of what is
+// left and the 8 bits that are left then, and a token's bf16 element times any of them is exact in fp32. So three bf16 matrix
+// instructions 16 deep (32 cycles each) give the fp32 products that eight fp32 ones 2 deep (64 cycles each) do, and their
+// sums are rounded once for 16 products instead of once for each. What bounds it: the splitting's vector work beside the matrix
+// instructions (11 a pair of gate values against 24 x 32 cycles a 16 deep chunk of 64 x 128) where the experts are many, x from
+// memory where they are few. Measured against the fp32 instruction, the tokens from memory (us): 8192 x 7168 x 256 316 -> 99, 16384 x
+// 4096 x 8 65 -> 30, 4096 x 4096 x 8 39 -> 17, 8192 x 4096 x 128 130 -> 45; error against float64 (2-norm) 7.5e-7 -> 4.6e-7, 5.4e-7 ->
+// 3.3e-7, 5.8e-7 -> 3.5e-7 and 5.8e-7 -> 3.5e-7, and smaller for each of 64 shapes of 65 to 16384 tokens, 512 to 7168 deep.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+__device__ __forceinline__ uint32_t upper_halves(float high, float low) {
+  return __builtin_amdgcn_perm(__float_as_uint(high), __float_as_uint(low), 0x07060302u);
+}
+__device__ __forceinline__ float below_upper(float value) { return value - __uint_as_float(__float_as_uint(value) & 0xFFFF0000u); }
+
+// The sums of a share of the depth, its steps of 16 x CHUNKS from `first` to `last`, for ROWS tiles of 32 tokens from t0 on and TILES tiles of
+// 32 experts. A lane's depths of a step are contiguous in its token's row (64 bytes of four chunks, so that every line of x is asked
+// for once); a chunk's instructions take 8 of each half's. Its experts are TILES neighbours, one a tile, from `column` on: one load a depth.
+// WHOLE: the depth is whole steps.
+template <int ROWS, int TILES, int AHEAD, int CHUNKS, bool WHOLE>
+__device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const float* __restrict__ kernel, int tokens, int depth, int experts,
+                                            int t0, int column, int first, int last, f32x16 (&acc)[ROWS][TILES]) {
+  struct __attribute__((packed, aligned(4))) Neighbours {
+    float of[TILES];
+  };
+  constexpr int kStep = 16 * CHUNKS;
+  const int lane = threadIdx.x % 64, half = kStep / 2 * (lane / 32);
   const bf16_t* a_src[ROWS];
 #pragma unroll
-  for (int r = 0; r < ROWS; ++r) a_src[r] = x + static_cast<size_t>(row[r]) * depth + 8 * (lane / 32);
-  int column[TILES];
-  const int tile0 = blockIdx.y * TILES;  // (a decode step's blocks take one tile each: the gate kernel's bytes spread over the CUs)
-#pragma unroll
-  for (int c = 0; c < TILES; ++c) column[c] = min(32 * (tile0 + c) + lane % 32, experts - 1);
-  f32x16 acc[ROWS][TILES];
+  for (int r = 0; r < ROWS; ++r)  // (rows past the tokens repeat the last one; they are not stored)
+    a_src[r] = x + static_cast<size_t>(min(t0 + 32 * r + lane % 32, tokens - 1)) * depth;
 #pragma unroll
   for (int r = 0; r < ROWS; ++r)
 #pragma unroll
     for (int c = 0; c < TILES; ++c)
 #pragma unroll
       for (int i = 0; i < 16; ++i) acc[r][c][i] = 0.0f;
-  // A chunk's operands are loaded while the chunk before it multiplies (a block may be alone on its CU: nothing else
-  // would hide the loads).
-  u32x4 a_words[2][ROWS];
-  float b[2][TILES][8];
-  auto load = [&](int buffer, int chunk) __attribute__((always_inline)) {
-#pragma unroll
-    for (int r = 0; r < ROWS; ++r) a_words[buffer][r] = *reinterpret_cast<const u32x4*>(a_src[r] + chunk * 16);
-    const float* b_src = kernel + static_cast<size_t>(chunk * 16 + 8 * (lane / 32)) * experts;
-#pragma unroll
-    for (int c = 0; c < TILES; ++c)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) b[buffer][c][j] = b_src[static_cast<size_t>(j) * experts + column[c]];
-  };
-  auto multiply = [&](int buffer) __attribute__((always_inline)) {
-    float a[ROWS][8];
+  if (first >= last) return;
+  // Loads return in order, so the gate's, which the L2 holds, wait for the rows', which come from memory, and both are asked for the
+  // same time ahead: AHEAD steps. A chunk's gate values are split one chunk ahead, between the matrix instructions of the chunk before.
+  constexpr int kSets = 2 * AHEAD;
+  u32x4 a_words[kSets][ROWS][CHUNKS];
+  Neighbours g[AHEAD][CHUNKS][8];
+  bf16x8 terms[2][TILES][3];
+  auto load_rows = [&](int set, int step) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < ROWS; ++r)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        a[r][2 * i] = __uint_as_float(a_words[buffer][r][i] << 16);
-        a[r][2 * i + 1] = __uint_as_float(a_words[buffer][r][i] & 0xFFFF0000u);
-      }
-#pragma unroll
-    for (int c = 0; c < TILES; ++c)
-#pragma unroll
-      for (int r = 0; r < ROWS; ++r)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[r][j], b[buffer][c][j], acc[r][c], 0, 0, 0);
+      for (int c = 0; c < CHUNKS; ++c)  // (past the depth: its last 8, which are multiplied as zeros)
+        a_words[set][r][c] = *reinterpret_cast<const u32x4*>(a_src[r] + (WHOLE ? kStep * step + half + 8 * c : min(kStep * step + half + 8 * c, depth - 8)));
   };
-  if constexpr (WAVES == 16) {  // a decode step's wavefronts walk a few chunks each (loads kept further ahead changed nothing: the matrix pipe is the limit)
-    for (int chunk = first; chunk < last; ++chunk) {
-      load(0, chunk);
-      multiply(0);
+  auto load_gate = [&](int set, int step, int chunk) __attribute__((always_inline)) {
+    const int at = kStep * step + 8 * chunk;  // (the same for the wavefront: a load's address is a scalar base and the lane's own offset)
+    const float* b_src = kernel + static_cast<size_t>(WHOLE ? at : min(at, depth - 8)) * experts;
+    const uint32_t lower = (WHOLE || at + half < depth ? half * experts : 0) + column;
+#pragma unroll
+    for (int j = 0; j < 8; ++j, b_src += experts) g[set][chunk][j] = *reinterpret_cast<const Neighbours*>(b_src + lower);
+  };
+  auto split = [&](int set, int chunk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) {
+      float most[8], rest[8], least[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) most[j] = g[set][chunk][j].of[c];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) rest[j] = below_upper(most[j]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) least[j] = below_upper(rest[j]);
+      auto fragment = [](const float (&v)[8]) __attribute__((always_inline)) {
+        return __builtin_bit_cast(bf16x8, u32x4{upper_halves(v[1], v[0]), upper_halves(v[3], v[2]), upper_halves(v[5], v[4]), upper_halves(v[7], v[6])});
+      };
+      terms[chunk % 2][c][0] = fragment(least);
+      terms[chunk % 2][c][1] = fragment(rest);
+      terms[chunk % 2][c][2] = fragment(most);
     }
-  } else {
-    if (first < last) load(0, first);
-    for (int chunk = first; chunk < last; chunk += 2) {
-      load(1, min(chunk + 1, last - 1));
-      multiply(0);
-      load(0, min(chunk + 2, last - 1));
-      if (chunk + 1 < last) multiply(1);
+  };
+  auto walk = [&](int set, int step, bool more) __attribute__((always_inline)) {
+    if (more) load_rows((set + AHEAD) % kSets, min(step + AHEAD, last - 1));  // (behind the last step: that step again, which multiplies nothing)
+#pragma unroll
+    for (int chunk = 0; chunk < CHUNKS; ++chunk) {
+      const uint32_t kept = WHOLE || kStep * step + half + 8 * chunk < depth ? 0xFFFFFFFFu : 0u;
+#pragma unroll
+      for (int term = 0; term < 3; ++term)
+#pragma unroll
+        for (int c = 0; c < TILES; ++c)
+#pragma unroll
+          for (int r = 0; r < ROWS; ++r)
+            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a_words[set][r][chunk] & kept), terms[chunk % 2][c][term],
+                                                                acc[r][c], 0, 0, 0);
+      const int next = chunk < CHUNKS - 1 ? set % AHEAD : (set + 1) % AHEAD;  // the set of the chunk behind this one
+      if (more || chunk < CHUNKS - 1) split(next, (chunk + 1) % CHUNKS);
+      if (more) load_gate(next, min(step + AHEAD + (chunk == CHUNKS - 1), last - 1), (chunk + 1) % CHUNKS);
     }
+  };
+#pragma unroll
+  for (int ahead = 0; ahead < AHEAD; ++ahead) {
+    load_rows(ahead, min(first + ahead, last - 1));
+#pragma unroll
+    for (int chunk = 0; chunk < CHUNKS; ++chunk) load_gate(ahead, min(first + ahead, last - 1), chunk);
   }
-  // register i of lane l is the sum of token 8 (i / 4) + 4 (l / 32) + i % 4, expert column l % 32 of the tile. A tile's
-  // partial sums go through LDS; every thread then finishes its share of the tile's 1024 sums, adding the wavefronts'
-  // partial sums in wavefront order.
+  split(0, 0);
+  if (CHUNKS < 4 && last - first == 1) {  // (a share of a short depth: nothing behind it is asked for)
+    walk(0, first, false);
+    return;
+  }
+  load_gate(0, min(first + AHEAD, last - 1), 0);
+  int step = first;
+  for (; step + kSets <= last; step += kSets) {  // (no way out in the middle: every load would be waited for there)
+#pragma unroll
+    for (int set = 0; set < kSets; ++set) walk(set, step + set, true);
+  }
+#pragma unroll
+  for (int set = 0; set < kSets - 1; ++set)
+    if (step + set < last) walk(set, step + set, AHEAD > 1);
+}
+
+// A sum that is no finite number again, product by product in fp32: an infinity among the operands meets a term that is zero, and a
+// gate value's terms are not those of an infinity or a NaN.
+__device__ __forceinline__ float finite_or_plain(float sum, const bf16_t* __restrict__ row, const float* __restrict__ column, int experts, int from,
+                                                 int to) {
+  if (__builtin_isfinite(sum)) return sum;
+  sum = 0.0f;
+  for (int d = from; d < to; ++d) sum = fmaf(bf16_to_f32(row[d]), column[static_cast<size_t>(d) * experts], sum);
+  return sum;
+}
+
+// WAVES wavefronts a block split the depth; their sums meet in LDS in wavefront order, WAVES registers of the tiles at a time.
+template <int ROWS, int TILES, int WAVES, int AHEAD, int CHUNKS, bool WHOLE>
+__global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf16_t* __restrict__ x, const float* __restrict__ kernel,
+                                                                        const float* __restrict__ bias, float* __restrict__ logits,
+                                                                        int tokens, int depth, int experts) {
+  struct __attribute__((packed, aligned(4))) Neighbours {
+    float of[TILES];
+  };
+  __shared__ float partial[WAVES][WAVES][TILES][64];  // [wavefront][register][tile][lane]
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int t0 = blockIdx.x * 32 * ROWS, e0 = TILES * (32 * blockIdx.y + lane % 32);
+  // (lanes past the experts repeat the last ones: what they share with the lane before is the same sum)
+  const int column = min(e0, experts - TILES);
+  const int steps = (depth + 16 * CHUNKS - 1) / (16 * CHUNKS);
+  f32x16 acc[ROWS][TILES];
+  logit_terms<ROWS, TILES, AHEAD, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, column, steps * wave / WAVES, steps * (wave + 1) / WAVES, acc);
+  // register i of lane l is the sum of token 8 (i / 4) + 4 (l / 32) + i % 4 and the lane's expert
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
 #pragma unroll
-    for (int c = 0; c < TILES; ++c) {
-      if (32 * (tile0 + c) >= experts) continue;  // (the same for every wavefront of the block: the barriers below stay matched)
+    for (int i0 = 0; i0 < 16; i0 += WAVES) {
+      if (r + i0 > 0) __syncthreads();
+#pragma unroll
+      for (int i = 0; i < WAVES; ++i)
+#pragma unroll
+        for (int c = 0; c < TILES; ++c) partial[wave][i][c][lane] = acc[r][c][i0 + i];
       __syncthreads();
+      const int i = i0 + wave, t = t0 + 32 * r + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
+      Neighbours sums;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) partial[wave][i][lane] = acc[r][c][i];
-      __syncthreads();
+      for (int c = 0; c < TILES; ++c) {
+        float sum = partial[0][wave][c][lane];
 #pragma unroll
-      for (int k = 0; k < 16 / WAVES; ++k) {
-        const int i = wave + WAVES * k;
-        float sum = partial[0][i][lane];
+        for (int w = 1; w < WAVES; ++w) sum += partial[w][wave][c][lane];
+        sums.of[c] = sum;
+      }
+      if (t < tokens && e0 < experts) {
 #pragma unroll
-        for (int w = 1; w < WAVES; ++w) sum += partial[w][i][lane];
-        const int t = t0 + 32 * r + 8 * (i / 4) + 4 * (lane / 32) + i % 4, e = 32 * (tile0 + c) + lane % 32;
-        // a biased router (GPT-OSS's, src/dew/nn/gpt_oss.py:163-165) adds its fp32 bias to the finished sum
-        if (t < tokens && e < experts) logits[static_cast<size_t>(t) * experts + e] = bias ? sum + bias[e] : sum;
+        for (int c = 0; c < TILES; ++c) {
+          sums.of[c] = finite_or_plain(sums.of[c], x + static_cast<size_t>(t) * depth, kernel + column + c, experts, 0, depth);
+          // a biased router (GPT-OSS's, src/dew/nn/gpt_oss.py:163-165) adds its fp32 bias to the finished sum
+          if (bias) sums.of[c] += bias[column + c];
+        }
+        *reinterpret_cast<Neighbours*>(logits + static_cast<size_t>(t) * experts + column) = sums;
       }
     }
   }
@@ -122,6 +197,17 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kShares = kLogitShares;  // the depth's shares, one a wavefront
+
+// Sixteen shares of a short depth take steps of 32: in steps of 64 a depth of 512 leaves half of them without one (a layer's pass over
+// 2048 tokens of a 512 x 8 gate 49.4 us, 48.5 with them).
+static bool short_shares(int depth) { return depth < 1024; }
+
+// 32 x 32 tiles few enough that sixteen shares of the depth spread them over the CUs. (Few experts' shares are few bytes: a layer of 4096
+// tokens and 8 experts leaves them too.)
+static bool share_tiles(int tokens, int experts) {
+  const long long tiles = static_cast<long long>((tokens + 31) / 32) * ((experts + 31) / 32);
+  return tokens <= 2048 ? tiles < 112 : experts <= 32 && tiles <= 128;
+}
 
 // The sums of share `share` of the depth for 16 tokens from t0 on and 16 experts from e0 on.
 __device__ __forceinline__ f32x4 fine_share(const bf16_t* __restrict__ x, const float* __restrict__ kernel, int tokens, int depth, int experts,
@@ -201,45 +287,32 @@ __global__ __launch_bounds__(64) void router_logit_shares_kernel(const bf16_t* _
   }
 }
 
-// The shares of router_logits_mfma_kernel<1, 16> the same way: 32 tokens x 32 experts of one share of the depth a wavefront, for
-// the few hundred tokens whose tiles with sixteen wavefronts each leave CUs without one. The partial sums are that kernel's and are
-// added in its order: the same bits.
+// The shares of router_logits_mfma_kernel<1, 1, 16, 1, CHUNKS> the same way: 32 tokens x 32 experts of one share of the depth a wavefront,
+// for the few hundred tokens whose tiles with sixteen wavefronts each leave CUs without one. The partial sums are that kernel's and
+// are added in its order: the same bits.
+template <int CHUNKS, bool WHOLE>
 __global__ __launch_bounds__(64) void router_logit_tile_shares_kernel(const bf16_t* __restrict__ x, const float* __restrict__ kernel,
                                                                       float* __restrict__ partial, int tokens, int depth, int experts) {
-  const int lane = threadIdx.x, t0 = blockIdx.x * 32, e0 = blockIdx.y * 32, share = blockIdx.z;
-  const int chunks = depth / 16;
-  const int first = static_cast<int>(static_cast<long long>(chunks) * share / kShares);
-  const int last = static_cast<int>(static_cast<long long>(chunks) * (share + 1) / kShares);
-  const bf16_t* a_src = x + static_cast<size_t>(min(t0 + lane % 32, tokens - 1)) * depth + 8 * (lane / 32);
-  const float* b_src = kernel + static_cast<size_t>(8 * (lane / 32)) * experts + min(e0 + lane % 32, experts - 1);
-  f32x16 acc;
+  const int lane = threadIdx.x, t0 = blockIdx.x * 32, share = blockIdx.z;
+  const int steps = (depth + 16 * CHUNKS - 1) / (16 * CHUNKS), first = steps * share / kShares, last = steps * (share + 1) / kShares;
+  f32x16 acc[1][1];
+  logit_terms<1, 1, 1, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, min(32 * static_cast<int>(blockIdx.y) + lane % 32, experts - 1), first, last, acc);
+  const int e = 32 * blockIdx.y + lane % 32;
+  if (e >= experts) return;
+  float zero = 0.0f;  // (a NaN where any sum is no finite number)
 #pragma unroll
-  for (int i = 0; i < 16; ++i) acc[i] = 0.0f;
-  u32x4 words[2];
-  float b[2][8];
-  auto load = [&](int set, int chunk) __attribute__((always_inline)) {
-    words[set] = *reinterpret_cast<const u32x4*>(a_src + chunk * 16);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) b[set][j] = b_src[static_cast<size_t>(chunk * 16 + j) * experts];
-  };
-  auto multiply = [&](int set) __attribute__((always_inline)) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const uint32_t word = words[set][j / 2];
-      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(j % 2 ? word & 0xFFFF0000u : word << 16), b[set][j], acc, 0, 0, 0);
-    }
-  };
-  if (first < last) load(0, first);
-  for (int chunk = first; chunk < last; chunk += 2) {  // (past the share: the last chunk again, which multiplies nothing)
-    load(1, min(chunk + 1, last - 1));
-    multiply(0);
-    load(0, min(chunk + 2, last - 1));
-    if (chunk + 1 < last) multiply(1);
-  }
+  for (int i = 0; i < 16; ++i) zero = fmaf(0.0f, acc[0][0][i], zero);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
-    const int t = t0 + 8 * (i / 4) + 4 * (lane / 32) + i % 4, e = e0 + lane % 32;
-    if (t < tokens && e < experts) partial[(static_cast<size_t>(share) * tokens + t) * experts + e] = acc[i];
+    const int t = t0 + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
+    if (t < tokens) partial[(static_cast<size_t>(share) * tokens + t) * experts + e] = acc[0][0][i];
+  }
+  if (zero == 0.0f) return;
+  for (int i = 0; i < 16; ++i) {
+    const int t = t0 + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
+    if (t >= tokens) continue;
+    float* sum = partial + (static_cast<size_t>(share) * tokens + t) * experts + e;
+    *sum = finite_or_plain(*sum, x + static_cast<size_t>(t) * depth, kernel + e, experts, 16 * CHUNKS * first, min(16 * CHUNKS * last, depth));
   }
 }
 
@@ -252,13 +325,15 @@ LogitShares logit_shares(int tokens, int depth, int experts) {
   if (depth % 16 != 0) return kNoShares;
   if (tokens <= kShareTokens) return kFineShares;
   const long long blocks = static_cast<long long>((tokens + 31) / 32) * ((experts + 31) / 32);
-  if (depth < 64 || tokens > 2048 || blocks >= 112) return kNoShares;
+  if (depth < 64 || !share_tiles(tokens, experts)) return kNoShares;
   return blocks < 64 ? kFineShares : kTileShares;
 }
 
 int router_logit_shares(const void* x, const float* kernel, float* partial, int tokens, int depth, int experts, hipStream_t stream) {
   if (logit_shares(tokens, depth, experts) == kTileShares) {
-    hipLaunchKernelGGL(router_logit_tile_shares_kernel, dim3((tokens + 31) / 32, (experts + 31) / 32, kShares), dim3(64), 0, stream,
+    auto routine = short_shares(depth) ? (depth % 32 == 0 ? router_logit_tile_shares_kernel<2, true> : router_logit_tile_shares_kernel<2, false>)
+                                       : (depth % 64 == 0 ? router_logit_tile_shares_kernel<4, true> : router_logit_tile_shares_kernel<4, false>);
+    hipLaunchKernelGGL(routine, dim3((tokens + 31) / 32, (experts + 31) / 32, kShares), dim3(64), 0, stream,
                        static_cast<const bf16_t*>(x), kernel, partial, tokens, depth, experts);
     return launched("router_logit_tile_shares_kernel");
   }
@@ -350,20 +425,29 @@ extern "C" int dew_moe_router_logits(const void* x, const float* kernel, const f
                          static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts);
       return launched("router_logits_fine_kernel");
     }
-    if (tokens <= 2048) {  // at most 64 token blocks: a block takes one tile, its sixteen wavefronts share the depth
-      hipLaunchKernelGGL((router_logits_mfma_kernel<1, 16>), dim3((tokens + 31) / 32, tiles), dim3(1024), 0, s, static_cast<const bf16_t*>(x),
-                         kernel, bias, logits, tokens, depth, experts);
-      return launched("router_logits_mfma_kernel");
-    }
-    // (more than four tiles: blocks of four tiles beside each other, 64 accumulators a lane, several blocks a CU)
-    auto launch = [&](auto routine, int tiles_a_block, int rows_a_block) {
-      hipLaunchKernelGGL(routine, dim3((tokens + 32 * rows_a_block - 1) / (32 * rows_a_block), (tiles + tiles_a_block - 1) / tiles_a_block),
-                         dim3(256), 0, s, static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts);
+    auto launch = [&](auto whole, auto ragged, int step, int tokens_a_block, int tiles_a_block, int waves) {
+      hipLaunchKernelGGL(depth % step == 0 ? whole : ragged, dim3((tokens + tokens_a_block - 1) / tokens_a_block, (tiles + tiles_a_block - 1) / tiles_a_block),
+                         dim3(64 * waves), 0, s, static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts);
     };
-    if (tiles == 1) launch(router_logits_mfma_kernel<1, 4>, 1, 1);
-    else if (tiles == 2) launch(router_logits_mfma_kernel<2, 4>, 2, 1);
-    else if (static_cast<long long>(tokens / 64) * ((tiles + 3) / 4) >= 256) launch(router_logits_mfma_kernel<4, 4, 2>, 4, 2);  // still a block a CU
-    else launch(router_logits_mfma_kernel<4, 4>, 4, 1);
+#define DEW_LOGITS(ROWS, TILES, WAVES, AHEAD, CHUNKS)                       \
+  launch(router_logits_mfma_kernel<ROWS, TILES, WAVES, AHEAD, CHUNKS, true>, \
+         router_logits_mfma_kernel<ROWS, TILES, WAVES, AHEAD, CHUNKS, false>, 16 * CHUNKS, 32 * ROWS, TILES, WAVES)
+    auto blocks = [&](int rows, int beside) { return static_cast<long long>((tokens + 32 * rows - 1) / (32 * rows)) * ((tiles + beside - 1) / beside); };
+    // The largest tile that still gives most CUs a block: it reads x and the gate least often and splits a gate value for most rows.
+    // Measured (us; rows x tiles): 8192 x 7168 x 256 (256 blocks of 2 x 4) 104, in 2 x 2 129; 4096 x 7168 x 256 (256 of 2 x 2) 67, in
+    // 2 x 4 86; 3000 x 4096 x 256 (188 of 2 x 2) 42, in 2 x 1 49; 2112 x 7168 x 160 (165 of 2 x 1) 45, in 2 x 2 64, in 1 x 1 49; 5000 x
+    // 7168 x 32 (157 of 1 x 1) 35, in 2 x 1 50. Up to 2048 tokens eight wavefronts, whose shorter sums keep the error below the fp32
+    // instruction's on sixteen: 2048 x 7168 x 256 45 in 2 x 1, 88 there.
+    if (share_tiles(tokens, experts)) {  // (whose sums a layer's shares are)
+      if (short_shares(depth)) DEW_LOGITS(1, 1, 16, 1, 2);
+      else DEW_LOGITS(1, 1, 16, 1, 4);
+    } else if (tokens <= 2048 && blocks(2, 1) >= 128) DEW_LOGITS(2, 1, 8, 1, 4);
+    else if (tokens <= 2048) DEW_LOGITS(1, 1, 8, 1, 4);
+    else if (tiles >= 4 && blocks(2, 4) >= 224) DEW_LOGITS(2, 4, 4, 1, 4);
+    else if (tiles >= 2 && blocks(2, 2) >= 160) DEW_LOGITS(2, 2, 4, 2, 4);
+    else if (blocks(2, 1) >= 160) DEW_LOGITS(2, 1, 4, 2, 4);
+    else DEW_LOGITS(1, 1, 4, 2, 4);
+#undef DEW_LOGITS
     return launched("router_logits_mfma_kernel");
   }
   const dim3 grid((tokens + LT - 1) / LT, (experts + LE - 1) / LE);

@@ -1,0 +1,64 @@
+"""The gate's logits from three bf16 terms of the fp32 kernel, at the edges of every launch that forms them so: against the product in
+float64, with operands whose terms are not the value's (infinities, NaN, the largest magnitudes), and in a layer's shares."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+# tokens, depth, experts: the launch each shape takes stands behind it (tiles of 32 tokens x tiles of 32 experts, wavefronts a tile)
+SHAPES = [(14400, 80, 128),    # 2 x 4, 4; the depth ends inside a step
+          (14400, 320, 131),   # the last lane's experts overlap the lane's before it
+          (10300, 144, 40),    # 2 x 2, 4
+          (10300, 448, 20),    # 2 x 1, 4; steps left over behind the unrolled ones
+          (4200, 1088, 9),     # 1 x 1, 4
+          (2000, 208, 300),    # 2 x 1, 8
+          (1900, 112, 63),     # 1 x 1, 8
+          (2040, 80, 32),      # 1 x 1, 16 in steps of 32
+          (2100, 1040, 8)]     # 1 x 1, 16 in steps of 64
+
+
+@pytest.mark.parametrize("tokens,depth,experts", SHAPES)
+def test_three_terms_are_the_fp32_products(tokens, depth, experts):
+    """2^-19 of the summed magnitudes, as for the other launches: products exact in fp32, a few roundings a sum of up to 7168."""
+    from dew_amd import ops
+
+    generator = torch.Generator("cuda").manual_seed(depth + experts)
+    x = torch.randn((tokens, depth), generator=generator, device="cuda").to(torch.bfloat16)
+    kernel = torch.randn((depth, experts), generator=generator, device="cuda") * depth ** -0.5
+    bias = torch.randn(experts, generator=generator, device="cuda")
+    got = ops.router_logits(x, kernel, bias)
+    exact = x.double() @ kernel.double() + bias.double()
+    magnitudes = x.double().abs() @ kernel.double().abs() + bias.double().abs()
+    assert bool(((got.double() - exact).abs() <= 2.0 ** -19 * magnitudes).all())
+    assert torch.equal(got, ops.router_logits(x, kernel, bias))
+
+    x[3, depth - 1], x[tokens - 1, 0], x[7, 5] = float("inf"), float("nan"), -3.0e38
+    x[3, 2] = x[7, 2] = 0.0                              # (no product that overflows in fp32 alone meets an infinity of the other sign)
+    kernel[1, 0], kernel[depth - 1, experts - 1], kernel[2, 2], kernel[:, 4] = float("-inf"), float("nan"), 3.4028e38, 0.0
+    kernel.view(torch.int32)[9, 5] = 0x7F800001          # a NaN whose upper half is an infinity's
+    got = ops.router_logits(x, kernel)
+    exact = x.double() @ kernel.double()
+    assert torch.equal(got.isnan(), exact.isnan())
+    infinite = exact.abs() > torch.finfo(torch.float32).max
+    assert torch.equal(got[infinite].double(), exact[infinite].sign() * float("inf"))
+    plain = ~(infinite | exact.isnan())
+    magnitudes = x.double().nan_to_num(0, 0, 0).abs() @ kernel.double().nan_to_num(0, 0, 0).abs()
+    assert bool(((got.double() - exact)[plain].abs() <= 2.0 ** -19 * magnitudes[plain]).all())
+
+
+@pytest.mark.parametrize("tokens,depth", [(2040, 512), (2040, 1088), (2100, 1088)])
+def test_a_layers_shares_are_the_launchs_sums(tokens, depth):
+    from dew_amd import formats, moe
+
+    generator = torch.Generator("cuda").manual_seed(tokens + depth)
+    normal = lambda *shape: torch.randn(shape, generator=generator, device="cuda")
+    experts, hidden = 32 if tokens <= 2048 else 8, 128
+    layer = moe.SparseMLP(num_experts=experts, top_k=2, hidden_features=hidden, out_features=depth)
+    shapes = {"gate_proj": (depth, hidden), "up_proj": (depth, hidden), "down_proj": (hidden, depth)}
+    variables = {"params": {"gate": {"kernel": normal(depth, experts) * depth ** -0.5}},
+                 "quantization": {"experts": {n: {"kernel": formats.Bf16((normal(experts, *s) * 0.05).to(torch.bfloat16))} for n, s in shapes.items()}}}
+    x = normal(tokens, depth).to(torch.bfloat16)
+    x[5, 7], x[tokens - 1, depth - 1] = float("inf"), float("nan")
+    want, got = layer._bound(variables, ())(x), layer._applied(variables, x)
+    assert got is not None and torch.equal(got.nan_to_num(nan=9.0), want.nan_to_num(nan=9.0)) and bool(got[8].any())
