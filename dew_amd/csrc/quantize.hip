@@ -307,14 +307,12 @@ __global__ __launch_bounds__(256) void nvfp4_largest_kernel(const u32x4_t* __res
 // that contracts each group's tokens (reference src/dew/nn/kernels/projections.py:211-224 `rows_quantized(x.T)`, and
 // :263-275 `MxFp8.quantized(x.T)`). MX false: the blockwise FP8 recipe's 1 x 128 tiles (128 tokens of one column under
 // the scale rule of quantize_rows_fp8_kernel, its byte written for each of the tile's four 32-token blocks); MX true: OCP
-// MX blocks of 32 tokens (quantize_rows_mxfp8_kernel's rule). BANK false writes the lhs_t operand: codes [dim, tokens]
-// in the row operand's order within each 128 tokens (see the head of this file) and scales [dim, tokens / 32]. BANK true
-// writes the rhs_t operand as a prepared MXFP8 bank of one expert, depth = tokens, width = dim: codes as 32 column x 32
-// token atoms [dim / 32][tokens / 32][64 lanes][16 bytes] (lane 32 g + c holds tokens 16 g .. 16 g + 15 of column c) and
-// scales [dim / 32][tokens / 128][32 columns][4 bytes].
-// A block takes 128 tokens x 64 columns through the LDS: thread (column c, quarter a) owns the 32 tokens of block a.
-// HBM-bound: 2 bytes read and 1 written per element.
-template <bool MX, bool BANK>
+// MX blocks of 32 tokens (quantize_rows_mxfp8_kernel's rule).
+//
+// As the lhs_t operand, rows of tokens: codes [dim, tokens] in the row operand's order within each 128 tokens (see the head of this
+// file) and scales [dim, tokens / 32]. A block takes 128 tokens x 64 columns through the LDS: thread (column c, quarter a) owns the
+// 32 tokens of block a. HBM-bound: 2 bytes read and 1 written per element.
+template <bool MX>
 __global__ __launch_bounds__(256) void quantize_columns_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes,
                                                                uint32_t* __restrict__ scales, int tokens, int dim) {
   __shared__ uint32_t tile[128][33];     // 128 tokens x 64 columns of bf16, a dword of padding a row
@@ -364,23 +362,122 @@ __global__ __launch_bounds__(256) void quantize_columns_kernel(const bf16_t* __r
   }
   atomicOr(&scale_word[c], byte << (8 * quarter));
   const u32x4_t low = {packed[0], packed[1], packed[2], packed[3]}, high = {packed[4], packed[5], packed[6], packed[7]};
-  if constexpr (BANK) {
-    uint8_t* atom = codes + ((static_cast<size_t>((d0 + c) / 32) * (tokens / 32) + t0 / 32 + quarter) * 64 + c % 32) * 16;
-    *reinterpret_cast<u32x4_t*>(atom) = low;
-    *reinterpret_cast<u32x4_t*>(atom + 512) = high;
-    __syncthreads();
-    if (tid < 64) scales[(static_cast<size_t>((d0 + tid) / 32) * (tokens / 128) + t0 / 128) * 32 + tid % 32] = scale_word[tid];
-  } else {
-    // tokens 32 a + 16 g + b of the 128 sit at byte 16 (4 g + a) + b
-    staged[c][quarter ^ (c & 7)] = low;
-    staged[c][(4 + quarter) ^ (c & 7)] = high;
-    __syncthreads();
+  // tokens 32 a + 16 g + b of the 128 sit at byte 16 (4 g + a) + b
+  staged[c][quarter ^ (c & 7)] = low;
+  staged[c][(4 + quarter) ^ (c & 7)] = high;
+  __syncthreads();
 #pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int item = tid + 256 * k, row = item / 8, chunk = item % 8;
-      *reinterpret_cast<u32x4_t*>(codes + static_cast<size_t>(d0 + row) * tokens + t0 + chunk * 16) = staged[row][chunk ^ (row & 7)];
+  for (int k = 0; k < 2; ++k) {
+    const int item = tid + 256 * k, row = item / 8, chunk = item % 8;
+    *reinterpret_cast<u32x4_t*>(codes + static_cast<size_t>(d0 + row) * tokens + t0 + chunk * 16) = staged[row][chunk ^ (row & 7)];
+  }
+  if (tid < 64) scales[static_cast<size_t>(d0 + tid) * (tokens / 128) + t0 / 128] = scale_word[tid];
+}
+
+// As the rhs_t operand (or either operand of the launch that takes two such), a prepared MXFP8 bank of one expert, depth = tokens, width =
+// dim: codes as 32 column x 32 token atoms [dim / 32][tokens / 32][64 lanes][16 bytes] (lane 32 g + c holds tokens 16 g .. 16 g + 15 of
+// column c) and scales [dim / 32][tokens / 128][32 columns][4 bytes]; and, ROWS, along its rows too from the same read, which the
+// cotangent's other product takes (quantize_rows_fp8_kernel's and quantize_rows_mxfp8_kernel's bytes). A block takes 128 tokens x 128
+// columns: eight neighbours of a row a thread as they arrive, for the rows; then, through the LDS, 16 tokens of two neighbouring columns,
+// whose codes are 32 bytes of an atom. Every XCD's blocks walk along the columns of its own tokens, so that the few bytes of scales that a
+// block writes of a row meet in that XCD's L2. HBM-bound: 2 bytes read and 1 (ROWS: 2) written an element, at 4.8 to 5.8 TB/s. Measured (us): a
+// cotangent both ways, MXFP8, 32 768 x 14 336 567 by a launch each way, 368 here, FP8, 32 768 x 2048 80 and 46; along the tokens alone (once 128
+// tokens x 64 columns a block, a half word of the LDS a read) 32 768 x 4096 96 -> 80, 32 768 x 2048 45 -> 39, 32 768 x 14 336 274 -> 271.
+template <bool MX, bool ROWS>
+__global__ __launch_bounds__(512) void quantize_bank_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes, uint32_t* __restrict__ scales,
+                                                            uint8_t* __restrict__ row_codes, uint8_t* __restrict__ row_scales, int tokens, int dim,
+                                                            int pitch) {
+  constexpr int kRow = 68;              // dwords of a row of 128 columns as it is staged
+  __shared__ u32x4_t tile[128 * kRow / 4];
+  __shared__ float largest[8][128];     // of 16 tokens of a column
+  const int tid = threadIdx.x, across = dim / 128, tiles = tokens / 128 * across, run = (tiles + 7) / 8;
+  const int at = blockIdx.x % 8 * run + blockIdx.x / 8;  // (workgroup b runs on XCD b mod 8)
+  if (at >= tiles) return;
+  const int t0 = at / across * 128, d0 = at % across * 128;
+  const int chunk = tid % 16;
+  u32x4_t words[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) words[k] = *reinterpret_cast<const u32x4_t*>(x + static_cast<size_t>(t0 + tid / 16 + 32 * k) * dim + d0 + chunk * 8);
+  auto low = [](uint32_t word) { return __uint_as_float(word << 16); };
+  auto high = [](uint32_t word) { return __uint_as_float(word & 0xFFFF0000u); };
+  auto scale_byte = [](float most) -> uint32_t {
+    if (MX) return min(max(static_cast<int>(__float_as_uint(most) >> 23) - 8, 0), 254);
+    const uint32_t bits = __float_as_uint(fmaxf(most, 1e-4f) * 0x1.24924ap-9f);  // f32(1 / 448)
+    return min(max((bits >> 23) + ((bits & 0x7FFFFFu) != 0u ? 1u : 0u), 1u), 253u);
+  };
+  auto code4 = [](float a, float b, float c, float d, float inverse) {
+    float q[4] = {a * inverse, b * inverse, c * inverse, d * inverse};
+    if (MX) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q[i] = fminf(fmaxf(q[i], -448.0f), 448.0f);
     }
-    if (tid < 64) scales[static_cast<size_t>(d0 + tid) * (tokens / 128) + t0 / 128] = scale_word[tid];
+    const uint32_t half = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
+    return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], half, true));
+  };
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const int row = tid / 16 + 32 * k;
+    tile[row * (kRow / 4) + chunk] = words[k];
+    if constexpr (ROWS) {
+      float most = 0.0f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) most = fmaxf(most, fmaxf(fabsf(low(words[k][i])), fabsf(high(words[k][i]))));
+#pragma unroll
+      for (int offset = 1; offset < (MX ? 4 : 16); offset <<= 1) most = fmaxf(most, __shfl_xor(most, offset, 64));
+      const uint32_t byte = scale_byte(most);
+      const float inverse = __uint_as_float((254u - byte) << 23);
+      const u32x2_t packed = {code4(low(words[k][0]), high(words[k][0]), low(words[k][1]), high(words[k][1]), inverse),
+                              code4(low(words[k][2]), high(words[k][2]), low(words[k][3]), high(words[k][3]), inverse)};
+      const int half = chunk / 8, piece = chunk % 8 / 4, group = chunk % 4 / 2;  // (the operand order of the head of this file)
+      *reinterpret_cast<u32x2_t*>(row_codes + static_cast<size_t>(t0 + row) * dim + d0 + 16 * (4 * group + 2 * half + piece) + 8 * (chunk % 2)) = packed;
+      if constexpr (MX) {
+        uint32_t word = byte << (8 * (chunk / 4));
+        word |= __shfl_xor(word, 4, 64);
+        word |= __shfl_xor(word, 8, 64);
+        if (chunk == 0) *reinterpret_cast<uint32_t*>(row_scales + static_cast<size_t>(t0 + row) * (dim / 32) + d0 / 32) = word;
+      } else {
+        if (chunk == 0) row_scales[static_cast<size_t>(t0 + row) * pitch + d0 / 128] = static_cast<uint8_t>(byte);
+      }
+    }
+  }
+  __syncthreads();
+  const int pair = tid % 64, sixteen = tid / 64;
+  uint32_t column[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) column[i] = reinterpret_cast<const uint32_t*>(tile)[(16 * sixteen + i) * kRow + pair];
+  float first = 0.0f, second = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    first = fmaxf(first, fabsf(low(column[i])));
+    second = fmaxf(second, fabsf(high(column[i])));
+  }
+  largest[sixteen][2 * pair] = first;
+  largest[sixteen][2 * pair + 1] = second;
+  __syncthreads();
+  auto most_of = [&](int c, int thirty_two) {  // a column's block of 32 tokens, or its 128
+    if (MX) return fmaxf(largest[2 * thirty_two][c], largest[2 * thirty_two + 1][c]);
+    float most = largest[0][c];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) most = fmaxf(most, largest[i][c]);
+    return most;
+  };
+  const float inverse_first = __uint_as_float((254u - scale_byte(most_of(2 * pair, sixteen / 2))) << 23);
+  const float inverse_second = __uint_as_float((254u - scale_byte(most_of(2 * pair + 1, sixteen / 2))) << 23);
+  u32x4_t of_first, of_second;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    of_first[w] = code4(low(column[4 * w]), low(column[4 * w + 1]), low(column[4 * w + 2]), low(column[4 * w + 3]), inverse_first);
+    of_second[w] = code4(high(column[4 * w]), high(column[4 * w + 1]), high(column[4 * w + 2]), high(column[4 * w + 3]), inverse_second);
+  }
+  const int c = d0 + 2 * pair;
+  uint8_t* atom = codes + ((static_cast<size_t>(c / 32) * (tokens / 32) + t0 / 32 + sixteen / 2) * 64 + 32 * (sixteen % 2) + c % 32) * 16;
+  *reinterpret_cast<u32x4_t*>(atom) = of_first;
+  *reinterpret_cast<u32x4_t*>(atom + 16) = of_second;
+  if (tid < 128) {
+    uint32_t word = 0;
+#pragma unroll
+    for (int quarter = 0; quarter < 4; ++quarter) word |= scale_byte(most_of(tid, quarter)) << (8 * quarter);
+    scales[(static_cast<size_t>((d0 + tid) / 32) * (tokens / 128) + t0 / 128) * 32 + tid % 32] = word;
   }
 }
 
@@ -566,24 +663,30 @@ static int transpose_columns(const char* who, bool nvfp4, const void* x, void* o
   return launched("transpose_columns_kernel");
 }
 
-static int quantize_columns(const char* who, bool mx, const void* x, void* codes, void* scales, int tokens, int dim, int as_bank,
-                            void* stream) {
+// x [tokens, dim] along the tokens, as rows of tokens or as a bank, and with `row_codes` (as a bank) along its rows too.
+static int quantize_columns(const char* who, bool mx, const void* x, void* codes, void* scales, int tokens, int dim, int as_bank, void* stream,
+                            void* row_codes = nullptr, void* row_scales = nullptr) {
   DEW_REQUIRE(tokens >= 0 && tokens % 128 == 0, "%s: %d tokens are not whole 128-token blocks", who, tokens);
   DEW_REQUIRE(dim >= 128 && dim % 128 == 0, "%s: %d columns (whole 128s)", who, dim);
   if (tokens == 0) return DEW_MOE_OK;
   DEW_REQUIRE(tokens / 128 <= 65535 * 32, "%s: %d tokens", who, tokens);
   DEW_REQUIRE(x && codes && scales, "%s: x, codes and scales must not be null", who);
   DEW_REQUIRE(aligned16(x) && aligned16(codes) && aligned16(scales), "%s: x, codes and scales must be 16-byte aligned", who);
-  const dim3 grid(tokens / 128, dim / 64);
   hipStream_t s = static_cast<hipStream_t>(stream);
-  auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, static_cast<const bf16_t*>(x), static_cast<uint8_t*>(codes),
-                       static_cast<uint32_t*>(scales), tokens, dim);
-  };
-  if (mx && as_bank) launch(quantize_columns_kernel<true, true>);
-  else if (mx) launch(quantize_columns_kernel<true, false>);
-  else if (as_bank) launch(quantize_columns_kernel<false, true>);
-  else launch(quantize_columns_kernel<false, false>);
+  const bf16_t* from = static_cast<const bf16_t*>(x);
+  uint8_t* to = static_cast<uint8_t*>(codes);
+  uint32_t* scales_to = static_cast<uint32_t*>(scales);
+  if (as_bank) {
+    const long long tiles = static_cast<long long>(tokens / 128) * (dim / 128);
+    DEW_REQUIRE(tiles < (1ll << 30), "%s: %d tokens of %d columns", who, tokens, dim);
+    auto kernel = row_codes ? (mx ? quantize_bank_kernel<true, true> : quantize_bank_kernel<false, true>)
+                            : (mx ? quantize_bank_kernel<true, false> : quantize_bank_kernel<false, false>);
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>((tiles + 7) / 8 * 8)), dim3(512), 0, s, from, to, scales_to, static_cast<uint8_t*>(row_codes),
+                       static_cast<uint8_t*>(row_scales), tokens, dim, (dim / 128 + 15) / 16 * 16);
+    return launched("quantize_bank_kernel");
+  }
+  auto kernel = mx ? quantize_columns_kernel<true> : quantize_columns_kernel<false>;
+  hipLaunchKernelGGL(kernel, dim3(tokens / 128, dim / 64), dim3(256), 0, s, from, to, scales_to, tokens, dim);
   return launched("quantize_columns_kernel");
 }
 
@@ -614,6 +717,15 @@ extern "C" int dew_moe_quantize_columns_fp8(const void* x, void* codes, void* sc
 extern "C" int dew_moe_quantize_columns_mxfp8(const void* x, void* codes, void* scales, int32_t tokens, int32_t dim, int32_t as_bank,
                                               void* stream) {
   return dew::quantize_columns("dew_moe_quantize_columns_mxfp8", true, x, codes, scales, tokens, dim, as_bank, stream);
+}
+
+extern "C" int dew_moe_quantize_rows_and_columns(const void* x, void* row_codes, uint8_t* row_scales, void* codes, void* scales, int32_t tokens, int32_t dim,
+                                                 int32_t mx, void* stream) {
+  using namespace dew;
+  const char* who = "dew_moe_quantize_rows_and_columns";
+  DEW_REQUIRE(tokens == 0 || (row_codes && row_scales && aligned16(row_codes) && aligned16(row_scales)),
+              "%s: the rows' codes and scales must not be null and must be 16-byte aligned", who);
+  return quantize_columns(who, mx != 0, x, codes, scales, tokens, dim, 1, stream, row_codes, row_scales);
 }
 
 extern "C" int dew_moe_quantize_rows_nvfp4(const void* x, void* values, float* tensor_scale, uint32_t* workspace, int32_t rows,

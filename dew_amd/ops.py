@@ -989,16 +989,37 @@ def quantize_columns(x: torch.Tensor, *, mx: bool, as_bank: bool):
     call = _lib.library().dew_moe_quantize_columns_mxfp8 if mx else _lib.library().dew_moe_quantize_columns_fp8
     name = "dew_moe_quantize_columns_mxfp8" if mx else "dew_moe_quantize_columns_fp8"
     if as_bank:
-        buffer = torch.empty(max(tokens * dim + tokens // 32 * dim, 16), dtype=torch.uint8, device=x.device)
-        codes, scales = buffer[:tokens * dim], buffer[tokens * dim:tokens * dim + tokens // 32 * dim]
+        buffer, codes, scales = _columns_bank(x)
     else:
         codes = torch.empty((dim, tokens), dtype=torch.uint8, device=x.device)
         scales = torch.empty((dim, tokens // 32), dtype=torch.uint8, device=x.device)
     _lib.check(call(_ptr(x), _ptr(codes), _ptr(scales), tokens, dim, int(as_bank), _stream()), name)
-    if not as_bank:
-        return codes, scales
+    return _columns_prepared(x, buffer, codes, scales) if as_bank else (codes, scales)
+
+
+def _columns_bank(x: torch.Tensor):
+    tokens, dim = x.shape
+    buffer = torch.empty(max(tokens * dim + tokens // 32 * dim, 16), dtype=torch.uint8, device=x.device)
+    return buffer, buffer[:tokens * dim], buffer[tokens * dim:tokens * dim + tokens // 32 * dim]
+
+
+def _columns_prepared(x: torch.Tensor, buffer: torch.Tensor, codes: torch.Tensor, scales: torch.Tensor) -> PreparedBank:
+    tokens, dim = x.shape
     view = _lib.Bank(_lib.W_MXFP8, _lib.LAYOUT_PREPARED, 1, tokens, dim, _ptr(codes), _ptr(scales), None)
     return PreparedBank(view, (1, tokens, dim), (buffer,))
+
+
+def quantize_rows_and_columns(x: torch.Tensor, *, mx: bool) -> tuple[torch.Tensor, torch.Tensor, PreparedBank]:
+    """Both of a cotangent's quantizations from one read of it, bf16 `[tokens, dim]` of whole 128s: (`codes`, `scales`) as
+    `quantize_rows_mxfp8` (`mx`) or `quantize_rows_fp8` writes them, and `quantize_columns(x, mx=mx, as_bank=True)`."""
+    _device(x, "x", torch.bfloat16)
+    tokens, dim = x.shape
+    row_codes = torch.empty((tokens, dim), dtype=torch.uint8, device=x.device)
+    row_scales = torch.empty((tokens, dim // 32 if mx else block_scale_pitch(dim)), dtype=torch.uint8, device=x.device)
+    buffer, codes, scales = _columns_bank(x)
+    _lib.check(_lib.library().dew_moe_quantize_rows_and_columns(_ptr(x), _ptr(row_codes), _ptr(row_scales), _ptr(codes), _ptr(scales), tokens, dim,
+                                                                int(mx), _stream()), "dew_moe_quantize_rows_and_columns")
+    return row_codes, row_scales, _columns_prepared(x, buffer, codes, scales)
 
 
 def kernel_gradient_mxfp8(codes: torch.Tensor, scales: torch.Tensor, rhs_t: PreparedBank, offsets: torch.Tensor, *,

@@ -289,9 +289,13 @@ def kernel_gradient(x: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, m
     1 x 128 tiles (`rows_quantized(x.T)`, `blockwise_fp8_kernel_gradient`, src/dew/nn/kernels/projections.py:220-223)
     or, `mx`, MXFP8's blocks of 32 tokens (src/dew/nn/kernels/projections.py:268-274). Group `g` holds
     `group_blocks[g]` whole 128-token blocks; an empty group's gradient is zero."""
-    offsets = _groups(group_blocks, x.device).offsets
     bank = ops.quantize_columns(cotangent.contiguous(), mx=mx, as_bank=True)
-    if out_dtype in (torch.bfloat16, torch.float32) and ops.kernel_gradient_takes_banks(x.shape[0], x.shape[1], cotangent.shape[1], offsets.numel() - 1):
+    return _contracted(x, bank, cotangent.shape[1], _groups(group_blocks, x.device).offsets, mx, out_dtype)
+
+
+def _contracted(x: torch.Tensor, bank: ops.PreparedBank, width: int, offsets: torch.Tensor, mx: bool, out_dtype) -> torch.Tensor:
+    """`kernel_gradient` of a cotangent that is a bank already."""
+    if out_dtype in (torch.bfloat16, torch.float32) and ops.kernel_gradient_takes_banks(x.shape[0], x.shape[1], width, offsets.numel() - 1):
         return ops.kernel_gradient_mxfp8_banks(ops.quantize_columns(x.contiguous(), mx=mx, as_bank=True), bank, offsets, out_dtype=out_dtype)
     codes, scales = ops.quantize_columns(x.contiguous(), mx=mx, as_bank=False)
     return ops.kernel_gradient_mxfp8(codes, scales, bank, offsets, out_dtype=out_dtype)
@@ -303,16 +307,34 @@ def blockwise_fp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.T
     scale transpose as they are; the quantizer reads `w` where it lies, either way round); the matrices' is
     `kernel_gradient`."""
     group_blocks = _groups(group_blocks, x.device)    # once for both products
-    d_x = blockwise_fp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
-    return d_x, kernel_gradient(x, cotangent, group_blocks, mx=False, out_dtype=out_dtype)
+    if not _quantized_both_ways(cotangent):
+        d_x = blockwise_fp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
+        return d_x, kernel_gradient(x, cotangent, group_blocks, mx=False, out_dtype=out_dtype)
+    matrices = _bank(w.transpose(1, 2), "blockwise_fp8", (formats.Fp8Blocks, ops.PreparedBank), blocks_quantized)
+    *rows, columns = ops.quantize_rows_and_columns(cotangent.contiguous(), mx=False)
+    d_x = blockwise_fp8_product(QuantizedRows(*rows), matrices, group_blocks, out_dtype=x.dtype)
+    return d_x, _contracted(x, columns, cotangent.shape[1], group_blocks.offsets, False, out_dtype)
+
+
+def _quantized_both_ways(cotangent: torch.Tensor) -> bool:
+    """Whether a cotangent is one that `ops.quantize_rows_and_columns` takes; the others are quantized by a launch each way, which refuse
+    what no launch takes."""
+    return (cotangent.is_cuda and cotangent.dtype == torch.bfloat16 and cotangent.dim() == 2 and cotangent.shape[0] > 0 and cotangent.shape[1] > 0
+            and cotangent.shape[0] % SCALE_DEPTH == 0 and cotangent.shape[1] % SCALE_DEPTH == 0
+            and not (cotangent.is_contiguous() and cotangent.data_ptr() % 16))
 
 
 def mxfp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):
     """`_mx_backward` (src/dew/nn/kernels/projections.py:263-275) -> (d_x, d_w): the MXFP8 product of the cotangent and
     the matrices, both quantized along the width, and `kernel_gradient` with a scale every 32 tokens."""
     group_blocks = _groups(group_blocks, x.device)    # once for both products
-    d_x = mxfp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
-    return d_x, kernel_gradient(x, cotangent, group_blocks, mx=True, out_dtype=out_dtype)
+    if not _quantized_both_ways(cotangent):
+        d_x = mxfp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
+        return d_x, kernel_gradient(x, cotangent, group_blocks, mx=True, out_dtype=out_dtype)
+    matrices = _bank(w.transpose(1, 2), "mxfp8", (formats.MxFp8, ops.PreparedBank), formats.MxFp8.quantized)
+    *rows, columns = ops.quantize_rows_and_columns(cotangent.contiguous(), mx=True)
+    d_x = mxfp8_product(MxFp8Rows(*rows), matrices, group_blocks, out_dtype=x.dtype)
+    return d_x, _contracted(x, columns, cotangent.shape[1], group_blocks.offsets, True, out_dtype)
 
 
 def _contracted_in_place(tokens: int, depth: int, width: int, groups: int) -> bool:

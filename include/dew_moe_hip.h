@@ -422,6 +422,9 @@ int dew_moe_grouped_gemm_mxfp8_rows(const void* x_codes, const uint8_t* x_scales
  * [dim / 32][tokens / 32][64][16] bytes, then scales [dim / 32][tokens / 128][32][4]; wrap them in a dew_moe_bank
  * {MXFP8, PREPARED, experts 1, depth tokens, width dim}. tokens whole 128s (a recipe pads each group to them), dim
  * whole 128s.
+ * dew_moe_quantize_rows_and_columns: both of a cotangent's quantizations from one read of it: row_codes and row_scales as
+ * dew_moe_quantize_rows_fp8 writes them (mx: dew_moe_quantize_rows_mxfp8), codes and scales as dew_moe_quantize_columns_fp8
+ * (_mxfp8) does with as_bank 1; the same bytes.
  * dew_moe_kernel_gradient_mxfp8: out [groups, depth, width] (bf16, or fp32 where out_is_f32) from the lhs_t operand
  * [depth, tokens] and the rhs_t bank [width, tokens]; group g contracts tokens offsets[g] .. offsets[g + 1], whole
  * 128-token blocks (device int32 [groups + 1]); an empty group's matrix is zero. Both operands enter
@@ -432,6 +435,8 @@ int dew_moe_quantize_columns_fp8(const void* x /* bf16 [tokens, dim] */, void* c
                                  int32_t dim, int32_t as_bank, void* stream);
 int dew_moe_quantize_columns_mxfp8(const void* x /* bf16 [tokens, dim] */, void* codes, void* scales, int32_t tokens,
                                    int32_t dim, int32_t as_bank, void* stream);
+int dew_moe_quantize_rows_and_columns(const void* x /* bf16 [tokens, dim] */, void* row_codes, uint8_t* row_scales, void* codes,
+                                      void* scales, int32_t tokens, int32_t dim, int32_t mx, void* stream);
 int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint8_t* lhs_t_scales, const dew_moe_bank* rhs_t,
                                   const int32_t* offsets, void* out, int32_t out_is_f32, int32_t depth, int32_t groups,
                                   void* stream);

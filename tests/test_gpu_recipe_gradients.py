@@ -269,3 +269,21 @@ def test_kernel_gradients_over_more_groups_than_a_block_has_threads(ops, kind):
         bar = 2.0 ** -18
     assert np.abs(got - want).max() <= bar * np.abs(want).max()
     assert not got[blocks == 0].any()
+
+
+@pytest.mark.parametrize("tokens,dim", [(128, 128), (256, 384), (128, 2176), (1152, 640)])
+@pytest.mark.parametrize("mx", [False, True], ids=["fp8", "mxfp8"])
+def test_one_read_quantizes_a_cotangent_both_ways(ops, tokens, dim, mx):
+    """The same bytes as by the rows' quantizer and, along the tokens, the oracle's; one tile, tiles in no whole eighths, 17 across."""
+    x = tokens_case(tokens, dim, seed=tokens + dim).cuda()
+    x[3, 5], x[tokens - 1, dim - 2] = float("inf"), float("nan")
+    x[64:96, 32:64] = 0.0
+    codes, scales, bank = ops.quantize_rows_and_columns(x, mx=mx)
+    want_codes, want_scales = ops.quantize_rows_mxfp8(x) if mx else ops.quantize_rows_fp8(x)
+    held = dim // 32 if mx else dim // 128                  # (the FP8 rows' pitch is padding from there on)
+    assert torch.equal(codes, want_codes) and torch.equal(scales[:, :held], want_scales[:, :held])
+    lhs_codes, lhs_scales = ops.quantize_columns(x, mx=mx, as_bank=False)
+    got_codes, got_scales = bank_codes(bank, tokens, dim)
+    assert np.array_equal(got_codes, ops.depth_order_fp8(lhs_codes).cpu().numpy()) and np.array_equal(got_scales, lhs_scales.cpu().numpy())
+    alone_codes, alone_scales = bank_codes(ops.quantize_columns(x, mx=mx, as_bank=True), tokens, dim)
+    assert np.array_equal(got_codes, alone_codes) and np.array_equal(got_scales, alone_scales)
