@@ -352,20 +352,29 @@ static bool few_tiles(int rows, int groups, int width) {  // about so many of 12
   return (rows / 128 + groups / 2 + 1) * static_cast<long long>((width + 255) / 256) <= kFewTiles;
 }
 
-// 256 x 256 tiles (wide.hip) where they fill the CUs over the rounds that they take, on groups of at least about half a tile's rows
-// (of 64 to 97 rows 0.82 to 0.98 times as fast). Measured against the tiles below on some 250 shapes (64 to 7168 deep, 1 to 64 groups; us,
-// there and here). Natural order, from 0.57 on: 4608 rows of 1 x 1024 x 2048, 148 tiles, 32.1 and 25.5, 4300 of 4 x 4096 x 2048 97.4 and 77.3,
-// 10 000 of 4 x 512 x 2048, 328 tiles, 33.7 and 30.9, 8192 of 8 x 4096 x 2048, 288, 159 and 162, 9000 of 1 x 4096 x 4096, 570, 290 and 262; below it 4096
-// of 1 x 4096 x 2048, 132, 67.5 and 80.3, 8300 of 4 x 4096 x 2048, 275, 158 and 164. K-major matrices, which the tiles below read half a cache line
-// at a step, from 0.51 on: 4608 of 1 x 4096 x 2048 121 and 78, 8300 of 4 x 4096 x 2048 184 and 162, 8448 of 1 x 7168 x 2048, 268 tiles, 318 and 278;
-// 4096 of 1 x 4096 x 2048, 132 tiles, 75.6 and 79.9, 3300 of 4, 119, 72.3 and 72.9.
+// 256 x 256 tiles (wide.hip) on groups of at least about half a tile's rows (of 64 to 97 rows 0.82 to 0.98 times as fast) but where they
+// are a first round of whole ones that is half empty. Measured against the tiles below (us, there and here). Whole tiles, natural order, from
+// 146 on: 4608 rows of 1 x 1024 x 2048, 148 tiles, 32.1 and 25.5, 4300 of 4 x 4096 x 2048 97.4 and 77.3; below it 4096 of 1 x 4096 x 2048, 132, 67.5
+// and 80.3, 3584 of 4, 136, 69.5 and 83.2. K-major matrices, which the tiles below read half a cache line at a step, from 129: 4096 of 1 x 4096 x 2048, 132,
+// 75.6 and 79.9, of 4, 136, 81.4 and 77.0. A second round begun: 4352 rows of 1 x 4096 x 4096, 272 tiles, 165 and 125. In quarters alone, natural and
+// K-major, up to one a block: 512 rows of 1 x 4096 x 4096, 32 tiles, 42.2 and 42.7 -> 29.4 and 29.1, 1024, 64, 67.7 and 74.8 -> 37.0 and 37.6, 1024 x 4096, 25.1
+// and 27.0 -> 17.7 and 20.3, 1024 of 8 x 4096 x 2048 53.0 and 58.2 -> 31.2 and 31.8; up to two where the walk is long: 1536 of 1 x 4096 x 4096, 96, 67.3 and
+// 74.1 -> 60.6 and 60.4, 2560 of 4 x 1024 x 2048, 88, 24.7 and 26.7 -> 23.6 and 23.4, 1732 of 8 x 1152 x 1792, 70, natural, 20.0 and 22.6. Of 90 shapes of 128 to
+// 16 384 rows in 1 to 16 groups (steps of one forward product, one input's gradient and one kernel's) these rules make the three 1.09, 1.11 and
+// 1.09 times as fast; furthest off 3127 of 1 x 3584 x 1152, 65 tiles, 46 and 50.
 static bool wide_product(int rows, int groups, int depth, int width, bool kmajor) {
-  return wide_extents(groups, depth, width) && rows / groups >= 112 && fills_rounds(product_tiles(rows, groups, width), kmajor ? 51 : 57, kGuessed);
+  const double tiles = product_tiles(rows, groups, width);
+  const int quarters = depth >= (kmajor ? 1024 : 2048) ? 128 : 64;
+  return wide_extents(groups, depth, width) && rows / groups >= 112 && (tiles + (groups > 1 ? kGuessed : 0) <= quarters || tiles >= (kmajor ? 129 : 146));
 }
 
-// A kernel's gradient; groups of fewer than 256 rows, four steps, are all start and end either way (0.91 to 1.18 times as fast).
+// A kernel's gradient; groups of fewer than 256 rows, four steps, are all start and end either way (0.91 to 1.18 times as fast), and in quarters those of
+// fewer than 512 (813 rows of 3 x 640 x 2176, 81 tiles, 10.7 and 13.3; us, there and here, 4096 of 2 x 512 x 2048, 32 tiles, 32.1 and 17.9, of 1 x 1024 x 4096, 64,
+// 57.5 and 35.5, 1 x 2048 x 4096, 128, 81.6 and 67.2; 512 12.5 and 11.3, 16.9 and 17.1). Whole tiles from over half a round on: 144 of 512 rows 20.1 and
+// 18.4, of 8192 207 and 169.
 static bool wide_gradient(int rows, int groups, int depth, int width) {
-  return wide_extents(groups, depth, width) && rows / groups >= 256 && fills_rounds(gradient_tiles(groups, depth, width), kGradientRounds);
+  const double tiles = gradient_tiles(groups, depth, width);
+  return wide_extents(groups, depth, width) && rows / groups >= (tiles <= 128 ? 512 : 256) && (tiles <= 128 || tiles >= 141);
 }
 
 }  // namespace dew

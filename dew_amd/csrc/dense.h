@@ -14,6 +14,7 @@ struct DenseParams {
   void* out;
   const float *factor0, *factor1;  // a kernel gradient's sums times *factor0 * *factor1 (each may be null)
   int groups, rows, inner, outer_m, outer_n, m_tiles, group_m;
+  int quarter_turns;  // 256 x 256 tiles: the last round in quarters where a block has at most so many
 };
 
 // 256 x 256 tiles on blocks that stay (wide.hip), of rows that are neither gathered nor scattered; `across`: a kernel gradient; `kmajor`:

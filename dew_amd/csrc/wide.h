@@ -46,8 +46,9 @@ struct WideTiles {
   static constexpr int kRounds = kWideGroups / 64;
   int first_tile[kRounds], first_row[kRounds], group_size[kRounds];
   int gradient_tiles, strips, total, held;  // `held`: rows in all groups
+  int whole;                                // tiles that leave as such; those behind them in quarters
 
-  __device__ __forceinline__ void find(const int32_t* offsets, const int32_t* sizes, int groups, int outer_m, int outer_n) {
+  __device__ __forceinline__ void find(const int32_t* offsets, const int32_t* sizes, int groups, int outer_m, int outer_n, int quarter_turns) {
     const int lane = threadIdx.x % 64;
     gradient_tiles = (outer_m + kWideTile - 1) / kWideTile;
     int m_tiles = 0;
@@ -73,6 +74,19 @@ struct WideTiles {
     if (!sizes) held = offsets[groups];
     strips = (outer_n + kWideTile - 1) / kWideTile;
     total = __builtin_amdgcn_readfirstlane(m_tiles * strips);
+    const int blocks = gridDim.x, behind = total % blocks;
+    whole = behind <= blocks * quarter_turns / 4 ? total - behind : total;
+  }
+
+  // The block's quarter tile number `turn` of those behind the whole ones, false past its last: its tile, and which quarter. Neighbours
+  // are an XCD's, and share their operands in its L2.
+  __device__ __forceinline__ bool quarter_at(int turn, int group_m, WidePlace& out, int& quarter) const {
+    const int xcds = 8, slots = gridDim.x / xcds, count = 4 * (total - whole), run = (count + xcds - 1) / xcds, slot = blockIdx.x / xcds + turn * slots;
+    const int order = __builtin_amdgcn_readfirstlane(slot < run ? blockIdx.x % xcds * run + slot : count);
+    if (order >= count) return false;
+    quarter = order % 4;
+    place(whole + order / 4, group_m, out);
+    return true;
   }
 
   // The block's tile number `turn`, false past its last. A round of one tile a block is chunks of group_m row tiles x 8 strips, one an XCD;
@@ -81,9 +95,14 @@ struct WideTiles {
   // of a product's 222, [11 264, 12 800] x 1280, 159 -> 152.)
   __device__ __forceinline__ bool at(int turn, int group_m, WidePlace& out) const {
     const int xcds = 8, slots = gridDim.x / xcds, begun = turn * slots * xcds;
-    const int run = min((total - begun + xcds - 1) / xcds, slots), slot = blockIdx.x / xcds;
-    const int order = __builtin_amdgcn_readfirstlane(slot < run ? begun + blockIdx.x % xcds * run + slot : total);
-    if (order >= total) return false;
+    const int run = min((whole - begun + xcds - 1) / xcds, slots), slot = blockIdx.x / xcds;
+    const int order = __builtin_amdgcn_readfirstlane(slot < run ? begun + blockIdx.x % xcds * run + slot : whole);
+    if (order >= whole) return false;
+    place(order, group_m, out);
+    return true;
+  }
+
+  __device__ __forceinline__ void place(int order, int group_m, WidePlace& out) const {
     const int across = order / strips;  // (the tiles of a group are in a row: this many before it at most)
     int group = -1;
 #pragma unroll
@@ -100,7 +119,6 @@ struct WideTiles {
     const int place_in_group = order - before * strips;
     const int band = place_in_group / (group_m * strips), band_tiles = min(group_m, tiles - band * group_m), within = place_in_group % (group_m * strips);
     out = WidePlace{group, start, size, band * group_m + within % band_tiles, within / band_tiles};
-    return true;
   }
 };
 
@@ -115,15 +133,16 @@ __device__ __forceinline__ void clear_unowned(bf16_t* out, int held, int rows, i
 }
 
 // The sums are zero: sixteen products of zeros, in half the time of as many moves (each of its own, or the compiler makes one and copies it).
-__device__ __forceinline__ void clear_sums(f32x16_t (&acc)[4][4]) {
+template <int kTiles>
+__device__ __forceinline__ void clear_sums(f32x16_t (&acc)[kTiles][kTiles]) {
   bf16x8_t zero = __builtin_bit_cast(bf16x8_t, u32x4_t{0, 0, 0, 0});
   f32x16_t none;
 #pragma unroll
   for (int q = 0; q < 16; ++q) none[q] = 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < kTiles; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
+    for (int j = 0; j < kTiles; ++j) {
       asm volatile("" : "+v"(zero));
       acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(zero, zero, none, 0, 0, 0);
     }
@@ -156,8 +175,8 @@ __device__ __forceinline__ void across_quads(uint32_t (&v)[4]) {
 // steps and a store a tile, FP8, 32 768 tokens of 32 x 7168 x 2048, 561 -> 526 (396 without any store), of 8 x 4096 x 14 336 1510 -> 1487;
 // of products, deeper, 1 to 2 % less. `out_row0`, `valid_rows`: the block's tile (what lies past the buffer's end, the rows
 // past its last, and the columns sent there are not stored); `tile_row`, `column0`: the wavefront's place in it and in the row.
-template <bool kOutF32>
-__device__ __forceinline__ void leave(f32x16_t (&acc)[4][4], void* to_rows, size_t out_row0, int valid_rows, int width, int tile_row, int column0, float factor) {
+template <bool kOutF32, int kTiles>
+__device__ __forceinline__ void leave(f32x16_t (&acc)[kTiles][kTiles], void* to_rows, size_t out_row0, int valid_rows, int width, int tile_row, int column0, float factor) {
   int lane = threadIdx.x % 64;
   asm volatile("" : "+v"(lane));
   constexpr int kOutBytes = kOutF32 ? 4 : 2;
@@ -168,15 +187,15 @@ __device__ __forceinline__ void leave(f32x16_t (&acc)[4][4], void* to_rows, size
   auto stay = [&](int i) __attribute__((always_inline)) {
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) asm volatile("" : "+a"(acc[i][j]));
+    for (int j = 0; j < kTiles; ++j) asm volatile("" : "+a"(acc[i][j]));
 #endif
   };
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < kTiles; ++i) {
     stay(i);
     const uint32_t row = tile_row + 32 * i + lane % 32 / 4 * 4;
 #pragma unroll
-    for (int pair = 0; pair < 2; ++pair) {
+    for (int pair = 0; pair < kTiles / 2; ++pair) {
       // the lane's row of tile 2 pair + lane / 32, in pieces of 16 bytes
       constexpr int kPieces = kOutF32 ? 8 : 4;
       uint32_t pieces[kPieces][4];

@@ -56,7 +56,7 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_fp8_kernel(WideFp8Params
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)lds));
 
   WideTiles<kGradient> tiles;
-  tiles.find(p.offsets, nullptr, p.groups, p.rows, p.width);
+  tiles.find(p.offsets, nullptr, p.groups, p.rows, p.width, 0);
   if constexpr (!kGradient) clear_unowned(static_cast<bf16_t*>(p.out), tiles.held, p.rows, p.width);
 
   struct Tile {

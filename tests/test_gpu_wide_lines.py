@@ -24,6 +24,22 @@ def test_gradients(sizes, depth, width, out_dtype):
     test_gpu_wide.test_gradients(sizes, depth, width, out_dtype)
 
 
+# Quarters: a launch of nothing else (with a group of no rows and one of a row; whole quarters past a group's rows and past the width), two a
+# block, and behind a whole round, one a block and two; the depths are one step, an odd number and more than the ring holds.
+@pytest.mark.parametrize("depth,sizes,width", ((64, [129, 1000, 0, 383, 1, 700], 800), (320, [129, 1000, 383, 700], 800), (448, [600], 160),
+                                               (2112, [2100, 1900], 1504), (448, [4000], 4384), (1088, [3800, 200], 5472)))
+def test_products_in_quarters(monkeypatch, depth, sizes, width):
+    monkeypatch.setitem(test_gpu_wide.SIZES, "quarters", sizes)
+    monkeypatch.setitem(test_gpu_wide.WIDTHS, "quarters", width)
+    test_gpu_wide.test_products("quarters", depth)
+
+
+@pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("sizes,depth,width", (([600, 513, 1, 800], 264, 1032), ([2000, 1100], 1032, 2568), ([700, 800], 2056, 4104), ([1500, 900], 2504, 4400)))
+def test_gradients_in_quarters(sizes, depth, width, out_dtype):
+    test_gpu_wide.test_gradients(sizes, depth, width, out_dtype)
+
+
 @pytest.mark.parametrize("sizes", ([480, 600, 700, 500], [1900, 2050, 2100, 1950]))     # 97 tiles by the launch's guess, 275
 @pytest.mark.parametrize("recipe", ("blockwise_fp8", "mxfp8"))
 def test_recipes_products(monkeypatch, recipe, sizes):
