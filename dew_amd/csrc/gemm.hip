@@ -1311,20 +1311,20 @@ static bool few_gradient_blocks(const GemmParams& p) {
   return static_cast<long long>(p.experts) * ((p.window_rows + 255) / 256) * ((p.width + 255) / 256) <= 128;
 }
 
-// The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered: on groups of half
-// a tile's rows, wherever such tiles are enough to measure, from three eighths of a round on. Against the launches below (us, there and
-// here, 160 shapes of 512 to 32 768 rows, 1 to 51 groups, depths from 512): blockwise, [2560, 512] x 2048 of 4 groups, 96 tiles, 14.2 and 12.7, 4096
-// deep 46.5 and 42.3; [4608, 1024] x 2048, 148, 26.0 and 18.3; [8192, 4096] x 2048 of 2, 264 tiles of two rounds, 92.2 and 87.7; [32 768, 7168] x 2048 of
-// 32, forward 470 and 424, input's gradient 520 and 444; MXFP8, [32 768, 4096] x 14336 of 8 1636 and 1490. Least: [3584, 1024] x 2048, 116, blockwise, 18.5 and 18.3.
-constexpr int kFp8ProductRounds = 37;
-
+// The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered, on groups of half
+// a tile's rows, but for what two quarters a block of a short walk would take. Against the launches below (us, there and here). Whole tiles:
+// blockwise, [2560, 512] x 2048 of 4 groups, 96 tiles, 14.2 and 12.7; [4608, 1024] x 2048, 148, 26.0 and 18.3; [32 768, 7168] x 2048 of 32, forward 470
+// and 424, input's gradient 520 and 444; MXFP8, [32 768, 4096] x 14336 of 8 1636 and 1490. In quarters, up to one a block: [1024, 2944] x 640 of 2, 15
+// tiles, 19.5 and 14.1, [1792, 5504] x 896 of 11, 44, 31.9 and 23.3, [1408, 896] x 640 of 6, 21, 9.5 and 8.9; up to two: [1280, 3456] x 3840 of 2, 75, 43.7 and
+// 32.0, [3584, 2176] x 1920 of 4, 120, 29.6 and 24.0; but [1408, 1920] x 2688 of 2, 66, 17.6 and 21.7, [640, 1152] x 5248 of 4, 84, 14.0 and 16.7.
 static WideFp8Params wide_fp8_params(const GemmParams& p, int a_scale_pitch) {
   return WideFp8Params{reinterpret_cast<const uint8_t*>(p.x), p.a_scale, p.w0.codes, p.w0.scales, p.offsets, p.out, p.experts, p.rows, p.depth, p.width, a_scale_pitch};
 }
 
 static bool wide_fp8_product(const GemmParams& p) {
+  const double tiles = product_tiles(p.rows, p.experts, p.width);
   return forced_tile_rows == 0 && !p.gather && !p.scatter && !p.bias && wide_extents(p.experts, p.depth, p.width) && p.depth >= 512 &&
-         p.rows / p.experts >= 112 && fills_rounds(product_tiles(p.rows, p.experts, p.width), kFp8ProductRounds, kGuessed);
+         p.rows / p.experts >= 112 && (p.depth >= 2048 || tiles >= 95 || tiles + (p.experts > 1 ? kGuessed : 0) <= 64);
 }
 
 static bool wide_fp8_gradient_extents(int tokens, int depth, int width, int groups) {
@@ -1549,9 +1549,13 @@ extern "C" int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint
   return launch_tile<kFormatMxFp8Window, kPlain, 256, 128, 2, 2>(who, p, s);
 }
 
+// (In quarters up to one a block: us, there and here, 8064 tokens of 1920 x 1536, 48 tiles, 55.1 and 30.6, 4224 of 1792 x 640, 21, 31.6 and 17.7, 896 of
+// 6 x 1280 x 512, 60, 9.9 and 7.3; up to two they gain a little or lose: 5376 of 2 x 3456 x 896, 112, 29.4 and 27.9, 20 992 of 4 x 1152 x 1536, 120, 61 and 67.
+// Whole tiles from over half a round on: 144 of 512 tokens 20.1 and 16.5, of 8192 99.9 and 85.7; 130 of 4224 25.2 and 30.7.)
 extern "C" int dew_moe_kernel_gradient_takes_banks(int32_t tokens, int32_t depth, int32_t width, int32_t groups) {
   using namespace dew;
-  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && fills_rounds(gradient_tiles(groups, depth, width), kGradientRounds);
+  const double tiles = gradient_tiles(groups, depth, width);
+  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && (tiles <= 64 || tiles >= 141);
 }
 
 extern "C" int dew_moe_kernel_gradient_mxfp8_banks(const dew_moe_bank* lhs_t, const dew_moe_bank* rhs_t, const int32_t* offsets, void* out,

@@ -12,28 +12,23 @@ namespace dew {
 constexpr int kWideThreads = 256, kWideTile = 256;
 constexpr int kWideGroups = 256;  // groups that such a launch keeps the tiles of in registers
 
-// Whether `tiles` 256 x 256 tiles keep `percent` of the 256 CUs busy over the rounds that they take, one tile a CU and round. A kernel's
-// gradient knows its tiles; a product's are a guess, since its groups end where they end: kGuessed of them may not be there (two groups of
-// 1950 rows x 4096 columns are guessed 260 tiles and are 256: bf16, 1024 deep, 36.4 us in smaller tiles and 31.5; where they are 264, the
-// other way round, 45.8 and 49.4). Each launch has one line for all rounds, where both sides, timed in turn, meet.
+// The 256 x 256 tiles of a launch, of which a CU takes one a round. A kernel's gradient knows its tiles; a product's are a guess, since its
+// groups end where they end: about kGuessed of them may not be there, or more.
 constexpr int kGuessed = 8;
-inline bool fills_rounds(double tiles, int percent, int may_be_missing = 0) {
-  const double rounds = fmax(1.0, ceil((tiles - may_be_missing) / 256));
-  return tiles * 100 >= rounds * 256 * percent;
-}
-
 inline double product_tiles(int rows, int groups, int width) { return (rows / 256.0 + groups / 2.0) * ((width + 255) / 256); }
 
-// Of either type's kernel gradients: over half a round, up to which the launches of smaller tiles take half as large ones again (us, there and
-// here, e4m3 then bf16: 144 tiles of 512 tokens 20.1 and 16.5, 20.1 and 18.4, of 8192 99.9 and 85.7, 207 and 169; 128 of 1024 16.4 and 18.9, 24.9
-// and 28.0, of 8192 63.9 and 83.4, 153 and 169), and over half of two (288 of 1024 35.5 and 33.8, 53.3 and 49.9; 260 34.2 and 34.7, 50.2 and 53.3;
-// 264 of 33 x 512 x 1024 39.2 and 43.8, 53.1 and 65.9).
-constexpr int kGradientRounds = 55;
 inline double gradient_tiles(int groups, int depth, int width) { return static_cast<double>(groups) * ((depth + 255) / 256) * ((width + 255) / 256); }
 
 inline bool wide_extents(int groups, int a, int b) { return groups <= kWideGroups && a <= (1 << 20) && b <= (1 << 20); }  // (offsets within a tile are 32-bit)
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// Whether a kernel's gradient leaves its last tiles in quarters; its launch carries their code only then (the registers that it keeps for it
+// cost every other tile's start: e4m3, eight tiles of a few steps a block, 3 to 5 %). A product's tiles are known on the device alone.
+inline bool ends_in_quarters(int groups, int depth, int width, int quarter_turns) {
+  const int tiles = static_cast<int>(gradient_tiles(groups, depth, width));
+  return tiles % 256 != 0 && tiles % 256 <= 64 * quarter_turns;
+}
 
 struct WidePlace {
   int group, start, size;  // the tile's group: its first row and its rows

@@ -460,19 +460,19 @@ __device__ __forceinline__ void quarter_tiles(const DenseParams& p, const WideTi
   __builtin_amdgcn_s_waitcnt(7 << 4);  // (no load into the LDS outlives the block)
 }
 
-template <bool kAAcross, bool kBAcross, bool kOutF32>
+template <bool kAAcross, bool kBAcross, bool kOutF32, bool kQuarters>
 __global__ __launch_bounds__(kWideThreads, 1) void wide_kernel(DenseParams p) {
   extern __shared__ uint8_t lds[];
   WideTiles<kAAcross> tiles;
-  tiles.find(p.offsets, p.sizes, p.groups, p.outer_m, p.outer_n, p.quarter_turns);
+  tiles.find(p.offsets, p.sizes, p.groups, p.outer_m, p.outer_n, kQuarters ? p.quarter_turns : 0);
   if constexpr (!kAAcross) clear_unowned(static_cast<bf16_t*>(p.out), tiles.held, p.rows, p.outer_n);
   whole_tiles<kAAcross, kBAcross, kOutF32>(p, tiles, lds);
-  if (tiles.whole < tiles.total) quarter_tiles<kAAcross, kBAcross, kOutF32>(p, tiles, lds);
+  if (kQuarters && tiles.whole < tiles.total) quarter_tiles<kAAcross, kBAcross, kOutF32>(p, tiles, lds);
 }
 
-template <bool kAAcross, bool kBAcross, bool kOutF32>
+template <bool kAAcross, bool kBAcross, bool kOutF32, bool kQuarters>
 static int launch_wide_kernel(const char* who, const DenseParams& p, hipStream_t stream) {
-  auto kernel = wide_kernel<kAAcross, kBAcross, kOutF32>;
+  auto kernel = wide_kernel<kAAcross, kBAcross, kOutF32, kQuarters>;
   static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
   static hipError_t reserved = hipSuccess;
   std::call_once(configured, [&] {
@@ -491,8 +491,10 @@ int launch_wide(const char* who, const DenseParams& params, bool across, bool km
   // long as the whole tile or longer (2.7 rounds 110 -> 120, 0.66 228 -> 282).
   p.quarter_turns = (across ? p.rows / p.groups : p.inner) >= 1024 ? 2 : 1;
   p.group_m = 4;  // (4 row tiles x 8 strips are what an XCD's 32 CUs hold at once; 6 or 8 were 0 to 3 % slower)
-  if (across) return out_f32 ? launch_wide_kernel<true, true, true>(who, p, stream) : launch_wide_kernel<true, true, false>(who, p, stream);
-  return kmajor ? launch_wide_kernel<false, false, false>(who, p, stream) : launch_wide_kernel<false, true, false>(who, p, stream);
+  if (!across) return kmajor ? launch_wide_kernel<false, false, false, true>(who, p, stream) : launch_wide_kernel<false, true, false, true>(who, p, stream);
+  if (ends_in_quarters(p.groups, p.outer_m, p.outer_n, p.quarter_turns))
+    return out_f32 ? launch_wide_kernel<true, true, true, true>(who, p, stream) : launch_wide_kernel<true, true, false, true>(who, p, stream);
+  return out_f32 ? launch_wide_kernel<true, true, true, false>(who, p, stream) : launch_wide_kernel<true, true, false, false>(who, p, stream);
 }
 
 }  // namespace dew

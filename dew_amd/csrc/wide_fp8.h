@@ -13,6 +13,7 @@ struct WideFp8Params {
   const int32_t* offsets;      // [groups + 1] of the rows, or (a kernel gradient) of the depth
   void* out;
   int groups, rows, depth, width, a_scale_pitch;  // a kernel gradient's `rows`: every group's
+  int quarter_turns;           // the last round in quarters where a block has at most so many
 };
 
 int launch_wide_fp8(const char* who, const WideFp8Params& p, bool mx, bool gradient, bool out_f32, hipStream_t stream);

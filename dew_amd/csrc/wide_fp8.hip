@@ -12,6 +12,7 @@
 //    filled the L1 with as many lines as the rows themselves.
 //  * The pipe is 67 to 69 % busy at 1.9 GHz over 32 and more steps a tile of MXFP8 (2.6 to 2.7 PFLOP/s), 55 to 59 % at 2.0 to 2.3 over 16 and 56 of the blockwise
 //    recipe, 39 to 43 % over 8 at 2.1 to 2.4 (profiles/wide_tiles_mfma_utilisation.txt).
+//  * The tiles behind the last whole round are cut in quarters (`quarter_fp8_tiles`) where these go round.
 //  * Before a phase a wavefront waits for the loads of the phase before the last, and all of them meet: every load has one to two phases.
 #include <mutex>
 
@@ -48,16 +49,11 @@ __device__ __forceinline__ uint32_t read_scale(uint32_t at) {
 // bank. kGradient (kMx): every group contracts its own window of the depth of the same two matrices, both of them banks, whose
 // atoms a load takes 4 KB of at a time where a row of the tokens would give it a line (32 x 1024 tokens x 7168 x 2048: 604 -> 583 us).
 template <bool kMx, bool kGradient, bool kOutF32>
-__global__ __launch_bounds__(kWideThreads, 1) void wide_fp8_kernel(WideFp8Params p) {
+__device__ __forceinline__ void whole_fp8_tiles(const WideFp8Params& p, const WideTiles<kGradient>& tiles, uint8_t* lds) {
   constexpr int kScaleSteps = kMx ? 4 : 16;  // steps that a row's 16 bytes of scales are for
-  extern __shared__ uint8_t lds[];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int wave_row = wave / 2, wave_column = wave % 2;
   const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)lds));
-
-  WideTiles<kGradient> tiles;
-  tiles.find(p.offsets, nullptr, p.groups, p.rows, p.width, 0);
-  if constexpr (!kGradient) clear_unowned(static_cast<bf16_t*>(p.out), tiles.held, p.rows, p.width);
 
   struct Tile {
     int group, row0, valid_rows, n0, first_step, steps, empty;
@@ -373,9 +369,232 @@ __global__ __launch_bounds__(kWideThreads, 1) void wide_fp8_kernel(WideFp8Params
   }
 }
 
+// The tiles behind the last whole round, where these would leave most CUs without one: a quarter each, 2 x 2 wavefronts of 64 x 64. A
+// step's eight matrix instructions are one phase, in which the next step's fragments and scales are read and the loads go out four
+// steps ahead, into the stage that was read the phase before; the first two wavefronts fetch the rows' scales, the others the bank's.
+// Bound by the loads, 64 bytes a clock of the pipe's rate.
 template <bool kMx, bool kGradient, bool kOutF32>
+__device__ __forceinline__ void quarter_fp8_tiles(const WideFp8Params& p, const WideTiles<kGradient>& tiles, uint8_t* lds) {
+  constexpr int kScaleSteps = kMx ? 4 : 16;  // steps that a row's 16 bytes of scales are for
+  constexpr int kHalf = kWideTile / 2, kOperand = kHalf * kFp8Step, kStages = 4, kStage = 2 * kOperand, kLoads = 4;  // of each operand, a wavefront a step
+  constexpr int kScalesAt = kStages * kStage, kBankScales = kHalf * 16, kScales = 2 * kBankScales;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int wave_row = wave / 2, wave_column = wave % 2;
+  const uint32_t lds_base = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const void*)lds));
+  const int depth_steps = p.depth / kFp8Step, strips32 = p.width / 32, blocks = p.width / 128;
+  const size_t strip_bytes = static_cast<size_t>(p.depth) * 32;
+  uint32_t a_offset[kLoads], b_offset[kLoads];
+#pragma unroll
+  for (int i = 0; i < kLoads; ++i) {
+    const int row = 8 * (kLoads * wave + i) + lane / 8;
+    b_offset[i] = wave * static_cast<uint32_t>(strip_bytes) + i * kAtomBytes + lane * 16;
+    a_offset[i] = kGradient ? b_offset[i] : row * static_cast<uint32_t>(p.depth) + 16 * ((lane % 8) ^ (((row >> 1) & 7) ^ ((row & 1) << 2)));
+  }
+  const uint32_t strip_scale_offset = (wave % 2 * 2 + lane / 32) * static_cast<uint32_t>(depth_steps) * 128 + (lane % 32) * 16;
+  const uint32_t scale_offset = wave < 2 ? (kGradient ? strip_scale_offset : (64 * wave + lane) * static_cast<uint32_t>(p.a_scale_pitch))
+                                         : (kMx ? strip_scale_offset : lane * static_cast<uint32_t>(blocks) * 4);
+  auto buffer = [](const uint8_t* at, int bytes) __attribute__((always_inline)) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(at), 0, bytes, 0x00027000); };
+
+  WidePlace place;
+  for (int turn = 0, quarter = 0; tiles.quarter_at(turn, 4, place, quarter); ++turn) {
+    const int row_at = place.within * kWideTile + quarter / 2 * kHalf, n0 = place.strip * kWideTile + quarter % 2 * kHalf;
+    const int valid_rows = __builtin_amdgcn_readfirstlane(min(kHalf, (kGradient ? p.rows : place.size) - row_at));
+    if (valid_rows <= 0 || n0 >= p.width) continue;  // (the same for the whole block)
+    int first_step = 0, steps = depth_steps, row0 = row_at;
+    bool empty = false;
+    if constexpr (kGradient) {  // (an empty window: one step of zeros, as in the whole tiles)
+      first_step = min(max(place.start, 0), p.depth) / kFp8Step;
+      steps = __builtin_amdgcn_readfirstlane(min(max(place.start + place.size, 0), p.depth) / kFp8Step - first_step);
+      empty = steps <= 0;
+      if (empty) first_step = 0;
+      steps = max(steps, 1);
+    } else {
+      row0 += place.start;
+    }
+    const size_t strip = static_cast<size_t>(kGradient ? 0 : place.group) * strips32 + n0 / 32;
+    const int strips = empty ? 0 : min(kHalf / 32, strips32 - n0 / 32);
+    const uint8_t* a_next = p.a + static_cast<size_t>(row0) * p.depth + first_step * (kGradient ? 4 * kAtomBytes : kFp8Step);
+    const uint8_t* b_next = p.b + strip * strip_bytes + static_cast<size_t>(first_step) * 4 * kAtomBytes;
+    const int a_bytes = empty ? 0 : valid_rows * p.depth, b_bytes = strips * static_cast<int>(strip_bytes);
+    // this wavefront's scales: the rows', or the bank's
+    const uint8_t* scales = wave < 2 ? p.a_scale + static_cast<size_t>(row0) * p.a_scale_pitch
+                            : kMx    ? static_cast<const uint8_t*>(p.b_scale) + strip * depth_steps * 128
+                                     : static_cast<const uint8_t*>(p.b_scale) + (static_cast<size_t>(place.group) * depth_steps * blocks + n0 / 128) * 4;
+    const int scale_bytes = empty ? 0 : wave < 2 ? valid_rows * p.a_scale_pitch : kMx ? strips * depth_steps * 128 : (depth_steps * blocks - n0 / 128) * 4;
+    const int scale_step = wave < 2 ? (kGradient ? 128 : kMx ? 4 : 1) : (kMx ? 128 : blocks * 4);  // bytes from a step's to the next one's
+    int scale_shift[2] = {0, 0};  // where a buffer's first step stands in it
+    int fetched = 0, slot = 0;
+    __amdgpu_buffer_rsrc_t a_buffer, b_buffer;
+    auto begin = [&]() __attribute__((always_inline)) {  // (steps behind the last read as zeros)
+      const bool any = fetched < steps;
+      a_buffer = buffer(a_next, any ? a_bytes : 0);
+      b_buffer = buffer(b_next, any ? b_bytes : 0);
+      a_next += kGradient ? 4 * kAtomBytes : kFp8Step;
+      b_next += 4 * kAtomBytes;
+      if (fetched % kScaleSteps == 0 && any) {
+        const int scale_slot = fetched / kScaleSteps % 2, first = first_step + fetched;
+        const int from = kMx ? min(first, depth_steps - 4) : first;  // (a row's last 16 bytes end with it)
+        if (scale_slot)
+          scale_shift[1] = first - from;
+        else
+          scale_shift[0] = first - from;
+#if defined(__HIP_DEVICE_COMPILE__)
+        typedef __attribute__((address_space(3))) void* lds_t;
+        uint8_t* to = lds + kScalesAt + scale_slot * kScales + wave / 2 * kBankScales;
+        const __amdgpu_buffer_rsrc_t from_scales = buffer(scales + static_cast<size_t>(from) * scale_step, !kMx && wave >= 2 ? scale_bytes - from * scale_step : scale_bytes);
+        if (kMx || wave < 2)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(from_scales, (lds_t)(to + wave % 2 * 1024), 16, scale_offset, 0, 0, 0);
+        else if (wave == 2)  // (16 steps of the one column block; what the other lanes fetch is not read)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(from_scales, (lds_t)to, 4, scale_offset, 0, 0, 0);
+#endif
+      }
+      ++fetched;
+    };
+    auto load = [&](auto piece) __attribute__((always_inline)) {
+#if defined(__HIP_DEVICE_COMPILE__)
+      typedef __attribute__((address_space(3))) void* lds_t;
+      constexpr int i = decltype(piece)::value % kLoads;
+      uint8_t* to = lds + slot * kStage + (wave * kLoads + i) * 1024;
+      if constexpr (decltype(piece)::value < kLoads)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(a_buffer, (lds_t)to, 16, a_offset[i], 0, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(b_buffer, (lds_t)(to + kOperand), 16, b_offset[i], 0, 0, 0);
+#endif
+    };
+    auto turned = [&]() __attribute__((always_inline)) { slot = slot == kStages - 1 ? 0 : slot + 1; };
+
+    uint32_t a_at[4];  // of the row tiles' 16 bytes 2 * half + piece
+    uint32_t b_at = lds_base + kOperand + wave_column * 2 * 4 * kAtomBytes + lane * 16;
+    {
+      const int row = 64 * wave_row + lane % 32;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        a_at[i] = kGradient ? lds_base + wave_row * 2 * 4 * kAtomBytes + i * kAtomBytes + lane * 16
+                            : lds_base + row * 128 + (((4 * (lane / 32) + i) ^ (((row >> 1) & 7) ^ ((row & 1) << 2))) * 16);
+    }
+    constexpr int kRowTileScales = kGradient ? 512 : 32 * 16, kBankWords = kMx ? 2 : 1;
+    const uint32_t a_scale_at = lds_base + kScalesAt + (kGradient ? wave_row * 2 * 512 + (lane % 32) * 4 : (64 * wave_row + lane % 32) * 16);
+    const uint32_t b_scale_at = lds_base + kScalesAt + kBankScales + (kMx ? wave_column * 2 * 512 + (lane % 32) * 4 : 0);
+    f32x16_t acc[2][2];
+    i32x8_t a_frag[2][2][2], b_frag[2][2][2];
+    uint32_t a_read[2], b_read[kBankWords];
+    int a_word[2], b_word[kBankWords], unscalable = 0;
+    auto read = [&](auto set, auto piece) __attribute__((always_inline)) {
+      constexpr int h = decltype(piece)::value / 4, i = decltype(piece)::value % 2;
+      auto whole = [](const u32x4_t& low, const u32x4_t& high) __attribute__((always_inline)) {
+        return i32x8_t{static_cast<int>(low[0]), static_cast<int>(low[1]), static_cast<int>(low[2]), static_cast<int>(low[3]),
+                       static_cast<int>(high[0]), static_cast<int>(high[1]), static_cast<int>(high[2]), static_cast<int>(high[3])};
+      };
+      if constexpr (decltype(piece)::value % 4 < 2)
+        b_frag[set.value][h][i] = whole(read_quad<(4 * i + 2 * h) * kAtomBytes>(b_at), read_quad<(4 * i + 2 * h + 1) * kAtomBytes>(b_at));
+      else
+        a_frag[set.value][h][i] = whole(read_quad<i * 32 * kFp8Step>(a_at[2 * h]), read_quad<i * 32 * kFp8Step>(a_at[2 * h + 1]));
+    };
+    int taken = 0, read_slot = 0;
+    auto read_scales = [&]() __attribute__((always_inline)) {  // of step `taken`, and on to the next
+      const int scale_slot = taken / kScaleSteps % 2;
+      const uint32_t from = taken % kScaleSteps + (scale_slot ? scale_shift[1] : scale_shift[0]), buffer_at = scale_slot * kScales;
+      const uint32_t a_from = a_scale_at + (buffer_at + from * (kGradient ? 128 : kMx ? 4 : 1)), b_from = b_scale_at + (buffer_at + from * (kMx ? 128 : 4));
+      static_for<2>([&](auto i) __attribute__((always_inline)) { a_read[i.value] = read_scale<i.value * kRowTileScales, !kMx>(a_from); });
+      static_for<kBankWords>([&](auto j) __attribute__((always_inline)) { b_read[j.value] = read_scale<j.value * 512, false>(b_from); });
+      ++taken;
+    };
+    auto moves = [&]() __attribute__((always_inline)) {
+      const uint32_t move = read_slot == kStages - 1 ? -(kStages - 1) * kStage : kStage;
+      read_slot = read_slot == kStages - 1 ? 0 : read_slot + 1;
+      a_at[0] += move, a_at[1] += move, a_at[2] += move, a_at[3] += move, b_at += move;
+    };
+    // every wavefront's loads but its `younger` last are done, and so are its reads, which are the next phase's operands
+    auto landed = [&](auto younger, auto set) __attribute__((always_inline)) {
+      constexpr int n = decltype(younger)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt((n & 15) | ((n >> 4) << 14) | (7 << 4));  // vmcnt(n) lgkmcnt(0)
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) asm volatile("" : "+v"(a_frag[set.value][h][i]), "+v"(b_frag[set.value][h][i]));
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        asm volatile("" : "+v"(a_read[i]));
+        a_word[i] = static_cast<int>(kMx ? a_read[i] >> (8 * (lane / 32)) : a_read[i]);
+      }
+#pragma unroll
+      for (int j = 0; j < kBankWords; ++j) {
+        asm volatile("" : "+v"(b_read[j]));
+        b_word[j] = static_cast<int>(kMx ? b_read[j] >> (8 * (lane / 32)) : b_read[j] >> 23);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto phase = [&](auto from, auto into) __attribute__((always_inline)) {
+      if constexpr (!kMx) unscalable |= (b_read[0] & 0x807FFFFFu) | ((b_read[0] >> 23) == 0u) | ((b_read[0] >> 23) == 255u);
+      begin();
+      read_scales();
+      static_for<8>([&](auto m) __attribute__((always_inline)) {
+        constexpr int t = decltype(m)::value, h = t / 4, i = t % 4 / 2, j = t % 2, byte = kMx ? 2 * h : 0;
+        read(into, m);
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(b_frag[from.value][h][j], a_frag[from.value][h][i], acc[i][j], 0, 0, byte,
+                                                                     b_word[kMx ? j : 0], byte, a_word[i]);
+        load(m);
+        __builtin_amdgcn_sched_barrier(0);
+      });
+      turned();
+      moves();
+      // (in flight: the loads of the two steps behind the one that is read next)
+      landed(std::integral_constant<int, 2 * 2 * kLoads>{}, into);
+    };
+    constexpr std::integral_constant<int, 0> c0{};
+    constexpr std::integral_constant<int, 1> c1{};
+    // (the LDS is free of the last tile's reads and loads)
+    __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0) lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int ahead = 0; ahead < kStages; ++ahead) {
+      begin();
+      static_for<2 * kLoads>(load);
+      turned();
+    }
+    clear_sums(acc);
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::: "memory");
+    constexpr int kFirst = (kStages - 1) * 2 * kLoads;
+    __builtin_amdgcn_s_waitcnt((kFirst & 15) | ((kFirst >> 4) << 14) | (7 << 4));
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    read_scales();
+    static_for<8>([&](auto piece) __attribute__((always_inline)) { read(c0, piece); });
+    moves();
+    landed(std::integral_constant<int, 2 * 2 * kLoads>{}, c0);
+    int step = 0;
+    for (; step + 2 <= steps; step += 2) {
+      phase(c0, c1);
+      phase(c1, c0);
+    }
+    if (step < steps) phase(c0, c1);
+    float factor = 1.0f;
+    if constexpr (!kMx) factor = unscalable != 0 ? __uint_as_float(0x7FC00000u) : 1.0f;  // (NaN rather than the product under another scale)
+    const size_t out_row0 = kGradient ? static_cast<size_t>(place.group) * p.rows + row_at : row0;
+    leave<kOutF32>(acc, p.out, out_row0, valid_rows, p.width, 64 * wave_row, n0 + 64 * wave_column, factor);
+  }
+  __builtin_amdgcn_s_waitcnt(7 << 4);  // (no load into the LDS outlives the block)
+}
+
+template <bool kMx, bool kGradient, bool kOutF32, bool kQuarters>
+__global__ __launch_bounds__(kWideThreads, 1) void wide_fp8_kernel(WideFp8Params p) {
+  extern __shared__ uint8_t lds[];
+  WideTiles<kGradient> tiles;
+  tiles.find(p.offsets, nullptr, p.groups, p.rows, p.width, kQuarters ? p.quarter_turns : 0);
+  if constexpr (!kGradient) clear_unowned(static_cast<bf16_t*>(p.out), tiles.held, p.rows, p.width);
+  whole_fp8_tiles<kMx, kGradient, kOutF32>(p, tiles, lds);
+  if (kQuarters && tiles.whole < tiles.total) quarter_fp8_tiles<kMx, kGradient, kOutF32>(p, tiles, lds);
+}
+
+template <bool kMx, bool kGradient, bool kOutF32, bool kQuarters>
 static int launch_kernel(const char* who, const WideFp8Params& p, hipStream_t stream) {
-  auto kernel = wide_fp8_kernel<kMx, kGradient, kOutF32>;
+  auto kernel = wide_fp8_kernel<kMx, kGradient, kOutF32, kQuarters>;
   static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
   static hipError_t reserved = hipSuccess;
   std::call_once(configured, [&] {
@@ -386,9 +605,16 @@ static int launch_kernel(const char* who, const WideFp8Params& p, hipStream_t st
   return launched(who);
 }
 
-int launch_wide_fp8(const char* who, const WideFp8Params& p, bool mx, bool gradient, bool out_f32, hipStream_t stream) {
-  if (gradient) return out_f32 ? launch_kernel<true, true, true>(who, p, stream) : launch_kernel<true, true, false>(who, p, stream);
-  return mx ? launch_kernel<true, false, false>(who, p, stream) : launch_kernel<false, false, false>(who, p, stream);
+int launch_wide_fp8(const char* who, const WideFp8Params& params, bool mx, bool gradient, bool out_f32, hipStream_t stream) {
+  WideFp8Params p = params;
+  // A last round of at most a quarter of the CUs, or of half of them where a tile's walk is long enough to hide two starts. Measured (us): [21 888,
+  // 4992] x 2304 of 4, 3.02 rounds, 227 -> 202, [9088, 2816] x 1792 of 20, 1.12, 66 -> 51, [2816, 4608] x 7424 of 4, 1.36, 103 -> 95, [12 032, 896] x 1792 of
+  // 9, 1.37, 31.3 and 31.4; kernel gradients of 10 496 tokens, 6 x 4096 x 640, 1.12, 57 -> 43, 8320 of 2 x 2560 x 3456, 1.09, 99 -> 68.
+  p.quarter_turns = (gradient ? p.depth / p.groups : p.depth) >= 2048 ? 2 : 1;
+  if (!gradient) return mx ? launch_kernel<true, false, false, true>(who, p, stream) : launch_kernel<false, false, false, true>(who, p, stream);
+  if (ends_in_quarters(p.groups, p.rows, p.width, p.quarter_turns))
+    return out_f32 ? launch_kernel<true, true, true, true>(who, p, stream) : launch_kernel<true, true, false, true>(who, p, stream);
+  return out_f32 ? launch_kernel<true, true, true, false>(who, p, stream) : launch_kernel<true, true, false, false>(who, p, stream);
 }
 
 }  // namespace dew

@@ -52,3 +52,31 @@ def test_recipes_products(monkeypatch, recipe, sizes):
 @pytest.mark.parametrize("blocks,depth,width", (([1, 2, 0, 3, 1, 1, 2, 1, 4], 1024, 1024), ([1] * 9, 1024, 2048)))     # 144 tiles, 288
 def test_recipes_gradients(blocks, depth, width, mx, out_dtype):
     test_gpu_wide_fp8.test_gradients(blocks, depth, width, mx, out_dtype)
+
+
+# (whole and ragged groups of a scale load; one quarter a block and two, alone and behind a whole round)
+@pytest.mark.parametrize("depth,sizes,width", ((512, [129, 1000, 0, 383, 1, 700], 896), (640, [129, 1000, 383, 700], 896), (2176, [2100, 1900], 1408),
+                                               (640, [4000], 4480), (2176, [3800, 200], 5504)))
+@pytest.mark.parametrize("recipe", ("blockwise_fp8", "mxfp8"))
+def test_recipes_products_in_quarters(monkeypatch, recipe, depth, sizes, width):
+    monkeypatch.setitem(test_gpu_wide_fp8.SIZES, "quarters", (sizes, width))
+    test_gpu_wide_fp8.test_products(recipe, "quarters", depth)
+
+
+@pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
+@pytest.mark.parametrize("mx", (True, False))
+@pytest.mark.parametrize("blocks,depth,width", (([0, 1, 5, 3, 4], 640, 640), ([9, 2, 0], 640, 896), ([40, 1], 896, 4096), ([5, 4], 2176, 4096)))
+def test_recipes_gradients_in_quarters(blocks, depth, width, mx, out_dtype):
+    test_gpu_wide_fp8.test_gradients(blocks, depth, width, mx, out_dtype)
+
+
+def test_a_quarter_writes_nan_where_it_meets_a_scale_that_is_no_power_of_two():
+    from dew_amd import formats, gemm, ops
+
+    sizes, depth, width = [300, 400, 500], 640, 896
+    x, w, counts = test_gpu_wide_fp8.operands(sizes, depth, width)
+    factors = torch.ones((3, depth // 128, width // 128), device="cuda")
+    factors[1, 4, 3] = 1.5
+    bank = gemm.prepared(formats.Fp8Blocks((w.float() / 64).clamp(-448, 448).to(torch.float8_e4m3fn).view(torch.uint8).contiguous(), factors))
+    got = ops.grouped_gemm_fp8_rows(*ops.quantize_rows_fp8(x), bank, ops.group_offsets(counts))
+    assert bool(torch.isnan(got[300:700, 384:512]).all()) and int(torch.isnan(got).sum()) == 400 * 128
