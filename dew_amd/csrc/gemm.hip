@@ -128,7 +128,8 @@ __device__ __forceinline__ void schedule_phase() {
 // the same launch with the SwiGLU epilogue, and on the block tile: BM rows x BN columns of each matrix. The
 // four wavefronts sit WM x WN (1 x 4: side by side along the columns, so no two of them need the same weight
 // bytes); each owns (BM/WM) x (BN/WN) of every matrix as 32 x 32 MFMA tiles.
-template <int FORMAT, int MODE, int BM, int BN, int WM, int WN>
+// STREAM: the launch reads every weight byte once, with loads that say so.
+template <int FORMAT, int MODE, int BM, int BN, int WM, int WN, bool STREAM>
 __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 && ((MODE == kSwigluOfTwo || MODE == kSwigluOfTwoSplit) ? 2 : 1) * BN == 256) ? 2 : 1) void grouped_gemm_kernel(GemmParams p) {
   constexpr bool PAIRED = MODE == kSwigluOfTwo || MODE == kSwigluOfTwoSplit;
   constexpr bool kSplitOut = MODE == kSwigluOfTwoSplit;
@@ -334,10 +335,11 @@ __global__ __launch_bounds__(kThreads, (FORMAT != DEW_MOE_W_BF16 && BM == 128 &&
       for (int a = 0; a < kAtoms; ++a) {
         const u32x4_t* from = reinterpret_cast<const u32x4_t*>(b_src[t] + (static_cast<size_t>(step) * kAtoms + a) * kAtomBytes);
         // Decode-sized groups (the 32-row tiles) read every weight byte once: loaded as non-temporal the stream runs 3 to 6 %
-        // faster (a read-only stream of 16-byte loads measures 7.1 TB/s so hinted against 5.6 to 6.4 without). Taller
-        // tiles keep the plain load: their groups' tiles share weight strips through the L2 (128-row tiles: 2 to 4 % slower
-        // with the hint).
-        if constexpr (BM <= 32)
+        // faster (a read-only stream of 16-byte loads measures 7.1 TB/s so hinted against 5.6 to 6.4 without), and so does the
+        // launch of groups' last rows, one tile a group (a layer of 8192 tokens on 256 experts of 7168 x 2048, which has two such launches,
+        // 7539 -> 7513 and 7582 -> 7513 us, two runs of one side 0.1 % apart). Other taller tiles keep the plain load: their groups' tiles share weight strips through the L2 (with the
+        // hint 128-row tiles are 2 to 4 % slower, layers on 64-row tiles 2 % faster to 13 % slower).
+        if constexpr (STREAM)
           b_regs[set.value][t][a] = __builtin_nontemporal_load(from);
         else
           b_regs[set.value][t][a] = *from;
@@ -1108,13 +1110,13 @@ static int check_split_extents(const char* who, const dew_moe_bank* bank, const 
   return DEW_MOE_OK;
 }
 
-template <int FORMAT, int MODE, int BM, int BN, int WM, int WN>
+template <int FORMAT, int MODE, int BM, int BN, int WM, int WN, bool STREAM = BM <= 32>
 static int launch_tile(const char* who, GemmParams p, hipStream_t stream) {
   // block-scaled activations keep their tile's scales behind the ring (reserved at their largest: kMaxBlockScaleDepth)
   constexpr size_t kShared = shared_bytes<BM, BN, MODE>() +
                              (FORMAT == kFormatMxSplitBlocks || FORMAT == kFormatFp8Rows ? static_cast<size_t>(BM) * (block_scale_pitch(kMaxBlockScaleDepth) + (FORMAT == kFormatFp8Rows ? 4 : 0)) : 0) +
                              (FORMAT == kFormatMxFp8Rows || FORMAT == kFormatMxFp8Window ? 2 * static_cast<size_t>(BM) * 16 : 0);  // MXFP8 rows: four steps' dwords of each row, twice
-  auto kernel = grouped_gemm_kernel<FORMAT, MODE, BM, BN, WM, WN>;
+  auto kernel = grouped_gemm_kernel<FORMAT, MODE, BM, BN, WM, WN, STREAM>;
   static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel (whichever thread calls first)
   static hipError_t reserved = hipSuccess;
   std::call_once(configured, [&] {
@@ -1253,7 +1255,7 @@ static int launch_format(const char* who, const GemmParams& p, hipStream_t strea
       if (status != DEW_MOE_OK || !shared) return status;
       GemmParams rest = p;
       rest.tail_of = 128;
-      return launch_tile<FORMAT, MODE, 64, 128, 1, 4>(who, rest, stream);
+      return launch_tile<FORMAT, MODE, 64, 128, 1, 4, true>(who, rest, stream);
     }
   }
 }
