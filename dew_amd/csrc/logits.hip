@@ -318,7 +318,7 @@ __global__ __launch_bounds__(64) void router_logit_tile_shares_kernel(const bf16
 
 // How a layer's gate leaves its logits: in shares, by 16 x 16 tiles as the fine launch's (up to kShareTokens tokens, and wherever
 // dew_moe_router_logits takes that launch) or by 32 x 32 tiles as its sixteen wavefronts', or finished. Past some hundred such tiles
-// the shares' sixteen times the bytes cost more than the idle CUs do. A layer's pass (us): 200 tokens of a 2048 x 8 gate 85.0 -> 81.4,
+// the shares' sixteen times the bytes cost more than the idle CUs do. A layer's pass (us; tiles by the fp32 instruction still): 200 tokens of a 2048 x 8 gate 85.0 -> 81.4,
 // 100 of 7168 x 256 (32 tiles) 393 -> 381, 2048 of 512 x 8 (64) 52.0 -> 50.3, 1111 of 2048 x 64 (70) 134.5 -> 131.9, 1000 of 7168 x 128
 // (128) 489.5 and 490.4, 600 of 2048 x 256 (152) 284.6 and 288.
 LogitShares logit_shares(int tokens, int depth, int experts) {
