@@ -99,9 +99,12 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
   auto row_of = [&](int p) { return KMAJOR ? p * kGroups + group : group * kLoads + p; };
   const T* source = w + e * depth * width + static_cast<size_t>(KMAJOR ? n0 : k0) * pitch + (KMAJOR ? k0 : n0) + piece * kVec;
   const uint32_t share = kNv ? nvfp4_share(largest, kNvfp4Partials) : 0u;
+  // Bound by memory, and every weight is read once: non-temporal, so that the weights don't push out what the step's products read next. us of
+  // twelve drawn steps of the FP8 recipes 1.00 to 1.12 times as fast (252 -> 224, 535 -> 497, 228 -> 209). Non-temporal stores too, of codes that the
+  // product reads at once: no difference in steps of 400 us and more and of 113 and less, 5 to 10 % slower in those of 180 to 300.
   u32x4_t words[kLoads];
 #pragma unroll
-  for (int p = 0; p < kLoads; ++p) words[p] = *reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch);
+  for (int p = 0; p < kLoads; ++p) words[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch));
 
   float tensor = 1.0f;
   bool quick = false;  // (the same for the whole launch)

@@ -395,9 +395,10 @@ __global__ __launch_bounds__(512) void quantize_bank_kernel(const bf16_t* __rest
   if (at >= tiles) return;
   const int t0 = at / across * 128, d0 = at % across * 128;
   const int chunk = tid % 16;
+  // Read once, non-temporal (a blockwise step of 32 768 rows 2156 -> 2137 us, steps of 100 to 400 us 0 to 2 %).
   u32x4_t words[4];
 #pragma unroll
-  for (int k = 0; k < 4; ++k) words[k] = *reinterpret_cast<const u32x4_t*>(x + static_cast<size_t>(t0 + tid / 16 + 32 * k) * dim + d0 + chunk * 8);
+  for (int k = 0; k < 4; ++k) words[k] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(x + static_cast<size_t>(t0 + tid / 16 + 32 * k) * dim + d0 + chunk * 8));
   auto low = [](uint32_t word) { return __uint_as_float(word << 16); };
   auto high = [](uint32_t word) { return __uint_as_float(word & 0xFFFF0000u); };
   auto scale_byte = [](float most) -> uint32_t {
