@@ -28,6 +28,58 @@ __device__ __forceinline__ uint32_t upper_halves(float high, float low) {
 }
 __device__ __forceinline__ float below_upper(float value) { return value - __uint_as_float(__float_as_uint(value) & 0xFFFF0000u); }
 
+// The sums of depths `from` to `to` (whole 16s) for the tiles that `needed` names of a tile of 32 tokens beside TILES of 32 experts, `row` and
+// `column` the lane's own, on the fp32 instruction: what the terms cannot give. Bound by the matrix pipe, 512 cycles a tile and 16 deep
+// chunk, where a row of tiles is needed, by its loads, which go out two chunks ahead, where one is. Finite
+// operands, a token of NaN, and nothing else, us: 8192 x 7168 x 256 102, 218 and 317, 2048 x 7168 x 256 46, 81 and 119, 4096 x 4096 x 8 16, 38 and 43 (the
+// fp32 instruction alone 300, 92 and 34; where every such sum's lane walked the depth for it a token of NaN took 7057, 1696 and 339).
+template <int TILES>
+__device__ __forceinline__ void plain_sums(const bf16_t* __restrict__ row, const float* __restrict__ column, int experts, int from, int to, uint32_t needed,
+                                           f32x16 (&acc)[TILES]) {
+  struct __attribute__((packed, aligned(4))) Neighbours {
+    float of[TILES];
+  };
+  constexpr int kAhead = 2;  // chunks of a set
+  const int lower = 8 * (threadIdx.x % 64 / 32);
+#pragma unroll
+  for (int c = 0; c < TILES; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[c][i] = 0.0f;
+  u32x4 words[2][kAhead];
+  Neighbours g[2][kAhead][8];
+  auto load = [&](int set, int chunk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ahead = 0; ahead < kAhead; ++ahead) {
+      const int at = min(chunk + 16 * ahead, to - 16) + lower;  // (past the share: the last chunk again, which multiplies nothing)
+      words[set][ahead] = *reinterpret_cast<const u32x4*>(row + at);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) g[set][ahead][j] = *reinterpret_cast<const Neighbours*>(column + static_cast<size_t>(at + j) * experts);
+    }
+  };
+  auto multiply = [&](int set, int chunk) __attribute__((always_inline)) {
+#pragma unroll
+    for (int ahead = 0; ahead < kAhead; ++ahead) {
+      if (chunk + 16 * ahead >= to) continue;
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+        if (!(needed >> c & 1)) continue;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const uint32_t word = words[set][ahead][j / 2];
+          acc[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(j % 2 ? word & 0xFFFF0000u : word << 16), g[set][ahead][j].of[c], acc[c], 0, 0, 0);
+        }
+      }
+    }
+  };
+  load(0, from);
+  for (int chunk = from; chunk < to; chunk += 32 * kAhead) {
+    load(1, chunk + 16 * kAhead);
+    multiply(0, chunk);
+    load(0, chunk + 32 * kAhead);
+    multiply(1, chunk + 16 * kAhead);
+  }
+}
+
 // The sums of a share of the depth, its steps of 16 x CHUNKS from `first` to `last`, for ROWS tiles of 32 tokens from t0 on and TILES tiles of
 // 32 experts. A lane's depths of a step are contiguous in its token's row (64 bytes of four chunks, so that every line of x is asked
 // for once); a chunk's instructions take 8 of each half's. Its experts are TILES neighbours, one a tile, from `column` on: one load a depth.
@@ -116,27 +168,37 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
   split(0, 0);
   if (CHUNKS < 4 && last - first == 1) {  // (a share of a short depth: nothing behind it is asked for)
     walk(0, first, false);
-    return;
-  }
-  load_gate(0, min(first + AHEAD, last - 1), 0);
-  int step = first;
-  for (; step + kSets <= last; step += kSets) {  // (no way out in the middle: every load would be waited for there)
+  } else {
+    load_gate(0, min(first + AHEAD, last - 1), 0);
+    int step = first;
+    for (; step + kSets <= last; step += kSets) {  // (no way out in the middle: every load would be waited for there)
 #pragma unroll
-    for (int set = 0; set < kSets; ++set) walk(set, step + set, true);
-  }
+      for (int set = 0; set < kSets; ++set) walk(set, step + set, true);
+    }
 #pragma unroll
-  for (int set = 0; set < kSets - 1; ++set)
-    if (step + set < last) walk(set, step + set, AHEAD > 1);
-}
-
-// A sum that is no finite number again, product by product in fp32: an infinity among the operands meets a term that is zero, and a
-// gate value's terms are not those of an infinity or a NaN.
-__device__ __forceinline__ float finite_or_plain(float sum, const bf16_t* __restrict__ row, const float* __restrict__ column, int experts, int from,
-                                                 int to) {
-  if (__builtin_isfinite(sum)) return sum;
-  sum = 0.0f;
-  for (int d = from; d < to; ++d) sum = fmaf(bf16_to_f32(row[d]), column[static_cast<size_t>(d) * experts], sum);
-  return sum;
+    for (int set = 0; set < kSets - 1; ++set)
+      if (step + set < last) walk(set, step + set, AHEAD > 1);
+  }
+  // An infinity among the operands meets a term that is zero, and a gate value's terms are not those of an infinity or a NaN: tiles with
+  // a sum that is no finite number are formed again on the fp32 instruction, and that sum taken from there.
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    uint32_t needed = 0;
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) {
+      float zero = 0.0f;  // (a NaN where any sum is no finite number)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) zero = fmaf(0.0f, acc[r][c][i], zero);
+      if (__any(zero != 0.0f)) needed |= 1u << c;
+    }
+    if (needed == 0) continue;
+    f32x16 plain[TILES];
+    plain_sums<TILES>(a_src[r], kernel + column, experts, kStep * first, min(kStep * last, depth), needed, plain);
+#pragma unroll
+    for (int c = 0; c < TILES; ++c)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[r][c][i] = __builtin_isfinite(acc[r][c][i]) ? acc[r][c][i] : plain[c][i];
+  }
 }
 
 // WAVES wavefronts a block split the depth; their sums meet in LDS in wavefront order, WAVES registers of the tiles at a time.
@@ -177,11 +239,9 @@ __global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf
       }
       if (t < tokens && e0 < experts) {
 #pragma unroll
-        for (int c = 0; c < TILES; ++c) {
-          sums.of[c] = finite_or_plain(sums.of[c], x + static_cast<size_t>(t) * depth, kernel + column + c, experts, 0, depth);
+        for (int c = 0; c < TILES; ++c)
           // a biased router (GPT-OSS's, src/dew/nn/gpt_oss.py:163-165) adds its fp32 bias to the finished sum
           if (bias) sums.of[c] += bias[column + c];
-        }
         *reinterpret_cast<Neighbours*>(logits + static_cast<size_t>(t) * experts + column) = sums;
       }
     }
@@ -299,20 +359,10 @@ __global__ __launch_bounds__(64) void router_logit_tile_shares_kernel(const bf16
   logit_terms<1, 1, 1, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, min(32 * static_cast<int>(blockIdx.y) + lane % 32, experts - 1), first, last, acc);
   const int e = 32 * blockIdx.y + lane % 32;
   if (e >= experts) return;
-  float zero = 0.0f;  // (a NaN where any sum is no finite number)
-#pragma unroll
-  for (int i = 0; i < 16; ++i) zero = fmaf(0.0f, acc[0][0][i], zero);
 #pragma unroll
   for (int i = 0; i < 16; ++i) {
     const int t = t0 + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
     if (t < tokens) partial[(static_cast<size_t>(share) * tokens + t) * experts + e] = acc[0][0][i];
-  }
-  if (zero == 0.0f) return;
-  for (int i = 0; i < 16; ++i) {
-    const int t = t0 + 8 * (i / 4) + 4 * (lane / 32) + i % 4;
-    if (t >= tokens) continue;
-    float* sum = partial + (static_cast<size_t>(share) * tokens + t) * experts + e;
-    *sum = finite_or_plain(*sum, x + static_cast<size_t>(t) * depth, kernel + e, experts, 16 * CHUNKS * first, min(16 * CHUNKS * last, depth));
   }
 }
 
