@@ -13,18 +13,25 @@ namespace dew {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-// The exact split of the gate kernel: an fp32 value is the sum of three bf16 values, its upper 16 bits, the upper 16 of what is
-// left and the 8 bits that are left then, and a token's bf16 element times any of them is exact in fp32. So three bf16 matrix
-// instructions 16 deep (32 cycles each) give the fp32 products that eight fp32 ones 2 deep (64 cycles each) do, and their
-// sums are rounded once for 16 products instead of once for each. What bounds it: the splitting's vector work beside the matrix
-// instructions (11 a pair of gate values against 24 x 32 cycles a 16 deep chunk of 64 x 128) where the experts are many, x from
-// memory where they are few. Measured against the fp32 instruction, the tokens from memory (us): 8192 x 7168 x 256 316 -> 99, 16384 x
+// The exact split of the gate kernel: an fp32 value of 2^-110 and more is the sum of three bf16 values, its upper 16 bits, the upper 16 of what is
+// left and the 8 bits that are left then, and a token's bf16 element times any of them is exact in fp32 (a column with a smaller value,
+// whose last bits no term holds, is seen and formed on the fp32 instruction). So three bf16 matrix instructions 16 deep (32 cycles each) give the
+// fp32 products that eight fp32 ones 2 deep (64 cycles each) do; the sum of 16 products is cut off inside the instruction, where the fp32 ones
+// round after each. What bounds it: the splitting's vector work beside the matrix instructions (11 and a half a pair of gate values against 24 x 32
+// cycles a 16 deep chunk of 64 x 128) where the experts are many, x from memory where they are few. Measured against the fp32 instruction, the tokens from memory (us): 8192 x 7168 x 256 316 -> 99, 16384 x
 // 4096 x 8 65 -> 30, 4096 x 4096 x 8 39 -> 17, 8192 x 4096 x 128 130 -> 45; error against float64 (2-norm) 7.5e-7 -> 4.6e-7, 5.4e-7 ->
 // 3.3e-7, 5.8e-7 -> 3.5e-7 and 5.8e-7 -> 3.5e-7, and smaller for each of 64 shapes of 65 to 16384 tokens, 512 to 7168 deep.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ uint32_t upper_halves(float high, float low) {
   return __builtin_amdgcn_perm(__float_as_uint(high), __float_as_uint(low), 0x07060302u);
+}
+// The same, and the bits of both seen in `seen` (one block: apart, the compiler keeps the values for the second, and 8192 x 7168 x 256 takes 137 us
+// instead of 102).
+__device__ __forceinline__ uint32_t upper_halves(float high, float low, uint32_t& seen) {
+  uint32_t word;
+  asm("v_or3_b32 %0, %0, %2, %3\n\tv_perm_b32 %1, %2, %3, %4" : "+v"(seen), "=&v"(word) : "v"(high), "v"(low), "s"(0x07060302u));
+  return word;
 }
 __device__ __forceinline__ float below_upper(float value) { return value - __uint_as_float(__float_as_uint(value) & 0xFFFF0000u); }
 
@@ -83,10 +90,10 @@ __device__ __forceinline__ void plain_sums(const bf16_t* __restrict__ row, const
 // The sums of a share of the depth, its steps of 16 x CHUNKS from `first` to `last`, for ROWS tiles of 32 tokens from t0 on and TILES tiles of
 // 32 experts. A lane's depths of a step are contiguous in its token's row (64 bytes of four chunks, so that every line of x is asked
 // for once); a chunk's instructions take 8 of each half's. Its experts are TILES neighbours, one a tile, from `column` on: one load a depth.
-// WHOLE: the depth is whole steps.
+// `end`: the depth that the share goes to, up to three chunks behind its last step; WHOLE: none, as the depth is whole steps.
 template <int ROWS, int TILES, int AHEAD, int CHUNKS, bool WHOLE>
 __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const float* __restrict__ kernel, int tokens, int depth, int experts,
-                                            int t0, int column, int first, int last, f32x16 (&acc)[ROWS][TILES]) {
+                                            int t0, int column, int first, int last, int end, f32x16 (&acc)[ROWS][TILES]) {
   struct __attribute__((packed, aligned(4))) Neighbours {
     float of[TILES];
   };
@@ -109,17 +116,19 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
   u32x4 a_words[kSets][ROWS][CHUNKS];
   Neighbours g[AHEAD][CHUNKS][8];
   bf16x8 terms[2][TILES][3];
+  uint32_t dropped[TILES];  // the bits of a lane's gate values that no term holds, in its lower half
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) dropped[c] = 0;
   auto load_rows = [&](int set, int step) __attribute__((always_inline)) {
 #pragma unroll
     for (int r = 0; r < ROWS; ++r)
 #pragma unroll
-      for (int c = 0; c < CHUNKS; ++c)  // (past the depth: its last 8, which are multiplied as zeros)
-        a_words[set][r][c] = *reinterpret_cast<const u32x4*>(a_src[r] + (WHOLE ? kStep * step + half + 8 * c : min(kStep * step + half + 8 * c, depth - 8)));
+      for (int c = 0; c < CHUNKS; ++c) a_words[set][r][c] = *reinterpret_cast<const u32x4*>(a_src[r] + (kStep * step + half + 8 * c));
   };
   auto load_gate = [&](int set, int step, int chunk) __attribute__((always_inline)) {
-    const int at = kStep * step + 8 * chunk;  // (the same for the wavefront: a load's address is a scalar base and the lane's own offset)
-    const float* b_src = kernel + static_cast<size_t>(WHOLE ? at : min(at, depth - 8)) * experts;
-    const uint32_t lower = (WHOLE || at + half < depth ? half * experts : 0) + column;
+    // (the same for the wavefront: a load's address is a scalar base and the lane's own offset)
+    const float* b_src = kernel + static_cast<size_t>(kStep * step + 8 * chunk) * experts;
+    const uint32_t lower = half * experts + column;
 #pragma unroll
     for (int j = 0; j < 8; ++j, b_src += experts) g[set][chunk][j] = *reinterpret_cast<const Neighbours*>(b_src + lower);
   };
@@ -136,7 +145,8 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
       auto fragment = [](const float (&v)[8]) __attribute__((always_inline)) {
         return __builtin_bit_cast(bf16x8, u32x4{upper_halves(v[1], v[0]), upper_halves(v[3], v[2]), upper_halves(v[5], v[4]), upper_halves(v[7], v[6])});
       };
-      terms[chunk % 2][c][0] = fragment(least);
+      terms[chunk % 2][c][0] = __builtin_bit_cast(bf16x8, u32x4{upper_halves(least[1], least[0], dropped[c]), upper_halves(least[3], least[2], dropped[c]),
+                                                                upper_halves(least[5], least[4], dropped[c]), upper_halves(least[7], least[6], dropped[c])});
       terms[chunk % 2][c][1] = fragment(rest);
       terms[chunk % 2][c][2] = fragment(most);
     }
@@ -145,15 +155,13 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
     if (more) load_rows((set + AHEAD) % kSets, min(step + AHEAD, last - 1));  // (behind the last step: that step again, which multiplies nothing)
 #pragma unroll
     for (int chunk = 0; chunk < CHUNKS; ++chunk) {
-      const uint32_t kept = WHOLE || kStep * step + half + 8 * chunk < depth ? 0xFFFFFFFFu : 0u;
 #pragma unroll
       for (int term = 0; term < 3; ++term)
 #pragma unroll
         for (int c = 0; c < TILES; ++c)
 #pragma unroll
           for (int r = 0; r < ROWS; ++r)
-            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a_words[set][r][chunk] & kept), terms[chunk % 2][c][term],
-                                                                acc[r][c], 0, 0, 0);
+            acc[r][c] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a_words[set][r][chunk]), terms[chunk % 2][c][term], acc[r][c], 0, 0, 0);
       const int next = chunk < CHUNKS - 1 ? set % AHEAD : (set + 1) % AHEAD;  // the set of the chunk behind this one
       if (more || chunk < CHUNKS - 1) split(next, (chunk + 1) % CHUNKS);
       if (more) load_gate(next, min(step + AHEAD + (chunk == CHUNKS - 1), last - 1), (chunk + 1) % CHUNKS);
@@ -179,8 +187,12 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
     for (int set = 0; set < kSets - 1; ++set)
       if (step + set < last) walk(set, step + set, AHEAD > 1);
   }
-  // An infinity among the operands meets a term that is zero, and a gate value's terms are not those of an infinity or a NaN: tiles with
-  // a sum that is no finite number are formed again on the fp32 instruction, and that sum taken from there.
+  // An infinity among the operands meets a term that is zero, a gate value's terms are not those of an infinity or a NaN, and below 2^-110 its
+  // last bits lie under the least bf16 value: tiles with a sum that is no finite number, or with a column that dropped bits, are formed again on
+  // the fp32 instruction, and those sums taken from there.
+  bool inexact[TILES];
+#pragma unroll
+  for (int c = 0; c < TILES; ++c) inexact[c] = ((dropped[c] | __shfl_xor(dropped[c], 32, 64)) & 0xFFFFu) != 0;
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
     uint32_t needed = 0;
@@ -189,15 +201,23 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
       float zero = 0.0f;  // (a NaN where any sum is no finite number)
 #pragma unroll
       for (int i = 0; i < 16; ++i) zero = fmaf(0.0f, acc[r][c][i], zero);
-      if (__any(zero != 0.0f)) needed |= 1u << c;
+      if (__any(zero != 0.0f || inexact[c])) needed |= 1u << c;
     }
     if (needed == 0) continue;
     f32x16 plain[TILES];
-    plain_sums<TILES>(a_src[r], kernel + column, experts, kStep * first, min(kStep * last, depth), needed, plain);
+    plain_sums<TILES>(a_src[r], kernel + column, experts, kStep * first, kStep * last, needed, plain);
 #pragma unroll
     for (int c = 0; c < TILES; ++c)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) acc[r][c][i] = __builtin_isfinite(acc[r][c][i]) ? acc[r][c][i] : plain[c][i];
+      for (int i = 0; i < 16; ++i) acc[r][c][i] = __builtin_isfinite(acc[r][c][i]) && !inexact[c] ? acc[r][c][i] : plain[c][i];
+  }
+  if (WHOLE || end == kStep * last) return;
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) {
+    f32x16 plain[TILES];
+    plain_sums<TILES>(a_src[r], kernel + column, experts, kStep * last, end, (1u << TILES) - 1, plain);
+#pragma unroll
+    for (int c = 0; c < TILES; ++c) acc[r][c] += plain[c];
   }
 }
 
@@ -214,9 +234,9 @@ __global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf
   const int t0 = blockIdx.x * 32 * ROWS, e0 = TILES * (32 * blockIdx.y + lane % 32);
   // (lanes past the experts repeat the last ones: what they share with the lane before is the same sum)
   const int column = min(e0, experts - TILES);
-  const int steps = (depth + 16 * CHUNKS - 1) / (16 * CHUNKS);
+  const int steps = depth / (16 * CHUNKS), first = steps * wave / WAVES, last = steps * (wave + 1) / WAVES;
   f32x16 acc[ROWS][TILES];
-  logit_terms<ROWS, TILES, AHEAD, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, column, steps * wave / WAVES, steps * (wave + 1) / WAVES, acc);
+  logit_terms<ROWS, TILES, AHEAD, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, column, first, last, wave == WAVES - 1 ? depth : 16 * CHUNKS * last, acc);
   // register i of lane l is the sum of token 8 (i / 4) + 4 (l / 32) + i % 4 and the lane's expert
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
@@ -354,9 +374,10 @@ template <int CHUNKS, bool WHOLE>
 __global__ __launch_bounds__(64) void router_logit_tile_shares_kernel(const bf16_t* __restrict__ x, const float* __restrict__ kernel,
                                                                       float* __restrict__ partial, int tokens, int depth, int experts) {
   const int lane = threadIdx.x, t0 = blockIdx.x * 32, share = blockIdx.z;
-  const int steps = (depth + 16 * CHUNKS - 1) / (16 * CHUNKS), first = steps * share / kShares, last = steps * (share + 1) / kShares;
+  const int steps = depth / (16 * CHUNKS), first = steps * share / kShares, last = steps * (share + 1) / kShares;
   f32x16 acc[1][1];
-  logit_terms<1, 1, 1, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, min(32 * static_cast<int>(blockIdx.y) + lane % 32, experts - 1), first, last, acc);
+  logit_terms<1, 1, 1, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, min(32 * static_cast<int>(blockIdx.y) + lane % 32, experts - 1), first, last,
+                               share == kShares - 1 ? depth : 16 * CHUNKS * last, acc);
   const int e = 32 * blockIdx.y + lane % 32;
   if (e >= experts) return;
 #pragma unroll

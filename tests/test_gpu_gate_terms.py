@@ -14,8 +14,10 @@ SHAPES = [(14400, 80, 128),    # 2 x 4, 4; the depth ends inside a step
           (4200, 1088, 9),     # 1 x 1, 4
           (2000, 208, 300),    # 2 x 1, 8
           (1900, 112, 63),     # 1 x 1, 8
-          (2040, 80, 32),      # 1 x 1, 16 in steps of 32
-          (2100, 1040, 8)]     # 1 x 1, 16 in steps of 64
+          (2040, 80, 32),      # 1 x 1, 16 in steps of 32; a depth behind the last step
+          (2040, 96, 32),      # whole steps
+          (2100, 1072, 8),     # 1 x 1, 16 in steps of 64; three chunks behind the last step
+          (2100, 1088, 8)]     # whole steps
 
 
 @pytest.mark.parametrize("tokens,depth,experts", SHAPES)
@@ -97,4 +99,23 @@ def test_operands_that_are_no_finite_numbers_cost_what_one_instruction_does(toke
     assert torch.equal(got[:tokens // 2], want[:tokens // 2]) and bool(got[tokens // 2:].isnan().all())
     got = ops.router_logits(one, kernel)
     got[tokens // 3] = want[tokens // 3]
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("tokens,depth,experts", SHAPES)
+@pytest.mark.parametrize("exponent", (-100, -112, -126, -140))
+def test_a_gate_value_that_three_terms_do_not_hold(tokens, depth, experts, exponent):
+    """Below 2^-110 a value's last bits lie under bf16's least (its smallest subnormal is 2^-133), and under 2^-133 all of them. One column of such
+    values, beside others that keep their bits."""
+    from dew_amd import ops
+
+    generator = torch.Generator("cuda").manual_seed(depth + experts)
+    x = torch.randn((tokens, depth), generator=generator, device="cuda").to(torch.bfloat16) * 2.0 ** 60
+    kernel = torch.randn((depth, experts), generator=generator, device="cuda") * depth ** -0.5
+    want = ops.router_logits(x, kernel)
+    kernel[:, experts // 2] = (kernel[:, experts // 2].double() * 2.0 ** exponent).float()
+    got = ops.router_logits(x, kernel)
+    exact, magnitudes = x.double() @ kernel.double(), x.double().abs() @ kernel.double().abs()
+    assert bool(((got.double() - exact).abs() <= 2.0 ** -19 * magnitudes).all())
+    want[:, experts // 2] = got[:, experts // 2]
     assert torch.equal(got, want)
