@@ -5,11 +5,14 @@
 // result does not depend on timing. A decode step's few tokens take 16 x 16 tiles of the fp32 instruction (v_mfma_f32_16x16x4_f32),
 // four times the blocks: 64 tokens of GPT-OSS's 2880 x 32 gate in about 5 us. Depths in no whole 16s take the plain kernel below (a
 // 64-token x 64-expert tile, 16-deep LDS steps, fp32 FMA; 1.3 ms for 8192 tokens of a 7168 x 256 gate, where the terms take 99 us).
+#include <mutex>
+
 #include "common.h"
 #include "sort.h"
 
 namespace dew {
 
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -17,10 +20,12 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // left and the 8 bits that are left then, and a token's bf16 element times any of them is exact in fp32 (a column with a smaller value,
 // whose last bits no term holds, is seen and formed on the fp32 instruction). So three bf16 matrix instructions 16 deep (32 cycles each) give the
 // fp32 products that eight fp32 ones 2 deep (64 cycles each) do; the sum of 16 products is cut off inside the instruction, where the fp32 ones
-// round after each. What bounds it: the splitting's vector work beside the matrix instructions (11 and a half a pair of gate values against 24 x 32
-// cycles a 16 deep chunk of 64 x 128) where the experts are many, x from memory where they are few. Measured against the fp32 instruction, the tokens from memory (us): 8192 x 7168 x 256 316 -> 99, 16384 x
-// 4096 x 8 65 -> 30, 4096 x 4096 x 8 39 -> 17, 8192 x 4096 x 128 130 -> 45; error against float64 (2-norm) 7.5e-7 -> 4.6e-7, 5.4e-7 ->
-// 3.3e-7, 5.8e-7 -> 3.5e-7 and 5.8e-7 -> 3.5e-7, and smaller for each of 64 shapes of 65 to 16384 tokens, 512 to 7168 deep.
+// round after each, so that the cuts of a long chain of sums of one sign add up: chains end, in fp32, after at most 1024 depths (launch_logits).
+// What bounds it: the splitting's vector work beside the matrix instructions (11 and a half a pair of gate values against 24 x 32
+// cycles a 16 deep chunk of 64 x 128) where the experts are many, x from memory where they are few. Measured against the
+// fp32 instruction, the tokens from memory (us; error against float64, 2-norm, of normal tokens and gate and of positive ones): 8192 x 7168 x 256 327 -> 105
+// (7.5e-7 -> 3.2e-7, 3.0e-7 -> 1.1e-7), 16384 x 4096 x 8 65 -> 30 (6.2e-7 -> 3.7e-7, 2.5e-7 -> 2.1e-7), 4096 x 4096 x 8 36 -> 18 (5.6e-7 -> 1.8e-7, 2.5e-7 -> 7.5e-8),
+// 8192 x 4096 x 128 130 -> 45 (5.8e-7 -> 3.4e-7, 2.5e-7 -> 2.1e-7). The mean error, nil there, is -1e-8 to -5e-8 of normal logits' root mean square here.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 __device__ __forceinline__ uint32_t upper_halves(float high, float low) {
@@ -90,10 +95,11 @@ __device__ __forceinline__ void plain_sums(const bf16_t* __restrict__ row, const
 // The sums of a share of the depth, its steps of 16 x CHUNKS from `first` to `last`, for ROWS tiles of 32 tokens from t0 on and TILES tiles of
 // 32 experts. A lane's depths of a step are contiguous in its token's row (64 bytes of four chunks, so that every line of x is asked
 // for once); a chunk's instructions take 8 of each half's. Its experts are TILES neighbours, one a tile, from `column` on: one load a depth.
-// `end`: the depth that the share goes to, up to three chunks behind its last step; WHOLE: none, as the depth is whole steps.
+// `end`: the depth that the share goes to, up to three chunks behind its last step; WHOLE: none, as the depth is whole steps. `chain`: the
+// steps, whole sets of loads, after which sums go to `aside`, the lane's place in the LDS, and start from zero.
 template <int ROWS, int TILES, int AHEAD, int CHUNKS, bool WHOLE>
 __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const float* __restrict__ kernel, int tokens, int depth, int experts,
-                                            int t0, int column, int first, int last, int end, f32x16 (&acc)[ROWS][TILES]) {
+                                            int t0, int column, int first, int last, int end, int chain, f32x4* aside, f32x16 (&acc)[ROWS][TILES]) {
   struct __attribute__((packed, aligned(4))) Neighbours {
     float of[TILES];
   };
@@ -167,6 +173,30 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
       if (more) load_gate(next, min(step + AHEAD + (chunk == CHUNKS - 1), last - 1), (chunk + 1) % CHUNKS);
     }
   };
+  // Chains end between two loops or within one, by which the compiler keeps the loads in registers: 2 x 4 tiles 105 us between, 119 within (8192 x 7168 x
+  // 256), 2 x 1 43 and 46 (2112 x 7168 x 160), but 1 x 1 39 and 34 (5000 x 7168 x 32), and eight wavefronts 45 and 40 (2048 x 7168 x 256).
+  constexpr bool kBetween = ROWS * TILES * AHEAD >= 4;
+  auto put_aside = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int c = 0; c < TILES; ++c) {
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) aside[((r * TILES + c) * 4 + i / 4) * 64] = f32x4{acc[r][c][i], acc[r][c][i + 1], acc[r][c][i + 2], acc[r][c][i + 3]};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[r][c][i] = 0.0f;
+      }
+    aside += ROWS * TILES * 256;
+  };
+  auto take_back = [&]() __attribute__((always_inline)) {
+    aside -= ROWS * TILES * 256;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int c = 0; c < TILES; ++c)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[r][c][i] += aside[((r * TILES + c) * 4 + i / 4) * 64][i % 4];
+  };
 #pragma unroll
   for (int ahead = 0; ahead < AHEAD; ++ahead) {
     load_rows(ahead, min(first + ahead, last - 1));
@@ -179,13 +209,25 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
   } else {
     load_gate(0, min(first + AHEAD, last - 1), 0);
     int step = first;
-    for (; step + kSets <= last; step += kSets) {  // (no way out in the middle: every load would be waited for there)
+    int until = first + chain;
+    for (;;) {
+      const int stop = kBetween ? min(until, last) : last;
+      for (; step + kSets <= stop; step += kSets) {  // (no way out in the middle: every load would be waited for there)
 #pragma unroll
-      for (int set = 0; set < kSets; ++set) walk(set, step + set, true);
+        for (int set = 0; set < kSets; ++set) walk(set, step + set, true);
+        if (kBetween || step + kSets != until || until >= last) continue;
+        put_aside();
+        until += chain;
+      }
+      if (!kBetween || until >= last) break;
+      put_aside();
+      until += chain;
     }
 #pragma unroll
     for (int set = 0; set < kSets - 1; ++set)
       if (step + set < last) walk(set, step + set, AHEAD > 1);
+#pragma unroll 1
+    for (; until > first + chain; until -= chain) take_back();
   }
   // An infinity among the operands meets a term that is zero, a gate value's terms are not those of an infinity or a NaN, and below 2^-110 its
   // last bits lie under the least bf16 value: tiles with a sum that is no finite number, or with a column that dropped bits, are formed again on
@@ -225,7 +267,7 @@ __device__ __forceinline__ void logit_terms(const bf16_t* __restrict__ x, const 
 template <int ROWS, int TILES, int WAVES, int AHEAD, int CHUNKS, bool WHOLE>
 __global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf16_t* __restrict__ x, const float* __restrict__ kernel,
                                                                         const float* __restrict__ bias, float* __restrict__ logits,
-                                                                        int tokens, int depth, int experts) {
+                                                                        int tokens, int depth, int experts, int chain, int slots) {
   struct __attribute__((packed, aligned(4))) Neighbours {
     float of[TILES];
   };
@@ -234,9 +276,11 @@ __global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf
   const int t0 = blockIdx.x * 32 * ROWS, e0 = TILES * (32 * blockIdx.y + lane % 32);
   // (lanes past the experts repeat the last ones: what they share with the lane before is the same sum)
   const int column = min(e0, experts - TILES);
+  extern __shared__ f32x4 aside[];  // [wavefront][slot][row tile][tile][quad of registers][lane]
   const int steps = depth / (16 * CHUNKS), first = steps * wave / WAVES, last = steps * (wave + 1) / WAVES;
   f32x16 acc[ROWS][TILES];
-  logit_terms<ROWS, TILES, AHEAD, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, column, first, last, wave == WAVES - 1 ? depth : 16 * CHUNKS * last, acc);
+  logit_terms<ROWS, TILES, AHEAD, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, column, first, last, wave == WAVES - 1 ? depth : 16 * CHUNKS * last,
+                                                 chain, aside + wave * slots * (ROWS * TILES * 256) + lane, acc);
   // register i of lane l is the sum of token 8 (i / 4) + 4 (l / 32) + i % 4 and the lane's expert
 #pragma unroll
   for (int r = 0; r < ROWS; ++r) {
@@ -268,12 +312,33 @@ __global__ __launch_bounds__(64 * WAVES) void router_logits_mfma_kernel(const bf
   }
 }
 
+// The chains of a wavefront's share: of at most 1024 depths, and of 512 on eight wavefronts, as far as the LDS has room for the sums set aside (2 x 4
+// tiles up to 8192 deep, the others up to 12 288 and more). Sixteen wavefronts walk as much only from 16 384 depths on. Error against float64 (2-norm) of
+// positive tokens and gate, in one chain, in these, and by the fp32 instruction: 8192 x 7168 x 256 7.2e-7, 1.1e-7 and 3.0e-7, 3000 x 5120 x 128
+// 3.5e-7, 9.5e-8 and 2.8e-7, 2048 x 7168 x 256 1.1e-7, 6.6e-8 and 9.6e-8; at 1024 depths 2.1e-7 and 2.5e-7 (3000 x 4096 x 256).
+template <int ROWS, int TILES, int WAVES, int AHEAD, int CHUNKS, bool WHOLE>
+static int launch_logits(const bf16_t* x, const float* kernel, const float* bias, float* logits, int tokens, int depth, int experts, hipStream_t stream) {
+  auto routine = router_logits_mfma_kernel<ROWS, TILES, WAVES, AHEAD, CHUNKS, WHOLE>;
+  constexpr int kSlot = WAVES * ROWS * TILES * 64 * 16 * 4, kSlots = WAVES == 16 ? 0 : 131072 / kSlot;
+  static std::once_flag configured;  // dynamic LDS above 64 KiB must be opted into once per kernel
+  static hipError_t reserved = hipSuccess;
+  std::call_once(configured, [&] {
+    if (kSlots > 0) reserved = hipFuncSetAttribute(reinterpret_cast<const void*>(routine), hipFuncAttributeMaxDynamicSharedMemorySize, kSlots * kSlot);
+  });
+  if (reserved != hipSuccess) return fail(DEW_MOE_ELAUNCH, "dew_moe_router_logits: cannot reserve %d bytes of LDS", kSlots * kSlot);
+  constexpr int kChain = (WAVES == 8 ? 512 : 1024) / (16 * CHUNKS), kSets = 2 * AHEAD;
+  const int share = (depth / (16 * CHUNKS) + WAVES - 1) / WAVES, slots = min((share + kChain - 1) / kChain - 1, kSlots);
+  const int chain = slots > 0 ? (share + (slots + 1) * kSets - 1) / ((slots + 1) * kSets) * kSets : 1 << 30;
+  hipLaunchKernelGGL(routine, dim3((tokens + 32 * ROWS - 1) / (32 * ROWS), (experts + 32 * TILES - 1) / (32 * TILES)), dim3(64 * WAVES),
+                     static_cast<size_t>(max(slots, 0)) * kSlot, stream, x, kernel, bias, logits, tokens, depth, experts, chain, slots);
+  return launched("router_logits_mfma_kernel");
+}
+
 // The few tokens of a decode step on finer tiles: 16 tokens x 16 experts a block (v_mfma_f32_16x16x4_f32, the same
 // rate a CU as the 32 x 32 form), sixteen wavefronts a share of the depth each. A 32 x 32 tile's block keeps its whole
 // product on one CU's four matrix pipes (64 tokens of a 2880 x 32 gate: two blocks, 20 us); four times the blocks
 // finish in a quarter of that. Lane l multiplies token l % 16 and expert l % 16 over the depths 4 (l / 16) .. + 3 of a
 // 16-deep chunk, one depth an instruction; its four sums are tokens 4 (l / 16) + i of expert column l % 16.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kShares = kLogitShares;  // the depth's shares, one a wavefront
@@ -377,7 +442,7 @@ __global__ __launch_bounds__(64) void router_logit_tile_shares_kernel(const bf16
   const int steps = depth / (16 * CHUNKS), first = steps * share / kShares, last = steps * (share + 1) / kShares;
   f32x16 acc[1][1];
   logit_terms<1, 1, 1, CHUNKS, WHOLE>(x, kernel, tokens, depth, experts, t0, min(32 * static_cast<int>(blockIdx.y) + lane % 32, experts - 1), first, last,
-                               share == kShares - 1 ? depth : 16 * CHUNKS * last, acc);
+                               share == kShares - 1 ? depth : 16 * CHUNKS * last, 1 << 30, nullptr, acc);
   const int e = 32 * blockIdx.y + lane % 32;
   if (e >= experts) return;
 #pragma unroll
@@ -496,13 +561,9 @@ extern "C" int dew_moe_router_logits(const void* x, const float* kernel, const f
                          static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts);
       return launched("router_logits_fine_kernel");
     }
-    auto launch = [&](auto whole, auto ragged, int step, int tokens_a_block, int tiles_a_block, int waves) {
-      hipLaunchKernelGGL(depth % step == 0 ? whole : ragged, dim3((tokens + tokens_a_block - 1) / tokens_a_block, (tiles + tiles_a_block - 1) / tiles_a_block),
-                         dim3(64 * waves), 0, s, static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts);
-    };
-#define DEW_LOGITS(ROWS, TILES, WAVES, AHEAD, CHUNKS)                       \
-  launch(router_logits_mfma_kernel<ROWS, TILES, WAVES, AHEAD, CHUNKS, true>, \
-         router_logits_mfma_kernel<ROWS, TILES, WAVES, AHEAD, CHUNKS, false>, 16 * CHUNKS, 32 * ROWS, TILES, WAVES)
+#define DEW_LOGITS(ROWS, TILES, WAVES, AHEAD, CHUNKS) \
+  return (depth % (16 * CHUNKS) == 0 ? launch_logits<ROWS, TILES, WAVES, AHEAD, CHUNKS, true> : launch_logits<ROWS, TILES, WAVES, AHEAD, CHUNKS, false>)( \
+      static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts, s)
     auto blocks = [&](int rows, int beside) { return static_cast<long long>((tokens + 32 * rows - 1) / (32 * rows)) * ((tiles + beside - 1) / beside); };
     // The largest tile that still gives most CUs a block: it reads x and the gate least often and splits a gate value for most rows.
     // Measured (us; rows x tiles): 8192 x 7168 x 256 (256 blocks of 2 x 4) 104, in 2 x 2 129; 4096 x 7168 x 256 (256 of 2 x 2) 67, in
@@ -519,7 +580,6 @@ extern "C" int dew_moe_router_logits(const void* x, const float* kernel, const f
     else if (blocks(2, 1) >= 160) DEW_LOGITS(2, 1, 4, 2, 4);
     else DEW_LOGITS(1, 1, 4, 2, 4);
 #undef DEW_LOGITS
-    return launched("router_logits_mfma_kernel");
   }
   const dim3 grid((tokens + LT - 1) / LT, (experts + LE - 1) / LE);
   hipLaunchKernelGGL(router_logits_kernel, grid, dim3(256), 0, s, static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth,

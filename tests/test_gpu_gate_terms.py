@@ -17,7 +17,9 @@ SHAPES = [(14400, 80, 128),    # 2 x 4, 4; the depth ends inside a step
           (2040, 80, 32),      # 1 x 1, 16 in steps of 32; a depth behind the last step
           (2040, 96, 32),      # whole steps
           (2100, 1072, 8),     # 1 x 1, 16 in steps of 64; three chunks behind the last step
-          (2100, 1088, 8)]     # whole steps
+          (2100, 1088, 8),     # whole steps
+          # chains of sums that end before a wavefront's share does, once and more often, with a depth behind the last step and without
+          (14400, 4432, 128), (14400, 8512, 100), (10300, 4480, 40), (10300, 8464, 20), (4200, 4432, 9), (2000, 4432, 300), (1900, 8512, 63)]
 
 
 @pytest.mark.parametrize("tokens,depth,experts", SHAPES)
@@ -119,3 +121,31 @@ def test_a_gate_value_that_three_terms_do_not_hold(tokens, depth, experts, expon
     assert bool(((got.double() - exact).abs() <= 2.0 ** -19 * magnitudes).all())
     want[:, experts // 2] = got[:, experts // 2]
     assert torch.equal(got, want)
+
+
+# (what the fp32 instruction's sums, rounded after each product, are off)
+@pytest.mark.parametrize("tokens,depth,experts,bar", [(8192, 7168, 256, 3.0e-7), (4096, 7168, 256, 3.0e-7), (3000, 5120, 128, 2.7e-7), (2112, 7168, 160, 3.0e-7),
+                                                      (5000, 7168, 32, 3.0e-7), (2048, 7168, 256, 9.6e-8), (4100, 7168, 40, 3.0e-7)])
+def test_sums_of_one_sign_are_no_further_off_than_rounded_ones(tokens, depth, experts, bar):
+    """The instruction cuts its sums off, always to the same side: in one chain over a wavefront's share 7.2e-7 at 1792 depths."""
+    from dew_amd import ops
+
+    generator = torch.Generator("cuda").manual_seed(depth + experts)
+    x = torch.randn((tokens, depth), generator=generator, device="cuda").abs().to(torch.bfloat16)
+    kernel = torch.randn((depth, experts), generator=generator, device="cuda").abs() * depth ** -0.5
+    for sign in (1.0, -1.0):
+        exact = x.double() @ (sign * kernel).double()
+        assert float((ops.router_logits(x, sign * kernel).double() - exact).norm() / exact.norm()) <= bar
+
+
+@pytest.mark.parametrize("tokens,depth,experts", SHAPES)
+def test_every_term_of_a_product_is_in_the_sum(tokens, depth, experts):
+    """One product a sum, so that the sum is exact: all 24 bits of the gate's value times the token's."""
+    from dew_amd import ops
+
+    generator = torch.Generator("cuda").manual_seed(depth + experts)
+    x = torch.zeros((tokens, depth), dtype=torch.bfloat16, device="cuda")
+    at = torch.randint(0, depth, (tokens, 1), generator=generator, device="cuda")
+    x.scatter_(1, at, 2.0 ** torch.randint(-20, 20, (tokens, 1), generator=generator, device="cuda").to(torch.bfloat16))
+    kernel = torch.randn((depth, experts), generator=generator, device="cuda")
+    assert torch.equal(ops.router_logits(x, kernel), kernel[at[:, 0]] * x.gather(1, at).float())
