@@ -352,16 +352,13 @@ static bool few_tiles(int rows, int groups, int width) {  // about so many of 12
   return (rows / 128 + groups / 2 + 1) * static_cast<long long>((width + 255) / 256) <= kFewTiles;
 }
 
-// 256 x 256 tiles (wide.hip) on groups of at least about half a tile's rows (of 64 to 97 rows 0.82 to 0.98 times as fast) but where they
-// are a first round of whole ones that is half empty. Measured against the tiles below (us, there and here). Whole tiles, natural order, from
-// 146 on: 4608 rows of 1 x 1024 x 2048, 148 tiles, 32.1 and 25.5, 4300 of 4 x 4096 x 2048 97.4 and 77.3; below it 4096 of 1 x 4096 x 2048, 132, 67.5
-// and 80.3, 3584 of 4, 136, 69.5 and 83.2. K-major matrices, which the tiles below read half a cache line at a step, from 129: 4096 of 1 x 4096 x 2048, 132,
-// 75.6 and 79.9, of 4, 136, 81.4 and 77.0. A second round begun: 4352 rows of 1 x 4096 x 4096, 272 tiles, 165 and 125. In quarters alone, natural and
-// K-major, up to one a block: 512 rows of 1 x 4096 x 4096, 32 tiles, 42.2 and 42.7 -> 29.4 and 29.1, 1024, 64, 67.7 and 74.8 -> 37.0 and 37.6, 1024 x 4096, 25.1
-// and 27.0 -> 17.7 and 20.3, 1024 of 8 x 4096 x 2048 53.0 and 58.2 -> 31.2 and 31.8; up to two where the walk is long: 1536 of 1 x 4096 x 4096, 96, 67.3 and
-// 74.1 -> 60.6 and 60.4, 2560 of 4 x 1024 x 2048, 88, 24.7 and 26.7 -> 23.6 and 23.4, 1732 of 8 x 1152 x 1792, 70, natural, 20.0 and 22.6. Of 90 shapes of 128 to
-// 16 384 rows in 1 to 16 groups (steps of one forward product, one input's gradient and one kernel's) these rules make the three 1.09, 1.11 and
-// 1.09 times as fast; furthest off 3127 of 1 x 3584 x 1152, 65 tiles, 46 and 50.
+// Whether a product takes 256 x 256 tiles (wide.hip), on groups of at least about half a tile's rows (of 64 to 97 rows 0.82 to 0.98 times as fast):
+//  * whole tiles, but where a first round of them is half empty: from 146 on, K-major matrices, which the tiles below read half a cache line at a
+//    step, from 129;
+//  * quarters, up to one a block, and up to two where the walk is long enough to hide two starts.
+// us, the tiles below and here, natural order and K-major. Whole: 4608 rows of 1 x 1024 x 2048, 148 tiles, 32.1 and 25.5 (natural), 4096 of 1 x 4096 x 2048,
+// 132, 67.5 and 80.3, 75.6 and 79.9. One quarter a block: 1024 of 1 x 4096 x 4096 63 and 33, 70 and 33, 3127 of 1 x 3584 x 1152, 225 quarters of 65 tiles, 40 and 28,
+// 48 and 28. Two: 1536 of 1 x 4096 x 4096 64 and 56, 70 and 54, 2560 of 4 x 1024 x 2048 24 and 19 (K-major). Furthest off: 2205 of 14 x 4928 x 1184, 64 and 76, 64 and 59.
 static bool wide_product(int rows, int groups, int depth, int width, bool kmajor) {
   const double tiles = product_tiles(rows, groups, width);
   const int quarters = depth >= (kmajor ? 1024 : 2048) ? 128 : 64;

@@ -1314,11 +1314,9 @@ static bool few_gradient_blocks(const GemmParams& p) {
 }
 
 // The same products in 256 x 256 tiles on blocks that stay (wide_fp8.hip), of rows that are neither gathered nor scattered, on groups of half
-// a tile's rows, but for what two quarters a block of a short walk would take. Against the launches below (us, there and here). Whole tiles:
-// blockwise, [2560, 512] x 2048 of 4 groups, 96 tiles, 14.2 and 12.7; [4608, 1024] x 2048, 148, 26.0 and 18.3; [32 768, 7168] x 2048 of 32, forward 470
-// and 424, input's gradient 520 and 444; MXFP8, [32 768, 4096] x 14336 of 8 1636 and 1490. In quarters, up to one a block: [1024, 2944] x 640 of 2, 15
-// tiles, 19.5 and 14.1, [1792, 5504] x 896 of 11, 44, 31.9 and 23.3, [1408, 896] x 640 of 6, 21, 9.5 and 8.9; up to two: [1280, 3456] x 3840 of 2, 75, 43.7 and
-// 32.0, [3584, 2176] x 1920 of 4, 120, 29.6 and 24.0; but [1408, 1920] x 2688 of 2, 66, 17.6 and 21.7, [640, 1152] x 5248 of 4, 84, 14.0 and 16.7.
+// a tile's rows, but for what two quarters a block of a short walk would take. us, the launches below and here. Whole tiles: [2560, 512] x 2048 of 4
+// groups, 96 tiles, 14.2 and 12.7, [32 768, 7168] x 2048 of 32 470 and 424. One quarter a block: [1024, 2944] x 640 of 2 18.6 and 13.5, [6016, 2560] x 640, 235 quarters
+// of 72 tiles, 18.3 and 15.3. Two: [1280, 3456] x 3840 of 2, 75 tiles, 42.0 and 30.6; but [1408, 1920] x 2688 of 2, 66, 17.6 and 21.7.
 static WideFp8Params wide_fp8_params(const GemmParams& p, int a_scale_pitch) {
   return WideFp8Params{reinterpret_cast<const uint8_t*>(p.x), p.a_scale, p.w0.codes, p.w0.scales, p.offsets, p.out, p.experts, p.rows, p.depth, p.width, a_scale_pitch};
 }

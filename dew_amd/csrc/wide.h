@@ -19,6 +19,8 @@ inline double product_tiles(int rows, int groups, int width) { return (rows / 25
 
 inline double gradient_tiles(int groups, int depth, int width) { return static_cast<double>(groups) * ((depth + 255) / 256) * ((width + 255) / 256); }
 
+inline double gradient_quarters(int groups, int depth, int width) { return static_cast<double>(groups) * ((depth + 127) / 128) * ((width + 127) / 128); }
+
 inline bool wide_extents(int groups, int a, int b) { return groups <= kWideGroups && a <= (1 << 20) && b <= (1 << 20); }  // (offsets within a tile are 32-bit)
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -27,7 +29,7 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 // cost every other tile's start: e4m3, eight tiles of a few steps a block, 3 to 5 %). A product's tiles are known on the device alone.
 inline bool ends_in_quarters(int groups, int depth, int width, int quarter_turns) {
   const int tiles = static_cast<int>(gradient_tiles(groups, depth, width));
-  return tiles % 256 != 0 && tiles % 256 <= 64 * quarter_turns;
+  return (tiles % 256 != 0 && tiles % 256 <= 64 * quarter_turns) || (tiles < 256 && gradient_quarters(groups, depth, width) <= 256);
 }
 
 struct WidePlace {
@@ -42,45 +44,79 @@ struct WideTiles {
   int first_tile[kRounds], first_row[kRounds], group_size[kRounds];
   int gradient_tiles, strips, total, held;  // `held`: rows in all groups
   int whole;                                // tiles that leave as such; those behind them in quarters
+  bool fine;                                // the tiles are quarters themselves
 
-  __device__ __forceinline__ void find(const int32_t* offsets, const int32_t* sizes, int groups, int outer_m, int outer_n, int quarter_turns) {
+  // The groups' first tiles of `of` rows each; how many row tiles there are.
+  __device__ __forceinline__ int tabulate(int groups, int outer_m, int of) {
     const int lane = threadIdx.x % 64;
-    gradient_tiles = (outer_m + kWideTile - 1) / kWideTile;
+    gradient_tiles = (outer_m + of - 1) / of;
     int m_tiles = 0;
-    held = 0;
 #pragma unroll
     for (int round = 0; round < kRounds; ++round) {
       const int g = 64 * round + lane;
       first_tile[round] = 0x7FFFFFFF;
+      if (64 * round < groups) {
+        const int tiles = g >= groups ? 0 : kGradient ? gradient_tiles : (group_size[round] + of - 1) / of, inclusive = lanes_scanned(tiles);
+        if (g < groups) first_tile[round] = m_tiles + inclusive - tiles;
+        m_tiles += __builtin_amdgcn_readlane(inclusive, 63);
+      }
+    }
+    return m_tiles;
+  }
+
+  __device__ __forceinline__ void find(const int32_t* offsets, const int32_t* sizes, int groups, int outer_m, int outer_n, int quarter_turns) {
+    const int lane = threadIdx.x % 64;
+    held = 0;
+#pragma unroll
+    for (int round = 0; round < kRounds; ++round) {
+      const int g = 64 * round + lane;
       first_row[round] = group_size[round] = 0;
       if (64 * round < groups) {
         const int size = g >= groups ? 0 : sizes ? max(sizes[g], 0) : max(offsets[g + 1] - offsets[g], 0);
-        const int tiles = g >= groups ? 0 : kGradient ? gradient_tiles : (size + kWideTile - 1) / kWideTile;
-        const int rows = lanes_scanned(size), inclusive = lanes_scanned(tiles);
+        const int rows = lanes_scanned(size);
         if (g < groups) {
-          first_tile[round] = m_tiles + inclusive - tiles;
           first_row[round] = sizes ? held + rows - size : offsets[g];
           group_size[round] = size;
         }
-        m_tiles += __builtin_amdgcn_readlane(inclusive, 63);
         held += __builtin_amdgcn_readlane(rows, 63);
       }
     }
     if (!sizes) held = offsets[groups];
     strips = (outer_n + kWideTile - 1) / kWideTile;
-    total = __builtin_amdgcn_readfirstlane(m_tiles * strips);
+    total = __builtin_amdgcn_readfirstlane(tabulate(groups, outer_m, kWideTile) * strips);
     const int blocks = gridDim.x, behind = total % blocks;
     whole = behind <= blocks * quarter_turns / 4 ? total - behind : total;
+    fine = false;
+    // A launch of one quarter a block, though its tiles have more: those past a group's rows and the columns are left out, or blocks would wait
+    // a turn for them (us: 1348 rows' gradient of 2624 x 1496, 252 quarters of 66 tiles, 26.1 -> 16.4, a blockwise product of 768 rows of 2 x 5376 x 4352, 204
+    // of 68, 39.4 -> 23.1).
+    if (quarter_turns > 0 && total < blocks && 4 * total > blocks) {
+      int row_quarters = kGradient ? groups * ((outer_m + kWideTile / 2 - 1) / (kWideTile / 2)) : 0;
+#pragma unroll
+      for (int round = 0; round < kRounds; ++round)
+        if (!kGradient && 64 * round < groups) row_quarters += __builtin_amdgcn_readlane(lanes_scanned((group_size[round] + kWideTile / 2 - 1) / (kWideTile / 2)), 63);
+      const int strip_quarters = (outer_n + kWideTile / 2 - 1) / (kWideTile / 2);
+      if (row_quarters * strip_quarters <= blocks) {
+        tabulate(groups, outer_m, kWideTile / 2);
+        strips = strip_quarters;
+        total = __builtin_amdgcn_readfirstlane(row_quarters * strip_quarters);
+        whole = 0;
+        fine = true;
+      }
+    }
   }
 
-  // The block's quarter tile number `turn` of those behind the whole ones, false past its last: its tile, and which quarter. Neighbours
-  // are an XCD's, and share their operands in its L2.
-  __device__ __forceinline__ bool quarter_at(int turn, int group_m, WidePlace& out, int& quarter) const {
-    const int xcds = 8, slots = gridDim.x / xcds, count = 4 * (total - whole), run = (count + xcds - 1) / xcds, slot = blockIdx.x / xcds + turn * slots;
-    const int order = __builtin_amdgcn_readfirstlane(slot < run ? blockIdx.x % xcds * run + slot : count);
+  // The block's quarter tile number `turn`, false past its last: its tile, and the quarter's first row in the group and column. Neighbours
+  // are an XCD's, and share their operands in its L2. (Of a tile's four, some may lie past the group's rows or the columns; `fine` ones are all
+  // real.)
+  __device__ __forceinline__ bool quarter_at(int turn, int group_m, WidePlace& out, int& row_at, int& column) const {
+    const int xcds = 8, slots = gridDim.x / xcds, count = (fine ? 1 : 4) * (total - whole), run = (count + xcds - 1) / xcds;
+    const int slot = blockIdx.x / xcds + turn * slots, order = __builtin_amdgcn_readfirstlane(slot < run ? blockIdx.x % xcds * run + slot : count);
     if (order >= count) return false;
-    quarter = order % 4;
-    place(whole + order / 4, group_m, out);
+    const int quarter = fine ? 0 : order % 4, shift = fine ? 7 : 8;
+    place(fine ? order : whole + order / 4, fine ? 2 * group_m : group_m, shift, out);
+    row_at = (out.within << shift) + quarter / 2 * (kWideTile / 2);
+    column = (out.strip << shift) + quarter % 2 * (kWideTile / 2);
     return true;
   }
 
@@ -93,11 +129,11 @@ struct WideTiles {
     const int run = min((whole - begun + xcds - 1) / xcds, slots), slot = blockIdx.x / xcds;
     const int order = __builtin_amdgcn_readfirstlane(slot < run ? begun + blockIdx.x % xcds * run + slot : whole);
     if (order >= whole) return false;
-    place(order, group_m, out);
+    place(order, group_m, 8, out);
     return true;
   }
 
-  __device__ __forceinline__ void place(int order, int group_m, WidePlace& out) const {
+  __device__ __forceinline__ void place(int order, int group_m, int shift, WidePlace& out) const {
     const int across = order / strips;  // (the tiles of a group are in a row: this many before it at most)
     int group = -1;
 #pragma unroll
@@ -110,7 +146,7 @@ struct WideTiles {
         start = __builtin_amdgcn_readlane(first_row[round], group % 64);
         size = __builtin_amdgcn_readlane(group_size[round], group % 64);
       }
-    const int tiles = kGradient ? gradient_tiles : (size + kWideTile - 1) / kWideTile;
+    const int tiles = kGradient ? gradient_tiles : (size + (1 << shift) - 1) >> shift;
     const int place_in_group = order - before * strips;
     const int band = place_in_group / (group_m * strips), band_tiles = min(group_m, tiles - band * group_m), within = place_in_group % (group_m * strips);
     out = WidePlace{group, start, size, band * group_m + within % band_tiles, within / band_tiles};

@@ -335,8 +335,7 @@ __device__ __forceinline__ void quarter_tiles(const DenseParams& p, const WideTi
   if constexpr (kAAcross) factor = (p.factor0 ? *p.factor0 : 1.0f) * (p.factor1 ? *p.factor1 : 1.0f);
 
   WidePlace place;
-  for (int turn = 0, quarter = 0; tiles.quarter_at(turn, p.group_m, place, quarter); ++turn) {
-    const int row_at = place.within * kWideTile + quarter / 2 * kHalf, n0 = place.strip * kWideTile + quarter % 2 * kHalf;
+  for (int turn = 0, row_at = 0, n0 = 0; tiles.quarter_at(turn, p.group_m, place, row_at, n0); ++turn) {
     const int valid_rows = __builtin_amdgcn_readfirstlane(min(kHalf, (kAAcross ? p.outer_m : place.size) - row_at));
     if (valid_rows <= 0 || n0 >= p.outer_n) continue;  // (the same for the whole block)
     const uint8_t *a_next = reinterpret_cast<const uint8_t*>(p.a), *b_next = reinterpret_cast<const uint8_t*>(p.b);

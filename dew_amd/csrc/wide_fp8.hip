@@ -396,8 +396,7 @@ __device__ __forceinline__ void quarter_fp8_tiles(const WideFp8Params& p, const 
   auto buffer = [](const uint8_t* at, int bytes) __attribute__((always_inline)) { return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(at), 0, bytes, 0x00027000); };
 
   WidePlace place;
-  for (int turn = 0, quarter = 0; tiles.quarter_at(turn, 4, place, quarter); ++turn) {
-    const int row_at = place.within * kWideTile + quarter / 2 * kHalf, n0 = place.strip * kWideTile + quarter % 2 * kHalf;
+  for (int turn = 0, row_at = 0, n0 = 0; tiles.quarter_at(turn, 4, place, row_at, n0); ++turn) {
     const int valid_rows = __builtin_amdgcn_readfirstlane(min(kHalf, (kGradient ? p.rows : place.size) - row_at));
     if (valid_rows <= 0 || n0 >= p.width) continue;  // (the same for the whole block)
     int first_step = 0, steps = depth_steps, row0 = row_at;
