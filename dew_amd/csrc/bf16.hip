@@ -365,13 +365,19 @@ static bool wide_product(int rows, int groups, int depth, int width, bool kmajor
   return wide_extents(groups, depth, width) && rows / groups >= 112 && (tiles + (groups > 1 ? kGuessed : 0) <= quarters || tiles >= (kmajor ? 129 : 146));
 }
 
-// A kernel's gradient; groups of fewer than 256 rows, four steps, are all start and end either way (0.91 to 1.18 times as fast), and in quarters those of
-// fewer than 512 (813 rows of 3 x 640 x 2176, 81 tiles, 10.7 and 13.3; us, there and here, 4096 of 2 x 512 x 2048, 32 tiles, 32.1 and 17.9, of 1 x 1024 x 4096, 64,
-// 57.5 and 35.5, 1 x 2048 x 4096, 128, 81.6 and 67.2; 512 12.5 and 11.3, 16.9 and 17.1). Whole tiles from over half a round on: 144 of 512 rows 20.1 and
-// 18.4, of 8192 207 and 169.
+// The same of a kernel's gradient, whose tiles are known; groups of fewer than 256 rows, four steps, are all start and end either way:
+//  * up to 128 tiles, one quarter a block on groups of 512 rows and more, two where the walk is long (a launch takes two from 1024 rows on; of 1024 to
+//    2048 in several groups they are 0.8 to 1.2 times the time, 1.0 in the mean of 152 shapes, of more 0.93, in one group 0.87);
+//  * whole ones from over half a round on, and from 1.1, before which groups of fewer than 512 rows lose.
+// us, the tiles below and here. One quarter a block: 4096 rows of 2 x 512 x 2048 28.1 and 15.9, 2340 of 3 x 576 x 1952, 72 tiles, 14.3 and 11.1; 813 of 3 x 640 x
+// 2176 10.7 and 13.3. Two: 2048 of 1 x 2048 x 4096 41.0 and 35.9, 11 129 of 1 x 2048 x 2432 179 and 139, 16 329 of 2 x 1664 x 1344 137 and 111; 3531 of 4 x 960 x 1368
+// 21.2 and 24.0. Whole: 144 tiles of 512 rows 20.1 and 18.4, of 8192 207 and 169. Behind a round: 3364 of 1 x 2432 x 6672, 270 tiles, 141 and 106; 2221 of 5
+// x 3200 x 800, 260, 19.9 and 24.3.
 static bool wide_gradient(int rows, int groups, int depth, int width) {
-  const double tiles = gradient_tiles(groups, depth, width);
-  return wide_extents(groups, depth, width) && rows / groups >= (tiles <= 128 ? 512 : 256) && (tiles <= 128 || tiles >= 141);
+  const double tiles = gradient_tiles(groups, depth, width), quarters = gradient_quarters(groups, depth, width);
+  if (!wide_extents(groups, depth, width) || rows / groups < 256) return false;
+  if (tiles <= 128) return quarters <= 256 ? rows / groups >= 512 : quarters >= 280 && rows / groups >= (groups == 1 ? 1024 : 2048);
+  return tiles >= 282 || (tiles >= 141 && tiles <= 256) || (tiles > 256 && rows / groups >= 512);
 }
 
 }  // namespace dew
