@@ -1549,14 +1549,14 @@ extern "C" int dew_moe_kernel_gradient_mxfp8(const void* lhs_t_codes, const uint
   return launch_tile<kFormatMxFp8Window, kPlain, 256, 128, 2, 2>(who, p, s);
 }
 
-// (In quarters up to one a block: us, there and here, 8064 tokens of 1920 x 1536, 48 tiles, 55.1 and 30.6, 4224 of 1792 x 640, 21, 31.6 and 17.7, 896 of
-// 6 x 1280 x 512, 60, 9.9 and 7.3; up to two they gain a little or lose: 5376 of 2 x 3456 x 896, 112, 29.4 and 27.9, 20 992 of 4 x 1152 x 1536, 120, 61 and 67.
-// Whole tiles from over half a round on: 144 of 512 tokens 20.1 and 16.5, of 8192 99.9 and 85.7; 130 of 4224 25.2 and 30.7. Between one round and
-// 1.1 the answer is what it was before quarters; the recipes' gradients take banks there too, by a rule of their own.)
+// Quarters up to one a block, and whole tiles from over half a round on, a second round just begun among them, which leaves in quarters. us, operands as
+// rows and banks here: 8064 tokens of 1920 x 1536, 48 tiles, 55.1 and 30.6, 896 of 6 x 1280 x 512, 60, 9.9 and 7.3; two quarters a block gain a little or lose:
+// 5376 of 2 x 3456 x 896, 112, 29.4 and 27.9, 20 992 of 4 x 1152 x 1536, 120, 61 and 67. 144 of 512 tokens 20.1 and 16.5; 130 of 4224 25.2 and 30.7. 257 to 281, 38
+// shapes of 512 to 14 000 tokens: 0.65 to 1.14 times the time, 0.85 in the mean (3712 tokens of 2560 x 6656, 260, 88.5 and 60.6, 13 952 of 2 x 1536 x 5632, 264, 148 and 121).
 extern "C" int dew_moe_kernel_gradient_takes_banks(int32_t tokens, int32_t depth, int32_t width, int32_t groups) {
   using namespace dew;
   const double tiles = gradient_tiles(groups, depth, width);
-  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && (tiles <= 64 || (tiles >= 141 && tiles <= 256) || tiles >= 282);
+  return groups >= 1 && wide_fp8_gradient_extents(tokens, depth, width, groups) && (tiles <= 64 || tiles >= 141);
 }
 
 extern "C" int dew_moe_kernel_gradient_mxfp8_banks(const dew_moe_bank* lhs_t, const dew_moe_bank* rhs_t, const int32_t* offsets, void* out,

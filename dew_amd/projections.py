@@ -295,19 +295,10 @@ def kernel_gradient(x: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, m
 
 def _contracted(x: torch.Tensor, bank: ops.PreparedBank, width: int, offsets: torch.Tensor, mx: bool, out_dtype) -> torch.Tensor:
     """`kernel_gradient` of a cotangent that is a bank already."""
-    if out_dtype in (torch.bfloat16, torch.float32) and _gradient_of_banks(x.shape[0], x.shape[1], width, offsets.numel() - 1):
+    if out_dtype in (torch.bfloat16, torch.float32) and ops.kernel_gradient_takes_banks(x.shape[0], x.shape[1], width, offsets.numel() - 1):
         return ops.kernel_gradient_mxfp8_banks(ops.quantize_columns(x.contiguous(), mx=mx, as_bank=True), bank, offsets, out_dtype=out_dtype)
     codes, scales = ops.quantize_columns(x.contiguous(), mx=mx, as_bank=False)
     return ops.kernel_gradient_mxfp8(codes, scales, bank, offsets, out_dtype=out_dtype)
-
-
-def _gradient_of_banks(tokens: int, depth: int, width: int, groups: int) -> bool:
-    """Whether a kernel gradient takes both operands as banks: where the library says so, and where a second round of 256 x 256 tiles has just
-    begun, which leaves in quarters (us, rows and banks: 8320 tokens of 2 x 2560 x 3456, 280 tiles, 99 and 68; 4992 of 9 x 3712 x 512, 270, 28.8 and 22.0)."""
-    if ops.kernel_gradient_takes_banks(tokens, depth, width, groups):
-        return True
-    tiles = groups * -(-depth // 256) * -(-width // 256)
-    return 256 < tiles < 282 and groups <= 256 and 512 <= tokens <= 1 << 20
 
 
 def blockwise_fp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):
