@@ -72,7 +72,7 @@ __device__ __forceinline__ float saturated(float value, float inverse) {
   return value == value ? q : value;
 }
 
-template <int FORMAT, typename T, bool KMAJOR>
+template <int FORMAT, typename T, bool KMAJOR, bool CACHED>
 __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const T* __restrict__ w, uint8_t* __restrict__ codes,
                                                                          uint8_t* __restrict__ scales, const uint32_t* __restrict__ largest,
                                                                          float* __restrict__ tensor_scales, int depth, int width) {
@@ -100,11 +100,16 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
   const T* source = w + e * depth * width + static_cast<size_t>(KMAJOR ? n0 : k0) * pitch + (KMAJOR ? k0 : n0) + piece * kVec;
   const uint32_t share = kNv ? nvfp4_share(largest, kNvfp4Partials) : 0u;
   // Bound by memory, and every weight is read once: non-temporal, so that the weights don't push out what the step's products read next. us of
-  // twelve drawn steps of the FP8 recipes 1.00 to 1.12 times as fast (252 -> 224, 535 -> 497, 228 -> 209). Non-temporal stores too, of codes that the
-  // product reads at once: no difference in steps of 400 us and more and of 113 and less, 5 to 10 % slower in those of 180 to 300.
+  // twelve drawn steps of the FP8 recipes 1.00 to 1.12 times as fast (252 -> 224, 535 -> 497, 228 -> 209). CACHED: NVFP4's were just read for their largest
+  // magnitude, and where the 256 MB of the last-level cache hold them all, such loads only miss it (steps of 512 to 1024 rows, without and with them: 16 x 768 x
+  // 6912, 170 MB, 268 and 279 us, 22 x 768 x 4864, 164, 267 and 279; 31 x 5120 x 1024, 325, 531 and 515). Non-temporal stores too, of codes that the product
+  // reads at once: no difference in steps of 400 us and more and of 113 and less, 5 to 10 % slower in those of 180 to 300.
   u32x4_t words[kLoads];
 #pragma unroll
-  for (int p = 0; p < kLoads; ++p) words[p] = __builtin_nontemporal_load(reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch));
+  for (int p = 0; p < kLoads; ++p) {
+    const u32x4_t* from = reinterpret_cast<const u32x4_t*>(source + static_cast<size_t>(row_of(p)) * pitch);
+    words[p] = CACHED ? *from : __builtin_nontemporal_load(from);
+  }
 
   float tensor = 1.0f;
   bool quick = false;  // (the same for the whole launch)
@@ -297,10 +302,11 @@ static int quantize_matrices(const T* w, bool kmajor, int experts, int depth, in
     if (int rc = dew_moe_nvfp4_largest(w, static_cast<int64_t>(elements), sizeof(T) == 4, largest, s)) return rc;
   }
   const dim3 grid = kmajor ? dim3(depth / 128, width / 128, experts) : dim3(width / 128, depth / 128, experts);
-  if (kmajor)
-    hipLaunchKernelGGL((quantize_matrices_kernel<FORMAT, T, true>), grid, dim3(kMatrixThreads), 0, s, w, prepared, scales, largest, tensor_scales, depth, width);
-  else
-    hipLaunchKernelGGL((quantize_matrices_kernel<FORMAT, T, false>), grid, dim3(kMatrixThreads), 0, s, w, prepared, scales, largest, tensor_scales, depth, width);
+  constexpr bool kNv = FORMAT == DEW_MOE_W_NVFP4;
+  const bool cached = kNv && elements * sizeof(T) <= (size_t{256} << 20);
+  auto kernel = cached ? (kmajor ? quantize_matrices_kernel<FORMAT, T, true, kNv> : quantize_matrices_kernel<FORMAT, T, false, kNv>)
+                       : (kmajor ? quantize_matrices_kernel<FORMAT, T, true, false> : quantize_matrices_kernel<FORMAT, T, false, false>);
+  hipLaunchKernelGGL(kernel, grid, dim3(kMatrixThreads), 0, s, w, prepared, scales, largest, tensor_scales, depth, width);
   return launched("quantize_matrices_kernel");
 }
 

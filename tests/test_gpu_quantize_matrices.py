@@ -45,6 +45,18 @@ def test_the_bank_is_the_quantized_matrices_prepared(ops, recipe, dtype, turned,
         assert torch.equal(got.keep[2], want.keep[2])
 
 
+@pytest.mark.parametrize("turned", [False, True], ids=["natural", "kmajor"])
+def test_matrices_that_no_cache_holds(ops, turned):
+    """NVFP4's loads are others past 256 MB: every copy of a matrix has the codes and scales that it has alone."""
+    one = torch.randn((1, 2048, 2048), generator=torch.Generator("cuda").manual_seed(1), device="cuda").to(torch.bfloat16)
+    quantized = lambda w: ops.quantize_matrices(w.transpose(1, 2).contiguous().transpose(1, 2) if turned else w, "nvfp4").keep[0]
+    alone, bytes_of = quantized(one), one.numel() // 2
+    for copies in (32, 33):
+        got = quantized(one.expand(copies, -1, -1).contiguous())
+        assert bool((got[:copies * bytes_of].view(copies, -1) == alone[:bytes_of]).all())
+        assert bool((got[copies * bytes_of:copies * bytes_of * 9 // 8].view(copies, -1) == alone[bytes_of:bytes_of * 9 // 8]).all())
+
+
 @pytest.mark.parametrize("recipe", ["blockwise_fp8", "mxfp8", "nvfp4"])
 def test_a_nan_in_the_matrices_reaches_the_product(ops, recipe):
     from dew_amd import projections
