@@ -113,6 +113,30 @@ def test_the_input_gradient_is_the_recipes_own_product(ops, mx):
     assert (bf16_np(d_x) == want_x).mean() > 0.97 and (bf16_np(d_w) == want_w).mean() > 0.97
 
 
+@pytest.mark.parametrize("mx", [False, True], ids=["fp8", "mxfp8"])
+def test_a_cotangent_that_lies_otherwise_has_the_same_gradients(ops, mx):
+    """A transposed or strided cotangent is copied; one that begins off 16 bytes is refused, as its rows' quantizer alone refuses it."""
+    from dew_amd import projections
+
+    blocks, depth, width = (1, 0, 2, 1), 256, 384
+    tokens = 128 * sum(blocks)
+    x, dy = tokens_case(tokens, depth, seed=1).cuda(), tokens_case(tokens, width, seed=2).cuda()
+    w = tokens_case(len(blocks) * depth, width, seed=3).cuda().view(len(blocks), depth, width)
+    mirror = projections.mxfp8_gradients if mx else projections.blockwise_fp8_gradients
+    want = mirror(x, w, dy, blocks)
+    wider = torch.zeros((tokens, width + 8), dtype=torch.bfloat16, device="cuda")
+    wider[:, 4:width + 4] = dy                                       # rows 8 bytes off
+    for lies in (dy.T.contiguous().T, wider[:, 4:width + 4], dy[:, None].expand(-1, 2, -1)[:, 1]):
+        got = mirror(x, w, lies, blocks)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    flat = torch.zeros(tokens * width + 1, dtype=torch.bfloat16, device="cuda")
+    flat[1:] = dy.flatten()
+    with pytest.raises(ops.KernelError):
+        mirror(x, w, flat[1:].view(tokens, width), blocks)
+    with pytest.raises((ops.KernelError, ValueError)):
+        mirror(x, w, dy.float(), blocks)
+
+
 # ---- bf16 operands: the reference's gemm_t, and the NVFP4 recipe's kernel gradient ------------------------------
 
 

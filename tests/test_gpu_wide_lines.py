@@ -1,5 +1,6 @@
 """256 x 256 tiles on the lines from which they are taken: so few that half of the blocks have none, and a second round just begun. The
-comparisons are those of test_gpu_wide.py and test_gpu_wide_fp8.py, with the launches of smaller tiles (the same bits)."""
+comparisons are those of test_gpu_wide.py and test_gpu_wide_fp8.py, with the launches of smaller tiles (the same bits; a bf16 gradient's is the
+one of as many groups that each has fewer than 256 rows) and of gradients with products in fp32."""
 
 import pytest
 import test_gpu_wide
@@ -37,7 +38,7 @@ def test_products_in_quarters(monkeypatch, depth, sizes, width):
 
 
 @pytest.mark.parametrize("out_dtype", (torch.bfloat16, torch.float32))
-@pytest.mark.parametrize("sizes,depth,width", (([600, 513, 1, 800], 264, 1032), ([2000, 1100], 1032, 2568), ([700, 800], 2056, 4104), ([1500, 900], 2504, 4400),
+@pytest.mark.parametrize("sizes,depth,width", (([600, 513, 1, 800], 264, 1032), ([3000, 1800], 1032, 2568), ([700, 800], 2056, 4104), ([1500, 900], 2504, 4400),
                                                ([1348], 2624, 1496), ([600, 1513, 0, 1], 576, 1416)))     # (66 tiles, 252 real quarters; 72, 240)
 def test_gradients_in_quarters(sizes, depth, width, out_dtype):
     test_gpu_wide.test_gradients(sizes, depth, width, out_dtype)
