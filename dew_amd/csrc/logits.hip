@@ -1,10 +1,10 @@
-// Router gate logits: logits[t, e] = sum_d f32(x[t, d]) * kernel[d, e] in IEEE fp32
+// Router gate logits: logits[t, e] = sum_d f32(x[t, d]) * kernel[d, e], products exact in fp32 and summed in fp32
 // (reference src/dew/nn/moe.py:526-534: tokens widened to fp32, Precision.HIGHEST), and group offsets.
 // Depths in whole 16s run on the matrix unit, the fp32 gate as three bf16 terms (below): a block takes 32 (or 64) tokens and up to
 // four 32-expert tiles, its wavefronts a share of the depth each; the partial sums of a tile meet in LDS in wavefront order, so the
 // result does not depend on timing. A decode step's few tokens take 16 x 16 tiles of the fp32 instruction (v_mfma_f32_16x16x4_f32),
 // four times the blocks: 64 tokens of GPT-OSS's 2880 x 32 gate in about 5 us. Depths in no whole 16s take the plain kernel below (a
-// 64-token x 64-expert tile, 16-deep LDS steps, fp32 FMA; 1.3 ms for 8192 tokens of a 7168 x 256 gate, where the terms take 99 us).
+// 64-token x 64-expert tile, 16-deep LDS steps, fp32 FMA; 1.3 ms for 8192 tokens of a 7168 x 256 gate, where the terms take 102 us).
 #include <mutex>
 
 #include "common.h"
@@ -347,8 +347,10 @@ constexpr int kShares = kLogitShares;  // the depth's shares, one a wavefront
 // 2048 tokens of a 512 x 8 gate 49.4 us, 48.5 with them).
 static bool short_shares(int depth) { return depth < 1024; }
 
-// 32 x 32 tiles few enough that sixteen shares of the depth spread them over the CUs. (Few experts' shares are few bytes: a layer of 4096
-// tokens and 8 experts leaves them too.)
+// 32 x 32 tiles few enough that sixteen shares of the depth spread them over the CUs. Past 2048 tokens only few experts', whose shares are few
+// bytes: a layer's pass (us, finished logits and shares) of 7168 deep gates: 2100 tokens of 8 experts, 66 tiles, 159 and 147, 4096, 128, 258 and 251, 4500, 141, 266
+// and 264, 6000, 188, 306 and 307, 8192 294 and 298; of 32 experts, 4096 tokens 229 and 221, 8000 355 and 360; of 512 deep ones of 8 experts 128 tiles 43.7 and
+// 42.3, of 32 experts 40.6 and 41.9; of 64 experts, 132 tiles, 7168 deep 200 and 190, 512 deep 39.6 and 41.9.
 static bool share_tiles(int tokens, int experts) {
   const long long tiles = static_cast<long long>((tokens + 31) / 32) * ((experts + 31) / 32);
   return tokens <= 2048 ? tiles < 112 : experts <= 32 && tiles <= 128;
@@ -566,10 +568,9 @@ extern "C" int dew_moe_router_logits(const void* x, const float* kernel, const f
       static_cast<const bf16_t*>(x), kernel, bias, logits, tokens, depth, experts, s)
     auto blocks = [&](int rows, int beside) { return static_cast<long long>((tokens + 32 * rows - 1) / (32 * rows)) * ((tiles + beside - 1) / beside); };
     // The largest tile that still gives most CUs a block: it reads x and the gate least often and splits a gate value for most rows.
-    // Measured (us; rows x tiles): 8192 x 7168 x 256 (256 blocks of 2 x 4) 104, in 2 x 2 129; 4096 x 7168 x 256 (256 of 2 x 2) 67, in
-    // 2 x 4 86; 3000 x 4096 x 256 (188 of 2 x 2) 42, in 2 x 1 49; 2112 x 7168 x 160 (165 of 2 x 1) 45, in 2 x 2 64, in 1 x 1 49; 5000 x
-    // 7168 x 32 (157 of 1 x 1) 35, in 2 x 1 50. Up to 2048 tokens eight wavefronts, whose shorter sums keep the error below the fp32
-    // instruction's on sixteen: 2048 x 7168 x 256 45 in 2 x 1, 88 there.
+    // us, by 2 x 4, 2 x 2, 2 x 1 and 1 x 1 (rows x tiles, four wavefronts): 8192 x 7168 x 256 (256 blocks of 2 x 4) 101, 141, 168, 207; 4096 x 7168 x 256 (256 of
+    // 2 x 2) 87, 69, 84, 102; 3000 x 4096 x 256 (188 of 2 x 2) 49, 41, 50, 48; 2112 x 7168 x 160 (165 of 2 x 1) 80, 61, 41, 51; 5000 x 7168 x 32 (157 of 1 x 1) 81,
+    // 67, 48, 35. Up to 2048 tokens eight wavefronts, whose shorter sums keep the error below the fp32 instruction's on sixteen.
     if (share_tiles(tokens, experts)) {  // (whose sums a layer's shares are)
       if (short_shares(depth)) DEW_LOGITS(1, 1, 16, 1, 2);
       else DEW_LOGITS(1, 1, 16, 1, 4);

@@ -156,8 +156,9 @@ int dew_moe_route_blocks(const dew_moe_router* router /* host */, const float* l
 int dew_moe_balance_bias(const int32_t* counts /* [E] */, float* bias /* [E], updated in place */, float rate,
                          int32_t experts, void* stream);
 
-/* Gate logits (src/dew/nn/moe.py:526-534): logits[T,E] = f32(x[T,D] bf16) @ kernel[D,E] f32, IEEE fp32, plus
- * bias[E] where the router has one (GPT-OSS's, src/dew/nn/gpt_oss.py:163-165).                              */
+/* Gate logits (src/dew/nn/moe.py:526-534): logits[T,E] = f32(x[T,D] bf16) @ kernel[D,E] f32, plus bias[E] where the router
+ * has one (GPT-OSS's, src/dew/nn/gpt_oss.py:163-165). Every product is exact in fp32; sums are fp32 ones, those of 16 products cut off
+ * inside the matrix instruction where more than a decode step's tokens take it.                            */
 int dew_moe_router_logits(const void* x /* bf16 [T,D] */, const float* kernel /* [D,E] */,
                           const float* bias /* nullable [E] */, float* logits /* [T,E] */, int32_t tokens,
                           int32_t depth, int32_t experts, void* stream);
