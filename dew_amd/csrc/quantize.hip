@@ -16,87 +16,98 @@ namespace dew {
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
-constexpr int kQuantizeWaves = 4;  // rows per 256-thread block
+constexpr int kQuantizeWaves = 4;  // wavefronts a 256-thread block
 
-__global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_fp8_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes,
-                                                                              uint8_t* __restrict__ scales, int rows, int depth,
-                                                                              int pitch) {
-  const int lane = threadIdx.x % 64;
-  const int row = blockIdx.x * kQuantizeWaves + threadIdx.x / 64;
-  if (row >= rows) return;
-  const bf16_t* source = x + static_cast<size_t>(row) * depth;
-  uint8_t* target = codes + static_cast<size_t>(row) * depth;
-  // a lane takes 8 consecutive depths, 16 lanes a tile of 128, four tiles a pass of the wavefront
-  for (int chunk = lane; chunk < depth / 8; chunk += 64) {
-    const u32x4_t words = *reinterpret_cast<const u32x4_t*>(source + chunk * 8);
-    float v[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = __uint_as_float(words[i] << 16);
-      v[2 * i + 1] = __uint_as_float(words[i] & 0xFFFF0000u);
-    }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-#pragma unroll
-    for (int offset = 1; offset < 16; offset <<= 1) amax = fmaxf(amax, __shfl_xor(amax, offset, 64));
-    const uint32_t bits = __float_as_uint(fmaxf(amax, 1e-4f) * 0x1.24924ap-9f);  // f32(1 / 448)
-    const uint32_t field = min(max((bits >> 23) + ((bits & 0x7FFFFFu) != 0u ? 1u : 0u), 1u), 253u);
-    const float inverse = __uint_as_float((254u - field) << 23);  // 1 / scale, exactly
-    uint32_t packed[2];
-#pragma unroll
-    for (int w = 0; w < 2; ++w) {
-      packed[w] = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * w] * inverse, v[4 * w + 1] * inverse, 0, false);
-      packed[w] = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * w + 2] * inverse, v[4 * w + 3] * inverse, packed[w], true);
-    }
-    // depths 8 chunk .. 8 chunk + 7 of the row: eighth `within` of their 128-deep tile's sixteen
-    const int within = chunk % 16, half = within / 8, piece = (within % 8) / 4, group = (within % 4) / 2, low = within % 2;
-    *reinterpret_cast<u32x2_t*>(target + (chunk / 16) * 128 + 16 * (4 * group + 2 * half + piece) + 8 * low) = u32x2_t{packed[0], packed[1]};
-    if (within == 0) scales[static_cast<size_t>(row) * pitch + chunk / 16] = static_cast<uint8_t>(field);
-  }
+// What eight neighbouring lanes hold, taken together by `both` (which lane holds what must not matter).
+template <class Both>
+__device__ __forceinline__ uint32_t over_eight(uint32_t v, Both both) {
+  v = both(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true)));   // quad_perm 1 0 3 2
+  v = both(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true)));   // quad_perm 2 3 0 1
+  return both(v, static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true)));  // row_half_mirror
 }
 
-// The MXFP8 recipe's rows (OCP MX; reference src/dew/nn/kernels/formats.py:186-229): e4m3 codes under one E8M0 scale
+// MX: the MXFP8 recipe's rows (OCP MX; reference src/dew/nn/kernels/formats.py:186-229): e4m3 codes under one E8M0 scale
 // every 32 depths, the scale 2 to the largest magnitude's binary exponent less 8 (its fp32 exponent field less 8 is
 // the byte; a block of zeros, or one whose largest magnitude lies under 2^-119, takes byte 0), each value over its
 // scale rounded to e4m3, ties to even, saturating at +-448. Codes in the same operand order as above; the scale
 // bytes in depth order, depth / 32 a row (a 128-deep step's four bytes are one aligned dword).
-__global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_mxfp8_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes,
-                                                                                uint8_t* __restrict__ scales, int rows, int depth) {
-  const int lane = threadIdx.x % 64;
-  const int row = blockIdx.x * kQuantizeWaves + threadIdx.x / 64;
-  if (row >= rows) return;
-  const bf16_t* source = x + static_cast<size_t>(row) * depth;
-  uint8_t* target = codes + static_cast<size_t>(row) * depth;
-  for (int chunk = lane; chunk < depth / 8; chunk += 64) {  // 8 depths a lane, 4 lanes a block of 32
-    const u32x4_t words = *reinterpret_cast<const u32x4_t*>(source + chunk * 8);
-    float v[8];
+//
+// Rows are whole 128s, so the operand is one run of 128-deep tiles: eight lanes a tile, 16 depths each, which are 16 bytes of the operand
+// order, ITEMS such pieces a lane with all their loads in flight: two where that leaves four blocks a CU, more gave nothing. Bound by memory, 2 bytes read
+// and 1 written an element. (A wavefront a row, 8 depths a lane, had one load in flight and stored 8 bytes.) Measured (us, FP8, operands that the last-level
+// cache holds and ones it has lost): 4096 x 2048 4.7 and 8.8 -> 4.1 and 5.8, 8192 x 4096 16.5 and 27.6 -> 15.5 and 25.1, 32 768 x 7168 136 and 159 -> 124 and 149 (5.7 TB/s).
+template <bool MX, int ITEMS>
+__global__ __launch_bounds__(64 * kQuantizeWaves) void quantize_rows_kernel(const bf16_t* __restrict__ x, uint8_t* __restrict__ codes, uint8_t* __restrict__ scales,
+                                                                          long long pieces, uint32_t row_tiles, uint32_t pitch) {
+  const long long first = static_cast<long long>(blockIdx.x) * (64 * kQuantizeWaves * ITEMS) + threadIdx.x;
+  u32x4_t words[ITEMS][2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = __uint_as_float(words[i] << 16);
-      v[2 * i + 1] = __uint_as_float(words[i] & 0xFFFF0000u);
+  for (int k = 0; k < ITEMS; ++k) {
+    const u32x4_t* source = reinterpret_cast<const u32x4_t*>(x) + 2 * min(first + 64 * kQuantizeWaves * k, pieces - 1);
+    words[k][0] = source[0];
+    words[k][1] = source[1];
+  }
+#pragma unroll
+  for (int k = 0; k < ITEMS; ++k) {
+    const long long piece = first + 64 * kQuantizeWaves * k;
+    if (piece >= pieces) return;  // (eight lanes of a tile together)
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      v[2 * i] = __uint_as_float(words[k][i / 4][i % 4] << 16);
+      v[2 * i + 1] = __uint_as_float(words[k][i / 4][i % 4] & 0xFFFF0000u);
     }
-    float largest = 0.0f;
+    float most = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) largest = fmaxf(largest, fabsf(v[i]));
-    largest = fmaxf(largest, __shfl_xor(largest, 1, 64));
-    largest = fmaxf(largest, __shfl_xor(largest, 2, 64));
-    const int field = static_cast<int>(__float_as_uint(largest) >> 23);  // 0 for a zero or subnormal magnitude
-    const uint32_t byte = static_cast<uint32_t>(min(max(field - 8, 0), 254));
-    const float inverse = __uint_as_float((254u - byte) << 23);  // 2^(127 - byte), exactly (byte <= 247 for finite rows)
-    uint32_t packed[2];
+    for (int i = 0; i < 16; ++i) most = fmaxf(most, fabsf(v[i]));
+    const int within = threadIdx.x % 8;
+    const uint32_t tile = static_cast<uint32_t>(piece / 8);
+    uint32_t byte;
+    if constexpr (MX) {
+      most = fmaxf(most, __uint_as_float(__builtin_amdgcn_mov_dpp(__float_as_uint(most), 0xB1, 0xF, 0xF, true)));
+      byte = static_cast<uint32_t>(min(max(static_cast<int>(__float_as_uint(most) >> 23) - 8, 0), 254));  // (0 for a zero or subnormal magnitude; <= 247 for finite rows)
+      const uint32_t four = over_eight(byte << (8 * (within / 2)), [](uint32_t a, uint32_t b) { return a | b; });
+      if (within == 0) reinterpret_cast<uint32_t*>(scales)[tile] = four;
+    } else {
+      // (a magnitude's bits order as it does, and none here is a NaN: fmaxf left it out)
+      most = __uint_as_float(over_eight(__float_as_uint(most), [](uint32_t a, uint32_t b) { return max(a, b); }));
+      const uint32_t bits = __float_as_uint(fmaxf(most, 1e-4f) * 0x1.24924ap-9f);  // f32(1 / 448)
+      byte = min(max((bits >> 23) + ((bits & 0x7FFFFFu) != 0u ? 1u : 0u), 1u), 253u);
+      if (within == 0) scales[static_cast<size_t>(tile / row_tiles) * pitch + tile % row_tiles] = static_cast<uint8_t>(byte);
+    }
+    const float inverse = __uint_as_float((254u - byte) << 23);  // 1 / scale, exactly
+    u32x4_t packed;
 #pragma unroll
-    for (int w = 0; w < 2; ++w) {
+    for (int w = 0; w < 4; ++w) {
       float q[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) q[i] = fminf(fmaxf(v[4 * w + i] * inverse, -448.0f), 448.0f);
+      for (int i = 0; i < 4; ++i) {
+        q[i] = v[4 * w + i] * inverse;
+        if (MX) q[i] = fminf(fmaxf(q[i], -448.0f), 448.0f);
+      }
       packed[w] = __builtin_amdgcn_cvt_pk_fp8_f32(q[0], q[1], 0, false);
       packed[w] = __builtin_amdgcn_cvt_pk_fp8_f32(q[2], q[3], packed[w], true);
     }
-    const int within = chunk % 16, half = within / 8, piece = (within % 8) / 4, group = (within % 4) / 2, low = within % 2;
-    *reinterpret_cast<u32x2_t*>(target + (chunk / 16) * 128 + 16 * (4 * group + 2 * half + piece) + 8 * low) = u32x2_t{packed[0], packed[1]};
-    if (chunk % 4 == 0) scales[static_cast<size_t>(row) * (depth / 32) + chunk / 4] = static_cast<uint8_t>(byte);
+    const int half = within / 4, low = within % 4 / 2, group = within % 2;
+    *reinterpret_cast<u32x4_t*>(codes + static_cast<size_t>(tile) * 128 + 16 * (4 * group + 2 * half + low)) = packed;
   }
+}
+
+template <bool MX>
+static int quantize_rows(const char* who, const void* x, void* codes, uint8_t* scales, int rows, int depth, void* stream) {
+  DEW_REQUIRE(rows >= 0 && depth >= 128 && depth % 128 == 0, "%s: rows %d, depth %d (whole 128s)", who, rows, depth);
+  if (rows == 0) return DEW_MOE_OK;
+  DEW_REQUIRE(x && codes && scales, "%s: x, codes and scales must not be null", who);
+  DEW_REQUIRE(aligned16(x) && aligned16(codes) && aligned16(scales), "%s: x, codes and scales must be 16-byte aligned", who);
+  constexpr int kMany = 2, kThreads = 64 * kQuantizeWaves;
+  const long long pieces = static_cast<long long>(rows) * depth / 16;
+  const bool many = pieces >= 4ll * 256 * kThreads * kMany;
+  const long long blocks = (pieces + kThreads * (many ? kMany : 1) - 1) / (kThreads * (many ? kMany : 1));
+  DEW_REQUIRE(blocks < (1ll << 31) && pieces / 8 < (1ll << 32), "%s: %d rows of %d", who, rows, depth);
+  hipLaunchKernelGGL((many ? quantize_rows_kernel<MX, kMany> : quantize_rows_kernel<MX, 1>), dim3(static_cast<unsigned>(blocks)), dim3(kThreads), 0,
+                     static_cast<hipStream_t>(stream), static_cast<const bf16_t*>(x), static_cast<uint8_t*>(codes), scales, pieces,
+                     static_cast<uint32_t>(depth / 128), static_cast<uint32_t>((depth / 128 + 15) / 16 * 16));
+  return launched("quantize_rows_kernel");
 }
 
 // The NVFP4 recipe's rows (reference src/dew/nn/kernels/formats.py:263-274 over src/dew/algebra/bits.py:941-982):
@@ -306,8 +317,8 @@ __global__ __launch_bounds__(256) void nvfp4_largest_kernel(const u32x4_t* __res
 // A kernel gradient's operands: x [tokens, dim] quantized ALONG THE TOKENS and written transposed, for the product
 // that contracts each group's tokens (reference src/dew/nn/kernels/projections.py:211-224 `rows_quantized(x.T)`, and
 // :263-275 `MxFp8.quantized(x.T)`). MX false: the blockwise FP8 recipe's 1 x 128 tiles (128 tokens of one column under
-// the scale rule of quantize_rows_fp8_kernel, its byte written for each of the tile's four 32-token blocks); MX true: OCP
-// MX blocks of 32 tokens (quantize_rows_mxfp8_kernel's rule).
+// the scale rule of quantize_rows_kernel, its byte written for each of the tile's four 32-token blocks); MX true: OCP
+// MX blocks of 32 tokens (its MX rule).
 //
 // As the lhs_t operand, rows of tokens: codes [dim, tokens] in the row operand's order within each 128 tokens (see the head of this
 // file) and scales [dim, tokens / 32]. A block takes 128 tokens x 64 columns through the LDS: thread (column c, quarter a) owns the
@@ -377,7 +388,7 @@ __global__ __launch_bounds__(256) void quantize_columns_kernel(const bf16_t* __r
 // As the rhs_t operand (or either operand of the launch that takes two such), a prepared MXFP8 bank of one expert, depth = tokens, width =
 // dim: codes as 32 column x 32 token atoms [dim / 32][tokens / 32][64 lanes][16 bytes] (lane 32 g + c holds tokens 16 g .. 16 g + 15 of
 // column c) and scales [dim / 32][tokens / 128][32 columns][4 bytes]; and, ROWS, along its rows too from the same read, which the
-// cotangent's other product takes (quantize_rows_fp8_kernel's and quantize_rows_mxfp8_kernel's bytes). A block takes 128 tokens x 128
+// cotangent's other product takes (quantize_rows_kernel's bytes). A block takes 128 tokens x 128
 // columns: eight neighbours of a row a thread as they arrive, for the rows; then, through the LDS, 16 tokens of two neighbouring columns,
 // whose codes are 32 bytes of an atom. Every XCD's blocks walk along the columns of its own tokens, so that the few bytes of scales that a
 // block writes of a row meet in that XCD's L2. HBM-bound: 2 bytes read and 1 (ROWS: 2) written an element, at 4.8 to 5.8 TB/s. Measured (us): a
@@ -796,25 +807,9 @@ extern "C" int dew_moe_quantize_nvfp4(const void* x, const uint32_t* largest, vo
 }
 
 extern "C" int dew_moe_quantize_rows_mxfp8(const void* x, void* codes, uint8_t* scales, int32_t rows, int32_t depth, void* stream) {
-  using namespace dew;
-  DEW_REQUIRE(rows >= 0 && depth >= 128 && depth % 128 == 0, "dew_moe_quantize_rows_mxfp8: rows %d, depth %d (whole 128s)", rows, depth);
-  if (rows == 0) return DEW_MOE_OK;
-  DEW_REQUIRE(x && codes && scales, "dew_moe_quantize_rows_mxfp8: x, codes and scales must not be null");
-  DEW_REQUIRE(aligned16(x) && aligned16(codes) && aligned16(scales), "dew_moe_quantize_rows_mxfp8: x, codes and scales must be 16-byte aligned");
-  hipLaunchKernelGGL(quantize_rows_mxfp8_kernel, dim3((rows + kQuantizeWaves - 1) / kQuantizeWaves), dim3(64 * kQuantizeWaves), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const bf16_t*>(x), static_cast<uint8_t*>(codes), scales, rows, depth);
-  return launched("quantize_rows_mxfp8_kernel");
+  return dew::quantize_rows<true>("dew_moe_quantize_rows_mxfp8", x, codes, scales, rows, depth, stream);
 }
 
 extern "C" int dew_moe_quantize_rows_fp8(const void* x, void* codes, uint8_t* scales, int32_t rows, int32_t depth, void* stream) {
-  using namespace dew;
-  DEW_REQUIRE(rows >= 0 && depth >= 128 && depth % 128 == 0, "dew_moe_quantize_rows_fp8: rows %d, depth %d (whole 128s)", rows, depth);
-  if (rows == 0) return DEW_MOE_OK;
-  DEW_REQUIRE(x && codes && scales, "dew_moe_quantize_rows_fp8: x, codes and scales must not be null");
-  DEW_REQUIRE(aligned16(x) && aligned16(codes) && aligned16(scales), "dew_moe_quantize_rows_fp8: x, codes and scales must be 16-byte aligned");
-  const int pitch = (depth / 128 + 15) / 16 * 16;
-  hipLaunchKernelGGL(quantize_rows_fp8_kernel, dim3((rows + kQuantizeWaves - 1) / kQuantizeWaves), dim3(64 * kQuantizeWaves), 0,
-                     static_cast<hipStream_t>(stream), static_cast<const bf16_t*>(x), static_cast<uint8_t*>(codes), scales, rows, depth,
-                     pitch);
-  return launched("quantize_rows_fp8_kernel");
+  return dew::quantize_rows<false>("dew_moe_quantize_rows_fp8", x, codes, scales, rows, depth, stream);
 }

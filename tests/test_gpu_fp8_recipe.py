@@ -156,6 +156,18 @@ def test_mxfp8_rows_are_quantized_bit_for_bit(ops, rows, depth):
     assert np.array_equal(ops.depth_order_fp8(codes).cpu().numpy(), oracle.e4m3_bytes(want_values))
 
 
+@pytest.mark.parametrize("mx", [False, True])
+@pytest.mark.parametrize("rows,depth", [(6, 128), (2047, 4096), (2049, 4096)])
+def test_rows_on_either_side_of_two_pieces_a_lane_are_quantized_bit_for_bit(ops, rows, depth, mx):
+    """One 128-deep tile a row, a block's last lanes without a piece, and, from 2^23 elements on, two pieces a lane whose last block is part full."""
+    x = rows_case(rows, depth, seed=rows)
+    codes, scales = (ops.quantize_rows_mxfp8 if mx else ops.quantize_rows_fp8)(x.cuda())
+    want_values, want_scales = (oracle.mxfp8_quantized if mx else oracle.rows_quantized)(bf16_np(x))
+    got_scales = scales.cpu().numpy()[:, :want_scales.shape[1]]
+    assert np.array_equal(got_scales if mx else np.ldexp(np.float32(1), got_scales.astype(np.int32) - 127), want_scales)
+    assert np.array_equal(ops.depth_order_fp8(codes).cpu().numpy(), oracle.e4m3_bytes(want_values))
+
+
 @pytest.mark.parametrize("label,sizes", SIZES, ids=[s[0] for s in SIZES])
 @pytest.mark.parametrize("depth,width", [(256, 128), (1152, 384), (512, 512)])
 def test_the_mxfp8_product_matches_the_oracle(ops, label, sizes, depth, width):
