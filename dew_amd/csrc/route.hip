@@ -47,36 +47,83 @@ __device__ __forceinline__ float wave_max(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
-// Sum rounded once: fp64 partials per lane, then a butterfly; every lane ends with the same value.
+// Sum rounded once: fp64 partials per lane, then a butterfly over lanes 32, 16, 8, 4, 2 and 1 apart; every lane ends with the same value.
+// (Both halves of a swap are added where a lane would add its own and the other's, and once lanes 8 apart hold the same, four lanes on in a
+// row of 16 is four apart: the same additions as exchanges through the LDS crossbar, without its six round trips.)
 __device__ __forceinline__ float wave_sum_once(double v) {
-#pragma unroll
-  for (int offset = 32; offset >= 1; offset >>= 1) v = v + __shfl_xor(v, offset, kWave);
+  auto words = [](double value) { return __builtin_bit_cast(uint64_t, value); };
+  auto of = [](uint32_t low, uint32_t high) { return __builtin_bit_cast(double, static_cast<uint64_t>(high) << 32 | low); };
+  {
+    const uint32_t low = static_cast<uint32_t>(words(v)), high = static_cast<uint32_t>(words(v) >> 32);
+    const auto lows = __builtin_amdgcn_permlane32_swap(low, low, false, false), highs = __builtin_amdgcn_permlane32_swap(high, high, false, false);
+    v = of(lows[0], highs[0]) + of(lows[1], highs[1]);
+  }
+  {
+    const uint32_t low = static_cast<uint32_t>(words(v)), high = static_cast<uint32_t>(words(v) >> 32);
+    const auto lows = __builtin_amdgcn_permlane16_swap(low, low, false, false), highs = __builtin_amdgcn_permlane16_swap(high, high, false, false);
+    v = of(lows[0], highs[0]) + of(lows[1], highs[1]);
+  }
+  auto add_moved = [&](auto control) {
+    const uint32_t low = static_cast<uint32_t>(words(v)), high = static_cast<uint32_t>(words(v) >> 32);
+    v = v + of(__builtin_amdgcn_mov_dpp(low, decltype(control)::value, 0xF, 0xF, true), __builtin_amdgcn_mov_dpp(high, decltype(control)::value, 0xF, 0xF, true));
+  };
+  add_moved(std::integral_constant<int, 0x128>{});  // row_ror 8
+  add_moved(std::integral_constant<int, 0x124>{});  // row_ror 4
+  add_moved(std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  add_moved(std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
   return static_cast<float>(v);
 }
 
-struct Best {
-  float value;
-  int index;
-};
-
-__device__ __forceinline__ bool better(float v, int i, const Best& than) {
-  return v > than.value || (v == than.value && i < than.index);
+// A float as an unsigned key of the same order (-inf lowest of the non-NaN), never 0.
+__device__ __forceinline__ uint32_t ordered_key(float v) {
+  const uint32_t bits = __float_as_uint(v);
+  return (bits & 0x80000000u) ? ~bits : bits | 0x80000000u;
 }
 
-// The wavefront's best (value, index): the largest value by a butterfly of maxima, then the lowest index among the
-// lanes that hold it. Almost always one lane does, found by a ballot and read with one cross-lane move; ties walk
-// the ballot's set bits. Half the cross-lane traffic of reducing value and index together.
-__device__ __forceinline__ Best wave_best(Best b) {
-  const float top = wave_max(b.value);
-  unsigned long long holders = __ballot(b.value == top);
-  Best best;
-  best.value = top;
-  best.index = 0x7fffffff;
-  while (holders != 0ull) {
-    const int lane = __builtin_ctzll(holders);
-    best.index = min(best.index, __builtin_amdgcn_readlane(b.index, lane));
-    holders &= holders - 1ull;
+__device__ __forceinline__ float from_ordered_key(uint32_t key) {
+  if (key == 0u) return -__builtin_inff();  // no token wrote here
+  return __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);
+}
+
+// A selection as it competes: by its value, either zero the same, NaN as -inf; 0, below them all, is none.
+__device__ __forceinline__ uint32_t competing_key(float v) { return ordered_key(v == v ? v + 0.0f : -__builtin_inff()); }
+
+// The wavefront's largest key, the same register in every lane: as wave_max, an instruction a move.
+__device__ __forceinline__ uint32_t wave_max_key(uint32_t v) {
+  auto moved = [](uint32_t value, auto control, auto rows) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, value, decltype(control)::value, decltype(rows)::value, 0xF, false));
+  };
+  using std::integral_constant;
+  v = max(v, moved(v, integral_constant<int, 0xB1>{}, integral_constant<int, 0xF>{}));   // quad_perm [1,0,3,2]
+  v = max(v, moved(v, integral_constant<int, 0x4E>{}, integral_constant<int, 0xF>{}));   // quad_perm [2,3,0,1]
+  v = max(v, moved(v, integral_constant<int, 0x141>{}, integral_constant<int, 0xF>{}));  // row_half_mirror
+  v = max(v, moved(v, integral_constant<int, 0x140>{}, integral_constant<int, 0xF>{}));  // row_mirror
+  v = max(v, moved(v, integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{}));  // row_bcast15 into rows 1, 3
+  v = max(v, moved(v, integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{}));  // row_bcast31 into rows 2, 3
+  return static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), 63));
+}
+
+// The best of the wavefront's keys (key[i] of a lane is number lane + 64 i), ties to the lower number, taken out: its number, the same
+// register in every lane. One of them is not 0.
+// Bound by its chain: seven vector instructions one after another, a ballot a register and scalar ones. As values and numbers compared lane by
+// lane before a butterfly of float maxima (four instructions a move) a round of 128 experts took some 0.4 us, a wavefront alone on its SIMD. A launch's us with
+// that, sums through the LDS crossbar and a round trip of the gate's shares for every 64 experts, and now: one token of 128 experts, top 8, sorted too
+// 6.5 -> 4.7, 64 tokens 5.9 -> 4.6, 1111 of 64, top 6, 5.75 -> 5.05, 2048 of 8, top 2, 5.0 -> 4.4, 8192 of 256 in 8 groups, top 8, 30 -> 27.
+template <int kCount>
+__device__ __forceinline__ int take_best(uint32_t (&key)[kCount]) {
+  const int lane = threadIdx.x % kWave;
+  uint32_t mine = key[0];
+#pragma unroll
+  for (int i = 1; i < kCount; ++i) mine = max(mine, key[i]);
+  const uint32_t top = wave_max_key(mine);
+  int best = 0;
+#pragma unroll
+  for (int i = kCount - 1; i >= 0; --i) {
+    const unsigned long long holders = __ballot(key[i] == top);
+    if (holders != 0ull) best = kWave * i + __builtin_ctzll(holders);
   }
+#pragma unroll
+  for (int i = 0; i < kCount; ++i) key[i] = lane + kWave * i == best ? 0u : key[i];
   return best;
 }
 
@@ -110,17 +157,6 @@ struct RouteParams {
   const float* gate_bias;  // nullable [E]
 };
 
-// A float as an unsigned key of the same order (-inf lowest of the non-NaN), never 0.
-__device__ __forceinline__ uint32_t ordered_key(float v) {
-  const uint32_t bits = __float_as_uint(v);
-  return (bits & 0x80000000u) ? ~bits : bits | 0x80000000u;
-}
-
-__device__ __forceinline__ float from_ordered_key(uint32_t key) {
-  if (key == 0u) return -__builtin_inff();  // no token wrote here
-  return __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);
-}
-
 // The block a token routes with: its row's blocks are numbered from 0, padding (or an id past the row) is block `length`.
 __device__ __forceinline__ size_t block_of(const RouteParams& p, int token) {
   const int id = p.blocks[token];
@@ -136,24 +172,33 @@ template <int kPerLane>
 __device__ __forceinline__ void read_logits(const RouteParams& p, int token, float (&logit)[kPerLane]) {
   const int lane = threadIdx.x % kWave;
   const float* row = p.logits + static_cast<size_t>(token) * p.experts;
+  if (p.shares) {
+    constexpr int kAtOnce = kPerLane < 4 ? kPerLane : 4;
 #pragma unroll
-  for (int i = 0; i < kPerLane; ++i) {
-    const int e = lane + kWave * i, at = min(e, p.experts - 1);
-    float value;
-    if (p.shares) {
-      float share[kLogitShares];
+    for (int first = 0; first < kPerLane; first += kAtOnce) {
+      float share[kAtOnce][kLogitShares];
+      auto expert = [&](int i) { return min(lane + kWave * (first + i), p.experts - 1); };
 #pragma unroll
-      for (int s = 0; s < kLogitShares; ++s) share[s] = row[static_cast<size_t>(s) * p.tokens * p.experts + at];
+      for (int i = 0; i < kAtOnce; ++i)
+#pragma unroll
+        for (int s = 0; s < kLogitShares; ++s) share[i][s] = row[static_cast<size_t>(s) * p.tokens * p.experts + expert(i)];
       __builtin_amdgcn_sched_barrier(0);  // (all of them asked for before the first is waited for)
-      value = share[0];
 #pragma unroll
-      for (int s = 1; s < kLogitShares; ++s) value += share[s];
-      if (p.gate_bias != nullptr) value = value + p.gate_bias[at];
-    } else {
-      value = row[at];
+      for (int i = 0; i < kAtOnce; ++i) {
+        float value = share[i][0];
+#pragma unroll
+        for (int s = 1; s < kLogitShares; ++s) value += share[i][s];
+        if (p.gate_bias != nullptr) value = value + p.gate_bias[expert(i)];
+        logit[first + i] = value;
+      }
     }
-    logit[i] = e < p.experts ? value : -__builtin_inff();
+  } else {
+#pragma unroll
+    for (int i = 0; i < kPerLane; ++i) logit[i] = row[min(lane + kWave * i, p.experts - 1)];
   }
+#pragma unroll
+  for (int i = 0; i < kPerLane; ++i)
+    if (lane + kWave * i >= p.experts) logit[i] = -__builtin_inff();
 }
 
 // One token of a wavefront, from its logits (expert lane + 64 i in logit[i], -inf past the experts) to its experts and weights:
@@ -277,18 +322,10 @@ __device__ __forceinline__ Chosen routed_token(const RouteParams& p, int token, 
       group_score = p.group_by_max ? first : first + second;
     }
     unsigned long long kept = 0ull;
-    bool taken = false;
+    uint32_t group_key[1] = {lane < p.expert_groups && group_score == group_score ? competing_key(group_score) : 0u};
     for (int round = 0; round < p.groups_per_token; ++round) {
-      Best b;
-      b.value = ninf;
-      b.index = 0x7fffffff;
-      if (lane < p.expert_groups && !taken) {
-        b.value = group_score;
-        b.index = lane;
-      }
-      b = wave_best(b);
-      kept |= 1ull << b.index;
-      if (b.index == lane) taken = true;
+      if (__ballot(group_key[0] != 0u) == 0ull) break;  // (a group whose two best are infinities of either sign has no score)
+      kept |= 1ull << take_best(group_key);
     }
 #pragma unroll
     for (int i = 0; i < kPerLane; ++i) {
@@ -303,7 +340,6 @@ __device__ __forceinline__ Chosen routed_token(const RouteParams& p, int token, 
   // src/dew/nn/moe.py:202-224) and its sort drops the slot. Its reads below go to the nearest expert, to stay in range.
   const bool replayed = p.given != nullptr && (p.covered == nullptr || p.covered[token] != 0);
   // top-k: k rounds of a wave-wide argmax, ties to the lower index
-  unsigned taken_mask = 0u;
   int my_choice = 0, given_id = 0;
   bool in_range = true;
   if (replayed && lane < p.top_k) {
@@ -311,21 +347,14 @@ __device__ __forceinline__ Chosen routed_token(const RouteParams& p, int token, 
     in_range = given_id >= 0 && given_id < p.experts;
     my_choice = min(max(given_id, 0), p.experts - 1);
   }
-  for (int round = 0; round < (replayed ? 0 : p.top_k); ++round) {
-    Best b;
-    b.value = ninf;
-    b.index = 0x7fffffff;
+  if (!replayed) {
+    uint32_t key[kPerLane];
 #pragma unroll
-    for (int i = 0; i < kPerLane; ++i) {
-      const int e = lane + kWave * i;
-      if (e < p.experts && !((taken_mask >> i) & 1u) && better(select[i], e, b)) {
-        b.value = select[i];
-        b.index = e;
-      }
+    for (int i = 0; i < kPerLane; ++i) key[i] = lane + kWave * i < p.experts ? competing_key(select[i]) : 0u;
+    for (int round = 0; round < p.top_k; ++round) {
+      const int best = take_best(key);
+      if (lane == round) my_choice = best;
     }
-    b = wave_best(b);
-    if ((b.index % kWave) == lane) taken_mask |= 1u << (b.index / kWave);
-    if (lane == round) my_choice = min(b.index, p.experts - 1);
   }
 
   // gate weights: lane j < k owns the j-th choice
@@ -349,8 +378,9 @@ __device__ __forceinline__ Chosen routed_token(const RouteParams& p, int token, 
       if (p.bias_in_weights) weight = weight + p.bias[my_choice];
     }
     if (p.normalize) {
-      float total = __shfl(weight, 0, kWave);
-      for (int j = 1; j < p.top_k; ++j) total = total + __shfl(weight, j, kWave);
+      auto of_lane = [&](int j) { return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight), j)); };
+      float total = of_lane(0);
+      for (int j = 1; j < p.top_k; ++j) total = total + of_lane(j);
       total = total + p.sum_epsilon;
       if (p.sum_min != 0.0f) total = fmaxf(total, p.sum_min);
       weight = weight / total;
@@ -381,7 +411,7 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
 // The router and the sort of up to sixteen tokens in one block: a wavefront routes a token and leaves its experts in the LDS,
 // where the whole block then sorts them. They are two launches of 4 to 5 us otherwise, most of either its own latency. (More
 // tokens, several a wavefront, are slower than two launches: some 750 instructions a token on one CU's four SIMDs.)
-// Measured, one token of 128 experts, top 8: 8.8 us with the sort that counts, 6.8 with the one of few slots.
+// Measured, one token of 128 experts, top 8: 8.8 us with the sort that counts, 6.8 with the one of few slots, 4.7 with rounds of keys (take_best).
 constexpr int kSortWaves = kSmallThreads / kWave;
 template <int kPerLane>
 __global__ __launch_bounds__(kSmallThreads) void route_and_sort_kernel(RouteParams p, PermuteParams sort) {
@@ -411,27 +441,16 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void block_shortlist_kernel(con
   const int lane = threadIdx.x % kWave;
   const int block = blockIdx.x * kRouteWaves + threadIdx.x / kWave;
   if (block >= blocks) return;
-  float best[kMaxPerLane];
+  uint32_t key[kMaxPerLane];
 #pragma unroll
   for (int i = 0; i < kMaxPerLane; ++i) {
     const int e = lane + kWave * i;
-    best[i] = e < experts ? from_ordered_key(keys[static_cast<size_t>(block) * experts + e]) : -__builtin_inff();
+    key[i] = e < experts ? competing_key(from_ordered_key(keys[static_cast<size_t>(block) * experts + e])) : 0u;
   }
   unsigned taken = 0u;
   for (int round = 0; round < count; ++round) {
-    Best b;
-    b.value = -__builtin_inff();
-    b.index = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < kMaxPerLane; ++i) {
-      const int e = lane + kWave * i;
-      if (e < experts && !((taken >> i) & 1u) && better(best[i], e, b)) {
-        b.value = best[i];
-        b.index = e;
-      }
-    }
-    b = wave_best(b);
-    if ((b.index % kWave) == lane) taken |= 1u << (b.index / kWave);
+    const int best = take_best(key);
+    if (best % kWave == lane) taken |= 1u << (best / kWave);
   }
   allowed[static_cast<size_t>(block) * kWave + lane] = static_cast<uint8_t>(taken);
 }

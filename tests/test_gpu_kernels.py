@@ -72,6 +72,23 @@ def test_router_matches_the_oracle_bit_for_bit(ops, name, experts, k, settings, 
     assert np.array_equal(got_w.cpu().numpy().view(np.uint32), want_w.view(np.uint32))
 
 
+@pytest.mark.parametrize("experts,k", [(1, 1), (63, 63), (64, 64), (65, 64), (129, 9), (257, 64), (512, 8)])
+def test_rounds_of_ties_infinities_and_either_zero_take_the_lower_expert(ops, experts, k):
+    """Selections of a few values only, infinities and a fill of -0.0 beside selections of 0 among them: every round's best is one of
+    many, in any of a lane's registers, and the last rounds find -inf alone. Powers of two, so the weights are exact as well."""
+    rng = np.random.default_rng(experts)
+    logits = np.zeros((130, experts), np.float32)
+    bias = rng.choice(np.array([-0.5, 0.0, 0.25, np.inf, -np.inf], np.float32), size=experts)   # (a score of 0.5: selections 0, 0.5, 0.75, +-inf)
+    for settings in (dict(), dict(expert_groups=8, groups_per_token=2, group_score="max", excluded_group_score=-0.0)):
+        if experts % settings.get("expert_groups", 1) or k > 2 * experts // settings.get("expert_groups", 2):
+            continue
+        settings = dict(settings, score_function="sigmoid", normalize_weights=False)
+        want_w, want_i = oracle.route(logits, k, bias=bias, **settings)
+        got_w, got_i = ops.route(torch.from_numpy(logits).cuda(), k, bias=torch.from_numpy(bias).cuda(), **settings)
+        assert np.array_equal(got_i.cpu().numpy(), want_i)
+        assert np.array_equal(got_w.cpu().numpy(), want_w)
+
+
 @pytest.mark.parametrize("fill", [0.0, 0.3, None])
 @pytest.mark.parametrize("experts,groups,kept,k,group_score", [(64, 8, 2, 8, "top2"), (256, 8, 1, 8, "top2"), (32, 4, 2, 6, "max")])
 def test_an_excluded_groups_experts_compete_at_the_score_filled_in(ops, experts, groups, kept, k, group_score, fill):
