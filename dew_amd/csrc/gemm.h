@@ -112,6 +112,26 @@ __device__ __forceinline__ void static_for(F&& f) {
   static_for_each(std::make_integer_sequence<int, N>{}, f);
 }
 
+constexpr int BK = 64;
+constexpr int kChunksPerRow = BK / 8;  // 16-byte chunks in an LDS row
+constexpr int kMaxDepthBlocks = 256;   // FP8 128 x 128 blocks: depth up to 32768
+
+// LDS index of 16-byte chunk `chunk` of row `row` (128-byte rows). The chunk is xor-swizzled by
+// f(row) = ((row >> 1) & 7) ^ ((row & 1) << 2), chosen against the measured service order of gfx950's LDS:
+// ds_read_b128 serves 16 lanes a pass over 64 banks, the passes being lanes {0-3,12-15,20-23,24-27},
+// {4-7,8-11,16-19,28-31} and the same + 32; ds_write_b128 serves 8 consecutive lanes a pass over 128 bytes.
+// With lane = row (mod 32) on the read side, f is injective on every read pass's rows of one parity, and a
+// store pass writes the 8 chunks of one row, so fragment reads and stores are conflict-free.
+__device__ __forceinline__ int swizzled(int row, int chunk) {
+  return row * kChunksPerRow + (chunk ^ (((row >> 1) & 7) ^ ((row & 1) << 2)));
+}
+
+// f(integral_constant<B>), f(integral_constant<B + 1>), ...: a loop whose index is a constant expression in its body.
+template <int B, int... Is, class F>
+__device__ __forceinline__ void static_range(std::integer_sequence<int, Is...>, F&& f) {
+  (f(std::integral_constant<int, B + Is>{}), ...);
+}
+
 // An inclusive sum over the lanes, by lane moves of the vector unit (a sixth of the time of as many trips through the LDS).
 __device__ __forceinline__ int lanes_scanned(int value) {
   value += __builtin_amdgcn_update_dpp(0, value, 0x111, 0xF, 0xF, false);  // row_shr:1
@@ -125,5 +145,8 @@ __device__ __forceinline__ int lanes_scanned(int value) {
 
 // The launch for few tiles of few rows (decode.hip); `mode`: kPlain, kSwigluOfTwo or kInterleavedGated.
 int launch_few_tiles(const char* who, const GemmParams& p, int format, int mode, hipStream_t stream);
+
+// The launch in tiles of up to 256 rows on eight wavefronts (tall.hip); of FP8 banks, one or two (gate and up, gated), or of one NVFP4 bank.
+int launch_tall(const char* who, const GemmParams& p, int format, bool paired, hipStream_t stream);
 
 }  // namespace dew
