@@ -64,21 +64,67 @@ __device__ __forceinline__ void clear_past_last(const GemmParams& p, int m_tile,
   }
 }
 
-template <int FORMAT, int MODE>
-__global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
+// The down product of a few tokens and their weighted sums as one launch (COMBINED): a block is a token's 32 output columns, a wavefront one of the
+// token's slots, whose row it multiplies as a tile of its own; the slots' rounded outputs meet in the LDS and are summed as the combine's
+// own launch sums them (combine.hip), so the bits are the two launches'. What bounds a step on small experts is its launches, one behind the
+// other, and the host that issues them: one of 2 to 3 us, and some 3 us of the host's, fall away (`combines_few`).
+struct CombineParams {
+  const float* weights;  // [tokens, top_k]
+  bf16_t* out;           // [tokens, width]
+  int tokens, top_k, shared;
+};
+
+// (each product and each sum rounded by itself)
+__device__ __forceinline__ float weighted_sum(const float* values, int pitch, const float* weights, int top_k) {
+#pragma clang fp contract(off)
+  float sum = 0.0f;
+  for (int j = 0; j < top_k; ++j) {
+    const float product = values[j * pitch] * weights[j];
+    sum = sum + product;
+  }
+  return sum;
+}
+
+// The tile of a slot's one row: its sorted position, and the group that holds it.
+__device__ __forceinline__ FewTile slot_tile(const GemmParams& p, int slot) {
+  const int lane = threadIdx.x % 64;
+  FewTile tile{0, 0, 0, 0, 0};
+  for (int base = 0; base < p.rows; base += 64) {
+    const unsigned long long hit = __ballot(base + lane < p.rows && p.scatter[min(base + lane, p.rows - 1)] == slot);
+    if (hit != 0ull) tile.row0 = base + __builtin_ctzll(hit);
+  }
+  for (int base = 0; base < p.experts; base += 64) {
+    const int e = min(base + lane, p.experts - 1);
+    const int begin = p.offsets[e], end = p.offsets[e + 1];
+    const unsigned long long hit = __ballot(base + lane < p.experts && tile.row0 >= begin && tile.row0 < end);
+    if (hit != 0ull) tile.expert = base + __builtin_ctzll(hit);
+  }
+  tile.end = tile.row0 + 1;
+  return tile;
+}
+
+template <int FORMAT, int MODE, bool COMBINED>
+__device__ __forceinline__ void few_tile_product(const GemmParams& p, const CombineParams& c) {
+  static_assert(!COMBINED || MODE == kPlain, "the down product");
   constexpr bool kPaired = MODE == kSwigluOfTwo, kGated = MODE == kInterleavedGated;
   constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4 || FORMAT == DEW_MOE_W_MXFP4, kBf16 = FORMAT == DEW_MOE_W_BF16;
   constexpr int kMatrices = kPaired ? 2 : 1;
   constexpr int kAtomK = kFp4 ? 64 : kBf16 ? 16 : 32, kAtoms = 64 / kAtomK;  // 16-byte loads a lane makes per matrix and 64 depths
   constexpr int kAhead = kMatrices * kAtoms >= 8 ? 4 : kMatrices * kAtoms >= 4 ? 6 : 8;  // steps of 64 depths in flight
-  const int lane = threadIdx.x;
-  const int strips = p.width / 32, m_tile = blockIdx.x / strips, strip = blockIdx.x % strips;
+  const int lane = COMBINED ? threadIdx.x % 64 : threadIdx.x, wave = COMBINED ? __builtin_amdgcn_readfirstlane(threadIdx.x / 64) : 0;
+  const int strips = p.width / 32, m_tile = blockIdx.x / strips /* COMBINED: the token */, strip = blockIdx.x % strips;
+  // (the shared expert's rows are the last slots)
+  const int slot = !COMBINED ? 0 : wave < c.top_k ? m_tile * c.top_k + wave : c.tokens * c.top_k + m_tile;
 
-  const FewTile tile = few_tile(p, m_tile);
+  FewTile tile;
+  if constexpr (COMBINED)
+    tile = slot_tile(p, slot);
+  else
+    tile = few_tile(p, m_tile);
   const int expert = tile.expert, row0 = tile.row0;
   const int out_width = kGated ? p.width / 2 : p.width;
   constexpr int kOutColumns = kGated ? 16 : 32;
-  if (expert < 0) {
+  if (!COMBINED && expert < 0) {
     clear_past_last<kOutColumns>(p, m_tile, tile, strip, out_width);
     return;
   }
@@ -150,7 +196,8 @@ __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
   };
   static_for<kAhead>([&](auto set) { load(set, min(decltype(set)::value, steps - 1)); });
   // where the rows' results go, asked for behind the first loads
-  const int out_row = p.scatter ? p.scatter[sorted_row] : sorted_row;
+  const int out_row = !COMBINED && p.scatter ? p.scatter[sorted_row] : sorted_row;
+  const float share = COMBINED && wave < c.top_k ? c.weights[slot] : 0.0f;
   int step = 0;
   for (; step + 2 * kAhead <= steps; step += kAhead)
     static_for<kAhead>([&](auto set) {
@@ -170,6 +217,18 @@ __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
   const int column = strip * 32 + lane % 32;
   float bias = (!kPaired && p.bias) ? p.bias[static_cast<size_t>(expert) * p.width + column] : 0.0f;
   if (p.round_bias) bias = bf16_round(bias);
+  if constexpr (COMBINED) {
+    __shared__ float outputs[kMostCombinedSlots][32];
+    __shared__ float shares[kMostCombinedSlots];
+    if (lane < 32) outputs[wave][lane] = bf16_round(acc[0][0] * factor0 + bias);  // (row 0 of the tile, whose rows are all the slot's)
+    if (lane == 0) shares[wave] = share;
+    __syncthreads();
+    if (threadIdx.x < 32) {
+      const float sum = weighted_sum(&outputs[0][lane], 32, shares, c.top_k);
+      c.out[static_cast<size_t>(m_tile) * p.width + column] = c.shared ? f32_to_bf16(bf16_round(sum) + outputs[c.top_k][lane]) : f32_to_bf16(sum);
+    }
+    return;
+  }
 #pragma unroll
   for (int q = 0; q < 16; ++q) {
     if (8 * (q / 4) >= valid_rows) continue;  // (the same for every lane)
@@ -187,6 +246,16 @@ __global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
     }
     if (row < valid_rows && (!kGated || lane % 2 == 0)) p.out[static_cast<size_t>(to) * out_width + (kGated ? column / 2 : column)] = value;
   }
+}
+
+template <int FORMAT, int MODE>
+__global__ __launch_bounds__(64) void few_tiles_kernel(GemmParams p) {
+  few_tile_product<FORMAT, MODE, false>(p, CombineParams{});
+}
+
+template <int FORMAT>
+__global__ __launch_bounds__(64 * kMostCombinedSlots) void few_combined_kernel(GemmParams p, CombineParams c) {
+  few_tile_product<FORMAT, kPlain, true>(p, c);
 }
 
 // Where strips are so few that most CUs have none, a block owns the 32 columns: of a pair each matrix has wavefronts of its own, and
@@ -416,6 +485,19 @@ int launch_few_tiles(const char* who, const GemmParams& p, int format, int mode,
     case kInterleavedGated: return launch_few_format<kInterleavedGated>(who, p, format, stream);
     default: return launch_few_format<kPlain>(who, p, format, stream);
   }
+}
+
+int launch_few_combined(const char* who, const GemmParams& p, int format, const float* weights, int tokens, int top_k, bool shared, void* out, hipStream_t stream) {
+  const CombineParams c{weights, static_cast<bf16_t*>(out), tokens, top_k, shared ? 1 : 0};
+  const dim3 grid(tokens * (p.width / 32)), block(64 * (top_k + c.shared));
+  switch (format) {
+    case DEW_MOE_W_FP8_BLOCK: hipLaunchKernelGGL(few_combined_kernel<DEW_MOE_W_FP8_BLOCK>, grid, block, 0, stream, p, c); break;
+    case DEW_MOE_W_FP8_CHANNEL: hipLaunchKernelGGL(few_combined_kernel<DEW_MOE_W_FP8_CHANNEL>, grid, block, 0, stream, p, c); break;
+    case DEW_MOE_W_MXFP4: hipLaunchKernelGGL(few_combined_kernel<DEW_MOE_W_MXFP4>, grid, block, 0, stream, p, c); break;
+    case DEW_MOE_W_BF16: hipLaunchKernelGGL(few_combined_kernel<DEW_MOE_W_BF16>, grid, block, 0, stream, p, c); break;
+    default: hipLaunchKernelGGL(few_combined_kernel<DEW_MOE_W_NVFP4>, grid, block, 0, stream, p, c);
+  }
+  return launched(who);
 }
 
 }  // namespace dew

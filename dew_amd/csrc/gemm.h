@@ -146,6 +146,11 @@ __device__ __forceinline__ int lanes_scanned(int value) {
 // The launch for few tiles of few rows (decode.hip); `mode`: kPlain, kSwigluOfTwo or kInterleavedGated.
 int launch_few_tiles(const char* who, const GemmParams& p, int format, int mode, hipStream_t stream);
 
+constexpr int kMostCombinedSlots = 8;  // wavefronts of a block: more have no registers for eight steps of weights each in flight
+// The down product and the combine as one launch (decode.hip); `p.scatter`: the sorted positions' slots, `p.rows` of them.
+int launch_few_combined(const char* who, const GemmParams& p, int format, const float* weights, int tokens, int top_k, bool shared, void* out,
+                        hipStream_t stream);
+
 // The launch in tiles of up to 256 rows on eight wavefronts (tall.hip); of FP8 banks, one or two (gate and up, gated), or of one NVFP4 bank.
 int launch_tall(const char* who, const GemmParams& p, int format, bool paired, hipStream_t stream);
 

@@ -30,6 +30,7 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "sort.h"
 #include "wide_fp8.h"
 
 namespace dew {
@@ -1355,6 +1356,28 @@ static int grouped_gemm_of(const char* who, const void* x, const int32_t* gather
   if (int rc = fill_single(who, p, x, gather, offsets, w, bias, scatter, out, rows, sizes)) return rc;
   p.round_bias = round_bias ? 1 : 0;
   return launch<kPlain>(who, p, w->format, static_cast<hipStream_t>(stream));
+}
+
+// A block holds all of a token's slots, so their weights pass through one CU, and each token reads its own: small experts only. us a layer's pass,
+// two launches and one, 2 of 8 experts of 512 x 512 (FP8, 33 KB a block) 22.7 -> 18.3 for one token and 23.1 -> 20.1 for 16; MXFP4, 7 of 256 of
+// 2048 x 512 (61 KB) one token 29.6 -> 28.0, four 38.6 -> 32.8, eight (31 MB in all) 46.3 -> 45.8, twelve 52.8 -> 58.7; 2 of 16 of 4096 x 2048 (70 KB)
+// one 31.3 -> 29.5, three 35.6 -> 35.3, eight 46.6 -> 47.9. Past the first line, FP8, 8 of 128 of 2048 x 768 (196 KB): one 26.4 -> 28.7, three 41.1 -> 38.3,
+// eight 63.9 -> 68.8; 8 of 32 of 7168 x 2048 (524 KB) two 106 -> 116.
+bool dew::combines_few(const dew_moe_bank* down, int tokens, int top_k, bool shared) {
+  const int slots = top_k + (shared ? 1 : 0);
+  if (forced_tile_rows != 0 || slots > kMostCombinedSlots || tokens > 16 || down->format == DEW_MOE_W_MXFP8) return false;
+  const double bytes = down->format == DEW_MOE_W_BF16 ? 2.0 : down->format == DEW_MOE_W_MXFP4 || down->format == DEW_MOE_W_NVFP4 ? 0.53 : 1.0;
+  const double block = 32.0 * slots * down->depth * bytes;
+  return block <= 72 * 1024 && block * (down->width / 32) * tokens <= 32e6;
+}
+
+int dew::down_and_combine(const char* who, const void* hidden, const int32_t* offsets, const dew_moe_bank* down, const float* bias, const int32_t* order,
+                          const float* weights, int tokens, int top_k, bool shared, void* out, hipStream_t stream) {
+  if (int rc = check_bank(who, down, "down")) return rc;
+  GemmParams p{};
+  if (int rc = fill_single(who, p, hidden, nullptr, offsets, down, bias, order, out, tokens * (top_k + (shared ? 1 : 0)))) return rc;
+  p.round_bias = 1;
+  return launch_few_combined(who, p, down->format, weights, tokens, top_k, shared, out, stream);
 }
 
 extern "C" int dew_moe_grouped_gemm_bias(const void* x, const int32_t* gather, const int32_t* offsets,

@@ -151,6 +151,8 @@ extern "C" int dew_moe_layer_forward(const dew_moe_layer* layer, const void* x, 
     } else {
       if (int rc = dew_moe_gateup_gated(x, gather, offsets, nullptr, gate, up, layer->gating, layer->limit, hidden, rows, stream)) return rc;
     }
+    if (combines_few(down, tokens, top_k, layer->shared != 0))
+      return down_and_combine(who, hidden, offsets, down, down_bias, order, weights, tokens, top_k, layer->shared != 0, out, s);
     if (int rc = dew_moe_grouped_gemm_param_bias(hidden, nullptr, offsets, nullptr, down, down_bias, order, slots, rows, stream)) return rc;
   }
   const void* addend = layer->shared ? slots + static_cast<size_t>(slots_count) * down->width * 2 : nullptr;

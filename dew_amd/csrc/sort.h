@@ -190,6 +190,10 @@ LogitShares logit_shares(int tokens, int depth, int experts);
 int router_logit_shares(const void* x, const float* kernel, float* partial, int tokens, int depth, int experts, hipStream_t stream);
 int route_shares(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
                  float* weights, int32_t* indices, hipStream_t stream);
+// A layer's last two launches as one, for a few tokens (decode.hip, gemm.hip): whether they are, and that launch.
+bool combines_few(const dew_moe_bank* down, int tokens, int top_k, bool shared);
+int down_and_combine(const char* who, const void* hidden, const int32_t* offsets, const dew_moe_bank* down, const float* bias, const int32_t* order,
+                     const float* weights, int tokens, int top_k, bool shared, void* out, hipStream_t stream);
 int route_and_sort(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
                    bool shared, float* weights, int32_t* sizes, int32_t* offsets, int32_t* order, int32_t* rows, hipStream_t stream);
 

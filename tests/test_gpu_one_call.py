@@ -25,6 +25,11 @@ CASES = {
     "shares, 63 tiles": dict(tokens=2016, experts=32, top_k=2, quant="fp8_block"),
     "shares, 111 tiles": dict(tokens=1184, experts=96, top_k=1, quant="fp8_block"),
     "no shares, 112 tiles": dict(tokens=1792, experts=64, top_k=1, quant="fp8_block"),
+    # the down product and the combine in one launch, in every format, with a shared expert, at the most slots and tokens
+    "combined, fp8 channels, 16 tokens": dict(tokens=16, experts=8, top_k=8, quant="fp8_channel"),
+    "combined, bf16, shared": dict(tokens=3, experts=8, top_k=3, quant="bf16", shared=256),
+    "combined, mxfp4, one slot": dict(tokens=5, experts=16, top_k=1, quant="mxfp4"),
+    "combined, nvfp4, shared, 70 experts": dict(tokens=16, experts=70, top_k=7, quant="nvfp4", shared=256),
     "300 experts": dict(tokens=64, experts=300, top_k=6, quant="fp8_block"),
 }
 DEPTH, HIDDEN = 512, 256
