@@ -528,23 +528,8 @@ __global__ __launch_bounds__(256) void router_logits_kernel(const bf16_t* __rest
     }
 }
 
-// offsets[0] = 0, offsets[e + 1] = offsets[e] + unit * sizes[e]: one wavefront, 64 sizes a round, the next round's asked for
-// while this one's are added up. (One lane walking the sizes took a memory round trip each few of them: 5 us for 16 groups.)
 __global__ __launch_bounds__(64) void group_offsets_kernel(const int32_t* __restrict__ sizes, int32_t* __restrict__ offsets, int experts, int unit) {
-  const int lane = threadIdx.x;
-  int running = 0, next = lane < experts ? sizes[lane] : 0;
-  if (lane == 0) offsets[0] = 0;
-  for (int base = 0; base < experts; base += 64) {
-    int through = unit * next;
-    next = base + 64 + lane < experts ? sizes[base + 64 + lane] : 0;
-#pragma unroll
-    for (int offset = 1; offset < 64; offset <<= 1) {
-      const int below = __shfl_up(through, offset, 64);
-      if (lane >= offset) through += below;
-    }
-    if (base + lane < experts) offsets[base + lane + 1] = running + through;
-    running += __shfl(through, 63, 64);
-  }
+  write_group_offsets(sizes, offsets, experts, unit);
 }
 
 }  // namespace dew

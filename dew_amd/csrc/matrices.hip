@@ -18,6 +18,7 @@
 // element, nvfp4.h; the general form, which fp32 matrices and operands out of range take, is thirty: 67 us here.)
 #include "common.h"
 #include "nvfp4.h"
+#include "sort.h"
 
 namespace dew {
 
@@ -72,10 +73,18 @@ __device__ __forceinline__ float saturated(float value, float inverse) {
   return value == value ? q : value;
 }
 
+// A step's groups, counted in blocks of `unit` rows, and where their offsets go (null: none): the matrices' launch writes them beside its codes, or
+// the step would take a launch of 5 us for a few words.
+struct StepGroups {
+  const int32_t* blocks;
+  int32_t* offsets;
+  int groups, unit;
+};
+
 template <int FORMAT, typename T, bool KMAJOR, bool CACHED>
 __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const T* __restrict__ w, uint8_t* __restrict__ codes,
                                                                          uint8_t* __restrict__ scales, const uint32_t* __restrict__ largest,
-                                                                         float* __restrict__ tensor_scales, int depth, int width) {
+                                                                         float* __restrict__ tensor_scales, int depth, int width, StepGroups step) {
   constexpr bool kBlocks = FORMAT == DEW_MOE_W_FP8_BLOCK, kNv = FORMAT == DEW_MOE_W_NVFP4;
   constexpr int kVec = 16 / sizeof(T);                   // elements of a load, along the memory's inner axis
   constexpr int kLanes = kMatrixTile / kVec;             // lanes a row of the tile
@@ -285,6 +294,7 @@ __global__ __launch_bounds__(kMatrixThreads) void quantize_matrices_kernel(const
       }
     }
   }
+  if (step.blocks && tid < 64 && blockIdx.x + blockIdx.y + blockIdx.z == 0) write_group_offsets(step.blocks, step.offsets, step.groups, step.unit);
 }
 
 // An NVFP4 bank's buffer: codes, block scales, then the partial largest magnitudes and the tensor scales.
@@ -292,13 +302,14 @@ static size_t nvfp4_scales_at(size_t elements) { return elements / 2; }
 static size_t nvfp4_largest_at(size_t elements) { return elements / 2 + elements / 16; }
 
 template <int FORMAT, typename T>
-static int quantize_matrices(const T* w, bool kmajor, int experts, int depth, int width, uint8_t* prepared, dew_moe_bank* out, hipStream_t s) {
+static int quantize_matrices(const T* w, bool kmajor, int experts, int depth, int width, const uint32_t* known_largest, const StepGroups& step, uint8_t* prepared,
+                             dew_moe_bank* out, hipStream_t s) {
   const size_t elements = static_cast<size_t>(experts) * depth * width;
   uint8_t* scales = prepared + (FORMAT == DEW_MOE_W_NVFP4 ? nvfp4_scales_at(elements) : elements);
   uint32_t* largest = reinterpret_cast<uint32_t*>(prepared + nvfp4_largest_at(elements));
   float* tensor_scales = reinterpret_cast<float*>(largest + kNvfp4Partials);
   *out = dew_moe_bank{FORMAT, DEW_MOE_LAYOUT_PREPARED, experts, depth, width, prepared, scales, FORMAT == DEW_MOE_W_NVFP4 ? tensor_scales : nullptr};
-  if (FORMAT == DEW_MOE_W_NVFP4) {
+  if (FORMAT == DEW_MOE_W_NVFP4 && !known_largest) {
     if (int rc = dew_moe_nvfp4_largest(w, static_cast<int64_t>(elements), sizeof(T) == 4, largest, s)) return rc;
   }
   const dim3 grid = kmajor ? dim3(depth / 128, width / 128, experts) : dim3(width / 128, depth / 128, experts);
@@ -306,7 +317,7 @@ static int quantize_matrices(const T* w, bool kmajor, int experts, int depth, in
   const bool cached = kNv && elements * sizeof(T) <= (size_t{256} << 20);
   auto kernel = cached ? (kmajor ? quantize_matrices_kernel<FORMAT, T, true, kNv> : quantize_matrices_kernel<FORMAT, T, false, kNv>)
                        : (kmajor ? quantize_matrices_kernel<FORMAT, T, true, false> : quantize_matrices_kernel<FORMAT, T, false, false>);
-  hipLaunchKernelGGL(kernel, grid, dim3(kMatrixThreads), 0, s, w, prepared, scales, largest, tensor_scales, depth, width);
+  hipLaunchKernelGGL(kernel, grid, dim3(kMatrixThreads), 0, s, w, prepared, scales, known_largest ? known_largest : largest, tensor_scales, depth, width, step);
   return launched("quantize_matrices_kernel");
 }
 
@@ -319,8 +330,9 @@ extern "C" size_t dew_moe_quantized_matrices_bytes(int32_t format, int32_t exper
   return dew_moe_prepared_bytes(format, experts, depth, width);
 }
 
-extern "C" int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
-                                         int32_t width, void* prepared, dew_moe_bank* out, void* stream) {
+extern "C" int dew_moe_quantize_step_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
+                                              int32_t width, const uint32_t* largest, const int32_t* blocks, int32_t groups, int32_t unit,
+                                              int32_t* offsets, void* prepared, dew_moe_bank* out, void* stream) {
   using namespace dew;
   const char* who = "dew_moe_quantize_matrices";
   DEW_REQUIRE(w && prepared && out, "%s: w, the prepared buffer and out must not be null", who);
@@ -330,14 +342,21 @@ extern "C" int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t 
   DEW_REQUIRE(depth >= 128 && depth % 128 == 0 && width >= 128 && width % 128 == 0 && depth / 128 <= 65535 && width / 128 <= 65535,
               "%s: matrices of %d x %d (whole 128s)", who, depth, width);
   DEW_REQUIRE(aligned16(w) && (reinterpret_cast<uintptr_t>(prepared) & 255u) == 0, "%s: w must be 16-byte and the prepared buffer 256-byte aligned", who);
+  DEW_REQUIRE(!blocks || (offsets && groups >= 1 && unit >= 1), "%s: offsets must not be null, %d groups in units of %d", who, groups, unit);
+  const StepGroups step{blocks, offsets, groups, unit};
   hipStream_t s = static_cast<hipStream_t>(stream);
   uint8_t* buffer = static_cast<uint8_t*>(prepared);
   auto of = [&](auto* typed) {
     switch (format) {
-      case DEW_MOE_W_FP8_BLOCK: return quantize_matrices<DEW_MOE_W_FP8_BLOCK>(typed, kmajor != 0, experts, depth, width, buffer, out, s);
-      case DEW_MOE_W_MXFP8: return quantize_matrices<DEW_MOE_W_MXFP8>(typed, kmajor != 0, experts, depth, width, buffer, out, s);
-      default: return quantize_matrices<DEW_MOE_W_NVFP4>(typed, kmajor != 0, experts, depth, width, buffer, out, s);
+      case DEW_MOE_W_FP8_BLOCK: return quantize_matrices<DEW_MOE_W_FP8_BLOCK>(typed, kmajor != 0, experts, depth, width, largest, step, buffer, out, s);
+      case DEW_MOE_W_MXFP8: return quantize_matrices<DEW_MOE_W_MXFP8>(typed, kmajor != 0, experts, depth, width, largest, step, buffer, out, s);
+      default: return quantize_matrices<DEW_MOE_W_NVFP4>(typed, kmajor != 0, experts, depth, width, largest, step, buffer, out, s);
     }
   };
   return w_is_f32 ? of(static_cast<const float*>(w)) : of(static_cast<const bf16_t*>(w));
+}
+
+extern "C" int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
+                                         int32_t width, void* prepared, dew_moe_bank* out, void* stream) {
+  return dew_moe_quantize_step_matrices(w, format, w_is_f32, kmajor, experts, depth, width, nullptr, nullptr, 0, 0, nullptr, prepared, out, stream);
 }

@@ -288,9 +288,16 @@ __global__ __launch_bounds__(256) void quantize_tokens_nvfp4_kernel(const bf16_t
   for (int t = 0; t < 16; ++t) *reinterpret_cast<u32x2_t*>(tokens_out + at + static_cast<size_t>(t) * dim) = words[t];
 }
 
-// An operand's partial largest magnitudes, bf16 or fp32, a partial a block.
+// Operands' partial largest magnitudes, bf16 or fp32, a partial a block: blockIdx.y is the operand. A step quantizes two or three operands, whose
+// magnitudes one launch forms side by side: 8192 rows' step on 8 x 2048 x 4096 had five launches of 8 to 26 us, 89 in all, and has two.
+constexpr int kMostOperands = 3;
+struct LargestOperands {
+  const u32x4_t* x[kMostOperands];
+  long long chunks[kMostOperands];
+  int f32[kMostOperands];
+};
 template <bool F32>
-__global__ __launch_bounds__(256) void nvfp4_largest_kernel(const u32x4_t* __restrict__ x, long long chunks, uint32_t* __restrict__ partials) {
+__device__ __forceinline__ uint32_t largest_of(const u32x4_t* __restrict__ x, long long chunks) {
   uint32_t mine = 0;
   auto take = [&](const u32x4_t& words) {
 #pragma unroll
@@ -306,12 +313,17 @@ __global__ __launch_bounds__(256) void nvfp4_largest_kernel(const u32x4_t* __res
     for (int k = 0; k < 8; ++k) take(words[k]);
   }
   for (; chunk < chunks; chunk += stride) take(x[chunk]);
+  return mine;
+}
+__global__ __launch_bounds__(256) void nvfp4_largest_kernel(LargestOperands of, uint32_t* __restrict__ partials) {
+  const int operand = blockIdx.y;
+  uint32_t mine = of.f32[operand] ? largest_of<true>(of.x[operand], of.chunks[operand]) : largest_of<false>(of.x[operand], of.chunks[operand]);
 #pragma unroll
   for (int offset = 32; offset >= 1; offset >>= 1) mine = max(mine, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mine), offset, 64)));
   __shared__ uint32_t waves[4];
   if (threadIdx.x % 64 == 0) waves[threadIdx.x / 64] = mine;
   __syncthreads();
-  if (threadIdx.x == 0) partials[blockIdx.x] = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
+  if (threadIdx.x == 0) partials[operand * kNvfp4Partials + blockIdx.x] = max(max(waves[0], waves[1]), max(waves[2], waves[3]));
 }
 
 // A kernel gradient's operands: x [tokens, dim] quantized ALONG THE TOKENS and written transposed, for the product
@@ -763,19 +775,26 @@ extern "C" int dew_moe_quantize_rows_nvfp4(const void* x, void* values, float* t
 
 extern "C" int dew_moe_nvfp4_partials(void) { return dew::kNvfp4Partials; }
 
-extern "C" int dew_moe_nvfp4_largest(const void* operand, int64_t elements, int32_t is_f32, uint32_t* partials, void* stream) {
+extern "C" int dew_moe_nvfp4_largest_of(const void* const* operands, const int64_t* elements, const int32_t* is_f32, int32_t count, uint32_t* partials,
+                                        void* stream) {
   using namespace dew;
   const char* who = "dew_moe_nvfp4_largest";
+  DEW_REQUIRE(operands && elements && is_f32 && count >= 1 && count <= kMostOperands, "%s: %d operands (1 to %d)", who, count, kMostOperands);
   DEW_REQUIRE(partials, "%s: the partials must not be null", who);
-  DEW_REQUIRE(elements >= 0 && elements % 8 == 0, "%s: an operand of %lld elements (whole 8s)", who, static_cast<long long>(elements));
-  DEW_REQUIRE(elements == 0 || (operand && aligned16(operand)), "%s: the operand must not be null and must be 16-byte aligned", who);
-  const u32x4_t* x = static_cast<const u32x4_t*>(operand);
-  hipStream_t s = static_cast<hipStream_t>(stream);
-  if (is_f32)
-    hipLaunchKernelGGL(nvfp4_largest_kernel<true>, dim3(kNvfp4Partials), dim3(256), 0, s, x, elements / 4, partials);
-  else
-    hipLaunchKernelGGL(nvfp4_largest_kernel<false>, dim3(kNvfp4Partials), dim3(256), 0, s, x, elements / 8, partials);
+  LargestOperands of{};
+  for (int i = 0; i < count; ++i) {
+    DEW_REQUIRE(elements[i] >= 0 && elements[i] % 8 == 0, "%s: an operand of %lld elements (whole 8s)", who, static_cast<long long>(elements[i]));
+    DEW_REQUIRE(elements[i] == 0 || (operands[i] && aligned16(operands[i])), "%s: the operand must not be null and must be 16-byte aligned", who);
+    of.x[i] = static_cast<const u32x4_t*>(operands[i]);
+    of.chunks[i] = elements[i] / (is_f32[i] ? 4 : 8);
+    of.f32[i] = is_f32[i];
+  }
+  hipLaunchKernelGGL(nvfp4_largest_kernel, dim3(kNvfp4Partials, count), dim3(256), 0, static_cast<hipStream_t>(stream), of, partials);
   return launched("nvfp4_largest_kernel");
+}
+
+extern "C" int dew_moe_nvfp4_largest(const void* operand, int64_t elements, int32_t is_f32, uint32_t* partials, void* stream) {
+  return dew_moe_nvfp4_largest_of(&operand, &elements, &is_f32, 1, partials, stream);
 }
 
 extern "C" int dew_moe_quantize_nvfp4(const void* x, const uint32_t* largest, void* row_values, void* token_values, float* tensor_scale,

@@ -3,6 +3,7 @@ contiguity), allocates its outputs with torch (device memory and streams are tor
 the library's) and calls the C ABI on torch's current stream. No function reads a device value on the host."""
 
 import contextlib
+import ctypes
 import dataclasses
 
 import torch
@@ -364,10 +365,11 @@ RECIPE_FORMATS = {"blockwise_fp8": _lib.W_FP8_BLOCK, "mxfp8": _lib.W_MXFP8, "nvf
 """The bank a recipe's product multiplies."""
 
 
-def quantize_matrices(w: torch.Tensor, recipe: str) -> PreparedBank:
+def quantize_matrices(w: torch.Tensor, recipe: str, *, largest: torch.Tensor | None = None, blocks: torch.Tensor | None = None, unit: int = 128):
     """`w [E, K, N]` (bf16 or fp32; contiguous, or the transpose of contiguous memory, read where it lies) quantized for a
     recipe's product straight into its prepared bank (`dew_moe_quantize_matrices`): the bytes that quantizing `w` to the
-    recipe's bank of `formats` and preparing that would give."""
+    recipe's bank of `formats` and preparing that would give. `largest`: `nvfp4_largest`'s of `w`, where a step has formed them already.
+    With `blocks`, a step's groups counted in blocks of `unit` rows, the bank and their `block_offsets`, from the same launch."""
     kmajor = not w.is_contiguous()
     _device(w.transpose(1, 2) if kmajor else w, "w")
     if w.dtype not in (torch.bfloat16, torch.float32):
@@ -377,15 +379,25 @@ def quantize_matrices(w: torch.Tensor, recipe: str) -> PreparedBank:
     fmt = RECIPE_FORMATS[recipe]
     experts, depth, width = w.shape
     lib = _lib.library()
+    if largest is not None:
+        _partials(largest), _device(largest, "largest", torch.int32)
+    groups, offsets = 0, None
+    if blocks is not None:
+        _device(blocks, "group_blocks", torch.int32)
+        groups = blocks.numel()
+        offsets = torch.empty(groups + 1, dtype=torch.int32, device=w.device)
+        if groups == 0:
+            raise KernelError("a step has one group at least")
     buffer = torch.empty(max(lib.dew_moe_quantized_matrices_bytes(fmt, experts, depth, width), 16), dtype=torch.uint8, device=w.device)
     out = _lib.Bank()
-    _lib.check(lib.dew_moe_quantize_matrices(_ptr(w), fmt, int(w.dtype == torch.float32), int(kmajor), experts, depth, width, _ptr(buffer), out,
-                                             _stream()), "dew_moe_quantize_matrices")
+    _lib.check(lib.dew_moe_quantize_step_matrices(w.data_ptr(), fmt, int(w.dtype == torch.float32), int(kmajor), experts, depth, width, _ptr(largest),
+                                                  _ptr(blocks), groups, unit, _ptr(offsets), buffer.data_ptr(), out, _stream()), "dew_moe_quantize_matrices")
     tensor = None
     if fmt == _lib.W_NVFP4:
         at = out.tensor_scale - buffer.data_ptr()
         tensor = buffer[at:at + 4 * experts].view(torch.float32)
-    return PreparedBank(out, (experts, depth, width), (buffer, None, tensor))
+    bank = PreparedBank(out, (experts, depth, width), (buffer, None, tensor))
+    return bank if blocks is None else (bank, offsets)
 
 
 # ---- products -----------------------------------------------------------------------------------------
@@ -915,12 +927,33 @@ def quantize_rows_nvfp4(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
 
 def nvfp4_largest(x: torch.Tensor) -> torch.Tensor:
     """The partial largest magnitudes (words) of `x`, bf16 or fp32, that `quantize_nvfp4` takes its tensor scale from."""
-    _device(x, "x")
-    if x.dtype not in (torch.bfloat16, torch.float32):
-        raise KernelError(f"x must be torch.bfloat16 or torch.float32, got {x.dtype}")
-    partials = torch.empty(_lib.library().dew_moe_nvfp4_partials(), dtype=torch.int32, device=x.device)
-    _lib.check(_lib.library().dew_moe_nvfp4_largest(_ptr(x), x.numel(), int(x.dtype == torch.float32), _ptr(partials), _stream()), "dew_moe_nvfp4_largest")
+    return nvfp4_largest_of(x)[0]
+
+
+MOST_OPERANDS = 3
+"""The most operands whose magnitudes one launch forms (`kMostOperands`, csrc/quantize.hip)."""
+
+
+def nvfp4_largest_of(*operands: torch.Tensor) -> torch.Tensor:
+    """`nvfp4_largest` of each of up to three operands, in one launch: a row of words each. (An operand may be the transpose of contiguous
+    memory, as `quantize_matrices`' matrices are.)"""
+    count = len(operands)
+    for x in operands:
+        _device(x if x.is_contiguous() or x.dim() != 3 else x.transpose(1, 2), "x")
+        if x.dtype not in (torch.bfloat16, torch.float32):
+            raise KernelError(f"x must be torch.bfloat16 or torch.float32, got {x.dtype}")
+    partials = torch.empty((count, _lib.library().dew_moe_nvfp4_partials()), dtype=torch.int32, device=operands[0].device)
+    _lib.check(_lib.library().dew_moe_nvfp4_largest_of((ctypes.c_void_p * count)(*(x.data_ptr() for x in operands)),
+                                                       (ctypes.c_int64 * count)(*(x.numel() for x in operands)),
+                                                       (ctypes.c_int32 * count)(*(int(x.dtype == torch.float32) for x in operands)), count,
+                                                       partials.data_ptr(), _stream()), "dew_moe_nvfp4_largest")
     return partials
+
+
+def _partials(largest: torch.Tensor) -> None:
+    words = _lib.library().dew_moe_nvfp4_partials()
+    if largest.numel() != words:    # (every one of them is read)
+        raise KernelError(f"largest has {largest.numel()} words, not nvfp4_largest's {words}")
 
 
 def quantize_nvfp4(x: torch.Tensor, largest: torch.Tensor, *, rows: bool, tokens: bool, bank: PreparedBank | None = None):
@@ -929,9 +962,7 @@ def quantize_nvfp4(x: torch.Tensor, largest: torch.Tensor, *, rows: bool, tokens
     fp32 `[1]`, the tensor scales of `bank`, which the rows will multiply, times it, or None)."""
     if x.dim() != 2:
         raise KernelError(f"x is {tuple(x.shape)}, not [rows, depth]")
-    words = _lib.library().dew_moe_nvfp4_partials()
-    if largest.numel() != words:    # (every one of them is read)
-        raise KernelError(f"largest has {largest.numel()} words, not nvfp4_largest's {words}")
+    _partials(largest)
     if bank is not None:
         bank._carries_tensor_scales()
     _device(x, "x", torch.bfloat16), _device(largest, "largest", torch.int32)

@@ -81,6 +81,16 @@ def _bank(w, recipe: str, bank_types: tuple, quantized):
     return quantized(w) if matrices is None else ops.quantize_matrices(matrices, recipe)
 
 
+def _bank_and_groups(w, recipe: str, bank_types: tuple, quantized, group_blocks, device):
+    """`_bank` and `_groups`, the groups' offsets from the launch that quantizes the matrices, where one does."""
+    if not (isinstance(group_blocks, gemm.GroupSizes) or isinstance(w, bank_types)):
+        matrices = _read_by_the_quantizer(w, recipe)
+        if matrices is not None and matrices.device == device:
+            bank, offsets = ops.quantize_matrices(matrices, recipe, blocks=_counts(group_blocks, device), unit=SCALE_DEPTH)
+            return bank, gemm.GroupSizes(None, offsets)
+    return _bank(w, recipe, bank_types, quantized), _groups(group_blocks, device)
+
+
 def _read_by_the_quantizer(w: torch.Tensor, recipe: str):
     """`w` as the device's quantizer of matrices reads it (as it lies, or a copy), None where its extents do not fit."""
     whole = SCALE_DEPTH * (2 if recipe == "nvfp4" else 1)    # (an NVFP4 bank's depth is whole 256s)
@@ -104,7 +114,11 @@ def _groups(group_blocks, device) -> gemm.GroupSizes:
     that a product reads of them."""
     if isinstance(group_blocks, gemm.GroupSizes):
         return group_blocks
-    return gemm.GroupSizes(None, ops.block_offsets(torch.as_tensor(group_blocks, device=device).to(torch.int32).contiguous(), SCALE_DEPTH))
+    return gemm.GroupSizes(None, ops.block_offsets(_counts(group_blocks, device), SCALE_DEPTH))
+
+
+def _counts(group_blocks, device) -> torch.Tensor:
+    return torch.as_tensor(group_blocks, device=device).to(torch.int32).contiguous()
 
 
 def blockwise_fp8_product(lhs: QuantizedRows, kernel, group_sizes, *, out_dtype=torch.bfloat16, bias=None,
@@ -125,8 +139,8 @@ def blockwise_fp8_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torc
     """Each group's rows of `x [rows, depth]` times its matrix of `w [groups, depth, width]` in the blockwise FP8
     recipe; group `g` holds `group_blocks[g]` whole 128-row blocks, in order (src/dew/nn/kernels/projections.py:
     50-60). `w` is the weights (quantized here, `blocks_quantized`) or a bank already quantized."""
-    bank = _bank(w, "blockwise_fp8", (formats.Fp8Blocks, ops.PreparedBank), blocks_quantized)
-    return blockwise_fp8_product(rows_quantized(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
+    bank, groups = _bank_and_groups(w, "blockwise_fp8", (formats.Fp8Blocks, ops.PreparedBank), blocks_quantized, group_blocks, x.device)
+    return blockwise_fp8_product(rows_quantized(x), bank, groups, out_dtype=out_dtype)
 
 
 def recipe_projection(rows: torch.Tensor, matrix, group_sizes=None, *, out_dtype=torch.bfloat16, bias=None,
@@ -206,8 +220,8 @@ def mxfp8_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torch.bfloat
     """Each group's rows of `x [rows, depth]` times its matrix of `w [groups, depth, width]` in the MXFP8 recipe, both
     quantized along the depth (src/dew/nn/kernels/projections.py:231-258); group `g` holds `group_blocks[g]` whole
     128-row blocks. `w` is the weights (quantized here) or an MXFP8 bank already quantized."""
-    bank = _bank(w, "mxfp8", (formats.MxFp8, ops.PreparedBank), formats.MxFp8.quantized)
-    return mxfp8_product(mxfp8_rows(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
+    bank, groups = _bank_and_groups(w, "mxfp8", (formats.MxFp8, ops.PreparedBank), formats.MxFp8.quantized, group_blocks, x.device)
+    return mxfp8_product(mxfp8_rows(x), bank, groups, out_dtype=out_dtype)
 
 
 # ---- the NVFP4 recipe ------------------------------------------------------------------------------------
@@ -262,9 +276,29 @@ def nvfp4_projection(x: torch.Tensor, w, group_blocks, *, out_dtype=torch.bfloat
         bank = _bank(w, "nvfp4", (formats.NvFp4, ops.PreparedBank), nvfp4_matrices)
         return nvfp4_block_product(nvfp4_rows(x), bank, _groups(group_blocks, x.device), out_dtype=out_dtype)
     x = x.contiguous()
-    bank = ops.quantize_matrices(matrices, "nvfp4")
-    values, _, _, scales = ops.quantize_nvfp4(x, ops.nvfp4_largest(x), rows=True, tokens=False, bank=bank)
-    return _nvfp4_product(values, bank.under(scales), _groups(group_blocks, x.device), out_dtype)
+    (x_largest,), bank, groups = _nvfp4_step((x,), matrices, group_blocks)
+    values, _, _, scales = ops.quantize_nvfp4(x, x_largest(), rows=True, tokens=False, bank=bank)
+    return _nvfp4_product(values, bank.under(scales), groups, out_dtype)
+
+
+CACHED_BYTES = 256 << 20
+"""What the last-level cache holds."""
+
+
+def _nvfp4_step(operands: tuple, matrices: torch.Tensor, group_blocks):
+    """Each operand's largest magnitudes (a call for them), the quantized matrices and the groups, which the matrices' launch leaves offsets of. The
+    magnitudes of operands that the last-level cache holds all of come from one launch (five of them were 89 us of a step of 589, 8192 rows of
+    8 x 2048 x 4096); larger ones are read for theirs right before they are quantized, while the cache holds the most of them."""
+    together = (*operands, matrices)
+    if sum(x.numel() * x.element_size() for x in together) <= CACHED_BYTES:
+        *known, of_matrices = ops.nvfp4_largest_of(*together)
+        largest = tuple(lambda words=words: words for words in known)
+    else:
+        of_matrices, largest = None, tuple(lambda x=x: ops.nvfp4_largest(x) for x in operands)
+    if isinstance(group_blocks, gemm.GroupSizes):
+        return largest, ops.quantize_matrices(matrices, "nvfp4", largest=of_matrices), group_blocks
+    bank, offsets = ops.quantize_matrices(matrices, "nvfp4", largest=of_matrices, blocks=_counts(group_blocks, operands[0].device), unit=SCALE_DEPTH)
+    return largest, bank, gemm.GroupSizes(None, offsets)
 
 
 def _quantized_in_place(x: torch.Tensor) -> bool:
@@ -306,11 +340,11 @@ def blockwise_fp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.T
     recipe's own product of the requantized cotangent and the matrices' blocks transposed (a 128 x 128 block and its
     scale transpose as they are; the quantizer reads `w` where it lies, either way round); the matrices' is
     `kernel_gradient`."""
-    group_blocks = _groups(group_blocks, x.device)    # once for both products
     if not _quantized_both_ways(cotangent):
+        group_blocks = _groups(group_blocks, x.device)    # once for both products
         d_x = blockwise_fp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
         return d_x, kernel_gradient(x, cotangent, group_blocks, mx=False, out_dtype=out_dtype)
-    matrices = _bank(w.transpose(1, 2), "blockwise_fp8", (formats.Fp8Blocks, ops.PreparedBank), blocks_quantized)
+    matrices, group_blocks = _bank_and_groups(w.transpose(1, 2), "blockwise_fp8", (formats.Fp8Blocks, ops.PreparedBank), blocks_quantized, group_blocks, x.device)
     *rows, columns = ops.quantize_rows_and_columns(cotangent.contiguous(), mx=False)
     d_x = blockwise_fp8_product(QuantizedRows(*rows), matrices, group_blocks, out_dtype=x.dtype)
     return d_x, _contracted(x, columns, cotangent.shape[1], group_blocks.offsets, False, out_dtype)
@@ -327,11 +361,11 @@ def _quantized_both_ways(cotangent: torch.Tensor) -> bool:
 def mxfp8_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, group_blocks, *, out_dtype=torch.bfloat16):
     """`_mx_backward` (src/dew/nn/kernels/projections.py:263-275) -> (d_x, d_w): the MXFP8 product of the cotangent and
     the matrices, both quantized along the width, and `kernel_gradient` with a scale every 32 tokens."""
-    group_blocks = _groups(group_blocks, x.device)    # once for both products
     if not _quantized_both_ways(cotangent):
+        group_blocks = _groups(group_blocks, x.device)    # once for both products
         d_x = mxfp8_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
         return d_x, kernel_gradient(x, cotangent, group_blocks, mx=True, out_dtype=out_dtype)
-    matrices = _bank(w.transpose(1, 2), "mxfp8", (formats.MxFp8, ops.PreparedBank), formats.MxFp8.quantized)
+    matrices, group_blocks = _bank_and_groups(w.transpose(1, 2), "mxfp8", (formats.MxFp8, ops.PreparedBank), formats.MxFp8.quantized, group_blocks, x.device)
     *rows, columns = ops.quantize_rows_and_columns(cotangent.contiguous(), mx=True)
     d_x = mxfp8_product(MxFp8Rows(*rows), matrices, group_blocks, out_dtype=x.dtype)
     return d_x, _contracted(x, columns, cotangent.shape[1], group_blocks.offsets, True, out_dtype)
@@ -360,19 +394,21 @@ def nvfp4_gradients(x: torch.Tensor, w: torch.Tensor, cotangent: torch.Tensor, g
     and the matrices, both quantized along the width; and each group's tokens contracted over `x` and the cotangent
     quantized along the tokens, every 16 a scale. The decoded operands short of their tensor scales are exact in bf16,
     so the contraction is the bf16 kernel gradient with both tensor scales applied to its fp32 sums."""
-    group_blocks = _groups(group_blocks, x.device)    # once for both products
     matrices = None if isinstance(w, (formats.NvFp4, ops.PreparedBank)) else _read_by_the_quantizer(w.transpose(1, 2), "nvfp4")
     if matrices is None or not (_quantized_in_place(x) and _quantized_in_place(cotangent)):
+        group_blocks = _groups(group_blocks, x.device)    # once for both products
         d_x = nvfp4_projection(cotangent, w.transpose(1, 2), group_blocks, out_dtype=x.dtype)
         return d_x, _nvfp4_transposed_gradient(x.contiguous(), cotangent.contiguous(), group_blocks, out_dtype)
     x, cotangent = x.contiguous(), cotangent.contiguous()
-    bank = ops.quantize_matrices(matrices, "nvfp4")
-    in_place = _contracted_in_place(x.shape[0], x.shape[1], cotangent.shape[1], group_blocks.offsets.numel() - 1)
+    group_blocks = group_blocks if isinstance(group_blocks, gemm.GroupSizes) else _counts(group_blocks, x.device)
+    groups = group_blocks.offsets.numel() - 1 if isinstance(group_blocks, gemm.GroupSizes) else group_blocks.numel()
+    in_place = _contracted_in_place(x.shape[0], x.shape[1], cotangent.shape[1], groups)
+    (of_cotangent, *of_x), bank, group_blocks = _nvfp4_step((cotangent, x) if in_place else (cotangent,), matrices, group_blocks)
     # the cotangent's two quantizations from one read
-    values, columns, columns_scale, scales = ops.quantize_nvfp4(cotangent, ops.nvfp4_largest(cotangent), rows=True, tokens=in_place, bank=bank)
+    values, columns, columns_scale, scales = ops.quantize_nvfp4(cotangent, of_cotangent(), rows=True, tokens=in_place, bank=bank)
     d_x = _nvfp4_product(values, bank.under(scales), group_blocks, x.dtype)
     if not in_place:
         return d_x, _nvfp4_transposed_gradient(x, cotangent, group_blocks, out_dtype)
-    _, rows, rows_scale, _ = ops.quantize_nvfp4(x, ops.nvfp4_largest(x), rows=False, tokens=True)
+    _, rows, rows_scale, _ = ops.quantize_nvfp4(x, of_x[0](), rows=False, tokens=True)
     d_w = ops.dense_gradient(rows, columns, group_blocks.offsets, lhs_scale=rows_scale, rhs_scale=columns_scale, out_dtype=out_dtype)
     return d_x, d_w

@@ -234,6 +234,12 @@ int dew_moe_prepare_bank(const dew_moe_bank* reference, void* prepared, dew_moe_
 size_t dew_moe_quantized_matrices_bytes(int32_t format, int32_t experts, int32_t depth, int32_t width);
 int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
                               int32_t width, void* prepared, dew_moe_bank* out /* host */, void* stream);
+/* The same as a step's launch: an NVFP4 bank's tensor scale from partial magnitudes formed already (`largest`, dew_moe_nvfp4_largest_of's
+ * words for w, or null), and the offsets [groups + 1] of groups counted in blocks of `unit` rows written beside the codes
+ * (dew_moe_block_offsets; `blocks` null: none).                                                                       */
+int dew_moe_quantize_step_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
+                                   int32_t width, const uint32_t* largest, const int32_t* blocks, int32_t groups, int32_t unit,
+                                   int32_t* offsets, void* prepared, dew_moe_bank* out /* host */, void* stream);
 
 /* The descriptor of a bank prepared earlier, from the buffer alone: for a binding that holds the prepared bytes as an
  * opaque array (an XLA buffer) and the bank's format tag and extents as static attributes. `format` is the PREPARED
@@ -490,6 +496,9 @@ int dew_moe_quantize_rows_nvfp4(const void* x /* bf16 [rows, K] */, void* values
  * the [experts] tensor scales of the bank that the rows will multiply; products [experts] receives them times the rows'.      */
 int dew_moe_nvfp4_partials(void);
 int dew_moe_nvfp4_largest(const void* operand, int64_t elements, int32_t is_f32, uint32_t* partials, void* stream);
+/* The same of up to three operands in one launch (the arrays are the host's): partials [count][dew_moe_nvfp4_partials()].  */
+int dew_moe_nvfp4_largest_of(const void* const* operands, const int64_t* elements, const int32_t* is_f32, int32_t count, uint32_t* partials,
+                             void* stream);
 int dew_moe_quantize_nvfp4(const void* x, const uint32_t* largest, void* row_values, void* token_values, float* tensor_scale,
                            const float* bank_scales, float* products, int32_t experts, int32_t rows, int32_t depth, void* stream);
 int dew_moe_quantize_rows_fp8(const void* x /* bf16 [rows, K] */, void* codes /* [rows, K] bytes */,

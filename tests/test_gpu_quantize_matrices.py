@@ -76,6 +76,21 @@ def test_block_offsets(ops, groups):
     assert torch.equal(ops.group_offsets(blocks).cpu().long() * 128, want)
 
 
+@pytest.mark.parametrize("groups", [1, 64, 65, 1000])
+@pytest.mark.parametrize("recipe", ["blockwise_fp8", "mxfp8", "nvfp4"])
+@pytest.mark.parametrize("turned", [False, True])
+def test_a_steps_launch_leaves_its_groups_offsets(ops, recipe, groups, turned):
+    blocks = torch.randint(0, 9, (groups,), generator=torch.Generator().manual_seed(groups), dtype=torch.int32).cuda()
+    w = torch.randn((3, 256, 512), device="cuda", generator=torch.Generator("cuda").manual_seed(groups)).to(torch.bfloat16)
+    w = w.transpose(1, 2).contiguous().transpose(1, 2) if turned else w
+    of_x, of_w, of_wide = ops.nvfp4_largest_of(w[0].contiguous() * 3, w, w.float())
+    assert torch.equal(of_w, ops.nvfp4_largest(w.contiguous() if not turned else w.transpose(1, 2))) and int(of_wide.max()) == int(of_w.max())
+    assert int(of_x.max()) == int(ops.nvfp4_largest(w[0].contiguous() * 3).max())
+    bank, offsets = ops.quantize_matrices(w, recipe, largest=of_w if recipe == "nvfp4" else None, blocks=blocks)
+    assert torch.equal(offsets, ops.block_offsets(blocks, 128))
+    assert torch.equal(bank.keep[0][:w.numel() // 2], ops.quantize_matrices(w, recipe).keep[0][:w.numel() // 2])
+
+
 def test_what_cannot_be_quantized_is_refused(ops):
     for w, recipe in ((torch.zeros((1, 128, 64), dtype=torch.bfloat16, device="cuda"), "mxfp8"),
                       (torch.zeros((1, 128, 128), dtype=torch.float16, device="cuda"), "mxfp8"),
