@@ -6,8 +6,18 @@
 // 128-row tiles of gemm.hip. Of a paired launch (gate and up, SwiGLU) wavefronts 0 to 3 hold the gate's 128 columns and 4 to 7
 // the up projection's, and they exchange rounded sums through the LDS in the epilogue.
 //
-// Tiles follow their groups: a group of n rows is ceil(n / 256) tiles of equally many 32-row tiles (each count its own copy of
-// the main loop), so that a group's last rows need neither a launch of their own nor a tile that is mostly empty.
+// Unquantized banks, whose launches are bound by their weights' bytes, gain otherwise: a group of 130 to 220 rows reads them once, not
+// twice, and one of 70 multiplies 96 rows, not 128.
+//
+// Tiles follow their groups: a group of n rows is ceil(n / 256) tiles (of at most 224 rows on unquantized banks) of equally many 32-row
+// tiles (each count its own copy of the main loop), so that a group's last rows need neither a launch of their own nor a tile that is
+// mostly empty.
+//
+// Cycles of a tile of 256 rows, FP8, 2048 deep (one bank): 7800 until its first step, 74 000 in 32 steps (the matrix pipe 88 % busy),
+// 7400 until its last store; paired 96 000, of which 13 000 are both matrices' sums' arithmetic. Tried and not kept, all the same to a
+// percent: several strips a block with the next one's loads under the epilogue (the clock gives back what the wait took: the chip's power
+// is the bound); blocks of four wavefronts, two a CU (quantized banks 4 % slower, their rows are fetched twice as often).
+#include <algorithm>
 #include <mutex>
 
 #include "common.h"
@@ -15,8 +25,7 @@
 
 namespace dew {
 
-constexpr int kTallThreads = 512, kTallRows = 256, kTallStages = 3;
-constexpr int kTallStageChunks = kTallRows * kChunksPerRow;
+constexpr int kTallThreads = 512, kTallRows = 256;
 constexpr int kScaleRow = kMaxDepthBlocks + 1;  // a column block's scales; the last step reads one past the deepest bank's (and drops it)
 
 // Dynamic LDS: the ring of A rows, or the staged output tile, behind it the sums that the halves of a paired launch exchange, and
@@ -63,13 +72,26 @@ __device__ __forceinline__ void schedule_slice() {
   }
 }
 
+// How far ahead of their use a tile of TI 32-row tiles asks for its rows (kAhead steps, a ring of one stage more) and its weights (kSets register
+// sets, kAhead + 1 steps). Quantized banks: two steps of 300 to 2400 cycles, with the vector unit the bound. Unquantized ones are bound by the weights'
+// stream, four times the bytes a step, and their steps are the shorter: as many as the registers hold.
+template <int FORMAT, int TI>
+struct TallDepth {
+  static constexpr int kAhead = FORMAT != DEW_MOE_W_BF16 || TI > 6 ? 2 : TI > 4 ? 3 : 4, kStages = kAhead + 1, kSets = kAhead + 2;
+  static constexpr int kRowLoads = (TI + 1) / 2;                     // A rows' loads a lane issues a step (of an odd TI the last wavefronts' fetch rows again)
+  static constexpr int kStageChunks = 64 * kRowLoads * kChunksPerRow;
+};
+// 32-row tiles of a tile at most: of unquantized banks the registers that a step's weights take leave seven.
+template <int FORMAT>
+constexpr int kMostTiles = FORMAT == DEW_MOE_W_BF16 ? 7 : 8;
+
 template <int FORMAT, bool PAIRED, int TI>
 __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile tile, u32x4_t* lds, float* depth_scales) {
-  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4;
+  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4, kBf16 = FORMAT == DEW_MOE_W_BF16;
   constexpr bool kBlockBank = FORMAT == DEW_MOE_W_FP8_BLOCK;
-  constexpr int kAtomK = kFp4 ? 64 : 32, kAtoms = BK / kAtomK;
-  constexpr int kRowLoads = (TI + 1) / 2;   // A rows' loads a lane issues a step (of an odd TI the last wavefronts' fetch rows again)
-  constexpr int kSets = 4;
+  constexpr int kAtomK = kFp4 ? 64 : kBf16 ? 16 : 32, kAtoms = BK / kAtomK;
+  using Depth = TallDepth<FORMAT, TI>;
+  constexpr int kAhead = Depth::kAhead, kStages = Depth::kStages, kSets = Depth::kSets, kRowLoads = Depth::kRowLoads, kStageChunks = Depth::kStageChunks;
   constexpr int kLoadsB = kAtoms + (kFp4 ? 1 : 0);
 
   const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64);
@@ -96,7 +118,10 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
   auto load_b = [&](auto set, int step) __attribute__((always_inline)) {
     const uint8_t* from = b_src + static_cast<size_t>(step) * (kAtoms * kAtomBytes);
 #pragma unroll
-    for (int a = 0; a < kAtoms; ++a) b_regs[set.value][a] = *reinterpret_cast<const u32x4_t*>(from + a * kAtomBytes + lane * 16);
+    for (int a = 0; a < kAtoms; ++a) {
+      const u32x4_t* at = reinterpret_cast<const u32x4_t*>(from + a * kAtomBytes + lane * 16);
+      b_regs[set.value][a] = kBf16 ? __builtin_nontemporal_load(at) : *at;  // (unquantized: taken where most groups are one tile, which reads them once)
+    }
     if constexpr (kFp4) s_regs[set.value] = *reinterpret_cast<const uint16_t*>(b_scale_src + static_cast<size_t>(step) * 128 + lane * 2);
   };
 
@@ -122,10 +147,7 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
   }
   constexpr std::integral_constant<int, 0> c0{};
   constexpr std::integral_constant<int, 1> c1{};
-  constexpr std::integral_constant<int, 2> c2{};
-  load_b(c0, 0);
-  load_b(c1, min(1, steps - 1));
-  load_b(c2, min(2, steps - 1));
+  static_for<kSets - 1>([&](auto set) __attribute__((always_inline)) { load_b(set, min(decltype(set)::value, steps - 1)); });
   const bf16_t* a_src[kRowLoads];
 #pragma unroll
   for (int i = 0; i < kRowLoads; ++i) {
@@ -150,7 +172,7 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
   uint32_t slice_at[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk)
-    slice_at[kk] = 16 * swizzled(lane % 32, kFp4 ? 4 * (lane / 32) + kk : 4 * (kk / 2) + 2 * (lane / 32) + kk % 2);
+    slice_at[kk] = 16 * swizzled(lane % 32, kFp4 ? 4 * (lane / 32) + kk : kBf16 ? 2 * kk + lane / 32 : 4 * (kk / 2) + 2 * (lane / 32) + kk % 2);
   auto fetch = [&](uint32_t stage, auto kk) __attribute__((always_inline)) {  // (`stage` in bytes)
     const uint8_t* from = reinterpret_cast<const uint8_t*>(lds) + (slice_at[kk.value] + stage);
 #pragma unroll
@@ -160,7 +182,8 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
   float block_scale = 1.0f;  // FP8 blocks: the scale of the step whose slices are brought to bf16
   auto dequantize = [&](auto set, auto kk, auto part) __attribute__((always_inline)) {
     u32x4_t& fragment = b_frag[kk.value % 2];
-    if constexpr (kFp4) {
+    if constexpr (kBf16) {  // (the atoms are the fragments)
+    } else if constexpr (kFp4) {
       if constexpr (kk.value % 2 == 0 && part.value == 0) {  // slices 0, 1 lie in the lane's first 16-deep block, 2, 3 in its second
         const float scale = kk.value == 0 ? __builtin_amdgcn_cvt_f32_fp8(s_regs[set.value], 0) : __builtin_amdgcn_cvt_f32_fp8(s_regs[set.value], 1);
         fp4_scale = scale * 0.00390625f;
@@ -177,30 +200,30 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
   for (int i = 0; i < TI; ++i)
 #pragma unroll
     for (int q = 0; q < 16; ++q) acc[i][q] = 0.0f;
-  auto multiply = [&](auto kk) __attribute__((always_inline)) {
+  auto multiply = [&](auto set, auto kk) __attribute__((always_inline)) {
+    const bf16x8_t b = __builtin_bit_cast(bf16x8_t, kBf16 ? b_regs[set.value][kk.value % kAtoms] : b_frag[kk.value % 2]);
 #pragma unroll
-    for (int i = 0; i < TI; ++i) {
-      acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_frag[kk.value % 2][i], __builtin_bit_cast(bf16x8_t, b_frag[kk.value % 2]), acc[i], 0, 0, 0);
-    }
+    for (int i = 0; i < TI; ++i) acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a_frag[kk.value % 2][i], b, acc[i], 0, 0, 0);
   };
 
-  // ---- pipeline: the ring and the waits of gemm.hip. A step's loads go out as A rows (of step s + 2) and then weights (of step
-  // s + 3), all before the barrier in front of the step's last phase, which waits for the A rows that step s - 1 asked for: younger
-  // are that step's weights and all loads of this one. So the weights of step s + 1, asked for in step s - 2, have landed there
-  // too, and the last phase brings their first slice to bf16. ----
-  constexpr int kYounger = 2 * kLoadsB + kRowLoads;
+  // ---- pipeline: the ring and the waits of gemm.hip. A step's loads go out as A rows (of step s + kAhead) and then weights (of step
+  // s + kAhead + 1), all before the barrier in front of the step's last slice, which waits for the A rows of step s + 1, asked for in step
+  // s + 1 - kAhead: younger are that step's weights and all loads since. So the weights of step s + 1, asked for one step before those
+  // rows, have landed there too, and the last slice brings their first one to bf16. ----
+  constexpr int kYounger = (kAhead - 1) * (kRowLoads + kLoadsB) + kLoadsB;
+  static_assert(kYounger < 64, "vmcnt is a 6-bit counter");
   constexpr int kWaitLanded = (kYounger & 0xF) | (7 << 4) | (0 << 8) | ((kYounger >> 4) << 14);
   constexpr int kWaitAll = (0 & 0xF) | (7 << 4) | (0 << 8) | (0 << 14);
   int stage_index = 0;
   auto iterate = [&](auto set, int step, auto last_steps) __attribute__((always_inline)) {
     constexpr std::integral_constant<int, (set.value + 1) % kSets> following{};
     constexpr std::integral_constant<int, (set.value + kSets - 1) % kSets> filling{};
-    const int next_index = stage_index == kTallStages - 1 ? 0 : stage_index + 1;
-    const int fill_index = next_index == kTallStages - 1 ? 0 : next_index + 1;
-    uint32_t current = stage_index * (kTallStageChunks * 16), next = next_index * (kTallStageChunks * 16);
+    const int next_index = stage_index == kStages - 1 ? 0 : stage_index + 1;
+    const int fill_index = stage_index == 0 ? kStages - 1 : stage_index - 1;
+    uint32_t current = stage_index * (kStageChunks * 16), next = next_index * (kStageChunks * 16);
     asm volatile("" : "+s"(current), "+s"(next));  // (formed here: hoisted out of the loop, every stage's and slice's addresses fill registers)
-    u32x4_t* fill = lds + fill_index * kTallStageChunks;
-    const int ahead_a = min(step + 2, steps - 1), ahead_b = min(step + kSets - 1, steps - 1);
+    u32x4_t* fill = lds + fill_index * kStageChunks;
+    const int ahead_a = min(step + kAhead, steps - 1), ahead_b = min(step + kSets - 1, steps - 1);
     static_range<0>(std::make_integer_sequence<int, 4>{}, [&](auto kk) __attribute__((always_inline)) {
       constexpr int slice = decltype(kk)::value;
       constexpr bool kLast = slice == 3;
@@ -217,7 +240,7 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
       if constexpr (kBlockBank && kLast) block_scale = next_scale;
       dequantize(deq_set, next_kk, c0);
       dequantize(deq_set, next_kk, c1);
-      multiply(kk);
+      multiply(set, kk);
       if constexpr (kBlockBank && slice == 2) next_scale = depth_scales[side * kScaleRow + (step + 1) / (128 / BK)];
       constexpr int a_each = (kRowLoads + 1) / 2;
       constexpr int a_begin = slice * a_each < kRowLoads ? slice * a_each : kRowLoads;
@@ -226,14 +249,15 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
       load_a(fill, ahead_a, std::integral_constant<int, a_begin>{}, std::integral_constant<int, a_end>{});
       if constexpr (kWeights) load_b(filling, ahead_b);
       constexpr int kLoads = a_end - a_begin + (kWeights ? kLoadsB : 0);
-      schedule_slice<0, TI, TI + (kBlockBank && slice == 2 ? 1 : 0), 17 + 2 * kLoads, kLoads>();
+      schedule_slice<0, TI, TI + (kBlockBank && slice == 2 ? 1 : 0), (kBf16 ? 0 : 17) + 2 * kLoads, kLoads>();
       __builtin_amdgcn_sched_barrier(0);
     });
     stage_index = next_index;
   };
   constexpr std::integral_constant<int, kRowLoads> every_row{};
-  load_a(lds, 0, c0, every_row);
-  load_a(lds + kTallStageChunks, min(1, steps - 1), c0, every_row);
+  static_for<kAhead>([&](auto stage) __attribute__((always_inline)) {
+    load_a(lds + decltype(stage)::value * kStageChunks, min(decltype(stage)::value, steps - 1), c0, every_row);
+  });
   if constexpr (kBlockBank) {
     static_assert(2 * kMaxDepthBlocks <= kTallThreads, "one scale a thread");
     if (tid < 2 * depth_blocks) depth_scales[tid / depth_blocks * kScaleRow + tid % depth_blocks] = early_scale;
@@ -372,7 +396,7 @@ template <int FORMAT, bool PAIRED>
 __global__ __launch_bounds__(kTallThreads, 2) void tall_kernel(GemmParams p) {
   extern __shared__ u32x4_t lds[];
   __shared__ float depth_scales[FORMAT == DEW_MOE_W_FP8_BLOCK ? 2 * kScaleRow : 1];
-  constexpr int kColumns = TallStaging<PAIRED>::kColumns;
+  constexpr int kColumns = TallStaging<PAIRED>::kColumns, kMostRows = 32 * kMostTiles<FORMAT>;
   const int tid = threadIdx.x, lane = tid % 64;
 
   // block -> (m-tile, strip), as in gemm.hip: chunks of group_m m-tiles x 8 strips dealt round-robin to the XCDs
@@ -403,13 +427,13 @@ __global__ __launch_bounds__(kTallThreads, 2) void tall_kernel(GemmParams p) {
       start = carried_rows + rows - size;
       carried_rows += __builtin_amdgcn_readlane(rows, 63);
     }
-    const int tiles = (size + kTallRows - 1) / kTallRows;
+    const int tiles = (size + kMostRows - 1) / kMostRows;
     const int inclusive = lanes_scanned(tiles), first = carried + inclusive - tiles;
     const unsigned long long hit = __ballot(m_tile >= first && m_tile < first + tiles);
     if (hit != 0ull) {
       const int owner = __builtin_ctzll(hit);
       expert = base + owner;
-      const int group_size = __builtin_amdgcn_readlane(size, owner), group_tiles = (group_size + kTallRows - 1) / kTallRows;
+      const int group_size = __builtin_amdgcn_readlane(size, owner), group_tiles = (group_size + kMostRows - 1) / kMostRows;
       const int rows_each = ((group_size + 31) / 32 + group_tiles - 1) / group_tiles * 32;  // equally many 32-row tiles each
       const int begin = (m_tile - __builtin_amdgcn_readlane(first, owner)) * rows_each;
       row0 = __builtin_amdgcn_readlane(start, owner) + begin;
@@ -420,8 +444,8 @@ __global__ __launch_bounds__(kTallThreads, 2) void tall_kernel(GemmParams p) {
   }
   asm volatile("" : "+s"(expert), "+s"(row0), "+s"(valid_rows));  // (the loop ends here: the tile's code is not to be laid inside it)
   if (expert < 0) {  // past the last tile: the rows no expert owns are zero
-    const int tail_begin = (p.sizes ? carried_rows : p.offsets[p.experts]) + (m_tile - carried) * kTallRows;
-    const int tail_end = min(tail_begin + kTallRows, p.rows);
+    const int tail_begin = (p.sizes ? carried_rows : p.offsets[p.experts]) + (m_tile - carried) * kMostRows;
+    const int tail_end = min(tail_begin + kMostRows, p.rows);
     for (int item = tid; item < (tail_end - tail_begin) * (kColumns / 8); item += kTallThreads) {
       const int sorted = tail_begin + item / (kColumns / 8), at = n0 + (item % (kColumns / 8)) * 8;
       const int row = p.scatter ? p.scatter[sorted] : sorted;
@@ -432,7 +456,9 @@ __global__ __launch_bounds__(kTallThreads, 2) void tall_kernel(GemmParams p) {
   if (valid_rows <= 0) return;  // (a group whose equal tiles end before its last one)
   const TallTile tile{expert, row0, valid_rows, n0};
   switch ((valid_rows + 31) / 32) {
-    case 8: return tall_tile<FORMAT, PAIRED, 8>(p, tile, lds, depth_scales);
+    case 8:
+      if constexpr (kMostTiles<FORMAT> == 8) return tall_tile<FORMAT, PAIRED, 8>(p, tile, lds, depth_scales);
+      return;
     case 7: return tall_tile<FORMAT, PAIRED, 7>(p, tile, lds, depth_scales);
     case 6: return tall_tile<FORMAT, PAIRED, 6>(p, tile, lds, depth_scales);
     case 5: return tall_tile<FORMAT, PAIRED, 5>(p, tile, lds, depth_scales);
@@ -442,17 +468,25 @@ __global__ __launch_bounds__(kTallThreads, 2) void tall_kernel(GemmParams p) {
   }
 }
 
+template <int FORMAT, int... TILES>
+constexpr size_t largest_ring(std::integer_sequence<int, TILES...>) {
+  size_t most = 0;
+  ((most = std::max(most, static_cast<size_t>(TallDepth<FORMAT, TILES + 1>::kStages) * TallDepth<FORMAT, TILES + 1>::kStageChunks * 16)), ...);
+  return most;
+}
+
 template <int FORMAT, bool PAIRED>
 static int launch_tall_kernel(const char* who, GemmParams p, hipStream_t stream) {
-  constexpr size_t ring = static_cast<size_t>(kTallStages) * kTallStageChunks * 16;
-  constexpr size_t kShared = TallStaging<PAIRED>::kBytes > ring ? TallStaging<PAIRED>::kBytes : ring;
+  constexpr size_t kShared = TallStaging<PAIRED>::kBytes;
+  static_assert(largest_ring<FORMAT>(std::make_integer_sequence<int, kMostTiles<FORMAT>>{}) <= kShared, "the rings fit what the staged tile takes");
   auto kernel = tall_kernel<FORMAT, PAIRED>;
   static std::once_flag configured;
   static hipError_t reserved = hipSuccess;
   std::call_once(configured, [&] { reserved = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kShared)); });
   if (reserved != hipSuccess) return fail(DEW_MOE_ELAUNCH, "%s: cannot reserve %zu bytes of LDS", who, kShared);
   constexpr int kColumns = TallStaging<PAIRED>::kColumns;
-  p.m_tile_bound = (p.rows + kTallRows - 1) / kTallRows + p.experts + 1;
+  constexpr int kMostRows = 32 * kMostTiles<FORMAT>;
+  p.m_tile_bound = (p.rows + kMostRows - 1) / kMostRows + p.experts + 1;
   p.group_m = 2;
   const int total = p.m_tile_bound * ((p.width + kColumns - 1) / kColumns), round = 64 * p.group_m;
   hipLaunchKernelGGL(kernel, dim3((total + round - 1) / round * round), dim3(kTallThreads), kShared, stream, p);
@@ -465,6 +499,8 @@ int launch_tall(const char* who, const GemmParams& p, int format, bool paired, h
       return paired ? launch_tall_kernel<DEW_MOE_W_FP8_BLOCK, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_FP8_BLOCK, false>(who, p, stream);
     case DEW_MOE_W_FP8_CHANNEL:
       return paired ? launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, false>(who, p, stream);
+    case DEW_MOE_W_BF16:
+      return paired ? launch_tall_kernel<DEW_MOE_W_BF16, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_BF16, false>(who, p, stream);
     default:
       return launch_tall_kernel<DEW_MOE_W_NVFP4, false>(who, p, stream);
   }
