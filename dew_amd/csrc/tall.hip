@@ -13,7 +13,7 @@
 // tiles (each count its own copy of the main loop), so that a group's last rows need neither a launch of their own nor a tile that is
 // mostly empty.
 //
-// Cycles of a tile of 256 rows, FP8, 2048 deep (one bank): 7800 until its first step, 74 000 in 32 steps (the matrix pipe 88 % busy),
+// Cycles of a tile of 256 rows, FP8, 2048 deep (one bank): some 7000 until its first step, 74 000 in 32 steps (the matrix pipe 88 % busy),
 // 7400 until its last store; paired 96 000, of which 13 000 are both matrices' sums' arithmetic. Tried and not kept, all the same to a
 // percent: several strips a block with the next one's loads under the epilogue (the clock gives back what the wait took: the chip's power
 // is the bound); blocks of four wavefronts, two a CU (quantized banks 4 % slower, their rows are fetched twice as often).
@@ -395,8 +395,11 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
   }
 }
 
-template <int FORMAT, bool PAIRED>
-__global__ __launch_bounds__(kTallThreads, 2) void tall_kernel(GemmParams p) {
+// (MODE: kPlain or kSwigluOfTwo; gemm.hip's kernels of the same name are the shorter tiles', of four wavefronts)
+template <int FORMAT, int MODE, int WAVES>
+__global__ __launch_bounds__(64 * WAVES, 2) void grouped_gemm_kernel(GemmParams p) {
+  constexpr bool PAIRED = MODE == kSwigluOfTwo;
+  static_assert(64 * WAVES == kTallThreads, "eight wavefronts");
   extern __shared__ u32x4_t lds[];
   __shared__ float depth_scales[FORMAT == DEW_MOE_W_FP8_BLOCK ? 2 * kScaleRow : 1];
   constexpr int kColumns = TallStaging<PAIRED>::kColumns, kMostRows = 32 * kMostTiles<FORMAT>;
@@ -482,7 +485,7 @@ template <int FORMAT, bool PAIRED>
 static int launch_tall_kernel(const char* who, GemmParams p, hipStream_t stream) {
   constexpr size_t kShared = TallStaging<PAIRED>::kBytes;
   static_assert(largest_ring<FORMAT>(std::make_integer_sequence<int, kMostTiles<FORMAT>>{}) <= kShared, "the rings fit what the staged tile takes");
-  auto kernel = tall_kernel<FORMAT, PAIRED>;
+  auto kernel = grouped_gemm_kernel<FORMAT, PAIRED ? kSwigluOfTwo : kPlain, kTallThreads / 64>;
   static std::once_flag configured;
   static hipError_t reserved = hipSuccess;
   std::call_once(configured, [&] { reserved = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kShared)); });
