@@ -152,7 +152,7 @@ int launch_few_combined(const char* who, const GemmParams& p, int format, const 
                         hipStream_t stream);
 
 // The launch in tiles of up to 256 rows on eight wavefronts (tall.hip); of FP8 or bf16 banks, one or two (gate and up,
-// gated), or of one FP4 bank.
+// gated), or of one NVFP4 bank.
 int launch_tall(const char* who, const GemmParams& p, int format, bool paired, hipStream_t stream);
 
 }  // namespace dew

@@ -1200,8 +1200,8 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 // four, 32 x 244 of 3584 x 2816 paired 341 -> 394, 32 x 359 of 6656 x 4352 670 -> 706); above, no faster (36 x 1820 of 4096 x 7936 7045, 7084).
 // General NVFP4 in one bank, groups of 130 to 1100 rows on 2304 deep or more: 70 x 209 of 2304 x 7424 739 -> 553, 64 x 295 of 2560 x 4096 455 ->
 // 396, 64 x 1024 of 2304 x 3840 1062 -> 1042; shallower or smaller ones lose up to 14 %, paired ones 2 to 8 %.
-// MXFP4 in one bank, groups of 70 to 300 rows on 3000 deep or more in two and a half rounds: 32 x 239 of 4352 x 7168 574 -> 455, 69 x 179 of 6144 x 2816
-// 515 -> 435, 145 x 94 of 5376 x 1536 280 -> 272; its codes cost so little that pairs and smaller launches lose up to 20 %.
+// MXFP4 codes cost the vector unit so little that the shorter tiles, two blocks a CU, are the faster ones: over 626 shapes of 70 to 300 rows a group, 3000 deep
+// or more, in two and a half rounds and more, 1.06 times as fast in the mean (128 x 265 of 3328 x 896 213 -> 277, 64 x 194 of 3584 x 2176 203 -> 265).
 // Unquantized, 110 shapes: groups of up to 300 rows in whole rounds of blocks or many, from 45 rows and 1000 deep on in one bank and 28 and 2500
 // paired: 25 x 126 of 5120 x 4608 304 -> 242, 256 x 132 of 1280 x 1280 250 -> 203, 24 x 60 of 3584 x 6912 252 -> 224; paired 32 x 181 of 6656 x 1280
 // 374 -> 273, 16 x 131 of 4096 x 7936 566 -> 437, 25 x 29 of 4864 x 4864 458 -> 380; at worst 183 x 238 of 2560 x 1280 418 -> 436. Outside the lines: a
@@ -1216,7 +1216,7 @@ static bool tall_tiles(const GemmParams& p, int format, bool paired) {
     return average < 300 && (paired ? average >= 28 && p.depth >= 2500 : average >= 45 && p.depth >= 1000) && rounds >= 0.85 &&
            (rounds >= 5 || rounds >= 0.8 * ceil(rounds));
   }
-  if (format == DEW_MOE_W_MXFP4) return average >= 70 && average <= 300 && p.depth >= 3000 && tiles >= 680;
+  if (format == DEW_MOE_W_MXFP4) return false;
   if (format == DEW_MOE_W_NVFP4) return average >= 130 && average <= 1100 && p.depth >= 2304 && tiles >= 560;
   return p.depth >= 2048 && average >= 76 && average <= 450 && tiles >= (average > 200 ? 1800 : paired ? 336 : 190);
 }
@@ -1228,7 +1228,7 @@ static int launch_format(const char* who, const GemmParams& p, hipStream_t strea
   // than one 256-row block; a one-bank launch the same there and 4 to 7 % slower on 4096-row groups, so it keeps the taller tile)
   constexpr bool kPaired = MODE == kSwigluOfTwo;
   constexpr bool kFp4 = FORMAT == DEW_MOE_W_MXFP4 || FORMAT == DEW_MOE_W_BF16 || (FORMAT == DEW_MOE_W_NVFP4 && !kPaired);
-  constexpr bool kTall = FORMAT == DEW_MOE_W_BF16 || FORMAT == DEW_MOE_W_FP8_BLOCK || FORMAT == DEW_MOE_W_FP8_CHANNEL || ((FORMAT == DEW_MOE_W_NVFP4 || FORMAT == DEW_MOE_W_MXFP4) && !kPaired);
+  constexpr bool kTall = FORMAT == DEW_MOE_W_BF16 || FORMAT == DEW_MOE_W_FP8_BLOCK || FORMAT == DEW_MOE_W_FP8_CHANNEL || (FORMAT == DEW_MOE_W_NVFP4 && !kPaired);
   if constexpr (kTall && (MODE == kPlain || kPaired)) {
     if (tall_tiles(p, FORMAT, kPaired)) return launch_tall(who, p, FORMAT, kPaired, stream);
   }
@@ -1351,6 +1351,17 @@ static bool wide_fp8_gradient_extents(int tokens, int depth, int width, int grou
 }
 
 }  // namespace dew
+
+extern "C" int dew_moe_takes_tall_tiles(const dew_moe_bank* bank, int32_t paired, int32_t rows) {
+  using namespace dew;
+  if (!bank || bank->layout != DEW_MOE_LAYOUT_PREPARED || bank->experts < 1 || rows < 1) return 0;
+  GemmParams p{};
+  p.experts = bank->experts;
+  p.depth = bank->depth;
+  p.width = bank->width;
+  p.rows = rows;
+  return tall_tiles(p, bank->format, paired != 0) ? 1 : 0;
+}
 
 extern "C" int dew_moe_tile_rows(int32_t rows) {
   using namespace dew;

@@ -43,17 +43,14 @@ struct TallTile {
   int expert, row0, valid_rows, n0;
 };
 
-// Half of a slice's fragment (words 2 part, 2 part + 1: four of the lane's eight weights), with the arithmetic of fragment_fp8,
-// fragment_fp4 and fragment_fp4_pow2.
+// Half of a slice's fragment (words 2 part, 2 part + 1: four of the lane's eight weights), with the arithmetic of fragment_fp8 and
+// fragment_fp4.
 template <int FORMAT, int PART>
 __device__ __forceinline__ void dequantize_half(u32x4_t& fragment, uint32_t word, float scale) {
   if constexpr (FORMAT == DEW_MOE_W_NVFP4) {
     const f32x2_t a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 2 * PART), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, 2 * PART + 1);
     fragment[2 * PART] = pack_bf16(a.x * scale, a.y * scale);
     fragment[2 * PART + 1] = pack_bf16(b.x * scale, b.y * scale);
-  } else if constexpr (FORMAT == DEW_MOE_W_MXFP4) {
-    fragment[2 * PART] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, 2 * PART));
-    fragment[2 * PART + 1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, 2 * PART + 1));
   } else {
     const f32x2_t a = __builtin_amdgcn_cvt_pk_f32_fp8(word, false), b = __builtin_amdgcn_cvt_pk_f32_fp8(word, true);
     fragment[2 * PART] = pack_bf16(a.x * scale, a.y * scale);
@@ -90,7 +87,7 @@ constexpr int kMostTiles = FORMAT == DEW_MOE_W_BF16 ? 7 : 8;
 
 template <int FORMAT, bool PAIRED, int TI>
 __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile tile, u32x4_t* lds, float* depth_scales) {
-  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4 || FORMAT == DEW_MOE_W_MXFP4, kBf16 = FORMAT == DEW_MOE_W_BF16;
+  constexpr bool kFp4 = FORMAT == DEW_MOE_W_NVFP4, kBf16 = FORMAT == DEW_MOE_W_BF16;
   constexpr bool kBlockBank = FORMAT == DEW_MOE_W_FP8_BLOCK;
   constexpr int kAtomK = kFp4 ? 64 : kBf16 ? 16 : 32, kAtoms = BK / kAtomK;
   using Depth = TallDepth<FORMAT, TI>;
@@ -252,7 +249,7 @@ __device__ __forceinline__ void tall_tile(const GemmParams& p, const TallTile ti
       load_a(fill, ahead_a, std::integral_constant<int, a_begin>{}, std::integral_constant<int, a_end>{});
       if constexpr (kWeights) load_b(filling, ahead_b);
       constexpr int kLoads = a_end - a_begin + (kWeights ? kLoadsB : 0);
-      schedule_slice<0, TI, TI + (kBlockBank && slice == 2 ? 1 : 0), (kBf16 ? 0 : FORMAT == DEW_MOE_W_MXFP4 ? 5 : 17) + 2 * kLoads, kLoads>();
+      schedule_slice<0, TI, TI + (kBlockBank && slice == 2 ? 1 : 0), (kBf16 ? 0 : 17) + 2 * kLoads, kLoads>();
       __builtin_amdgcn_sched_barrier(0);
     });
     stage_index = next_index;
@@ -507,8 +504,6 @@ int launch_tall(const char* who, const GemmParams& p, int format, bool paired, h
       return paired ? launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, false>(who, p, stream);
     case DEW_MOE_W_BF16:
       return paired ? launch_tall_kernel<DEW_MOE_W_BF16, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_BF16, false>(who, p, stream);
-    case DEW_MOE_W_MXFP4:
-      return launch_tall_kernel<DEW_MOE_W_MXFP4, false>(who, p, stream);
     default:
       return launch_tall_kernel<DEW_MOE_W_NVFP4, false>(who, p, stream);
   }

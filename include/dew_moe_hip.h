@@ -254,6 +254,10 @@ int dew_moe_prepared_view(int32_t format, int32_t experts, int32_t depth, int32_
  * default, chooses per launch from the rows, experts and width. The setting is thread-local: other threads' launches
  * (an FFI thread pool's) keep their own choice.                                                              */
 int dew_moe_tile_rows(int32_t rows);
+/* Whether a product of `rows` bf16 rows in all with this bank (`paired`: with it and a second one of its extents, gated) is launched by the
+ * calling thread in tiles of up to 256 rows on eight wavefronts (csrc/tall.hip; 1) or in shorter ones (0): the launches' own rule, for
+ * tests. Only the descriptor's format, layout and extents are read.                                                                   */
+int dew_moe_takes_tall_tiles(const dew_moe_bank* bank, int32_t paired, int32_t rows);
 
 /* ---- Grouped products (src/dew/nn/moe.py:666-770 expert_projection / paired_projections; replaces the
  *      launches of kernels/cutlass/ffi.cu:180-220 behind src/dew/nn/kernels/grouped_matmul.py:1826-1831) --

@@ -14,10 +14,10 @@ SIZES = {"fp8": [0, 1, 31, 32, 33, 64, 65, 96, 97, 128, 161, 192, 193, 224, 256,
 
 
 def banks(form, experts, depth, width, count):
-    from dew_amd import codecs, formats
+    from dew_amd import formats
 
     quantized = {"block": formats.Fp8Blocks.quantized, "channel": formats.Fp8Channels.quantized, "nvfp4": formats.NvFp4.quantized,
-                 "mxfp4": lambda w: formats.Mxfp4Blocks(*codecs.quantize_mxfp4(w)), "bf16": lambda w: formats.Bf16(w.to(torch.bfloat16))}[form]
+                 "bf16": lambda w: formats.Bf16(w.to(torch.bfloat16))}[form]
     generator = torch.Generator(device="cuda").manual_seed(depth + width)
     return [formats.stacked([quantized(torch.randn(1, depth, width, device="cuda", generator=generator) * 0.02 * (e % 3 + 1)) for e in range(experts)])
             for _ in range(count)]
@@ -30,7 +30,6 @@ def banks(form, experts, depth, width, count):
     ("channel", "fp8", 2432, 3200, False, None),    # 38 steps
     ("block", "several tiles", 2048, 16640, True, None),
     ("nvfp4", "nvfp4", 2304, 8064, False, None),   # a last strip of 128 columns
-    ("mxfp4", "nvfp4", 3008, 9696, False, None),   # 47 steps; a last strip of 224 columns
     ("bf16", "fp8", 2560, 1568, True, None),        # 40 steps; a last strip of 32 columns; tiles of at most 224 rows
     ("bf16", "fp8", 2880, 1664, True, 0.75),        # 45 steps
     ("bf16", "fp8", 1088, 3232, False, None),       # 17 steps; a last strip of 160 columns

@@ -1,0 +1,29 @@
+"""Which launches take tiles of up to 256 rows on eight wavefronts (dew_moe_takes_tall_tiles, csrc/gemm.hip): a rule that can be asked without
+a GPU. The shapes are ones where both launches were timed; times in us, the shorter tiles' and the tall ones'."""
+
+import pytest
+
+from dew_amd import _lib
+
+BLOCK, CHANNEL, NVFP4, MXFP4, BF16 = _lib.W_FP8_BLOCK, _lib.W_FP8_CHANNEL, _lib.W_NVFP4, _lib.W_MXFP4, _lib.W_BF16
+
+
+def taken(form, experts, rows, depth, width, paired=False, layout=_lib.LAYOUT_PREPARED):
+    return bool(_lib.library().dew_moe_takes_tall_tiles(_lib.Bank(form, layout, experts, depth, width, None, None, None), paired, experts * rows))
+
+
+@pytest.mark.parametrize("experts,rows,depth,width", [
+    (128, 265, 3328, 896),     # 213 -> 277
+    (64, 194, 3584, 2176),     # 203 -> 265
+    (128, 284, 3968, 896),     # 267 -> 345
+    (32, 239, 4352, 7168)])
+def test_mxfp4_banks_stay_on_the_shorter_tiles(experts, rows, depth, width):
+    assert not taken(MXFP4, experts, rows, depth, width)
+    assert not taken(MXFP4, experts, rows, depth, width, paired=True)
+
+
+def test_what_is_no_prepared_bank_or_has_no_rows_takes_none():
+    assert taken(BF16, 24, 112, 7040, 2432)                          # 233 -> 148
+    assert not taken(BF16, 24, 0, 7040, 2432) and not taken(BF16, 24, -112, 7040, 2432)
+    assert not taken(BF16, 24, 112, 7040, 2432, layout=_lib.LAYOUT_REFERENCE)
+    assert _lib.library().dew_moe_takes_tall_tiles(None, 0, 100) == 0
