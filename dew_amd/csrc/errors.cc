@@ -44,7 +44,7 @@ const char* dew_moe_kernels(void) {
          "permute_small|permute_count+scan+scatter,2048 slots/block,-,-,4,-,i32 ballot+LDS histogram\n"
          "grouped_gemm<large>,256,256 (paired 2x128),64,4 (1x4),v_mfma_f32_32x32x16_bf16,bf16 rows via global_load_lds x nvfp4|mxfp4 fragments from global; 1 block/CU\n"
          "grouped_gemm<medium>,128,256 (paired 2x128) | 128,64,4 (1x4),v_mfma_f32_32x32x16_bf16,bf16 x {fp8 block|fp8 channel|nvfp4|mxfp4}; 2 blocks/CU\n"
-         "grouped_gemm<tall>,up to 256 (a multiple of 32 a group),256 (paired 2x128),64,8 (1x8),v_mfma_f32_32x32x16_bf16,bf16 x {fp8 block|fp8 channel|nvfp4|bf16}: groups of 28 to 450 rows (nvfp4 to 1100); 1 block/CU\n"
+         "grouped_gemm<tall>,up to 256 (a multiple of 32 a group),256 (paired 2x128),64,8 (1x8),v_mfma_f32_32x32x16_bf16,bf16 x {fp8 block|fp8 channel|nvfp4|bf16}: groups of 28 to 450 rows (nvfp4 130 to 215); 1 block/CU\n"
          "grouped_gemm<decode>,32,128 (paired 2x128),64,4 (1x4),v_mfma_f32_32x32x16_bf16,weight streaming for groups under 24 rows\n"
          "grouped_gemm epilogues,-,-,-,-,-,plain (+bias) | swiglu of two banks | interleaved gate/up clamped 1.702 gating (+bias); tile staged in LDS and stored as whole rows\n"
          "grouped_gemm<split rows>,128 (paired; 2 blocks/CU) | 256,256 (paired 2x128),64,4 (2x2),v_mfma_scale_f32_32x32x64_f8f6f4,two e4m3 terms per bf16 activation x mxfp4 codes as stored; SwiGLU rows written already split\n"

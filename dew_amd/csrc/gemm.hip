@@ -1198,8 +1198,10 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 // at worst 30 x 106 of 6656 x 5888 733 -> 758; of 0.4 rounds 8 x 105 of 4096 x 3328 44 -> 66, depths of 768 to 1536 4 % slower); to 450 rows
 // only with seven rounds, whose last is a small part (114 x 298 of 5120 x 2048 paired 1560 -> 1495, 203 x 277 of 2560 x 2304 749 -> 725; at
 // four, 32 x 244 of 3584 x 2816 paired 341 -> 394, 32 x 359 of 6656 x 4352 670 -> 706); above, no faster (36 x 1820 of 4096 x 7936 7045, 7084).
-// General NVFP4 in one bank, groups of 130 to 1100 rows on 2304 deep or more: 70 x 209 of 2304 x 7424 739 -> 553, 64 x 295 of 2560 x 4096 455 ->
-// 396, 64 x 1024 of 2304 x 3840 1062 -> 1042; shallower or smaller ones lose up to 14 %, paired ones 2 to 8 %.
+// General NVFP4 in one bank, groups of 130 to 215 rows, one tile each where the shorter launch has two of 128, on 2304 deep or more and from 2.2
+// rounds on: 1.07 times as fast in the mean of 488 shapes (128 x 156 of 3072 x 1024 194 -> 138, 32 x 184 of 3072 x 4096 217 -> 160; at worst 16 x 133 of
+// 2560 x 11776 174 -> 204). Larger groups are 1.4 % slower in the mean of 1310 shapes to 1100 rows (64 x 533 of 3328 x 1280 284 -> 331, 48 x 844 of 2304 x
+// 1536 270 -> 306), shallower or smaller ones lose up to 14 %, paired ones 2 to 8 %.
 // MXFP4 codes cost the vector unit so little that the shorter tiles, two blocks a CU, are the faster ones: over 626 shapes of 70 to 300 rows a group, 3000 deep
 // or more, in two and a half rounds and more, 1.06 times as fast in the mean (128 x 265 of 3328 x 896 213 -> 277, 64 x 194 of 3584 x 2176 203 -> 265).
 // Unquantized, 110 shapes: groups of up to 300 rows in whole rounds of blocks or many, from 45 rows and 1000 deep on in one bank and 28 and 2500
@@ -1217,7 +1219,7 @@ static bool tall_tiles(const GemmParams& p, int format, bool paired) {
            (rounds >= 5 || rounds >= 0.8 * ceil(rounds));
   }
   if (format == DEW_MOE_W_MXFP4) return false;
-  if (format == DEW_MOE_W_NVFP4) return average >= 130 && average <= 1100 && p.depth >= 2304 && tiles >= 560;
+  if (format == DEW_MOE_W_NVFP4) return !paired && average >= 130 && average <= 215 && p.depth >= 2304 && tiles >= 560;
   return p.depth >= 2048 && average >= 76 && average <= 450 && tiles >= (average > 200 ? 1800 : paired ? 336 : 190);
 }
 

@@ -22,6 +22,20 @@ def test_mxfp4_banks_stay_on_the_shorter_tiles(experts, rows, depth, width):
     assert not taken(MXFP4, experts, rows, depth, width, paired=True)
 
 
+@pytest.mark.parametrize("experts,rows,depth,width,tall", [
+    (64, 533, 3328, 1280, False),     # 284 -> 331
+    (48, 844, 2304, 1536, False),     # 270 -> 306
+    (64, 268, 3072, 1536, False),     # 170 -> 217
+    (8, 1024, 14336, 4096, False),    # 839 -> 839
+    (32, 216, 3072, 4096, False),
+    (128, 156, 3072, 1024, True),     # 194 -> 138
+    (64, 161, 3072, 2048, True),      # 195 -> 142
+    (16, 207, 2304, 8192, True)])     # 174 -> 128
+def test_nvfp4_banks_take_them_where_a_group_is_one_tile(experts, rows, depth, width, tall):
+    assert taken(NVFP4, experts, rows, depth, width) == tall
+    assert not taken(NVFP4, experts, rows, depth, width, paired=True)
+
+
 def test_what_is_no_prepared_bank_or_has_no_rows_takes_none():
     assert taken(BF16, 24, 112, 7040, 2432)                          # 233 -> 148
     assert not taken(BF16, 24, 0, 7040, 2432) and not taken(BF16, 24, -112, 7040, 2432)
