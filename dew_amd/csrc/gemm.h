@@ -151,8 +151,8 @@ constexpr int kMostCombinedSlots = 8;  // wavefronts of a block: more have no re
 int launch_few_combined(const char* who, const GemmParams& p, int format, const float* weights, int tokens, int top_k, bool shared, void* out,
                         hipStream_t stream);
 
-// The launch in tiles of up to 256 rows on eight wavefronts (tall.hip); of FP8 or bf16 banks, one or two (gate and up,
-// gated), or of one NVFP4 bank.
+// The launch in tiles of up to 256 rows on eight wavefronts (tall.hip); of FP8 block or bf16 banks, one or two (gate and up,
+// gated), or of one FP8 channel or NVFP4 bank.
 int launch_tall(const char* who, const GemmParams& p, int format, bool paired, hipStream_t stream);
 
 }  // namespace dew

@@ -1198,6 +1198,9 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 // at worst 30 x 106 of 6656 x 5888 733 -> 758; of 0.4 rounds 8 x 105 of 4096 x 3328 44 -> 66, depths of 768 to 1536 4 % slower); to 450 rows
 // only with seven rounds, whose last is a small part (114 x 298 of 5120 x 2048 paired 1560 -> 1495, 203 x 277 of 2560 x 2304 749 -> 725; at
 // four, 32 x 244 of 3584 x 2816 paired 341 -> 394, 32 x 359 of 6656 x 4352 670 -> 706); above, no faster (36 x 1820 of 4096 x 7936 7045, 7084).
+// One scale a channel costs the shorter tiles' loop less than one a block does: pairs gain nothing there (1195 shapes, 1.00 in the mean and 31 % of them more than
+// 5 % slower: 32 x 157 of 3072 x 1664 135 -> 152, 128 x 105 of 2560 x 1152 204 -> 251), nor do one bank's groups of more than 200 rows for certain (67 shapes, 1.04 in the
+// mean, a quarter of them slower, by up to 10 %).
 // General NVFP4 in one bank, groups of 130 to 215 rows, one tile each where the shorter launch has two of 128, on 2304 deep or more and from 2.2
 // rounds on: 1.07 times as fast in the mean of 488 shapes (128 x 156 of 3072 x 1024 194 -> 138, 32 x 184 of 3072 x 4096 217 -> 160; at worst 16 x 133 of
 // 2560 x 11776 174 -> 204). Larger groups are 1.4 % slower in the mean of 1310 shapes to 1100 rows (64 x 533 of 3328 x 1280 284 -> 331, 48 x 844 of 2304 x
@@ -1220,6 +1223,7 @@ static bool tall_tiles(const GemmParams& p, int format, bool paired) {
   }
   if (format == DEW_MOE_W_MXFP4) return false;
   if (format == DEW_MOE_W_NVFP4) return !paired && average >= 130 && average <= 215 && p.depth >= 2304 && tiles >= 560;
+  if (format == DEW_MOE_W_FP8_CHANNEL && (paired || average > 200)) return false;
   return p.depth >= 2048 && average >= 76 && average <= 450 && tiles >= (average > 200 ? 1800 : paired ? 336 : 190);
 }
 
@@ -1230,7 +1234,7 @@ static int launch_format(const char* who, const GemmParams& p, hipStream_t strea
   // than one 256-row block; a one-bank launch the same there and 4 to 7 % slower on 4096-row groups, so it keeps the taller tile)
   constexpr bool kPaired = MODE == kSwigluOfTwo;
   constexpr bool kFp4 = FORMAT == DEW_MOE_W_MXFP4 || FORMAT == DEW_MOE_W_BF16 || (FORMAT == DEW_MOE_W_NVFP4 && !kPaired);
-  constexpr bool kTall = FORMAT == DEW_MOE_W_BF16 || FORMAT == DEW_MOE_W_FP8_BLOCK || FORMAT == DEW_MOE_W_FP8_CHANNEL || (FORMAT == DEW_MOE_W_NVFP4 && !kPaired);
+  constexpr bool kTall = FORMAT == DEW_MOE_W_BF16 || FORMAT == DEW_MOE_W_FP8_BLOCK || ((FORMAT == DEW_MOE_W_FP8_CHANNEL || FORMAT == DEW_MOE_W_NVFP4) && !kPaired);
   if constexpr (kTall && (MODE == kPlain || kPaired)) {
     if (tall_tiles(p, FORMAT, kPaired)) return launch_tall(who, p, FORMAT, kPaired, stream);
   }

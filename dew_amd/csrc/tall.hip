@@ -501,7 +501,7 @@ int launch_tall(const char* who, const GemmParams& p, int format, bool paired, h
     case DEW_MOE_W_FP8_BLOCK:
       return paired ? launch_tall_kernel<DEW_MOE_W_FP8_BLOCK, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_FP8_BLOCK, false>(who, p, stream);
     case DEW_MOE_W_FP8_CHANNEL:
-      return paired ? launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, false>(who, p, stream);
+      return launch_tall_kernel<DEW_MOE_W_FP8_CHANNEL, false>(who, p, stream);
     case DEW_MOE_W_BF16:
       return paired ? launch_tall_kernel<DEW_MOE_W_BF16, true>(who, p, stream) : launch_tall_kernel<DEW_MOE_W_BF16, false>(who, p, stream);
     default:

@@ -26,7 +26,7 @@ def banks(form, experts, depth, width, count):
 @pytest.mark.parametrize("form,sizes,depth,width,paired,limit", [
     ("block", "fp8", 2176, 2944, True, None),       # 34 steps
     ("block", "fp8", 2048, 3200, False, None),      # a last strip of 128 columns
-    ("channel", "fp8", 2048, 2944, True, 0.75),
+    ("block", "fp8", 3072, 3328, True, 0.75),
     ("channel", "fp8", 2432, 3200, False, None),    # 38 steps
     ("block", "several tiles", 2048, 16640, True, None),
     ("nvfp4", "nvfp4", 2304, 8064, False, None),   # a last strip of 128 columns

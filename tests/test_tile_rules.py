@@ -22,6 +22,21 @@ def test_mxfp4_banks_stay_on_the_shorter_tiles(experts, rows, depth, width):
     assert not taken(MXFP4, experts, rows, depth, width, paired=True)
 
 
+@pytest.mark.parametrize("experts,rows,depth,width", [
+    (128, 105, 2560, 1152),    # 204 -> 251
+    (64, 91, 2688, 896),       # 85 -> 106
+    (32, 157, 3072, 1664),     # 135 -> 152
+    (64, 320, 4096, 3072),
+    (8, 147, 5376, 6400)])
+def test_pairs_of_channel_scaled_banks_stay_on_the_shorter_tiles(experts, rows, depth, width):
+    assert not taken(CHANNEL, experts, rows, depth, width, paired=True)
+
+
+def test_channel_scaled_banks_of_large_groups_stay_on_the_shorter_tiles():
+    assert not taken(CHANNEL, 128, 286, 2048, 7168) and not taken(CHANNEL, 64, 201, 4096, 7168)
+    assert taken(CHANNEL, 8, 147, 4480, 6912)                        # 149 -> 87
+
+
 @pytest.mark.parametrize("experts,rows,depth,width,tall", [
     (64, 533, 3328, 1280, False),     # 284 -> 331
     (48, 844, 2304, 1536, False),     # 270 -> 306
