@@ -1191,13 +1191,18 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 }
 
 // Whether a product runs in tiles of up to 256 rows on eight wavefronts (tall.hip), which bring a weight to bf16 once for all rows of the
-// tile, where 128-row tiles do it for every 128. Against the tiles below, over 230 shapes with sizes spread by two fifths around their mean
-// (us, below and there): the steady loop is 8 % faster, and a block alone on its CU shows its start and end, 9 us a tile. So it takes a depth
-// they are small beside. FP8, groups of 76 to 200 rows, one tile each: from 1.3 (paired) and 0.75 rounds of blocks on (16 x 156 rows of 2560 x
-// 3840 in one bank 83 -> 66, 54 x 137 of 6656 x 3328 522 -> 437, 16 x 181 of 6912 x 4864 paired 470 -> 440, 64 x 151 of 6912 x 1024 379 -> 357;
-// at worst 30 x 106 of 6656 x 5888 733 -> 758; of 0.4 rounds 8 x 105 of 4096 x 3328 44 -> 66, depths of 768 to 1536 4 % slower); to 450 rows
-// only with seven rounds, whose last is a small part (114 x 298 of 5120 x 2048 paired 1560 -> 1495, 203 x 277 of 2560 x 2304 749 -> 725; at
-// four, 32 x 244 of 3584 x 2816 paired 341 -> 394, 32 x 359 of 6656 x 4352 670 -> 706); above, no faster (36 x 1820 of 4096 x 7936 7045, 7084).
+// tile, where 128-row tiles do it for every 128. Against the tiles below, timed in turn over some 11 000 shapes with groups' sizes spread by 0.15 to 0.85 around
+// their mean, as balanced and favouring gates spread them (us, below and there): the steady loop is 8 % faster, a group's last tile is no taller than
+// its rows, and a block alone on its CU shows its start and end, 9 us a tile, and leaves a last round that few blocks share as long as a whole one.
+// So it takes a depth that start and end are small beside and rounds that are mostly full.
+// FP8 in one bank, groups of 76 to 200 rows, 2048 deep or more: from 0.75 rounds on, where the rounds' blocks, in whole strips of columns, fill 0.7
+// of the last, in banks of up to 64 experts (a block searches its tile among 64 groups a step, with a wait each). 1.09 times as fast in the mean of 1023 shapes
+// (16 x 141 of 2432 x 3712 85 -> 54, 32 x 197 of 2944 x 1536 101 -> 72, 8 x 150 of 6912 x 7168 216 -> 146); 8 % of them are more than 5 % slower, those whose real sizes come to
+// one round more (16 x 135 of 2560 x 3328, sizes spread by 0.85, 66 -> 82). Past the lines 1.02 in the mean and 42 % of them slower, at worst by
+// two fifths (24 x 95 of 3968 x 2688 103 -> 142, 64 x 145 of 2560 x 640 48 -> 63).
+// Blocks, to 450 rows with seven rounds, whose last is a small part: 1.08 in the mean of 157 shapes, two of them slower, by 5 % at most (203 x 277 of 2560 x 2304 749 ->
+// 725). FP8 block pairs: groups of 76 to 200 rows from 1.3 rounds on, of more with seven (54 x 137 of 6656 x 3328 522 -> 437, 114 x 298 of 5120 x 2048 1560 ->
+// 1495; at four, 32 x 244 of 3584 x 2816 341 -> 394); above, no faster (36 x 1820 of 4096 x 7936 7045, 7084).
 // One scale a channel costs the shorter tiles' loop less than one a block does: pairs gain nothing there (1195 shapes, 1.00 in the mean and 31 % of them more than
 // 5 % slower: 32 x 157 of 3072 x 1664 135 -> 152, 128 x 105 of 2560 x 1152 204 -> 251), nor do one bank's groups of more than 200 rows for certain (67 shapes, 1.04 in the
 // mean, a quarter of them slower, by up to 10 %).
@@ -1213,18 +1218,23 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 // layer of 64 x 104 rows of 2048 x 1408, 2.8 rounds of pairs and 2.03 behind them, 301 -> 318 us; 768 to 1536 deep pairs 8 to 28 % slower, groups of 600 rows 6.
 static bool tall_tiles(const GemmParams& p, int format, bool paired) {
   if (forced_tile_rows != 0) return false;
-  const int average = p.rows / p.experts, columns = paired ? 128 : 256;
-  const long long tiles = (p.rows / 256 + p.experts / 2) * static_cast<long long>((p.width + columns - 1) / columns);
+  const int average = p.rows / p.experts, columns = paired ? 128 : 256, strips = (p.width + columns - 1) / columns;
+  const long long tiles = (p.rows / 256 + p.experts / 2) * static_cast<long long>(strips);
+  // tiles of at most `height` rows that the groups come to, each group's last one half empty, or one a group
+  auto groups_tiles = [&](int height, double last) { return fmax(p.experts, static_cast<double>(p.rows) / height + last * p.experts); };
   if (format == DEW_MOE_W_BF16) {
-    const double most = p.experts > p.rows / 224.0 + 0.55 * p.experts ? p.experts : p.rows / 224.0 + 0.55 * p.experts;
-    const double rounds = most * ((p.width + columns - 1) / columns) / 256;  // of blocks, one a CU
+    const double rounds = groups_tiles(224, 0.55) * strips / 256;  // of blocks, one a CU
     return average < 300 && (paired ? average >= 28 && p.depth >= 2500 : average >= 45 && p.depth >= 1000) && rounds >= 0.85 &&
            (rounds >= 5 || rounds >= 0.8 * ceil(rounds));
   }
   if (format == DEW_MOE_W_MXFP4) return false;
   if (format == DEW_MOE_W_NVFP4) return !paired && average >= 130 && average <= 215 && p.depth >= 2304 && tiles >= 560;
   if (format == DEW_MOE_W_FP8_CHANNEL && (paired || average > 200)) return false;
-  return p.depth >= 2048 && average >= 76 && average <= 450 && tiles >= (average > 200 ? 1800 : paired ? 336 : 190);
+  if (p.depth < 2048 || average < 76) return false;
+  if (average > 200) return average <= 450 && tiles >= 1800;
+  if (paired) return tiles >= 336;
+  const double filled = groups_tiles(256, 0.5);
+  return tiles >= 190 && p.experts <= 64 && filled * p.width / columns >= 0.7 * 256 * ceil(filled * strips / 256);
 }
 
 template <int FORMAT, int MODE>

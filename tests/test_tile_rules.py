@@ -22,6 +22,22 @@ def test_mxfp4_banks_stay_on_the_shorter_tiles(experts, rows, depth, width):
     assert not taken(MXFP4, experts, rows, depth, width, paired=True)
 
 
+@pytest.mark.parametrize("experts,rows,depth,width,tall", [
+    (24, 95, 3968, 2688, False),      # 103 -> 142
+    (16, 91, 4608, 4608, False),      # 117 -> 154
+    (32, 170, 2944, 1664, False),     # 83 -> 109
+    (64, 145, 2560, 640, False),      # 48 -> 63: three strips, the third half empty
+    (256, 186, 2560, 512, False),     # 170 -> 189
+    (16, 150, 2560, 4352, False),     # 272 tiles of 256 CUs'
+    (8, 145, 2944, 7040, True),       # 97 -> 64
+    (24, 148, 2816, 2304, True),      # 97 -> 67
+    (32, 197, 2944, 1536, True),      # 101 -> 72
+    (8, 150, 6912, 7168, True)])      # 216 -> 146
+def test_one_fp8_bank_takes_them_where_the_last_round_is_mostly_full(experts, rows, depth, width, tall):
+    assert taken(BLOCK, experts, rows, depth, width) == tall
+    assert taken(CHANNEL, experts, rows, depth, width) == tall
+
+
 @pytest.mark.parametrize("experts,rows,depth,width", [
     (128, 105, 2560, 1152),    # 204 -> 251
     (64, 91, 2688, 896),       # 85 -> 106
