@@ -1201,8 +1201,12 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 // one round more (16 x 135 of 2560 x 3328, sizes spread by 0.85, 66 -> 82). Past the lines 1.02 in the mean and 42 % of them slower, at worst by
 // two fifths (24 x 95 of 3968 x 2688 103 -> 142, 64 x 145 of 2560 x 640 48 -> 63).
 // Blocks, to 450 rows with seven rounds, whose last is a small part: 1.08 in the mean of 157 shapes, two of them slower, by 5 % at most (203 x 277 of 2560 x 2304 749 ->
-// 725). FP8 block pairs: groups of 76 to 200 rows from 1.3 rounds on, of more with seven (54 x 137 of 6656 x 3328 522 -> 437, 114 x 298 of 5120 x 2048 1560 ->
-// 1495; at four, 32 x 244 of 3584 x 2816 341 -> 394); above, no faster (36 x 1820 of 4096 x 7936 7045, 7084).
+// 725). FP8 block pairs, whose shorter launch is the better the fuller its own rounds of two blocks a CU are: groups of 76 to 200 rows on 3072 deep or more from 1.3
+// rounds on, where the shorter tiles fill less than 0.9 of theirs: 1.08 in the mean of 462 shapes (8 x 147 of 5376 x 6400 284 -> 193, 64 x 132 of 5120 x 1024
+// 296 -> 202; a tenth of them more than 5 % slower, 24 x 115 of 6528 x 2048 spread by 0.85 201 -> 248). Past these lines 1.03 in the mean of 591, 30 % of
+// them slower (24 x 132 of 2048 x 1792 66 -> 86, 128 x 105 of 3968 x 768 239 -> 288). Groups of more rows with seven rounds, 3584 deep or more: 1.05 in the mean of
+// 171 (114 x 298 of 5120 x 2048 1560 -> 1495), where 213 shallower ones gain nothing and lose up to 11 % (64 x 322 of 2048 x 2560 464 -> 475); above, no faster
+// (36 x 1820 of 4096 x 7936 7045, 7084).
 // One scale a channel costs the shorter tiles' loop less than one a block does: pairs gain nothing there (1195 shapes, 1.00 in the mean and 31 % of them more than
 // 5 % slower: 32 x 157 of 3072 x 1664 135 -> 152, 128 x 105 of 2560 x 1152 204 -> 251), nor do one bank's groups of more than 200 rows for certain (67 shapes, 1.04 in the
 // mean, a quarter of them slower, by up to 10 %).
@@ -1231,8 +1235,11 @@ static bool tall_tiles(const GemmParams& p, int format, bool paired) {
   if (format == DEW_MOE_W_NVFP4) return !paired && average >= 130 && average <= 215 && p.depth >= 2304 && tiles >= 560;
   if (format == DEW_MOE_W_FP8_CHANNEL && (paired || average > 200)) return false;
   if (p.depth < 2048 || average < 76) return false;
-  if (average > 200) return average <= 450 && tiles >= 1800;
-  if (paired) return tiles >= 336;
+  if (average > 200) return average <= 450 && tiles >= 1800 && (!paired || p.depth >= 3584);
+  if (paired) {
+    const double shorter = fmax(p.experts, p.rows / 128.0 + 0.5 * p.experts) * (p.width / 128) / 512;
+    return p.depth >= 3072 && tiles >= 336 && shorter < 0.9 * ceil(shorter);
+  }
   const double filled = groups_tiles(256, 0.5);
   return tiles >= 190 && p.experts <= 64 && filled * p.width / columns >= 0.7 * 256 * ceil(filled * strips / 256);
 }

@@ -24,11 +24,11 @@ def banks(form, experts, depth, width, count):
 
 
 @pytest.mark.parametrize("form,sizes,depth,width,paired,limit", [
-    ("block", "fp8", 2176, 2944, True, None),       # 34 steps
+    ("block", "fp8", 3200, 3328, True, None),       # 50 steps
     ("block", "fp8", 2048, 3200, False, None),      # a last strip of 128 columns
     ("block", "fp8", 3072, 3328, True, 0.75),
     ("channel", "fp8", 2432, 3200, False, None),    # 38 steps
-    ("block", "several tiles", 2048, 16640, True, None),
+    ("block", "several tiles", 3584, 16640, True, None),
     ("nvfp4", "nvfp4", 2304, 8064, False, None),   # a last strip of 128 columns
     ("bf16", "fp8", 2560, 1568, True, None),        # 40 steps; a last strip of 32 columns; tiles of at most 224 rows
     ("bf16", "fp8", 2880, 1664, True, 0.75),        # 45 steps

@@ -38,6 +38,20 @@ def test_one_fp8_bank_takes_them_where_the_last_round_is_mostly_full(experts, ro
     assert taken(CHANNEL, experts, rows, depth, width) == tall
 
 
+@pytest.mark.parametrize("experts,rows,depth,width,tall", [
+    (24, 132, 2048, 1792, False),     # 66 -> 86
+    (128, 105, 3968, 768, False),     # 239 -> 288
+    (64, 103, 6016, 768, False),      # 176 -> 223
+    (48, 96, 3840, 1024, False),      # 118 -> 141
+    (64, 322, 2048, 2560, False),     # 464 -> 475
+    (8, 147, 5376, 6400, True),       # 284 -> 193
+    (64, 132, 5120, 1024, True),      # 296 -> 202
+    (48, 142, 5632, 1280, True),      # 315 -> 226
+    (114, 298, 5120, 2048, True)])    # 1560 -> 1495
+def test_fp8_block_pairs_take_them_where_deep_and_where_the_shorter_rounds_are_not_full(experts, rows, depth, width, tall):
+    assert taken(BLOCK, experts, rows, depth, width, paired=True) == tall
+
+
 @pytest.mark.parametrize("experts,rows,depth,width", [
     (128, 105, 2560, 1152),    # 204 -> 251
     (64, 91, 2688, 896),       # 85 -> 106
