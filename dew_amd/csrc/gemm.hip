@@ -1216,10 +1216,12 @@ static bool few_tiles(const GemmParams& p, bool unquantized) {
 // 1536 270 -> 306), shallower or smaller ones lose up to 14 %, paired ones 2 to 8 %.
 // MXFP4 codes cost the vector unit so little that the shorter tiles, two blocks a CU, are the faster ones: over 626 shapes of 70 to 300 rows a group, 3000 deep
 // or more, in two and a half rounds and more, 1.06 times as fast in the mean (128 x 265 of 3328 x 896 213 -> 277, 64 x 194 of 3584 x 2176 203 -> 265).
-// Unquantized, 110 shapes: groups of up to 300 rows in whole rounds of blocks or many, from 45 rows and 1000 deep on in one bank and 28 and 2500
-// paired: 25 x 126 of 5120 x 4608 304 -> 242, 256 x 132 of 1280 x 1280 250 -> 203, 24 x 60 of 3584 x 6912 252 -> 224; paired 32 x 181 of 6656 x 1280
-// 374 -> 273, 16 x 131 of 4096 x 7936 566 -> 437, 25 x 29 of 4864 x 4864 458 -> 380; at worst 183 x 238 of 2560 x 1280 418 -> 436. Outside the lines: a
-// layer of 64 x 104 rows of 2048 x 1408, 2.8 rounds of pairs and 2.03 behind them, 301 -> 318 us; 768 to 1536 deep pairs 8 to 28 % slower, groups of 600 rows 6.
+// Unquantized, in whole rounds of blocks or many: in one bank groups of 45 to 224 rows, one tile of seven each, on 1280 deep or more, 1.12 times as fast in the
+// mean of 1505 shapes, 3 % of them more than 5 % slower (24 x 112 of 7040 x 2432 233 -> 148, 32 x 74 of 3968 x 1792 127 -> 85, 25 x 126 of 5120 x 4608 304 -> 242; sizes spread by
+// 0.85, 24 x 69 of 2176 x 2560 60 -> 73); groups of 225 to 300 rows, two tiles each if their sizes are alike, or 1000 to 1279 deep, 1.05 in the mean of 803 and 17 % of them more
+// than 5 % slower, at worst 39 % (24 x 263 of 1664 x 1536 55 -> 76, 8 x 287 of 4096 x 4352 118 -> 156). Pairs of 28 to 300 rows, 2500 deep or more: 1.15 in the mean of 1989, 3 % of
+// them slower (32 x 181 of 6656 x 1280 374 -> 273, 16 x 131 of 4096 x 7936 566 -> 437, 25 x 29 of 4864 x 4864 458 -> 380). Outside the lines: a layer of 64 x 104 rows of 2048 x
+// 1408, 2.8 rounds of pairs and 2.03 behind them, 301 -> 318 us; 768 to 1536 deep pairs 8 to 28 % slower, groups of 600 rows 6.
 static bool tall_tiles(const GemmParams& p, int format, bool paired) {
   if (forced_tile_rows != 0) return false;
   const int average = p.rows / p.experts, columns = paired ? 128 : 256, strips = (p.width + columns - 1) / columns;
@@ -1228,7 +1230,7 @@ static bool tall_tiles(const GemmParams& p, int format, bool paired) {
   auto groups_tiles = [&](int height, double last) { return fmax(p.experts, static_cast<double>(p.rows) / height + last * p.experts); };
   if (format == DEW_MOE_W_BF16) {
     const double rounds = groups_tiles(224, 0.55) * strips / 256;  // of blocks, one a CU
-    return average < 300 && (paired ? average >= 28 && p.depth >= 2500 : average >= 45 && p.depth >= 1000) && rounds >= 0.85 &&
+    return (paired ? average >= 28 && average < 300 && p.depth >= 2500 : average >= 45 && average <= 224 && p.depth >= 1280) && rounds >= 0.85 &&
            (rounds >= 5 || rounds >= 0.8 * ceil(rounds));
   }
   if (format == DEW_MOE_W_MXFP4) return false;

@@ -32,8 +32,8 @@ def banks(form, experts, depth, width, count):
     ("nvfp4", "nvfp4", 2304, 8064, False, None),   # a last strip of 128 columns
     ("bf16", "fp8", 2560, 1568, True, None),        # 40 steps; a last strip of 32 columns; tiles of at most 224 rows
     ("bf16", "fp8", 2880, 1664, True, 0.75),        # 45 steps
-    ("bf16", "fp8", 1088, 3232, False, None),       # 17 steps; a last strip of 160 columns
-    ("bf16", "nvfp4", 1216, 5216, False, None),     # 19 steps; a last strip of 96 columns
+    ("bf16", "fp8", 1344, 3232, False, None),       # 21 steps; a last strip of 160 columns
+    ("bf16", "nvfp4", 1472, 5216, False, None),     # 23 steps; a last strip of 96 columns
 ])
 def test_tall_tiles_return_the_shorter_tiles_bits(form, sizes, depth, width, paired, limit):
     from dew_amd import gemm, ops

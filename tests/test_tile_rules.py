@@ -81,6 +81,20 @@ def test_nvfp4_banks_take_them_where_a_group_is_one_tile(experts, rows, depth, w
     assert not taken(NVFP4, experts, rows, depth, width, paired=True)
 
 
+@pytest.mark.parametrize("experts,rows,depth,width,paired,tall", [
+    (24, 263, 1664, 1536, False, False),    # 55 -> 76
+    (8, 287, 4096, 4352, False, False),     # 118 -> 156
+    (24, 49, 1152, 6528, False, False),     # 78 -> 83
+    (64, 104, 2048, 1408, True, False),     # with its down product 301 -> 318
+    (24, 112, 7040, 2432, False, True),     # 233 -> 148
+    (48, 73, 6656, 1280, False, True),      # 219 -> 141
+    (128, 97, 3200, 512, False, True),      # 130 -> 84
+    (32, 162, 2560, 1536, True, True),      # 156 -> 128
+    (25, 29, 4864, 4864, True, True)])      # 458 -> 380
+def test_unquantized_banks_take_them_in_whole_rounds_of_groups_of_one_tile(experts, rows, depth, width, paired, tall):
+    assert taken(BF16, experts, rows, depth, width, paired) == tall
+
+
 def test_what_is_no_prepared_bank_or_has_no_rows_takes_none():
     assert taken(BF16, 24, 112, 7040, 2432)                          # 233 -> 148
     assert not taken(BF16, 24, 0, 7040, 2432) and not taken(BF16, 24, -112, 7040, 2432)
