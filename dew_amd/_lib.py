@@ -24,7 +24,7 @@ EXPORTS = (
     "dew_moe_gateup_interleaved", "dew_moe_split_rows", "dew_moe_grouped_gemm_split", "dew_moe_gateup_swiglu_split", "dew_moe_gateup_swiglu_split_out", "dew_moe_split_rows_fp6", "dew_moe_gateup_swiglu_split_fp6_out", "dew_moe_grouped_gemm_split_blocks", "dew_moe_route_sown", "dew_moe_balance_bias", "dew_moe_quantize_rows_nvfp4", "dew_moe_nvfp4_partials", "dew_moe_nvfp4_largest", "dew_moe_quantize_nvfp4", "dew_moe_quantize_columns_fp8", "dew_moe_quantize_columns_mxfp8", "dew_moe_quantize_rows_and_columns", "dew_moe_kernel_gradient_mxfp8", "dew_moe_kernel_gradient_takes_banks", "dew_moe_kernel_gradient_mxfp8_banks", "dew_moe_transpose_columns", "dew_moe_transpose_groups", "dew_moe_quantize_columns_nvfp4", "dew_moe_kernel_gradient_bf16", "dew_moe_quantize_rows_mxfp8", "dew_moe_grouped_gemm_mxfp8_rows", "dew_moe_quantize_rows_fp8", "dew_moe_grouped_gemm_fp8_rows", "dew_moe_gateup_swiglu", "dew_moe_swiglu", "dew_moe_swiglu_clamped", "dew_moe_gated_product", "dew_moe_scale_rows", "dew_moe_gate_rows", "dew_moe_gate_rows_add_f32", "dew_moe_gateup_gated", "dew_moe_silu", "dew_moe_relu2", "dew_moe_prefers_split_rows", "dew_moe_swiglu_mlp_split_workspace_bytes", "dew_moe_swiglu_mlp_split", "dew_moe_gated_mlp_split", "dew_moe_capacity_admit", "dew_moe_route_with", "dew_moe_route_call", "dew_moe_route_blocks_workspace_bytes", "dew_moe_route_blocks", "dew_moe_combine",
     "dew_moe_rows_f16", "dew_moe_gateup_gated_f16", "dew_moe_split_rows_e2m3_pair", "dew_moe_gateup_swiglu_split_e2m3_pair_out",
     "dew_moe_block_offsets", "dew_moe_quantized_matrices_bytes", "dew_moe_quantize_matrices", "dew_moe_quantize_step_matrices", "dew_moe_nvfp4_largest_of",
-    "dew_moe_layer_workspace_bytes", "dew_moe_layer_forward", "dew_moe_dense_gemm", "dew_moe_dense_gradient",
+    "dew_moe_layer_workspace_bytes", "dew_moe_layer_forward", "dew_moe_combines_few", "dew_moe_dense_gemm", "dew_moe_dense_gradient",
 )
 """Every symbol include/dew_moe_hip.h declares."""
 
@@ -156,6 +156,7 @@ def library() -> ctypes.CDLL:
         "dew_moe_dense_gemm": (i32, [ptr, ptr, ptr, ptr, ptr, i32, ptr, ptr, i32, i32, i32, i32, ptr]),
         "dew_moe_dense_gradient": (i32, [ptr, ptr, ptr, ptr, ptr, ptr, ptr, i32, i32, i32, i32, i32, ptr]),
         "dew_moe_layer_workspace_bytes": (size, [ptr, ptr, ptr, ptr, i32, i32, i32]),
+        "dew_moe_combines_few": (i32, [bank, i32, i32, i32]),
         "dew_moe_layer_forward": (i32, [ptr] * 10 + [i32, i32, i32, ptr, ptr, size, ptr]),
         "dew_moe_combine": (i32, [ptr, ptr, ptr, ptr, i32, i32, i32, ptr]),
     }

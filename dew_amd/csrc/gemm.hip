@@ -1409,17 +1409,23 @@ static int grouped_gemm_of(const char* who, const void* x, const int32_t* gather
   return launch<kPlain>(who, p, w->format, static_cast<hipStream_t>(stream));
 }
 
-// A block holds all of a token's slots, so their weights pass through one CU, and each token reads its own: small experts only. us a layer's pass,
-// two launches and one, 2 of 8 experts of 512 x 512 (FP8, 33 KB a block) 22.7 -> 18.3 for one token and 23.1 -> 20.1 for 16; MXFP4, 7 of 256 of
-// 2048 x 512 (61 KB) one token 29.6 -> 28.0, four 38.6 -> 32.8, eight (31 MB in all) 46.3 -> 45.8, twelve 52.8 -> 58.7; 2 of 16 of 4096 x 2048 (70 KB)
-// one 31.3 -> 29.5, three 35.6 -> 35.3, eight 46.6 -> 47.9. Past the first line, FP8, 8 of 128 of 2048 x 768 (196 KB): one 26.4 -> 28.7, three 41.1 -> 38.3,
-// eight 63.9 -> 68.8; 8 of 32 of 7168 x 2048 (524 KB) two 106 -> 116.
+// A block holds all of a token's slots, so their weights pass through one CU, and each token reads its own: small experts only, in at most a block a
+// CU where a token has several slots. Both ways timed in turn over 790 layers of up to 16 tokens, 72 KB a block: inside the lines 1.13 times as fast in the
+// mean of 645, none more than 1.3 % slower (2 of 8 experts of 512 x 512, FP8, 33 KB a block, one token 22.7 -> 18.3 us; MXFP4, 7 of 256 of 2048 x 512, 61 KB, four 38.6 ->
+// 32.8); several slots in more blocks gain nothing, and a third lose (MXFP4, 6 of 32 of 1024 x 512, 11 tokens 23.1 -> 27.8, NVFP4, 5 of 64 of 2304 x 768, four 36.0 ->
+// 39.4, FP8, 2 of 16 of 4480 x 1024, two 30.6 -> 32.2). Past 72 KB, FP8, 8 of 128 of 2048 x 768 (196 KB): one 26.4 -> 28.7, three 41.1 -> 38.3, eight 63.9 -> 68.8; 8 of
+// 32 of 7168 x 2048 (524 KB) two 106 -> 116.
 bool dew::combines_few(const dew_moe_bank* down, int tokens, int top_k, bool shared) {
   const int slots = top_k + (shared ? 1 : 0);
   if (forced_tile_rows != 0 || slots > kMostCombinedSlots || tokens > 16 || down->format == DEW_MOE_W_MXFP8) return false;
   const double bytes = down->format == DEW_MOE_W_BF16 ? 2.0 : down->format == DEW_MOE_W_MXFP4 || down->format == DEW_MOE_W_NVFP4 ? 0.53 : 1.0;
   const double block = 32.0 * slots * down->depth * bytes;
-  return block <= 72 * 1024 && block * (down->width / 32) * tokens <= 32e6;
+  const int blocks = tokens * (down->width / 32);
+  return block <= 72 * 1024 && (slots == 1 || blocks <= 256) && block * blocks <= 32e6;
+}
+
+extern "C" int dew_moe_combines_few(const dew_moe_bank* down, int32_t tokens, int32_t top_k, int32_t shared) {
+  return down && down->layout == DEW_MOE_LAYOUT_PREPARED && tokens >= 1 && top_k >= 1 && dew::combines_few(down, tokens, top_k, shared != 0) ? 1 : 0;
 }
 
 int dew::down_and_combine(const char* who, const void* hidden, const int32_t* offsets, const dew_moe_bank* down, const float* bias, const int32_t* order,

@@ -615,6 +615,9 @@ int dew_moe_layer_forward(const dew_moe_layer* layer, const void* x /* bf16 [T,D
                           const dew_moe_bank* gate, const dew_moe_bank* up, const dew_moe_bank* down, const float* up_bias,
                           const float* down_bias, int32_t tokens, int32_t split_terms, int32_t f16_rows_from, void* out /* bf16 [T,D] */,
                           void* workspace, size_t workspace_bytes, void* stream);
+/* Whether dew_moe_layer_forward makes the down product and the combine of so many tokens one launch (1) or two (0): its own rule, for tests.
+ * Only the descriptor's format, layout and extents are read.                                                                            */
+int dew_moe_combines_few(const dew_moe_bank* down, int32_t tokens, int32_t top_k, int32_t shared);
 
 #ifdef __cplusplus
 }

@@ -1,5 +1,6 @@
-"""Which launches take tiles of up to 256 rows on eight wavefronts (dew_moe_takes_tall_tiles, csrc/gemm.hip): a rule that can be asked without
-a GPU. The shapes are ones where both launches were timed; times in us, the shorter tiles' and the tall ones'."""
+"""Which products take tiles of up to 256 rows on eight wavefronts (dew_moe_takes_tall_tiles), and which layers' down product and combine are one
+launch (dew_moe_combines_few): rules (csrc/gemm.hip) that can be asked without a GPU. The shapes are ones where both forms were timed; times in us,
+the shorter tiles' and the tall ones', or two launches' and one's."""
 
 import pytest
 
@@ -100,3 +101,22 @@ def test_what_is_no_prepared_bank_or_has_no_rows_takes_none():
     assert not taken(BF16, 24, 0, 7040, 2432) and not taken(BF16, 24, -112, 7040, 2432)
     assert not taken(BF16, 24, 112, 7040, 2432, layout=_lib.LAYOUT_REFERENCE)
     assert _lib.library().dew_moe_takes_tall_tiles(None, 0, 100) == 0
+
+
+@pytest.mark.parametrize("form,tokens,top_k,experts,depth,width,combined", [
+    (MXFP4, 11, 6, 32, 512, 1024, False),     # 23.1 -> 27.8
+    (NVFP4, 15, 6, 32, 512, 768, False),      # 26.9 -> 31.4
+    (NVFP4, 4, 5, 64, 768, 2304, False),      # 36.0 -> 39.4
+    (BLOCK, 2, 2, 16, 1024, 4480, False),     # 30.6 -> 32.2
+    (BLOCK, 8, 3, 8, 640, 2048, False),       # 26.2 -> 27.5
+    (BLOCK, 1, 8, 128, 768, 2048, False),     # 26.4 -> 28.7: 196 KB a block
+    (CHANNEL, 1, 2, 8, 512, 512, True),       # 22.7 -> 18.3
+    (NVFP4, 2, 3, 8, 1280, 6144, False),
+    (MXFP4, 4, 7, 256, 512, 2048, True),      # 38.6 -> 32.8
+    (CHANNEL, 13, 1, 8, 640, 2048, True),     # 25.1 -> 24.1: one slot
+    (BF16, 5, 1, 32, 512, 6016, True)])       # 41.7 -> 41.4
+def test_a_layers_last_two_launches_are_one_where_a_cu_has_one_block(form, tokens, top_k, experts, depth, width, combined):
+    down = _lib.Bank(form, _lib.LAYOUT_PREPARED, experts, depth, width, None, None, None)
+    assert bool(_lib.library().dew_moe_combines_few(down, tokens, top_k, 0)) == combined
+    assert not _lib.library().dew_moe_combines_few(down, 17, top_k, 0) and not _lib.library().dew_moe_combines_few(down, tokens, 8, 1)
+    assert not _lib.library().dew_moe_combines_few(down, 0, top_k, 0) and not _lib.library().dew_moe_combines_few(None, tokens, top_k, 0)
