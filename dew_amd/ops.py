@@ -927,7 +927,7 @@ def quantize_rows_nvfp4(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
 
 def nvfp4_largest(x: torch.Tensor) -> torch.Tensor:
     """The partial largest magnitudes (words) of `x`, bf16 or fp32, that `quantize_nvfp4` takes its tensor scale from."""
-    return nvfp4_largest_of(x)[0]
+    return nvfp4_largest_of(_device(x, "x"))[0]
 
 
 MOST_OPERANDS = 3

@@ -108,6 +108,16 @@ def test_nvfp4_magnitudes_of_another_length_are_refused(words):
         ops.quantize_nvfp4(torch.zeros((128, 128), dtype=torch.bfloat16), torch.zeros(words, dtype=torch.int32), rows=True, tokens=False)
 
 
+@pytest.mark.gpu
+def test_an_operand_whose_magnitudes_are_formed_lies_as_it_is_shaped():
+    """`nvfp4_largest` is a row quantizer's first read: contiguous, as `quantize_nvfp4` takes it. (`nvfp4_largest_of` takes matrices either way round.)"""
+    x = torch.ones((2, 128, 256), dtype=torch.bfloat16, device="cuda")
+    for turned in (x.transpose(1, 2), x.transpose(0, 1), x[0].transpose(0, 1)):
+        with pytest.raises(KernelError, match="x must be contiguous"):
+            ops.nvfp4_largest(turned)
+    assert torch.equal(ops.nvfp4_largest_of(x.transpose(1, 2))[0], ops.nvfp4_largest(x))
+
+
 @pytest.mark.parametrize("shape", [(128,), (2, 128, 128), ()])
 def test_an_nvfp4_operand_that_is_no_matrix_is_refused(shape):
     with pytest.raises(KernelError, match=r"not \[rows, depth\]"):
