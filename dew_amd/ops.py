@@ -938,6 +938,8 @@ def nvfp4_largest_of(*operands: torch.Tensor) -> torch.Tensor:
     """`nvfp4_largest` of each of up to three operands, in one launch: a row of words each. (An operand may be the transpose of contiguous
     memory, as `quantize_matrices`' matrices are.)"""
     count = len(operands)
+    if not 1 <= count <= MOST_OPERANDS:
+        raise KernelError(f"{count} operands: one launch forms the magnitudes of 1 to {MOST_OPERANDS}")
     for x in operands:
         _device(x if x.is_contiguous() or x.dim() != 3 else x.transpose(1, 2), "x")
         if x.dtype not in (torch.bfloat16, torch.float32):

@@ -108,6 +108,12 @@ def test_nvfp4_magnitudes_of_another_length_are_refused(words):
         ops.quantize_nvfp4(torch.zeros((128, 128), dtype=torch.bfloat16), torch.zeros(words, dtype=torch.int32), rows=True, tokens=False)
 
 
+@pytest.mark.parametrize("count", [0, 4])
+def test_one_launch_forms_the_magnitudes_of_one_to_three_operands(count):
+    with pytest.raises(KernelError, match=f"{count} operands: one launch forms the magnitudes of 1 to 3"):
+        ops.nvfp4_largest_of(*[torch.zeros((128, 128), dtype=torch.bfloat16)] * count)
+
+
 @pytest.mark.gpu
 def test_an_operand_whose_magnitudes_are_formed_lies_as_it_is_shaped():
     """`nvfp4_largest` is a row quantizer's first read: contiguous, as `quantize_nvfp4` takes it. (`nvfp4_largest_of` takes matrices either way round.)"""
