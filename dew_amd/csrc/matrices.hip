@@ -330,11 +330,10 @@ extern "C" size_t dew_moe_quantized_matrices_bytes(int32_t format, int32_t exper
   return dew_moe_prepared_bytes(format, experts, depth, width);
 }
 
-extern "C" int dew_moe_quantize_step_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
-                                              int32_t width, const uint32_t* largest, const int32_t* blocks, int32_t groups, int32_t unit,
-                                              int32_t* offsets, void* prepared, dew_moe_bank* out, void* stream) {
+static int quantize_matrices_of(const char* who, const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth, int32_t width,
+                                const uint32_t* largest, const int32_t* blocks, int32_t groups, int32_t unit, int32_t* offsets, void* prepared, dew_moe_bank* out,
+                                void* stream) {
   using namespace dew;
-  const char* who = "dew_moe_quantize_matrices";
   DEW_REQUIRE(w && prepared && out, "%s: w, the prepared buffer and out must not be null", who);
   DEW_REQUIRE(format == DEW_MOE_W_FP8_BLOCK || format == DEW_MOE_W_MXFP8 || format == DEW_MOE_W_NVFP4,
               "%s: format %d is none of the recipes' (FP8 blocks, MXFP8, NVFP4)", who, format);
@@ -342,6 +341,7 @@ extern "C" int dew_moe_quantize_step_matrices(const void* w, int32_t format, int
   DEW_REQUIRE(depth >= 128 && depth % 128 == 0 && width >= 128 && width % 128 == 0 && depth / 128 <= 65535 && width / 128 <= 65535,
               "%s: matrices of %d x %d (whole 128s)", who, depth, width);
   DEW_REQUIRE(aligned16(w) && (reinterpret_cast<uintptr_t>(prepared) & 255u) == 0, "%s: w must be 16-byte and the prepared buffer 256-byte aligned", who);
+  DEW_REQUIRE(!largest || format == DEW_MOE_W_NVFP4, "%s: a bank of format %d has no tensor scale to form from magnitudes", who, format);
   DEW_REQUIRE(!blocks || (offsets && groups >= 1 && unit >= 1), "%s: offsets must not be null, %d groups in units of %d", who, groups, unit);
   const StepGroups step{blocks, offsets, groups, unit};
   hipStream_t s = static_cast<hipStream_t>(stream);
@@ -358,5 +358,11 @@ extern "C" int dew_moe_quantize_step_matrices(const void* w, int32_t format, int
 
 extern "C" int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
                                          int32_t width, void* prepared, dew_moe_bank* out, void* stream) {
-  return dew_moe_quantize_step_matrices(w, format, w_is_f32, kmajor, experts, depth, width, nullptr, nullptr, 0, 0, nullptr, prepared, out, stream);
+  return quantize_matrices_of("dew_moe_quantize_matrices", w, format, w_is_f32, kmajor, experts, depth, width, nullptr, nullptr, 0, 0, nullptr, prepared, out, stream);
+}
+
+extern "C" int dew_moe_quantize_step_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
+                                              int32_t width, const uint32_t* largest, const int32_t* blocks, int32_t groups, int32_t unit,
+                                              int32_t* offsets, void* prepared, dew_moe_bank* out, void* stream) {
+  return quantize_matrices_of("dew_moe_quantize_step_matrices", w, format, w_is_f32, kmajor, experts, depth, width, largest, blocks, groups, unit, offsets, prepared, out, stream);
 }

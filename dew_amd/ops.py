@@ -391,7 +391,7 @@ def quantize_matrices(w: torch.Tensor, recipe: str, *, largest: torch.Tensor | N
     buffer = torch.empty(max(lib.dew_moe_quantized_matrices_bytes(fmt, experts, depth, width), 16), dtype=torch.uint8, device=w.device)
     out = _lib.Bank()
     _lib.check(lib.dew_moe_quantize_step_matrices(w.data_ptr(), fmt, int(w.dtype == torch.float32), int(kmajor), experts, depth, width, _ptr(largest),
-                                                  _ptr(blocks), groups, unit, _ptr(offsets), buffer.data_ptr(), out, _stream()), "dew_moe_quantize_matrices")
+                                                  _ptr(blocks), groups, unit, _ptr(offsets), buffer.data_ptr(), out, _stream()), "dew_moe_quantize_step_matrices")
     tensor = None
     if fmt == _lib.W_NVFP4:
         at = out.tensor_scale - buffer.data_ptr()

@@ -235,7 +235,7 @@ size_t dew_moe_quantized_matrices_bytes(int32_t format, int32_t experts, int32_t
 int dew_moe_quantize_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
                               int32_t width, void* prepared, dew_moe_bank* out /* host */, void* stream);
 /* The same as a step's launch: an NVFP4 bank's tensor scale from partial magnitudes formed already (`largest`, dew_moe_nvfp4_largest_of's
- * words for w, or null), and the offsets [groups + 1] of groups counted in blocks of `unit` rows written beside the codes
+ * words for w, or null, as for the other formats), and the offsets [groups + 1] of groups counted in blocks of `unit` rows written beside the codes
  * (dew_moe_block_offsets; `blocks` null: none).                                                                       */
 int dew_moe_quantize_step_matrices(const void* w, int32_t format, int32_t w_is_f32, int32_t kmajor, int32_t experts, int32_t depth,
                                    int32_t width, const uint32_t* largest, const int32_t* blocks, int32_t groups, int32_t unit,

@@ -108,6 +108,21 @@ def test_nvfp4_magnitudes_of_another_length_are_refused(words):
         ops.quantize_nvfp4(torch.zeros((128, 128), dtype=torch.bfloat16), torch.zeros(words, dtype=torch.int32), rows=True, tokens=False)
 
 
+def test_what_a_steps_launch_refuses_bears_its_name():
+    """Both entry points share their checks, each under its own name; magnitudes are an NVFP4 bank's alone. (Refused before any address is read.)"""
+    lib, bank, at = _lib.library(), _lib.Bank(), 4096
+    step = lambda w, form, largest, blocks, groups: lib.dew_moe_quantize_step_matrices(w, form, 0, 0, 1, 256, 256, largest, blocks, groups, 128, at, at, bank, None)
+    assert step(None, _lib.W_NVFP4, None, None, 0) != 0
+    assert lib.dew_moe_last_error().decode().startswith("dew_moe_quantize_step_matrices: w, the prepared buffer")
+    assert step(at, _lib.W_NVFP4, None, at, 0) != 0
+    assert lib.dew_moe_last_error().decode() == "dew_moe_quantize_step_matrices: offsets must not be null, 0 groups in units of 128"
+    for form in (_lib.W_FP8_BLOCK, _lib.W_MXFP8):
+        assert step(at, form, at, None, 0) == lib.dew_moe_quantize_matrices(None, form, 0, 0, 1, 256, 256, at, bank, None) != 0
+        assert lib.dew_moe_last_error().decode().startswith("dew_moe_quantize_matrices: w, the prepared buffer")
+        assert step(at, form, at, None, 0) != 0
+        assert lib.dew_moe_last_error().decode() == f"dew_moe_quantize_step_matrices: a bank of format {form} has no tensor scale to form from magnitudes"
+
+
 @pytest.mark.parametrize("count", [0, 4])
 def test_one_launch_forms_the_magnitudes_of_one_to_three_operands(count):
     with pytest.raises(KernelError, match=f"{count} operands: one launch forms the magnitudes of 1 to 3"):
