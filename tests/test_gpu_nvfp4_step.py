@@ -45,9 +45,12 @@ def test_largest_magnitude(shape):
 
 
 @pytest.mark.parametrize("blocks,depth,width", (([1], 256, 256), ([3, 0, 2, 4], 512, 768), ([5, 6, 7, 6], 1024, 2560), ([49], 256, 512)))    # (the last walks its tokens in transposed copies)
-def test_a_step_is_its_operands_products(blocks, depth, width):
+@pytest.mark.parametrize("cached", (True, False))     # magnitudes of all operands from one launch, or of each right before it is quantized
+def test_a_step_is_its_operands_products(blocks, depth, width, cached, monkeypatch):
     from dew_amd import ops, projections
 
+    if not cached:
+        monkeypatch.setattr(projections, "CACHED_BYTES", 0)
     counts = torch.tensor(blocks, dtype=torch.int32, device="cuda")
     tokens = 128 * sum(blocks)
     x, w, dy = drawn(tokens, depth, seed=4), drawn(len(blocks), depth, width, seed=5), drawn(tokens, width, seed=6)

@@ -1,4 +1,5 @@
-"""A layer's pass as one foreign call against its separate calls: the same launches on the same operands, so the same bits."""
+"""A layer's pass as one foreign call against its separate calls, bit for bit: the same launches on the same operands, but that a few tokens' router
+and sort, and small experts' down product and combine, are one launch each there, which form every sum in the same order."""
 
 import pytest
 import torch
@@ -30,6 +31,12 @@ CASES = {
     "combined, bf16, shared": dict(tokens=3, experts=8, top_k=3, quant="bf16", shared=256),
     "combined, mxfp4, one slot": dict(tokens=5, experts=16, top_k=1, quant="mxfp4"),
     "combined, nvfp4, shared, 70 experts": dict(tokens=16, experts=70, top_k=7, quant="nvfp4", shared=256),
+    # ... and through whole rounds of its weight registers: from 1024 depths on in FP8 and FP4, 768 in bf16
+    "combined, fp8 blocks, two slots, 16 steps": dict(tokens=3, experts=8, top_k=2, quant="fp8_block", hidden=1024),
+    "combined, fp8 channels, one slot, 36 steps": dict(tokens=7, experts=8, top_k=1, quant="fp8_channel", hidden=2304),
+    "combined, bf16, one slot, 17 steps": dict(tokens=5, experts=8, top_k=1, quant="bf16", hidden=1088),
+    "combined, mxfp4, one slot, 67 steps": dict(tokens=5, experts=8, top_k=1, quant="mxfp4", hidden=4288),
+    "combined, nvfp4, shared, 20 steps": dict(tokens=4, experts=8, top_k=2, quant="nvfp4", hidden=1280, shared=1280),
     "300 experts": dict(tokens=64, experts=300, top_k=6, quant="fp8_block"),
 }
 DEPTH, HIDDEN = 512, 256
@@ -48,16 +55,19 @@ def bank(experts, depth, width, quant, generator):
 
 @pytest.mark.parametrize("name", CASES)
 def test_one_call_returns_the_separate_calls_bits(name):
-    from dew_amd import moe
+    from dew_amd import _lib, gemm, moe
 
     case = dict(CASES[name])
     tokens, experts, top_k, quant = (case.pop(key) for key in ("tokens", "experts", "top_k", "quant"))
-    layer = moe.SparseMLP(num_experts=experts, top_k=top_k, hidden_features=HIDDEN, out_features=DEPTH, **case)
+    hidden = case.pop("hidden", HIDDEN)
+    layer = moe.SparseMLP(num_experts=experts, top_k=top_k, hidden_features=hidden, out_features=DEPTH, **case)
     generator = torch.Generator("cuda").manual_seed(7)
-    shapes = {"gate_proj": (DEPTH, HIDDEN), "up_proj": (DEPTH, HIDDEN), "down_proj": (HIDDEN, DEPTH)}
+    shapes = {"gate_proj": (DEPTH, hidden), "up_proj": (DEPTH, hidden), "down_proj": (hidden, DEPTH)}
     held = {"experts": {n: {"kernel": bank(experts, *s, quant, generator)} for n, s in shapes.items()}}
     if case.get("shared"):
         held["shared_experts"] = {n: {"kernel": bank(1, *s, quant, generator)} for n, s in shapes.items()}
+    if name.startswith("combined"):
+        assert _lib.library().dew_moe_combines_few(gemm.prepared(held["experts"]["down_proj"]["kernel"]).descriptor, tokens, top_k, "shared" in case) == 1
     variables = {"params": {"gate": {"kernel": torch.randn((DEPTH, experts), generator=generator, device="cuda") * DEPTH ** -0.5}},
                  "moe": {"gate": {"e_score_correction_bias": torch.randn(experts, generator=generator, device="cuda") * 0.05}},
                  "quantization": held}
@@ -75,12 +85,12 @@ def test_one_call_returns_the_separate_calls_bits(name):
     assert torch.equal(layer.apply(variables, shaped, logits=torch.stack((logits, logits))), torch.stack((want, want)))
 
 
-@pytest.mark.parametrize("tokens", (1, 24, 700))
-def test_gpt_oss_in_one_call(tokens):
+@pytest.mark.parametrize("tokens,hidden", ((1, 192), (24, 192), (700, 192), (3, 1024)))     # (the last: 16 steps of the combined launch)
+def test_gpt_oss_in_one_call(tokens, hidden):
     from dew_amd import gpt_oss
 
     generator = torch.Generator("cuda").manual_seed(8)
-    depth, hidden, experts = 320, 192, 8
+    depth, experts = 320, 8
     layer = gpt_oss.GptOssMLP(depth, hidden, experts, 4)
     normal = lambda *shape: torch.randn(shape, generator=generator, device="cuda")
     variables = {"params": {"router": {"kernel": normal(depth, experts) * 0.1, "bias": normal(experts) * 0.1},
