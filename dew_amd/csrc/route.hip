@@ -153,8 +153,7 @@ struct RouteParams {
   uint32_t* block_keys;    // [rows x (length + 1), E]: a block's best selection for every expert, as ordered keys (0: none yet)
   const uint8_t* allowed;  // [rows x (length + 1), 64]: bit i of byte `lane` set where expert lane + 64 i is on the block's shortlist
   int gather_blocks;       // this launch only gathers the blocks' best selections into block_keys
-  int shares;              // `logits` are kLogitShares partial sums of them, [share][T][E] (logits.hip), to which `gate_bias` is still due
-  const float* gate_bias;  // nullable [E]
+  const float* gate_bias;  // nullable [E]: still due to logits that come in shares
 };
 
 // The block a token routes with: its row's blocks are numbered from 0, padding (or an id past the row) is block `length`.
@@ -168,11 +167,11 @@ __device__ __forceinline__ float capped(float logit, float cap) { return cap > 0
 
 // A token's logits, expert lane + 64 i in logit[i]: as they are, or added up from the gate's shares of the depth in the order the
 // gate's own launch adds them.
-template <int kPerLane>
+template <int kPerLane, bool SHARES>  // SHARES: p.logits are kLogitShares partial sums of them, [share][T][E] (logits.hip)
 __device__ __forceinline__ void read_logits(const RouteParams& p, int token, float (&logit)[kPerLane]) {
   const int lane = threadIdx.x % kWave;
   const float* row = p.logits + static_cast<size_t>(token) * p.experts;
-  if (p.shares) {
+  if constexpr (SHARES) {
     constexpr int kAtOnce = kPerLane < 4 ? kPerLane : 4;
 #pragma unroll
     for (int first = 0; first < kPerLane; first += kAtOnce) {
@@ -390,7 +389,10 @@ __device__ __forceinline__ Chosen routed_token(const RouteParams& p, int token, 
   return Chosen{in_range ? weight : 0.0f, replayed ? given_id : my_choice};
 }
 
-template <int kPerLane>
+// (SHARES apart: the shares in flight take 98 registers of more than 128 experts' launches, four wavefronts a SIMD, where logits as they are take 42 and
+// eight. Of few tokens, each a chain alone, that costs nothing; in one launch for both forms the many tokens that come without shares paid for it: 32 768 of 256
+// experts in 8 groups, top 1, 47 us, apart 33, 16 384 of 192 22 and 16.)
+template <int kPerLane, bool SHARES>
 __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p) {
   extern __shared__ float shared[];  // [kRouteWaves][experts] selections, for the group scores
   const int lane = threadIdx.x % kWave;
@@ -399,7 +401,7 @@ __global__ __launch_bounds__(kWave* kRouteWaves) void route_kernel(RouteParams p
   const bool active = token_raw < p.tokens;
   const int token = active ? token_raw : p.tokens - 1;
   float logit[kPerLane];
-  read_logits<kPerLane>(p, token, logit);
+  read_logits<kPerLane, SHARES>(p, token, logit);
   const Chosen chosen = routed_token<kPerLane>(p, token, active, logit, shared + wave * p.experts);
   if (p.gather_blocks) return;
   if (active && lane < p.top_k) {
@@ -420,7 +422,7 @@ __global__ __launch_bounds__(kSmallThreads) void route_and_sort_kernel(RoutePara
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
   if (wave < p.tokens) {  // a wavefront a token; the others wait for the sort
     float logit[kPerLane];
-    read_logits<kPerLane>(p, wave, logit);
+    read_logits<kPerLane, true>(p, wave, logit);
     const Chosen chosen = routed_token<kPerLane>(p, wave, true, logit, reinterpret_cast<float*>(scratch) + wave * p.experts);
     if (lane < p.top_k) {
       p.weights[wave * p.top_k + lane] = chosen.weight;
@@ -546,20 +548,21 @@ static RouteParams route_params(const dew_moe_router* router, const float* logit
                 router->expert_groups, router->groups_per_token, router->group_score == DEW_MOE_GROUP_MAX ? 1 : 0, router->scaling, scores, log_z,
                 router->bias_in_weights ? 1 : 0, router->weight_sum_epsilon, router->weight_sum_min,
                 router->fill_excluded ? 1 : 0, router->excluded_group_score, router->logit_softcap, given, covered, media_bias, media,
-                by_block.blocks, by_block.length, by_block.keys, by_block.allowed, by_block.gather, 0, nullptr};
+                by_block.blocks, by_block.length, by_block.keys, by_block.allowed, by_block.gather, nullptr};
 }
 
+template <bool SHARES>
 static int launch_route(const RouteParams& p, hipStream_t s) {
   const size_t shared = p.expert_groups > 1 ? sizeof(float) * kRouteWaves * p.experts : 0;
   const dim3 grid((p.tokens + kRouteWaves - 1) / kRouteWaves), block(kWave * kRouteWaves);
   if (p.experts <= 64) {
-    hipLaunchKernelGGL(route_kernel<1>, grid, block, shared, s, p);
+    hipLaunchKernelGGL((route_kernel<1, SHARES>), grid, block, shared, s, p);
   } else if (p.experts <= 128) {
-    hipLaunchKernelGGL(route_kernel<2>, grid, block, shared, s, p);
+    hipLaunchKernelGGL((route_kernel<2, SHARES>), grid, block, shared, s, p);
   } else if (p.experts <= 256) {
-    hipLaunchKernelGGL(route_kernel<4>, grid, block, shared, s, p);
+    hipLaunchKernelGGL((route_kernel<4, SHARES>), grid, block, shared, s, p);
   } else {
-    hipLaunchKernelGGL(route_kernel<kMaxPerLane>, grid, block, shared, s, p);
+    hipLaunchKernelGGL((route_kernel<kMaxPerLane, SHARES>), grid, block, shared, s, p);
   }
   return launched("route_kernel");
 }
@@ -575,7 +578,7 @@ int dew::route_launch(const dew_moe_router* router, const float* logits, const f
   DEW_REQUIRE(tokens == 0 || (logits && weights && indices), "dew_moe_route: logits, weights and indices must not be null");
   if (tokens == 0) return DEW_MOE_OK;
   const RouteParams p = route_params(router, logits, bias, media_bias, media, given, covered, by_block, tokens, weights, indices, scores, log_z);
-  return launch_route(p, static_cast<hipStream_t>(stream));
+  return launch_route<false>(p, static_cast<hipStream_t>(stream));
 }
 
 int dew::route_shares(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
@@ -583,9 +586,8 @@ int dew::route_shares(const dew_moe_router* router, const float* partial, const 
   if (int rc = check_router(router, selection_bias, tokens)) return rc;
   RouteParams p = route_params(router, partial, selection_bias, nullptr, nullptr, nullptr, nullptr, BlockRouting{}, tokens, weights, indices, nullptr,
                                nullptr);
-  p.shares = 1;
   p.gate_bias = gate_bias;
-  return launch_route(p, stream);
+  return launch_route<true>(p, stream);
 }
 
 int dew::route_and_sort(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
@@ -595,7 +597,6 @@ int dew::route_and_sort(const dew_moe_router* router, const float* partial, cons
   DEW_REQUIRE(tokens >= 1 && tokens <= kRouteAndSortTokens && slots <= kSmallSlots, "route_and_sort: %d tokens, %d slots", tokens, slots);
   RouteParams p = route_params(router, partial, selection_bias, nullptr, nullptr, nullptr, nullptr, BlockRouting{}, tokens, weights, nullptr, nullptr,
                                nullptr);
-  p.shares = 1;
   p.gate_bias = gate_bias;
   const int groups = experts + (shared ? 1 : 0);
   const PermuteParams sort{nullptr, sizes, offsets, order, rows, nullptr, slots, tokens * router->top_k, experts, groups, router->top_k, 1, groups + 1, slots};
