@@ -1279,13 +1279,13 @@ static int launch_format(const char* who, const GemmParams& p, hipStream_t strea
     default: {
       // Last tiles of at most 64 rows can go to a second launch of 64-row tiles. That launch runs after the first, so
       // it pays only where it fills the chip by itself and most groups have such a last tile: the average group just
-      // over a whole number of tiles (256 groups of 256 +- 16 rows: 2.5 tiles a group become 2 and a 64-row one, 1.5
-      // to 2.5 % faster; at 160 or 200 rows a group the same two launches are 5 to 15 % slower than one, a bank of 8
-      // experts, whose few last tiles run their whole depth alone, 20 to 35 % slower, and groups of 1024 rows 1 %). Where a
-      // gate's preferences spread the sizes widely, half the groups have such a last tile whatever the average: 256 experts of
-      // 7168 x 2048 gain 2 %, 128 experts nothing, and 64 or 128 experts of 2048 to 4096 x 2048 lose 2 to 8 % (FP8 at 140 and 275
-      // rows a group 848 -> 777 and 1145 -> 1089 us a layer in one launch, NVFP4 at 256 918 -> 896, MXFP4 at 412 999 -> 939): from
-      // 3072 strips of tiles on.
+      // over a whole number of tiles, or sizes that a gate's preferences spread widely, so that half the groups have one whatever the average
+      // (at 160 or 200 rows a group the same two launches are 5 to 15 % slower than one, a bank of 8
+      // experts, whose few last tiles run their whole depth alone, 20 to 35 % slower, and groups of 1024 rows 1 %; 64 or 128 experts of 2048 to 4096 x
+      // 2048 lose 2 to 8 %, MXFP4 at 412 rows a group 999 -> 939 us a layer in one launch): from 3072 strips of tiles on. What still comes here
+      // is what tall_tiles leaves, 191 shapes of which timed both ways, sizes spread by 0.05 to 0.85: pairs gain, on NVFP4 banks 3.8 % in the mean and nearly
+      // always (256 to 296 rows a group 5.0, 384 to 424 2.2), on FP8 blocks 1.3, channels and MXFP4 0.9. In one bank NVFP4 and MXFP4 are the same to 0.3 %, FP8
+      // loses 1 to 2, all of it at depths under 1024 (2.5 to 3.4).
       const int average = p.rows / p.experts;
       const bool shared = forced_tile_rows == 0 && FORMAT != DEW_MOE_W_BF16 && average >= 192 && average < 512 && average % 128 <= 40 &&
                           static_cast<long long>(p.experts) * (p.width / 128) >= 3072;

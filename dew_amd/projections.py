@@ -288,7 +288,8 @@ CACHED_BYTES = 256 << 20
 def _nvfp4_step(operands: tuple, matrices: torch.Tensor, group_blocks):
     """Each operand's largest magnitudes (a call for them), the quantized matrices and the groups, which the matrices' launch leaves offsets of. The
     magnitudes of operands that the last-level cache holds all of come from one launch (five of them were 89 us of a step of 589, 8192 rows of
-    8 x 2048 x 4096); larger ones are read for theirs right before they are quantized, while the cache holds the most of them."""
+    8 x 2048 x 4096); larger ones are read for theirs right before they are quantized, while the cache holds the most of them. (Both ways,
+    over 70 steps: 1.00 to 1.07 times as fast in one launch up to 256 MiB, the most where they are small, 1.00 to 1.02 past it.)"""
     together = (*operands, matrices)
     if sum(x.numel() * x.element_size() for x in together) <= CACHED_BYTES:
         *known, of_matrices = ops.nvfp4_largest_of(*together)
