@@ -551,19 +551,16 @@ static RouteParams route_params(const dew_moe_router* router, const float* logit
                 by_block.blocks, by_block.length, by_block.keys, by_block.allowed, by_block.gather, nullptr};
 }
 
-template <bool SHARES>
-static int launch_route(const RouteParams& p, hipStream_t s) {
+// (Kernels lie in the library in the order of their first use here. With the four kernels of whole logits ahead of the four of shares the same instructions cost a
+// pass that takes shares more: 2048 tokens of 512 x 1024, 2 of 8 experts, replayed, 47.7 us, as here 46.9. With all four of shares first 22 tokens of 256 experts take 0.3 more.)
+static int launch_route(const RouteParams& p, bool shares, hipStream_t s) {
   const size_t shared = p.expert_groups > 1 ? sizeof(float) * kRouteWaves * p.experts : 0;
   const dim3 grid((p.tokens + kRouteWaves - 1) / kRouteWaves), block(kWave * kRouteWaves);
-  if (p.experts <= 64) {
-    hipLaunchKernelGGL((route_kernel<1, SHARES>), grid, block, shared, s, p);
-  } else if (p.experts <= 128) {
-    hipLaunchKernelGGL((route_kernel<2, SHARES>), grid, block, shared, s, p);
-  } else if (p.experts <= 256) {
-    hipLaunchKernelGGL((route_kernel<4, SHARES>), grid, block, shared, s, p);
-  } else {
-    hipLaunchKernelGGL((route_kernel<kMaxPerLane, SHARES>), grid, block, shared, s, p);
-  }
+  auto kernel = p.experts <= 64    ? (shares ? route_kernel<1, true> : route_kernel<1, false>)
+                : p.experts <= 128 ? (shares ? route_kernel<2, true> : route_kernel<2, false>)
+                : p.experts <= 256 ? (shares ? route_kernel<4, true> : route_kernel<4, false>)
+                                   : (shares ? route_kernel<kMaxPerLane, true> : route_kernel<kMaxPerLane, false>);
+  hipLaunchKernelGGL(kernel, grid, block, shared, s, p);
   return launched("route_kernel");
 }
 
@@ -578,7 +575,7 @@ int dew::route_launch(const dew_moe_router* router, const float* logits, const f
   DEW_REQUIRE(tokens == 0 || (logits && weights && indices), "dew_moe_route: logits, weights and indices must not be null");
   if (tokens == 0) return DEW_MOE_OK;
   const RouteParams p = route_params(router, logits, bias, media_bias, media, given, covered, by_block, tokens, weights, indices, scores, log_z);
-  return launch_route<false>(p, static_cast<hipStream_t>(stream));
+  return launch_route(p, false, static_cast<hipStream_t>(stream));
 }
 
 int dew::route_shares(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
@@ -587,7 +584,7 @@ int dew::route_shares(const dew_moe_router* router, const float* partial, const 
   RouteParams p = route_params(router, partial, selection_bias, nullptr, nullptr, nullptr, nullptr, BlockRouting{}, tokens, weights, indices, nullptr,
                                nullptr);
   p.gate_bias = gate_bias;
-  return launch_route<true>(p, stream);
+  return launch_route(p, true, stream);
 }
 
 int dew::route_and_sort(const dew_moe_router* router, const float* partial, const float* gate_bias, const float* selection_bias, int tokens,
